@@ -128,6 +128,7 @@ struct hg_mesh {
                                    {kMixedHeatTolerance, kMixedPoissonTolerance}};
   // Workspaces.
   CgWorkspace cg;
+  SpatialOrder cg_order;  // the iterated solves' row order, built on the first that wants it
   MarchWorkspace march;  // the band march of a system refused under the budget
   // The Poisson system's multigrid hierarchy, built on its first solve past the budget.
   std::unique_ptr<Multigrid> poisson_mg;
@@ -232,7 +233,7 @@ int64_t mesh_device_bytes(const hg_mesh& m) {
   total += m.heat_factor.bytes() + m.poisson_factor.bytes() + m.pinned_factor.bytes() +
            m.reg_factor.bytes();
   if (m.plan) total += m.plan->bytes();
-  total += m.cg.bytes() + m.solve.bytes() + m.solve_side.bytes() + m.null_space.bytes();
+  total += m.cg.bytes() + m.cg_order.bytes() + m.solve.bytes() + m.solve_side.bytes() + m.null_space.bytes();
   return total;
 }
 
@@ -619,6 +620,14 @@ HeatSystem heat_system(hg_mesh& m, bool pinned) {
   return {m.heat.ptr, m.heat32.ptr, m.heat_inv.ptr, &m.heat_factor, HG_SYSTEM_HEAT};
 }
 
+// The rows' spatial order for an iterated solve that makes use of one.
+void order_rows(hg_mesh& m, CgProblem& p) {
+  if (!wants_spatial_order(p.n, p.n_columns)) return;
+  if (!m.cg_order.order.ptr) spatial_order(m.xyz.ptr, m.n, m.cg_order, m.cg, m.stream);
+  p.order = m.cg_order.order.ptr;
+  p.inverse = m.cg_order.inverse.ptr;
+}
+
 int32_t diffuse_iterated(hg_mesh& m, const HeatSystem& sys, const double* rhs, double* x,
                          int64_t k) {
   PhaseScope scope(&m.timer, kPhaseCg, m.stream);
@@ -639,6 +648,7 @@ int32_t diffuse_iterated(hg_mesh& m, const HeatSystem& sys, const double* rhs, d
     p.check_rounds = m.check_rounds;
     p.change_tolerance = m.change_tolerance;
     p.settle_rounds = m.settle_window > 0 ? m.settle_window : m.settle_rounds;
+    order_rows(m, p);
     total = std::max(total, run_cg(p, m.cg, m.stream));
   }
   return total;
@@ -835,6 +845,7 @@ void solve_poisson(hg_mesh& m, double* rhs, double* x, int64_t k, int32_t mode,
         p.chebyshev_steps = kChebyshevSteps;
         p.lambda_min = lo;
         p.lambda_max = hi;
+        order_rows(m, p);
         rounds = std::max(rounds, run_cg(p, m.cg, m.stream));
       }
       m.stats.poisson_rounds = rounds;

@@ -10,6 +10,8 @@
 // with grid-wide barriers, so nothing returns to the host until the solve ends. Every block folds
 // the per-block partials in the same fixed order, so all blocks agree on alpha, beta and the stop
 // decision bit for bit (the redundant fold ordito uses instead of a barrier, here beside one).
+#include <hipcub/hipcub.hpp>
+
 #include "kernels.h"
 
 namespace hg {
@@ -37,6 +39,11 @@ struct CgArgs {
   double* res;
   double* da;
   double* db;
+  // cg_resident_kernel: the rows' spatial order and its inverse, and the exchanged words.
+  const int32_t* order;
+  const int32_t* inverse;
+  double* exchange;  // [kPhases][n]
+  double* slots;     // [kSlotPhases][G][kSlotWidth]
   double* partials;  // [k][G][3], then [G][2] for the settle check, then [k][G] for |b|^2
   // [0] stepped rounds, [1] set when a grid barrier gave up waiting, [2] barrier groups arrived
   // at the current barrier, [3] barrier generation, [4, 12) each group's blocks arrived; [1..12)
@@ -404,162 +411,393 @@ __global__ __launch_bounds__(kThreads) void cg_kernel(CgArgs a) {
   if (blockIdx.x == 0 && threadIdx.x == 0) a.counters[0] = stepped_rounds;
 }
 
-// One column of at most kRows * 1024 rows in one workgroup, the iteration of cg_kernel with its
-// state where one compute unit reaches it fastest: each thread's rows (tid + 1024 j, j < kRows)
-// keep x, r, u, p, s, prev and the Chebyshev residual in registers, and the vectors the products
-// read from every row (u, and the Chebyshev directions) live in LDS, so a product is one round
-// trip for the operator's entries (issued a row at a time, four or eight together) and LDS
-// gathers.
-// Same recurrences, stop rules, sums in fixed order (a thread's rows in order, then block_sum).
-constexpr int kSmallThreads = 1024;
-constexpr int kSmallRows = 3;  // rows a thread: systems of at most 3,072 rows
+// ---- one column, its whole state on the chip ---------------------------------------------------
+//
+// cg_kernel keeps the iteration's vectors in memory, and its grid barrier makes them visible to
+// the other XCDs by writing back and invalidating the L2s, so every round re-reads its vectors and
+// the operator from beyond the L2: 20-35 us a product on systems of 41-164 thousand rows whose
+// data would fit the compute units several times over. Here a thread owns R rows and keeps their
+// operator entries (E a row; longer rows read the rest through the L2) and their vectors in
+// registers and LDS for the whole solve. Only two things leave a block:
+//   - the values the products gather (u, or a Chebyshev direction) of rows that have a neighbour
+//     in another block, written through to `exchange` where that neighbour's thread waits for them;
+//   - a block's three partial sums, written through to `slots`, where every block waits for all.
+// Both are agent-scope relaxed stores and loads, which pass the L2s by on their own, so nothing is
+// written back or invalidated, and the read-only operator stays cached. A value is its own arrival
+// flag: every word holds kEmpty until it is published, so a reader polls the very word it needs
+// and one store-to-load latency replaces a barrier's several.
+//
+// Blocks own consecutive rows of a spatial order of the vertices (spatial_order), so nearly all
+// of a row's neighbours are its block's and read from LDS. A published word is emptied again two
+// phases later by its owner: product k reads phase k's words; having read its neighbours' phase
+// k - 1, a row's thread knows that they have read phase k - 2 (they publish k - 1 after it, and
+// the pattern is symmetric), so in phase k it empties its word of phase k - 2, waits for that store
+// before it publishes phase k + 1, and nobody polls phase k + 2 in that word before reading that.
+// So four buffers of n words serve. The sums' slots rotate over three in the same way: a block
+// publishes sum q - 1 once all its threads have read sum q - 2.
+//
+// Sums keep a fixed order (a thread's rows, then butterflies over lanes, waves and blocks), so a
+// solve repeats bit for bit. Every wait is bounded as the grid barrier's are.
+constexpr uint64_t kEmpty = 0x7FF4A5A5C3C3F00Dull;       // a signaling NaN no arithmetic returns
+constexpr uint64_t kQuietNan = 0x7FF8000000000000ull;
+constexpr int kPhases = 4, kSlotPhases = 3, kSlotWidth = 4;
 
-// The products of a thread's rows, kBatch entries of every row a step: each step's columns and
-// values of all the rows are loaded together (one round trip for the rows, where a row at a time
-// waited once per row), then gathered from LDS and summed, each row in entry order. kWide: the
-// operator's float64 values only (the Chebyshev instance's: the Poisson systems have no narrowed
-// copy), else the narrowed values when there are.
-template <int kRows, bool kWide>
-__device__ __forceinline__ void small_row_products(const CgArgs& a, const int32_t (&begin)[kRows],
-                                                   const int32_t (&end)[kRows],
-                                                   const double* __restrict__ vec,
-                                                   double (&out)[kRows]) {
-  constexpr int kBatch = kRows == 1 ? 8 : (kRows == 2 ? 4 : (kWide ? 2 : 3));  // no spills
-  int32_t longest = 0;
-#pragma unroll
-  for (int j = 0; j < kRows; ++j) {
-    out[j] = 0.0;
-    longest = max(longest, end[j] - begin[j]);
-  }
-  for (int32_t base = 0; base < longest; base += kBatch) {
-    int32_t col[kRows][kBatch];
-    double val[kRows][kBatch];
-#pragma unroll
-    for (int j = 0; j < kRows; ++j)
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        const bool has = begin[j] + base + u < end[j];
-        const int32_t e = has ? begin[j] + base + u : 0;
-        col[j][u] = has ? a.columns[e] : 0;
-        val[j][u] = !has ? 0.0
-                    : kWide || !a.values32 ? a.values64[e]
-                                           : static_cast<double>(a.values32[e]);
-      }
-#pragma unroll
-    for (int j = 0; j < kRows; ++j)
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u)
-        if (begin[j] + base + u < end[j]) out[j] += val[j][u] * vec[col[j][u]];
-  }
+__device__ __forceinline__ void publish(double* word, double v) {
+  uint64_t bits = __builtin_bit_cast(uint64_t, v);
+  if (bits == kEmpty) bits = kQuietNan;
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(word), bits, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int kRows, bool kCheb>
-__global__ __launch_bounds__(kSmallThreads) void cg_small_kernel(CgArgs a) {
-  constexpr int kWaves = kSmallThreads / 64;
-  constexpr int kN = kRows * kSmallThreads;
-  __shared__ double u_lds[kN];
-  __shared__ double d_lds[2][kN];
-  __shared__ double scratch[3 * kWaves];
+__device__ __forceinline__ void empty(double* word) {
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(word), kEmpty, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ uint64_t peek(const double* word) {
+  return __hip_atomic_load(reinterpret_cast<const uint64_t*>(word), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// This wave's stores have reached the point of coherence.
+__device__ __forceinline__ void drain_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// A wait's patience: false once it has polled past the limit or another wait has given up, which
+// it then tells everyone.
+__device__ __forceinline__ bool wait_on(const CgArgs& a, int32_t& polls, bool& aborted) {
+  if (aborted) return false;
+  if ((++polls & 255) == 0) {
+    int32_t* flag = a.counters + 1;
+    if (polls > a.spin_limit ||
+        __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+      __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      aborted = true;
+      return false;
+    }
+  }
+  return true;
+}
+
+// A thread's value of a vector for each of its rows, in registers or in LDS (l = the thread's
+// first entry, entries kStride apart).
+template <int R, int kStride, bool kLds>
+struct RowVector {
+  double reg[kLds ? 1 : R];
+  double* lds;
+  __device__ __forceinline__ double get(int j) const {
+    if constexpr (kLds) return lds[kStride * j];
+    else return reg[j];
+  }
+  __device__ __forceinline__ void set(int j, double v) {
+    if constexpr (kLds) lds[kStride * j] = v;
+    else reg[j] = v;
+  }
+};
+
+// T threads a block, R rows a thread, E operator entries of a row in registers, TV the operator's
+// values (float: the narrowed heat operator), kCheb the polynomial preconditioner, kGrid more than
+// one block. Instances with double values keep x, p, s and r in LDS: they are touched once a round,
+// and the registers are the operator's.
+template <int T, int R, int E, typename TV, bool kCheb, bool kGrid>
+__global__ __launch_bounds__(T) void cg_resident_kernel(CgArgs a) {
+  constexpr int L = R * T, kWaves = T / 64;
+  static_assert((kWaves & (kWaves - 1)) == 0, "the waves' sums fold in a butterfly");
+  constexpr bool kLds = sizeof(TV) == 8;
+  // The values the products gather, two phases; entry L stays zero (the padding of a short row).
+  __shared__ double vec[2][L + 1];
+  __shared__ double state[kLds ? 4 * L : 1];
+  __shared__ double scratch[2][3 * kWaves];
+  const int t = threadIdx.x, wave = t / 64, lane = t % 64;
   const int32_t n = static_cast<int32_t>(a.n);
-  const int t = threadIdx.x;
-  bool live[kRows];
-  int32_t begin[kRows], end[kRows];
-  // The Chebyshev residual and direction (the Poisson step) or the settle check's last iterate
-  // (the heat step): an instance holds one or the other.
-  constexpr int kCheck = kCheb ? 1 : kRows, kPoly = kCheb ? kRows : 1;
-  double x[kRows], r[kRows], u[kRows], p[kRows], sv[kRows], dinv[kRows];
-  double prev[kCheck], res[kPoly], dcur[kPoly];
-  double bb[1] = {0.0};
+  const int32_t G = static_cast<int32_t>(gridDim.x);
+  const int32_t block = kGrid ? xcd_block() : 0;
+  const int32_t per_block = kGrid ? (n + G - 1) / G : n;
+  const int32_t base = block * per_block;
+  const int32_t count = max(0, min(per_block, n - base));  // this block's rows
+  const TV* values = sizeof(TV) == 4 ? reinterpret_cast<const TV*>(a.values32)
+                                     : reinterpret_cast<const TV*>(a.values64);
+  bool aborted = false;
+  if (t < 2) vec[t][L] = 0.0;
+
+  // The thread's rows: local index t + T j, row base + t + T j of the order. An operator column is
+  // held as the byte offset of its value: >= 0 in a phase's LDS vector, < 0 (complemented) in a
+  // phase's exchange, for a row of another block.
+  int32_t old_row[R], begin[R], extra[R];  // extra: entries past E
+  int32_t col[R][E];
+  TV val[R][E];
 #pragma unroll
-  for (int j = 0; j < kRows; ++j) {
-    const int32_t i = t + kSmallThreads * j;
-    live[j] = i < n;
-    begin[j] = live[j] ? a.offsets[i] : 0;
-    end[j] = live[j] ? a.offsets[i + 1] : 0;
-    dinv[j] = live[j] ? a.inv_diag[i] : 0.0;
-    x[j] = live[j] && a.guess ? a.guess[i] : 0.0;
-    u_lds[i] = x[j];
-  }
-  __syncthreads();
-  // r = b - A x0 (x0 the guess, else zero).
-  double ax[kRows] = {};
-  if (a.guess) small_row_products<kRows, kCheb>(a, begin, end, u_lds, ax);
+  for (int j = 0; j < R; ++j)
 #pragma unroll
-  for (int j = 0; j < kRows; ++j) {
-    const int32_t i = t + kSmallThreads * j;
-    const double b = live[j] ? a.rhs[i] : 0.0;
-    r[j] = live[j] && a.guess ? b - ax[j] : b;
-    if (live[j]) a.x[i] = x[j];
-    p[j] = 0.0;
-    sv[j] = 0.0;
-    if constexpr (!kCheb) prev[j] = 0.0;
-    u[j] = dinv[j] * r[j];
-    bb[0] += b * b;
+    for (int e = 0; e < E; ++e) {
+      col[j][e] = 8 * L;
+      val[j][e] = TV(0);
+    }
+  double dinv[R];
+  uint32_t live = 0, outer = 0;  // row j exists; row j has a neighbour in another block
+  auto locate = [&](int32_t c) {
+    if constexpr (!kGrid) return 8 * c;
+    const int32_t at = a.inverse[c] - base;
+    return at >= 0 && at < count ? 8 * at : ~(8 * (at + base));
+  };
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int32_t l = t + T * j;
+    const bool has = l < count;
+    if (has) live |= 1u << j;
+    old_row[j] = has ? (kGrid ? a.order[base + l] : l) : 0;
+    begin[j] = has ? a.offsets[old_row[j]] : 0;
+    const int32_t degree = has ? a.offsets[old_row[j] + 1] - begin[j] : 0;
+    extra[j] = max(0, degree - E);
+    dinv[j] = has ? a.inv_diag[old_row[j]] : 0.0;
+    // Entries past the row's end load one that exists, so the loads need no branches.
+    const int32_t last = a.offsets[n] - 1;
+    if (last < 0) continue;
+    int32_t c[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) c[e] = a.columns[min(begin[j] + e, last)];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const bool stored = e < degree;
+      const TV v = values[min(begin[j] + e, last)];
+      const int32_t at = locate(c[e]);
+      col[j][e] = stored ? at : 8 * L;
+      val[j][e] = stored ? v : TV(0);
+      if (kGrid && stored && at < 0) outer |= 1u << j;
+    }
+    if (kGrid)
+#pragma unroll 1
+      for (int32_t e = E; e < degree; ++e)
+        if (locate(a.columns[begin[j] + e]) < 0) outer |= 1u << j;
   }
-  block_sum<kSmallThreads, 1>(bb, scratch);
-  const double atol_sq = a.tol_sq * bb[0];
-  double gamma_old = INFINITY, alpha_old = 1.0;
-  const double sigma = a.cheb_steps > 0 ? a.theta / a.delta : 0.0;
-  // u = p(D^-1 A) D^-1 r for the Poisson step's rounds (chebyshev_apply's recurrence).
+
+  // Phase k of the exchange: this thread's rows' values, into LDS and, for rows with a neighbour
+  // elsewhere, into the exchange.
+  int32_t phase = -1;
+  auto phase_words = [&](int32_t k) { return a.exchange + static_cast<int64_t>(k % kPhases) * n; };
+  auto offer = [&](int j, double v) {
+    vec[phase & 1][t + T * j] = v;
+    if (kGrid && (outer >> j & 1)) publish(phase_words(phase) + base + t + T * j, v);
+  };
+  // Before a phase's offers: the words emptied in the last product have landed.
+  auto next_phase = [&]() {
+    ++phase;
+    if (kGrid) drain_stores();
+  };
+  // out = A v over this thread's rows, v the current phase's values, each row in its entry order.
+  auto product = [&](double (&out)[R]) {
+    const char* local = reinterpret_cast<const char*>(vec[phase & 1]);
+    const char* remote = nullptr;
+    auto at_local = [&](int32_t c) {
+      return *reinterpret_cast<const uint64_t*>(local + static_cast<uint32_t>(c));
+    };
+    auto at_remote = [&](int32_t c) {
+      return peek(reinterpret_cast<const double*>(remote + static_cast<uint32_t>(~c)));
+    };
+    if (kGrid) {
+      remote = reinterpret_cast<const char*>(phase_words(phase));
+      double* spent = phase_words(phase + 2) + base + t;
+#pragma unroll
+      for (int j = 0; j < R; ++j)
+        if (outer >> j & 1) empty(spent + T * j);
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      uint64_t raw[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) raw[e] = at_local(kGrid ? max(col[j][e], 0) : col[j][e]);
+      if (kGrid && (outer >> j & 1)) {
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+          if (col[j][e] < 0) raw[e] = at_remote(col[j][e]);
+        int32_t polls = 0;
+        for (;;) {
+          bool waiting = false;
+#pragma unroll
+          for (int e = 0; e < E; ++e)
+            if (raw[e] == kEmpty) {  // only a remote word can read so
+              raw[e] = at_remote(col[j][e]);
+              waiting = true;
+            }
+          if (!waiting || !wait_on(a, polls, aborted)) break;
+        }
+      }
+      double sum = 0.0;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        // Widened here each time: the widened values of a whole row would not fit the registers.
+        if constexpr (sizeof(TV) == 4) asm volatile("" : "+v"(val[j][e]));
+        sum += static_cast<double>(val[j][e]) * __builtin_bit_cast(double, raw[e]);
+      }
+#pragma unroll 1
+      for (int32_t e = 0; e < extra[j]; ++e) {  // the rest of a long row
+        const int32_t c = locate(a.columns[begin[j] + E + e]);
+        uint64_t bits;
+        if (kGrid && c < 0) {
+          int32_t polls = 0;
+          while ((bits = at_remote(c)) == kEmpty && wait_on(a, polls, aborted)) {
+          }
+        } else {
+          bits = at_local(c);
+        }
+        sum += static_cast<double>(values[begin[j] + E + e]) * __builtin_bit_cast(double, bits);
+      }
+      out[j] = sum;
+    }
+  };
+
+  // The sums of v[0..2] over every thread of every block, v[0]'s maximum instead when kMax, left in
+  // v on every thread. Scratch alternates between calls, so one block barrier a fold suffices.
+  int32_t folds = 0, sums = 0;
+  auto fold_block = [&](double (&v)[3], bool max_first) {
+    double* mine = scratch[folds++ & 1];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int offset = 32; offset > 0; offset >>= 1) {
+        const double other = __shfl_xor(v[c], offset, 64);
+        v[c] = c == 0 && max_first ? fmax(v[c], other) : v[c] + other;
+      }
+    if (lane == 0)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) mine[c * kWaves + wave] = v[c];
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      v[c] = mine[c * kWaves + lane % kWaves];
+#pragma unroll
+      for (int offset = kWaves / 2; offset > 0; offset >>= 1) {
+        const double other = __shfl_xor(v[c], offset, kWaves);
+        v[c] = c == 0 && max_first ? fmax(v[c], other) : v[c] + other;
+      }
+    }
+  };
+  auto fold = [&](double (&v)[3], bool max_first = false) {
+    if (!kGrid) {
+      fold_block(v, max_first);
+      return;
+    }
+    const int32_t q = sums++;
+    double* slots = a.slots + static_cast<int64_t>(q % kSlotPhases) * G * kSlotWidth;
+    double* spent = a.slots + static_cast<int64_t>((q + 1) % kSlotPhases) * G * kSlotWidth;
+    if (t < 3) empty(spent + block * kSlotWidth + t);
+    fold_block(v, max_first);
+    if (t < 3) {
+      drain_stores();
+      publish(slots + block * kSlotWidth + t, t == 0 ? v[0] : t == 1 ? v[1] : v[2]);
+    }
+    uint64_t got[3] = {0, 0, 0};  // +0.0: the identity of these sums and of a maximum of magnitudes
+    if (t < G) {
+      const double* theirs = slots + t * kSlotWidth;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) got[c] = peek(theirs + c);
+      int32_t polls = 0;
+      while (got[0] == kEmpty || got[1] == kEmpty || got[2] == kEmpty) {
+        if (!wait_on(a, polls, aborted)) break;
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+          if (got[c] == kEmpty) got[c] = peek(theirs + c);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) v[c] = __builtin_bit_cast(double, got[c]);
+    fold_block(v, max_first);
+  };
+
+  RowVector<R, T, kLds> x, r, p, s;
+  x.lds = state + t;
+  r.lds = state + (kLds ? L : 0) + t;
+  p.lds = state + (kLds ? 2 * L : 0) + t;
+  s.lds = state + (kLds ? 3 * L : 0) + t;
+  double u[R];
+  // r = b - A x0 (x0 the guess, else zero); the guess is read where the caller holds it.
+  double norm[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const bool has = live >> j & 1;
+    const double b = has ? a.rhs[old_row[j]] : 0.0;
+    double ri = b, xi = 0.0;
+    if (a.guess && has) {
+      double ax = 0.0;
+      xi = a.guess[old_row[j]];
+#pragma unroll 1
+      for (int32_t e = begin[j]; e < a.offsets[old_row[j] + 1]; ++e)
+        ax += static_cast<double>(values[e]) * a.guess[a.columns[e]];
+      ri = b - ax;
+    }
+    x.set(j, xi);
+    r.set(j, ri);
+    p.set(j, 0.0);
+    s.set(j, 0.0);
+    u[j] = dinv[j] * ri;
+    norm[0] += b * b;
+  }
+  fold(norm);
+  const double atol_sq = a.tol_sq * norm[0];
+
+  // u = p(D^-1 A) D^-1 r (chebyshev_apply's recurrence).
+  const double sigma = kCheb ? a.theta / a.delta : 0.0;
   auto chebyshev = [&]() {
     if constexpr (kCheb) {
       double rho = 1.0 / sigma;
+      double res[R], d[R];
+      next_phase();
 #pragma unroll
-      for (int j = 0; j < kRows; ++j) {
-        const int32_t i = t + kSmallThreads * j;
-        const double c = dinv[j] * r[j];
-        const double d = c / a.theta;
-        res[j] = c;
-        dcur[j] = d;
-        u[j] = d;
-        if (live[j]) d_lds[0][i] = d;
+      for (int j = 0; j < R; ++j) {
+        res[j] = dinv[j] * r.get(j);
+        d[j] = res[j] / a.theta;
+        u[j] = d[j];
+        offer(j, d[j]);
       }
       __syncthreads();
-      int cur = 0;
       for (int32_t step = 1; step < a.cheb_steps; ++step) {
         const double rho_new = 1.0 / (2.0 * sigma - rho);
         const double keep = rho_new * rho;
         const double push = 2.0 * rho_new / a.delta;
-        double ad[kRows];
-        small_row_products<kRows, kCheb>(a, begin, end, d_lds[cur], ad);
+        double ad[R];
+        product(ad);
+        const bool more = step + 1 < a.cheb_steps;
+        if (more) next_phase();
 #pragma unroll
-        for (int j = 0; j < kRows; ++j) {
-          const int32_t i = t + kSmallThreads * j;
-          if (!live[j]) continue;
+        for (int j = 0; j < R; ++j) {
           res[j] = res[j] - dinv[j] * ad[j];
-          const double d = keep * dcur[j] + push * res[j];
-          dcur[j] = d;
-          u[j] += d;
-          d_lds[cur ^ 1][i] = d;
+          d[j] = keep * d[j] + push * res[j];
+          u[j] += d[j];
+          if (more) offer(j, d[j]);
         }
         rho = rho_new;
-        cur ^= 1;
-        __syncthreads();
+        if (more) __syncthreads();
       }
     }
   };
-  if (kCheb) chebyshev();
-#pragma unroll
-  for (int j = 0; j < kRows; ++j)
-    if (live[j]) u_lds[t + kSmallThreads * j] = u[j];
-  __syncthreads();
 
+  double prev[kCheb ? 1 : R];
+  if constexpr (!kCheb)
+#pragma unroll
+    for (int j = 0; j < R; ++j) prev[j] = 0.0;
+  double gamma_old = INFINITY, alpha_old = 1.0;
   int32_t stepped_rounds = 0;
   int64_t round = 0;
   double settle_previous = 0.0, reach_check = 0.0, checks = 0.0;
   bool running = true;
+  if (kCheb) chebyshev();
   while (running) {
     ++round;
-    double w[kRows];
-    double acc[3] = {0.0, 0.0, 0.0};
-    small_row_products<kRows, kCheb>(a, begin, end, u_lds, w);
+    // w = A u and the round's three dots.
+    next_phase();
 #pragma unroll
-    for (int j = 0; j < kRows; ++j) {
-      acc[0] += r[j] * u[j];
+    for (int j = 0; j < R; ++j) offer(j, u[j]);
+    if (__syncthreads_or(aborted ? 1 : 0)) break;
+    double w[R];
+    double acc[3] = {0.0, 0.0, 0.0};
+    product(w);
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const double rj = r.get(j);
+      acc[0] += rj * u[j];
       acc[1] += w[j] * u[j];
-      acc[2] += r[j] * r[j];
+      acc[2] += rj * rj;
     }
-    block_sum<kSmallThreads, 3>(acc, scratch);
+    fold(acc);
     double alpha = 0.0, beta = 0.0;
     bool step = false;
     if (acc[2] > atol_sq && round <= a.maxiter && acc[0] != 0.0) {
@@ -575,49 +813,130 @@ __global__ __launch_bounds__(kSmallThreads) void cg_small_kernel(CgArgs a) {
     alpha_old = alpha;
     ++stepped_rounds;
 #pragma unroll
-    for (int j = 0; j < kRows; ++j) {
-      p[j] = u[j] + beta * p[j];
-      sv[j] = w[j] + beta * sv[j];
-      x[j] += alpha * p[j];
-      r[j] = r[j] - alpha * sv[j];
-      if (!kCheb) u[j] = dinv[j] * r[j];
+    for (int j = 0; j < R; ++j) {
+      const double pj = u[j] + beta * p.get(j);
+      const double sj = w[j] + beta * s.get(j);
+      p.set(j, pj);
+      s.set(j, sj);
+      x.set(j, x.get(j) + alpha * pj);
+      const double rj = r.get(j) - alpha * sj;
+      r.set(j, rj);
+      if (!kCheb) u[j] = dinv[j] * rj;
     }
     if (round >= a.maxiter) running = false;
     if (kCheb) chebyshev();
-    if (!kCheb && a.settle && round % a.check_rounds == 0) {
-      double change = 0.0;
-      double reached[1] = {0.0};
+    if constexpr (!kCheb) {
+      if (a.settle && round % a.check_rounds == 0) {
+        double verdict[3] = {0.0, 0.0, 0.0};  // the largest relative change, entries reached
 #pragma unroll
-      for (int j = 0; j < kCheck; ++j) {
-        if (live[j] && x[j] != 0.0) {
-          change = fmax(change, fabs(x[j] - prev[j]) / fabs(x[j]));
-          reached[0] += 1.0;
+        for (int j = 0; j < R; ++j) {
+          const double xj = x.get(j);
+          if ((live >> j & 1) && xj != 0.0) {
+            verdict[0] = fmax(verdict[0], fabs(xj - prev[j]) / fabs(xj));
+            verdict[1] += 1.0;
+          }
+          prev[j] = xj;
         }
-        prev[j] = x[j];
-      }
-      const double c = block_max<kSmallThreads>(change, scratch);
-      block_sum<kSmallThreads, 1>(reached, scratch);
-      checks += 1.0;
-      const double total = reached[0] + 1.0;
-      if (total != settle_previous) {
-        settle_previous = total;
-        reach_check = checks;
-      } else {
-        const double idle = (checks - reach_check) * static_cast<double>(a.check_rounds);
-        if (c < a.change_tolerance || idle >= static_cast<double>(a.settle_rounds)) running = false;
+        fold(verdict, true);
+        checks += 1.0;
+        const double total = verdict[1] + 1.0;
+        if (total != settle_previous) {
+          settle_previous = total;
+          reach_check = checks;
+        } else {
+          const double idle = (checks - reach_check) * static_cast<double>(a.check_rounds);
+          if (verdict[0] < a.change_tolerance || idle >= static_cast<double>(a.settle_rounds))
+            running = false;
+        }
       }
     }
-    // The next round's product reads u from LDS: every thread is past this round's (block_sum's
-    // barriers), so the rows are rewritten, then published.
-#pragma unroll
-    for (int j = 0; j < kRows; ++j)
-      if (live[j]) u_lds[t + kSmallThreads * j] = u[j];
-    __syncthreads();
   }
 #pragma unroll
-  for (int j = 0; j < kRows; ++j)
-    if (live[j]) a.x[t + kSmallThreads * j] = x[j];
-  if (t == 0) a.counters[0] = stepped_rounds;
+  for (int j = 0; j < R; ++j)
+    if (live >> j & 1) a.x[old_row[j]] = x.get(j);
+  if (block == 0 && t == 0) a.counters[0] = stepped_rounds;
+}
+
+// ---- a spatial order of the vertices -----------------------------------------------------------
+
+// Order-preserving integers of floats, for atomic minima and maxima.
+__device__ __forceinline__ uint32_t ordered_bits(float v) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, v);
+  return b & 0x80000000u ? ~b : b | 0x80000000u;
+}
+
+__device__ __forceinline__ float from_ordered_bits(uint32_t b) {
+  return __builtin_bit_cast(float, b & 0x80000000u ? b & 0x7FFFFFFFu : ~b);
+}
+
+// The finite coordinates' bounds into bounds[0..3) (minima, held complemented) and [3..6)
+// (maxima), all zero at launch.
+__global__ __launch_bounds__(kBlock) void bounds_kernel(const float* __restrict__ xyz, int64_t n,
+                                                        uint32_t* __restrict__ bounds) {
+  uint32_t best[6] = {0, 0, 0, 0, 0, 0};
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * kBlock)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const float v = xyz[3 * i + d];
+      if (!(fabsf(v) < INFINITY)) continue;
+      const uint32_t b = ordered_bits(v);
+      best[d] = max(best[d], ~b);
+      best[3 + d] = max(best[3 + d], b);
+    }
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+#pragma unroll
+    for (int offset = 32; offset > 0; offset >>= 1)
+      best[c] = max(best[c], static_cast<uint32_t>(__shfl_xor(static_cast<int>(best[c]), offset, 64)));
+    if (threadIdx.x % 64 == 0) atomicMax(bounds + c, best[c]);
+  }
+}
+
+__device__ __forceinline__ uint32_t spread3(uint32_t v) {  // ten bits, two zeros after each
+  v = (v | v << 16) & 0x030000FFu;
+  v = (v | v << 8) & 0x0300F00Fu;
+  v = (v | v << 4) & 0x030C30C3u;
+  return (v | v << 2) & 0x09249249u;
+}
+
+// Each vertex's Morton code over the bounds' cube, ten bits an axis (a non-finite coordinate in the
+// first cell), and its index.
+__global__ __launch_bounds__(kBlock) void morton_kernel(const float* __restrict__ xyz, int64_t n,
+                                                        const uint32_t* __restrict__ bounds,
+                                                        uint32_t* __restrict__ keys,
+                                                        int32_t* __restrict__ ids) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  if (i >= n) return;
+  float extent = 0.0f, low[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    low[d] = from_ordered_bits(~bounds[d]);
+    extent = fmaxf(extent, from_ordered_bits(bounds[3 + d]) - low[d]);
+  }
+  const float scale = extent > 0.0f ? 1024.0f / extent : 0.0f;
+  uint32_t key = 0;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const float cell = (xyz[3 * i + d] - low[d]) * scale;
+    const uint32_t c = cell > 0.0f ? static_cast<uint32_t>(fminf(cell, 1023.0f)) : 0u;
+    key |= spread3(c) << d;
+  }
+  keys[i] = key;
+  ids[i] = static_cast<int32_t>(i);
+}
+
+__global__ __launch_bounds__(kBlock) void invert_kernel(const int32_t* __restrict__ order, int64_t n,
+                                                        int32_t* __restrict__ inverse) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  if (i < n) inverse[order[i]] = static_cast<int32_t>(i);
+}
+
+__global__ __launch_bounds__(kBlock) void fill_empty_kernel(uint64_t* __restrict__ words,
+                                                            int64_t count) {
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < count;
+       i += static_cast<int64_t>(gridDim.x) * kBlock)
+    words[i] = kEmpty;
 }
 
 // Componentwise backward error flag (kernels/linalg.py:1128-1230): "not within" so NaN flags.
@@ -695,23 +1014,115 @@ int32_t cooperative_grid(int64_t n) {
 // wait.
 constexpr int64_t kSpinLimit = int64_t{1} << 21;
 
+using CgKernel = void (*)(CgArgs);
+
+// The resident kernel for a one-column problem: its threads, rows a thread and function, by size.
+// Up to 1,024 rows one block, which exchanges nothing (and up to 3,072 where there is no spatial
+// order; with one, 2,562 rows took 1.04 ms for both solves of a one-shot call in one block, which
+// reads three rows' entries out of one compute unit's LDS, and 0.88 ms in eleven of 256 threads).
+// Up to 65,536 rows a row a thread in blocks of 256, as few blocks as hold them (icosphere(6),
+// 40,962 rows: 3.51 ms; blocks of 512, 3.56; of 1024, 4.73). Past that every compute unit gets a
+// block of 512 threads with two rows each (icosphere(7), 163,842 rows: 11.7 ms; as few blocks as
+// hold them 12.0, 1024 threads with one row 12.1, 256 with four 15.2), or four with seven entries
+// in registers (torus of 524,288 rows, the heat solve: 10.8 ms; nine entries spill, 13.4 ms; 1024
+// threads with two rows 13.6 and 18.8 ms).
+// Blocks of a resident solve at most: one a compute unit, and no more than a block has threads to
+// read the sums of.
+int64_t resident_units() {
+  int device = 0, cus = 0;
+  HG_HIP(hipGetDevice(&device));
+  HG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+  return std::min<int64_t>(cus, 256);
+}
+
+struct ResidentChoice {
+  CgKernel kernel = nullptr;
+  int32_t threads = 0, rows = 0;  // rows a block
+};
+
+template <int T, int R, int E, bool kGrid>
+ResidentChoice resident_choice(bool cheb, bool narrow) {
+  ResidentChoice c;
+  c.threads = T;
+  c.rows = T * R;
+  if (cheb) c.kernel = cg_resident_kernel<T, R, E, double, true, kGrid>;
+  else if (narrow) c.kernel = cg_resident_kernel<T, R, E, float, false, kGrid>;
+  else if constexpr (!kGrid) c.kernel = cg_resident_kernel<T, R, E, double, false, kGrid>;
+  return c;
+}
+
+ResidentChoice choose_resident(const CgProblem& p) {
+  const bool cheb = p.chebyshev_steps > 0, narrow = p.values32 != nullptr;
+  if (p.n_columns != 1 || (cheb && narrow)) return {};
+  if (p.n <= 1024) return resident_choice<1024, 1, 9, false>(cheb, narrow);
+  if (!p.order || !p.inverse) {
+    if (p.n <= 2048) return resident_choice<1024, 2, 9, false>(cheb, narrow);
+    if (p.n <= 3072) return resident_choice<1024, 3, 5, false>(cheb, narrow);
+    return {};
+  }
+  const int64_t units = resident_units();
+  if (p.n <= 256 * units) return resident_choice<256, 1, 9, true>(cheb, narrow);
+  if (p.n <= 1024 * units) return resident_choice<512, 2, 9, true>(cheb, narrow);
+  if (p.n <= 2048 * units) return resident_choice<512, 4, 7, true>(cheb, narrow);
+  return {};
+}
+
+// The exchange of a resident solve of n rows in at most 256 blocks, in doubles.
+int64_t exchange_words(int64_t n) { return kPhases * n + kSlotPhases * kSlotWidth * 256; }
+
+void reserve_exchange(CgWorkspace& ws, int64_t words) {
+  if (ws.exchange.size < words) ws.exchange.allocate(words);
+}
+
+int32_t launched_rounds(CgWorkspace& ws, hipStream_t stream) {
+  int32_t words[2] = {0, 0};
+  HG_HIP(hipMemcpyAsync(words, ws.counters.ptr, sizeof(words), hipMemcpyDeviceToHost, stream));
+  HG_HIP(hipStreamSynchronize(stream));
+  HG_REQUIRE(words[1] == 0, HG_ERR_RUNTIME,
+             "conjugate gradient: a grid barrier waited past its limit; the solve was abandoned");
+  return words[0];
+}
+
 }  // namespace
+
+bool wants_spatial_order(int64_t n, int64_t n_columns) {
+  return n_columns == 1 && n > 1024 && n <= 2048 * resident_units();
+}
+
+void spatial_order(const float* xyz, int64_t n, SpatialOrder& out, CgWorkspace& ws,
+                   hipStream_t stream) {
+  out.order.allocate(std::max<int64_t>(n, 1));
+  out.inverse.allocate(std::max<int64_t>(n, 1));
+  if (n == 0) return;
+  // Keys, sorted keys, indices, bounds and the sort's storage, in the exchange of the solve that
+  // follows.
+  size_t bytes = 0;
+  uint32_t* keys = nullptr;
+  int32_t* ids = nullptr;
+  HG_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, keys, keys, ids, out.order.ptr,
+                                            static_cast<int>(n), 0, 30, stream));
+  const int64_t head = (4 * (3 * n + 6) + 255) / 256 * 256;
+  reserve_exchange(ws, std::max(exchange_words(n), (head + static_cast<int64_t>(bytes) + 7) / 8));
+  keys = reinterpret_cast<uint32_t*>(ws.exchange.ptr);
+  ids = reinterpret_cast<int32_t*>(keys + 2 * n);
+  uint32_t* bounds = keys + 3 * n;
+  void* temp = reinterpret_cast<uint8_t*>(keys) + head;
+  const unsigned blocks = static_cast<unsigned>((n + kBlock - 1) / kBlock);
+  launch_zero(bounds, 6 * sizeof(uint32_t), stream);
+  bounds_kernel<<<std::min(blocks, 256u), kBlock, 0, stream>>>(xyz, n, bounds);
+  morton_kernel<<<blocks, kBlock, 0, stream>>>(xyz, n, bounds, keys, ids);
+  HG_HIP(hipGetLastError());
+  HG_HIP(hipcub::DeviceRadixSort::SortPairs(temp, bytes, keys, keys + n, ids, out.order.ptr,
+                                            static_cast<int>(n), 0, 30, stream));
+  invert_kernel<<<blocks, kBlock, 0, stream>>>(out.order.ptr, n, out.inverse.ptr);
+  HG_HIP(hipGetLastError());
+}
 
 int32_t run_cg(const CgProblem& problem, CgWorkspace& ws, hipStream_t stream) {
   const int64_t n = problem.n;
   const int64_t k = problem.n_columns;
   HG_REQUIRE(k >= 1 && k <= kMaxColumns, HG_ERR_VALUE, "conjugate gradient takes 1-64 columns");
   if (n == 0) return 0;
-  // Small systems run in one block of 1024 lanes with block barriers only.
-  const bool single = n <= 8192;
-  const int32_t G = single ? 1 : cooperative_grid(n);
-  const int64_t entries = n * k;
-  if (ws.capacity_entries < entries) {
-    ws.vectors.allocate(9 * entries);
-    ws.capacity_entries = entries;
-  }
-  const int64_t partial_size = k * G * 3 + 2 * G + k * G;
-  if (ws.partials.size < partial_size) ws.partials.allocate(partial_size);
   if (ws.counters.size < 4 + kBarrierGroups) ws.counters.allocate(4 + kBarrierGroups);
   CgArgs a{};
   a.n = n;
@@ -724,17 +1135,6 @@ int32_t run_cg(const CgProblem& problem, CgWorkspace& ws, hipStream_t stream) {
   a.rhs = problem.rhs;
   a.guess = problem.guess;
   a.x = problem.x;
-  double* base = ws.vectors.ptr;
-  a.r = base;
-  a.u = base + entries;
-  a.p = base + 2 * entries;
-  a.s = base + 3 * entries;
-  a.w = base + 4 * entries;
-  a.prev = base + 5 * entries;
-  a.res = base + 6 * entries;
-  a.da = base + 7 * entries;
-  a.db = base + 8 * entries;
-  a.partials = ws.partials.ptr;
   a.counters = ws.counters.ptr;
   a.spin_limit = kSpinLimit;
   a.settle = problem.settle;
@@ -748,30 +1148,60 @@ int32_t run_cg(const CgProblem& problem, CgWorkspace& ws, hipStream_t stream) {
   a.delta = 0.5 * (problem.lambda_max - problem.lambda_min);
   void* args[] = {&a};
   launch_zero(ws.counters.ptr, sizeof(int32_t) * (4 + kBarrierGroups), stream);
-  if (k == 1 && n <= static_cast<int64_t>(kSmallRows) * kSmallThreads) {
-    const int64_t rows = (n + kSmallThreads - 1) / kSmallThreads;
-    const bool cheb = a.cheb_steps > 0;
-    // The Chebyshev instance reads the float64 values only.
-    HG_REQUIRE(!cheb || a.values32 == nullptr, HG_ERR_RUNTIME,
-               "the Chebyshev-preconditioned solve takes float64 operator values");
-    auto kernel = rows == 1 ? (cheb ? cg_small_kernel<1, true> : cg_small_kernel<1, false>)
-                  : rows == 2 ? (cheb ? cg_small_kernel<2, true> : cg_small_kernel<2, false>)
-                              : (cheb ? cg_small_kernel<3, true> : cg_small_kernel<3, false>);
-    hipLaunchKernelGGL(kernel, dim3(1), dim3(kSmallThreads), 0, stream, a);
+  const ResidentChoice choice = choose_resident(problem);
+  if (choice.kernel) {
+    if (n <= choice.rows) {
+      hipLaunchKernelGGL(choice.kernel, dim3(1), dim3(choice.threads), 0, stream, a);
+      HG_HIP(hipGetLastError());
+      return launched_rounds(ws, stream);
+    }
+    const int64_t G = choice.rows > choice.threads ? resident_units()
+                                                   : (n + choice.rows - 1) / choice.rows;
+    const int64_t words = exchange_words(n);
+    reserve_exchange(ws, words);
+    a.order = problem.order;
+    a.inverse = problem.inverse;
+    a.exchange = ws.exchange.ptr;
+    a.slots = ws.exchange.ptr + kPhases * n;
+    fill_empty_kernel<<<static_cast<unsigned>(std::min<int64_t>((words + kBlock - 1) / kBlock, 2048)),
+                        kBlock, 0, stream>>>(reinterpret_cast<uint64_t*>(ws.exchange.ptr), words);
     HG_HIP(hipGetLastError());
-  } else if (single) {
+    // Cooperative: every block waits for words of the others, so all must be resident.
+    HG_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(choice.kernel),
+                                      dim3(static_cast<unsigned>(G)), dim3(choice.threads), args,
+                                      0, stream));
+    return launched_rounds(ws, stream);
+  }
+  // Several columns, systems past the compute units' registers, and systems with no spatial order:
+  // the state in memory. Small ones run in one block of 1024 lanes with block barriers only.
+  const bool single = n <= 8192;
+  const int32_t G = single ? 1 : cooperative_grid(n);
+  const int64_t entries = n * k;
+  if (ws.capacity_entries < entries) {
+    ws.vectors.allocate(9 * entries);
+    ws.capacity_entries = entries;
+  }
+  const int64_t partial_size = k * G * 3 + 2 * G + k * G;
+  if (ws.partials.size < partial_size) ws.partials.allocate(partial_size);
+  double* base = ws.vectors.ptr;
+  a.r = base;
+  a.u = base + entries;
+  a.p = base + 2 * entries;
+  a.s = base + 3 * entries;
+  a.w = base + 4 * entries;
+  a.prev = base + 5 * entries;
+  a.res = base + 6 * entries;
+  a.da = base + 7 * entries;
+  a.db = base + 8 * entries;
+  a.partials = ws.partials.ptr;
+  if (single) {
     hipLaunchKernelGGL((cg_kernel<1024, true>), dim3(1), dim3(1024), 0, stream, a);
     HG_HIP(hipGetLastError());
   } else {
     HG_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&cg_kernel<1024, false>),
                                       dim3(G), dim3(1024), args, 0, stream));
   }
-  int32_t words[2] = {0, 0};
-  HG_HIP(hipMemcpyAsync(words, ws.counters.ptr, sizeof(words), hipMemcpyDeviceToHost, stream));
-  HG_HIP(hipStreamSynchronize(stream));
-  HG_REQUIRE(words[1] == 0, HG_ERR_RUNTIME,
-             "conjugate gradient: a grid barrier waited past its limit; the solve was abandoned");
-  return words[0];
+  return launched_rounds(ws, stream);
 }
 
 void launch_backward_error(const int32_t* offsets, const int32_t* columns, const double* values,

@@ -187,6 +187,10 @@ struct CgProblem {
   const double* rhs = nullptr;
   const double* guess = nullptr;  // initial iterate (may alias x), or null for zero
   double* x = nullptr;
+  // The rows' spatial order (order[new] = row) and its inverse, or null. Only with a symmetric
+  // pattern.
+  const int32_t* order = nullptr;
+  const int32_t* inverse = nullptr;
   // Stop rule: settle (the heat step) or relative residual tol (the Poisson step).
   int32_t settle = 1;
   int32_t check_rounds = 16;
@@ -203,20 +207,33 @@ struct CgProblem {
 struct CgWorkspace {
   DeviceArray<double> vectors;   // r, u, p, s, w, prev, and two polynomial vectors
   DeviceArray<double> partials;
+  DeviceArray<double> exchange;  // the words the resident solve's blocks exchange
   DeviceArray<int32_t> counters;
   int64_t capacity_entries = 0;
   int32_t capacity_blocks = 0;
   int32_t capacity_columns = 0;
-  int64_t bytes() const { return vectors.bytes() + partials.bytes() + counters.bytes(); }
+  int64_t bytes() const { return vectors.bytes() + partials.bytes() + exchange.bytes() + counters.bytes(); }
   void release() {
     vectors.reset();
     partials.reset();
+    exchange.reset();
     counters.reset();
     capacity_entries = 0;
     capacity_blocks = 0;
     capacity_columns = 0;
   }
 };
+
+// A permutation of the vertices that keeps neighbours in space close (a Morton order), and its
+// inverse; `workspace` lends its exchange to the sort.
+struct SpatialOrder {
+  DeviceArray<int32_t> order, inverse;
+  int64_t bytes() const { return order.bytes() + inverse.bytes(); }
+};
+void spatial_order(const float* xyz, int64_t n, SpatialOrder& out, CgWorkspace& workspace,
+                   hipStream_t stream);
+// Whether run_cg makes use of one for a system of this size.
+bool wants_spatial_order(int64_t n, int64_t n_columns);
 
 // Runs the solve; returns the rounds that stepped.
 int32_t run_cg(const CgProblem& problem, CgWorkspace& workspace, hipStream_t stream);
