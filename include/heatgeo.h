@@ -194,6 +194,14 @@ int hg_set_memory_budget(hg_mesh* mesh, int64_t bytes);
 int hg_set_budget_probe(hg_mesh* mesh, int32_t probe);
 
 /*
+ * How often a one-launch sweep's waits poll before it gives up and its solve starts over level by
+ * level, as this mesh's solves then do from then on (default 2^21, about two seconds; 0 gives up at
+ * the first value not there yet). Setting it returns the mesh to one-launch sweeps. No counterpart
+ * in the reference.
+ */
+int hg_set_sweep_patience(hg_mesh* mesh, int64_t polls);
+
+/*
  * The settle rule of the heat solves' iteration (solve_spd_settled's check_rounds,
  * change_tolerance and settle_rounds, linalg.py:2490-2560): every check_rounds rounds the iterate
  * stops once each entry changed by less than change_tolerance of itself since the last check, or

@@ -973,7 +973,9 @@ std::vector<uintptr_t> graph_signature(const hg_mesh& m, int64_t k) {
   std::memcpy(tol, m.refine_tolerance, sizeof(tol));
   return {static_cast<uintptr_t>(k), p(m.fields.ptr), p(w.bp.ptr), p(w.xa.ptr), p(w.xb.ptr),
           p(w.r.ptr), p(w.y.ptr), p(w.d.ptr), p(w.fvec.ptr), p(w.bmax.ptr), p(w.partials.ptr),
-          p(w.pending.ptr), static_cast<uintptr_t>(w.capacity), p(m.d_sources.ptr),
+          p(w.pending.ptr), static_cast<uintptr_t>(w.capacity),
+          static_cast<uintptr_t>(w.level_sweeps), static_cast<uintptr_t>(m.solve_side.level_sweeps),
+          p(m.d_sources.ptr),
           p(m.d_owner.ptr), static_cast<uintptr_t>(m.d_owner.size), p(m.d_offsets.ptr),
           p(m.invalid.ptr), p(m.h_invalid.ptr), p(m.h_speculate.ptr), p(m.d_slots.ptr),
           p(m.h_slots.ptr), p(m.null_partials.ptr), p(m.heat_factor.w64.ptr),
@@ -1582,6 +1584,18 @@ int hg_set_budget_probe(hg_mesh* mesh, int32_t probe) {
   return guarded([&] {
     require_mesh(mesh);
     mesh->budget_probe = probe != 0;
+  });
+}
+
+int hg_set_sweep_patience(hg_mesh* mesh, int64_t polls) {
+  return guarded([&] {
+    require_mesh(mesh);
+    HG_REQUIRE(polls >= 0, HG_ERR_VALUE, "a negative number of polls");
+    invalidate_graphs(*mesh);
+    for (SolveWorkspace* ws : {&mesh->solve, &mesh->solve_side}) {
+      ws->patience = polls;
+      ws->level_sweeps = false;
+    }
   });
 }
 

@@ -13,6 +13,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include "kernels.h"
+#include "words.h"
 
 namespace hg {
 namespace {
@@ -422,10 +423,9 @@ __global__ __launch_bounds__(kThreads) void cg_kernel(CgArgs a) {
 //   - the values the products gather (u, or a Chebyshev direction) of rows that have a neighbour
 //     in another block, written through to `exchange` where that neighbour's thread waits for them;
 //   - a block's three partial sums, written through to `slots`, where every block waits for all.
-// Both are agent-scope relaxed stores and loads, which pass the L2s by on their own, so nothing is
-// written back or invalidated, and the read-only operator stays cached. A value is its own arrival
-// flag: every word holds kEmpty until it is published, so a reader polls the very word it needs
-// and one store-to-load latency replaces a barrier's several.
+// Both are words that are their own arrival flags (words.h), so one store-to-load latency replaces
+// a barrier's several, nothing is written back or invalidated, and the read-only operator stays
+// cached.
 //
 // Blocks own consecutive rows of a spatial order of the vertices (spatial_order), so nearly all
 // of a row's neighbours are its block's and read from LDS. A published word is emptied again two
@@ -438,45 +438,7 @@ __global__ __launch_bounds__(kThreads) void cg_kernel(CgArgs a) {
 //
 // Sums keep a fixed order (a thread's rows, then butterflies over lanes, waves and blocks), so a
 // solve repeats bit for bit. Every wait is bounded as the grid barrier's are.
-constexpr uint64_t kEmpty = 0x7FF4A5A5C3C3F00Dull;       // a signaling NaN no arithmetic returns
-constexpr uint64_t kQuietNan = 0x7FF8000000000000ull;
 constexpr int kPhases = 4, kSlotPhases = 3, kSlotWidth = 4;
-
-__device__ __forceinline__ void publish(double* word, double v) {
-  uint64_t bits = __builtin_bit_cast(uint64_t, v);
-  if (bits == kEmpty) bits = kQuietNan;
-  __hip_atomic_store(reinterpret_cast<uint64_t*>(word), bits, __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ void empty(double* word) {
-  __hip_atomic_store(reinterpret_cast<uint64_t*>(word), kEmpty, __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ uint64_t peek(const double* word) {
-  return __hip_atomic_load(reinterpret_cast<const uint64_t*>(word), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// This wave's stores have reached the point of coherence.
-__device__ __forceinline__ void drain_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
-// A wait's patience: false once it has polled past the limit or another wait has given up, which
-// it then tells everyone.
-__device__ __forceinline__ bool wait_on(const CgArgs& a, int32_t& polls, bool& aborted) {
-  if (aborted) return false;
-  if ((++polls & 255) == 0) {
-    int32_t* flag = a.counters + 1;
-    if (polls > a.spin_limit ||
-        __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-      __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      aborted = true;
-      return false;
-    }
-  }
-  return true;
-}
 
 // A thread's value of a vector for each of its rows, in registers or in LDS (l = the thread's
 // first entry, entries kStride apart).
@@ -618,7 +580,7 @@ __global__ __launch_bounds__(T) void cg_resident_kernel(CgArgs a) {
               raw[e] = at_remote(col[j][e]);
               waiting = true;
             }
-          if (!waiting || !wait_on(a, polls, aborted)) break;
+          if (!waiting || !wait_on(a.counters + 1, 1, a.spin_limit, polls, aborted)) break;
         }
       }
       double sum = 0.0;
@@ -634,7 +596,7 @@ __global__ __launch_bounds__(T) void cg_resident_kernel(CgArgs a) {
         uint64_t bits;
         if (kGrid && c < 0) {
           int32_t polls = 0;
-          while ((bits = at_remote(c)) == kEmpty && wait_on(a, polls, aborted)) {
+          while ((bits = at_remote(c)) == kEmpty && wait_on(a.counters + 1, 1, a.spin_limit, polls, aborted)) {
           }
         } else {
           bits = at_local(c);
@@ -692,7 +654,7 @@ __global__ __launch_bounds__(T) void cg_resident_kernel(CgArgs a) {
       for (int c = 0; c < 3; ++c) got[c] = peek(theirs + c);
       int32_t polls = 0;
       while (got[0] == kEmpty || got[1] == kEmpty || got[2] == kEmpty) {
-        if (!wait_on(a, polls, aborted)) break;
+        if (!wait_on(a.counters + 1, 1, a.spin_limit, polls, aborted)) break;
 #pragma unroll
         for (int c = 0; c < 3; ++c)
           if (got[c] == kEmpty) got[c] = peek(theirs + c);
@@ -1008,11 +970,6 @@ int32_t cooperative_grid(int64_t n) {
   const int64_t needed = (n + 1023) / 1024;
   return static_cast<int32_t>(std::max<int64_t>(1, std::min<int64_t>(cus, needed)));
 }
-
-// Polls of a grid barrier before it gives up: each poll is an agent-scope load plus a short sleep
-// (about a microsecond), so about two seconds, thousands of times a round's longest legitimate
-// wait.
-constexpr int64_t kSpinLimit = int64_t{1} << 21;
 
 using CgKernel = void (*)(CgArgs);
 

@@ -31,17 +31,18 @@ struct DevicePlan {
     std::vector<int32_t> level_ptr;   // product tasks per level
     std::vector<int32_t> reduce_ptr;  // reduction groups per level (empty level: no split)
     std::vector<int32_t> slots;       // partial slots each level uses
-    DeviceArray<int32_t> s, tile, k0, k1, slot;  // per product task; slot -1 writes directly
-    // The same per task with its front's figures, three int4 a task read in one round trip:
-    // {s, tile, k0, k1}, {slot, ncol, col_begin, ncol + nrow}, {w_off (two words), vec_off
-    // (forward) or row_ptr (backward) as two words}.
+    // Three int4 a task, read in one round trip: {front, tile, k0, k1}, {slot (-1 writes directly),
+    // ncol, col_begin, ncol + nrow}, {w_off (two words), vec_off (forward) or row_ptr (backward) as
+    // two words}.
     DeviceArray<int4> desc;
     // The reduction groups likewise: {s, tile, first slot, slot count}, {0, ncol, col_begin, m},
     // {0, 0, vec_off (forward) as two words}.
     DeviceArray<int4> rdesc;
-    DeviceArray<int32_t> rs, rtile, rfirst, rcount;  // per reduction group
   };
   SweepTasks fwd, bwd;
+  // The tasks of a sweep in one launch (flow.hip), three int4 each, the forward ones first.
+  DeviceArray<int4> flow_desc;
+  int32_t flow_forward = 0;
   int32_t max_slots = 0;
   int32_t split_target = kDefaultSplitTarget;
   // Forward gather lists: each front position's children contributions (absolute rows of the
@@ -75,7 +76,20 @@ struct Factor {
   }
 };
 
+// One sweep of at most kFlowColumns right-hand sides (rows interleaved, [row][kk]) as one launch:
+// forward from r into y and the update words fvec, backward into d and, with x, x_next = x + d.
+// Clears *pending, and sets its kFlowAborted bit if the launch gave up waiting (y and d are then
+// undefined).
+void flow_sweep(const DevicePlan& plan, const Factor& factor, bool use_fp32, const double* r,
+                double* fvec, double* y, double* d, const double* x, double* x_next, int32_t kk,
+                int32_t* pending, int64_t patience, hipStream_t stream);
+
+// Polls of a one-launch sweep's waits before it gives up: about two seconds.
+constexpr int64_t kSweepPatience = int64_t{1} << 21;
+
 struct SolveWorkspace {
+  int64_t patience = kSweepPatience;
+  bool level_sweeps = false;  // a one-launch sweep gave up here: level by level from then on
   DeviceArray<double> bp, xa, xb, r, y, d, fvec, bmax, partials;
   DeviceArray<int32_t> pending;
   int64_t capacity = 0, fcap = 0, pcap = 0;

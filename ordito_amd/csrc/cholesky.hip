@@ -17,6 +17,8 @@
 // product that updates the trailing matrix, and no separate triangular inversion is needed.
 #include <utility>
 
+#include <cstring>
+
 #include "cholesky.h"
 
 namespace hg {
@@ -526,6 +528,48 @@ void validate_sweeps(const Plan& plan, int32_t target_tasks) {
         fail("reduction slots out of range");
     }
   }
+  // The one-launch sweep: every output of each direction is one task's, over its whole inner range,
+  // and each task follows its front's children (forward) or its parent and the whole forward sweep
+  // (backward).
+  {
+    const HostFlow flow = flow_tasks(plan);
+    const int64_t tasks = static_cast<int64_t>(flow.desc.size()) / 12;
+    if (flow.desc.size() % 12 || flow.n_forward < 0 || flow.n_forward > tasks) fail("flow list");
+    for (const bool forward : {true, false}) {
+      std::vector<int32_t> next(S, 0);
+      auto extent = [&](int32_t s) { return plan.ncol[s] + (forward ? plan.nrow[s] : 0); };
+      for (int64_t t = forward ? 0 : flow.n_forward; t < (forward ? flow.n_forward : tasks); ++t) {
+        const int32_t* f = flow.desc.data() + 12 * t;
+        const int32_t shape = f[0], tile = f[1], s = f[7];
+        if (s < 0 || s >= S) fail("flow front out of range");
+        const int32_t nc = plan.ncol[s], m = nc + plan.nrow[s];
+        if (f[4] != nc || f[5] != plan.col_begin[s] || f[6] != m) fail("flow front figures");
+        const int64_t w = static_cast<int64_t>(static_cast<uint32_t>(f[8])) |
+                          (static_cast<int64_t>(f[9]) << 32);
+        const int64_t other = static_cast<int64_t>(static_cast<uint32_t>(f[10])) |
+                              (static_cast<int64_t>(f[11]) << 32);
+        if (w != plan.w_off[s] || other != (forward ? plan.vec_off[s] : plan.row_ptr[s]))
+          fail("flow offsets");
+        if (tile != next[s] || tile >= extent(s)) fail("flow tiles out of order");
+        if (forward) {
+          if (shape != 1 && shape != 4 && shape != 16) fail("forward flow shape");
+          next[s] = std::min(extent(s), tile + 256 / shape);
+          if (f[2] != std::min(nc, tile + 256 / shape)) fail("flow inner range");
+          const bool has = plan.child_ptr[s + 1] > plan.child_ptr[s];
+          if (f[3] != (has ? 1 : 0)) fail("flow gather flag");
+          for (int32_t k = plan.child_ptr[s]; k < plan.child_ptr[s + 1]; ++k)
+            if (next[plan.children[k]] != extent(plan.children[k])) fail("flow child order");
+        } else {
+          if (shape != 1 && shape != 4) fail("backward flow shape");
+          next[s] = std::min(extent(s), tile + 16 * shape);
+          const int32_t p = plan.parent[s];
+          if (p >= 0 && next[p] != extent(p)) fail("flow parent order");
+        }
+      }
+      for (int64_t s = 0; s < S; ++s)
+        if (next[s] != extent(static_cast<int32_t>(s))) fail("flow tiles missing");
+    }
+  }
   const HostGather g = gather_lists(plan);
   if (static_cast<int64_t>(g.ptr.size()) != plan.vec_size + 1) fail("gather offsets size");
   for (int32_t v : g.src)
@@ -696,15 +740,6 @@ void upload_sweep(const Plan& plan, bool forward, const HostSweep& h,
   out.level_ptr = h.level_ptr;
   out.reduce_ptr = h.reduce_ptr;
   out.slots = h.slots;
-  out.s.upload(h.s, stream);
-  out.tile.upload(h.tile, stream);
-  out.k0.upload(h.k0, stream);
-  out.k1.upload(h.k1, stream);
-  out.slot.upload(h.slot, stream);
-  out.rs.upload(h.rs, stream);
-  out.rtile.upload(h.rtile, stream);
-  out.rfirst.upload(h.rfirst, stream);
-  out.rcount.upload(h.rcount, stream);
 }
 
 }  // namespace
@@ -716,6 +751,11 @@ void DevicePlan::upload_sweeps(const Plan& plan, int32_t target_tasks, hipStream
   upload_sweep(plan, true, hf, fwd, stream);
   upload_sweep(plan, false, hb, bwd, stream);
   split_target = target_tasks;
+  const HostFlow flow = flow_tasks(plan);
+  flow_forward = flow.n_forward;
+  std::vector<int4> flow4(flow.desc.size() / 4);
+  if (!flow4.empty()) std::memcpy(flow4.data(), flow.desc.data(), sizeof(int4) * flow4.size());
+  flow_desc.upload(flow4, stream);
 }
 
 void DevicePlan::upload(const Plan& plan, const HostPattern& pattern, int32_t target_tasks,
@@ -809,10 +849,10 @@ int64_t DevicePlan::bytes() const {
          row_ptr.bytes() + rows.bytes() + child_ptr.bytes() + children.bytes() + rel.bytes() +
          level_nodes.bytes() + front_off.bytes() + w_off.bytes() + vec_off.bytes() +
          entry_src.bytes() + entry_dst.bytes() + entry_row.bytes() + entry_col.bytes() +
-         fwd.s.bytes() * 5 + fwd.rs.bytes() * 4 + bwd.s.bytes() * 5 + bwd.rs.bytes() * 4 +
          fwd.desc.bytes() + fwd.rdesc.bytes() + bwd.desc.bytes() + bwd.rdesc.bytes() +
          gather_ptr.bytes() + gather_src.bytes() + gather_pair.bytes() +
-         p_offsets.bytes() + p_columns.bytes() + p_src.bytes() + factor_tasks.bytes();
+         p_offsets.bytes() + p_columns.bytes() + p_src.bytes() + factor_tasks.bytes() +
+         flow_desc.bytes();
 }
 
 void factor_numeric(const DevicePlan& plan, const double* values, const int32_t* pinned_new,

@@ -209,6 +209,28 @@ struct HostGather {
 };
 HostGather gather_lists(const Plan& plan);
 
+// A whole sweep of a few right-hand sides as one launch's tasks (flow.hip), in an order in which
+// each follows everything it waits for: the forward tasks by level upwards, then the backward ones
+// downwards. Twelve int32 a task: {shape, tile, inner, gathers, ncol, col_begin, ncol + nrow,
+// front, w_off (two words), vec_off (forward) or row_ptr (backward) as two words}. A forward task
+// is rows [tile, tile + 256 / shape) over columns [0, inner), shape 1, 4 or 16 threads a row; a
+// backward task columns [tile, tile + 16 shape), shape 1 or 4.
+struct HostFlow {
+  int32_t n_forward = 0;
+  std::vector<int32_t> desc;
+};
+// The most right-hand sides such a sweep takes. Its products are on the vector units, a multiply a
+// column; level by level they are on the matrix cores, sixteen columns for the price of one. A sweep
+// of 4 columns takes 196 us against 407 on icosphere(7), 491 against 899 on the 524,288-row torus
+// and 2.14 ms against 3.58 on icosphere(9); of 8, 360 against 411, 927 against 900 and 4.22 ms
+// against 3.62.
+constexpr int32_t kFlowColumns = 4;
+// A level of this many 64-wide tiles keeps them (icosphere(7): 160 us a sweep; from 128 on 164, from
+// 2,048 on 161, never 187).
+constexpr int64_t kFlowWideTiles = 512;
+constexpr int32_t kFlowAborted = 2;      // the pending word's bit of a launch that gave up waiting
+HostFlow flow_tasks(const Plan& plan);
+
 // Checks every index the device sweeps form from the plan against its buffer; throws on the first
 // violation.
 void validate_sweeps(const Plan& plan, int32_t target_tasks = kDefaultSplitTarget);

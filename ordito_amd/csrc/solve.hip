@@ -101,20 +101,6 @@ struct SweepArgs {
   int32_t gathers;   // the level's fronts have children (forward sweep): f gathers their updates
 };
 
-// One gathered entry: v plus the children's update rows adding into front-vector row `row`,
-// column q, in ascending child order (the sources as in gather_pairs).
-__device__ __forceinline__ double gather1(const SweepArgs& a, int64_t row, int q, double v) {
-  const int2 p = reinterpret_cast<const int2*>(a.gather_pair)[row];
-  if (p.x >= 0) v += a.fvec[static_cast<int64_t>(p.x) * a.kk + q];
-  if (p.y >= 0) {
-    v += a.fvec[static_cast<int64_t>(p.y) * a.kk + q];
-  } else if (p.y == -2) {
-    for (int32_t g = a.gather_ptr[row] + 1; g < a.gather_ptr[row + 1]; ++g)
-      v += a.fvec[static_cast<int64_t>(a.gather_src[g]) * a.kk + q];
-  }
-  return v;
-}
-
 // The children's update rows that add into front-vector rows row[u] (u < 4), in two steps so a
 // caller can issue other loads between them: gather_pairs loads each row's first two sources
 // (inline in gather_pair; -1: none; -2 in the second: more than two, the rest in the lists after
@@ -585,110 +571,6 @@ __global__ __launch_bounds__(256) void bwd_reduce_kernel(const int4* __restrict_
   }
 }
 
-// One right-hand side: f gathered into LDS 256 entries at a time, then four lanes a row split the
-// inner range (j = lane mod 4), folded in lane order.
-template <typename TW>
-__global__ __launch_bounds__(256) void fwd_tile1_kernel(
-    const int32_t* __restrict__ task_s, const int32_t* __restrict__ task_r0,
-    const int32_t* __restrict__ task_k0, const int32_t* __restrict__ task_k1,
-    const int32_t* __restrict__ task_slot, const TW* __restrict__ w, SweepArgs a) {
-  __shared__ double Fs[256];
-  __shared__ double part[4][kTile];
-  const int32_t task = xcd_block();
-  const int32_t s = task_s[task];
-  const int32_t r0 = task_r0[task];
-  const int32_t k0 = task_k0[task], k1 = task_k1[task];
-  const int32_t slot = task_slot[task];
-  const int32_t nc = a.ncol[s], c0 = a.col_begin[s];
-  const int32_t m = nc + a.nrow[s];
-  const TW* W = w + a.w_off[s];
-  const int64_t vbase = a.vec_off[s];
-  const int ii = threadIdx.x % kTile, lane = threadIdx.x / kTile;
-  const int32_t i = r0 + ii;
-  double acc = 0.0;
-  for (int32_t j0 = k0; j0 < k1; j0 += 256) {
-    const int32_t j = j0 + threadIdx.x;
-    Fs[threadIdx.x] =
-        j < k1 ? (a.gathers ? gather1(a, vbase + j, 0, a.r[c0 + j]) : a.r[c0 + j]) : 0.0;
-    __syncthreads();
-    const int32_t jend = min(k1 - j0, 256);
-    if (i < m)
-      for (int32_t jj = lane; jj < jend; jj += 4)
-        acc += widen(W[static_cast<int64_t>(j0 + jj) * m + i]) * Fs[jj];
-    __syncthreads();
-  }
-  part[lane][ii] = acc;
-  __syncthreads();
-  if (lane == 0 && i < m) {
-    const double sum = ((part[0][ii] + part[1][ii]) + part[2][ii]) + part[3][ii];
-    if (slot >= 0) {
-      a.partials[static_cast<int64_t>(slot) * kTile + ii] = sum;
-    } else if (i < nc) {
-      a.y[c0 + i] = sum;
-    } else {
-      const int64_t row = vbase + i;
-      a.fvec[row] =
-          (a.gathers ? gather1(a, row, 0, 0.0) : 0.0) + sum;
-    }
-  }
-}
-
-template <typename TW>
-__global__ __launch_bounds__(256) void bwd_tile1_kernel(
-    const int32_t* __restrict__ task_s, const int32_t* __restrict__ task_j0,
-    const int32_t* __restrict__ task_k0, const int32_t* __restrict__ task_k1,
-    const int32_t* __restrict__ task_slot, const TW* __restrict__ w, SweepArgs a) {
-  constexpr int kStage = 1024;  // entries of g staged at a time
-  __shared__ double Gs[kStage];
-  const int32_t task = xcd_block();
-  const int32_t s = task_s[task];
-  const int32_t j0 = task_j0[task];
-  const int32_t k0 = task_k0[task], k1 = task_k1[task];
-  const int32_t slot = task_slot[task];
-  const int32_t nc = a.ncol[s], c0 = a.col_begin[s];
-  const int32_t m = nc + a.nrow[s];
-  const TW* W = w + a.w_off[s];
-  const int32_t* srows = a.rows + a.row_ptr[s];
-  // g = [y(cols); d(rows)] over the inner range is staged in LDS once (its structure-row gathers
-  // off the products' path); then sixteen lanes a solve-block column, each group of sixteen
-  // reading 16 consecutive entries of its column (contiguous in memory) a step. The 64 columns go
-  // in four passes of sixteen; each column's sixteen lane sums fold in a fixed butterfly.
-  const int sub = threadIdx.x % 16, grp = threadIdx.x / 16;
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int32_t s0 = k0; s0 < k1; s0 += kStage) {
-    const int32_t s1 = min(k1, s0 + kStage);
-    for (int32_t i = s0 + static_cast<int32_t>(threadIdx.x); i < s1; i += 256)
-      Gs[i - s0] = i < nc ? a.y[c0 + i] : a.d[srows[i - nc]];
-    __syncthreads();
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const int32_t j = j0 + grp + 16 * p;
-      if (j >= nc) continue;
-      const TW* wj = W + static_cast<int64_t>(j) * m;
-      // Rows above the diagonal of the inverse's leading block are zero: start at j's group.
-      const int32_t first = s0 + max(0, (j - s0) / 16 * 16);
-      for (int32_t i = first + sub; i < s1; i += 16) acc[p] += widen(wj[i]) * Gs[i - s0];
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int p = 0; p < 4; ++p)
-#pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) acc[p] += __shfl_xor(acc[p], off, 16);
-  if (sub != 0) return;
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    const int32_t jj = grp + 16 * p, j = j0 + jj;
-    if (j >= nc) continue;
-    if (slot >= 0) {
-      a.partials[static_cast<int64_t>(slot) * kTile + jj] = acc[p];
-    } else {
-      a.d[c0 + j] = acc[p];
-      if (a.x) a.x_next[c0 + j] = a.x[c0 + j] + acc[p];
-    }
-  }
-}
-
 // Raises *flag once per block that fails, and not at all once the flag reads set: with every row
 // failing in a solve's first rounds, an atomic a wave on one word serializes the whole launch.
 // Block-collective.
@@ -1115,14 +997,8 @@ void sweep(const DevicePlan& plan, const TW* w, SweepArgs a, hipStream_t stream)
     const int32_t tasks = F.level_ptr[level + 1] - t0;
     if (tasks == 0) continue;
     a.gathers = plan.level_gathers[level];
-    if (a.kk == 1) {
-      fwd_tile1_kernel<TW><<<tasks, 256, 0, stream>>>(F.s.ptr + t0, F.tile.ptr + t0,
-                                                      F.k0.ptr + t0, F.k1.ptr + t0,
-                                                      F.slot.ptr + t0, w, a);
-    } else {
-      auto tile = a.gathers ? fwd_tile_kernel<TW, true> : fwd_tile_kernel<TW, false>;
-      tile<<<tasks, 256, 0, stream>>>(F.desc.ptr + 3 * static_cast<int64_t>(t0), w, a);
-    }
+    auto tile = a.gathers ? fwd_tile_kernel<TW, true> : fwd_tile_kernel<TW, false>;
+    tile<<<tasks, 256, 0, stream>>>(F.desc.ptr + 3 * static_cast<int64_t>(t0), w, a);
     const int32_t r0 = F.reduce_ptr[level];
     const int32_t groups = F.reduce_ptr[level + 1] - r0;
     if (groups > 0) {
@@ -1135,14 +1011,8 @@ void sweep(const DevicePlan& plan, const TW* w, SweepArgs a, hipStream_t stream)
     const int32_t t0 = B.level_ptr[level];
     const int32_t tasks = B.level_ptr[level + 1] - t0;
     if (tasks == 0) continue;
-    if (a.kk == 1) {
-      bwd_tile1_kernel<TW><<<tasks, 256, 0, stream>>>(B.s.ptr + t0, B.tile.ptr + t0,
-                                                      B.k0.ptr + t0, B.k1.ptr + t0,
-                                                      B.slot.ptr + t0, w, a);
-    } else {
-      auto tile = a.x ? bwd_tile_kernel<TW, true> : bwd_tile_kernel<TW, false>;
-      tile<<<tasks, 256, 0, stream>>>(B.desc.ptr + 3 * static_cast<int64_t>(t0), w, a);
-    }
+    auto tile = a.x ? bwd_tile_kernel<TW, true> : bwd_tile_kernel<TW, false>;
+    tile<<<tasks, 256, 0, stream>>>(B.desc.ptr + 3 * static_cast<int64_t>(t0), w, a);
     const int32_t r0 = B.reduce_ptr[level];
     const int32_t groups = B.reduce_ptr[level + 1] - r0;
     if (groups > 0) {
@@ -1243,6 +1113,8 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
     double* x_cur = x_home;
     int32_t rounds = 0;
     while (rounds < max_rounds) {
+      // A few columns sweep in one launch (flow.hip), unless one such launch has given up here.
+      const bool flows = kk <= kFlowColumns && !ws.level_sweeps;
       double* x_next = x_cur == x_home ? ws.xa.ptr : x_home;
       if (rounds == 0) {
         a.r = bp;
@@ -1257,7 +1129,10 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
       }
       {
         PhaseScope scope(timer, sweep_phase, stream);
-        if (use_fp32) sweep<float>(plan, factor.w32.ptr, a, stream);
+        if (flows)
+          flow_sweep(plan, factor, use_fp32, a.r, a.fvec, a.y, a.d, a.x, a.x_next, kk,
+                     ws.pending.ptr, ws.patience, stream);
+        else if (use_fp32) sweep<float>(plan, factor.w32.ptr, a, stream);
         else sweep<double>(plan, factor.w64.ptr, a, stream);
       }
       if (rounds > 0) x_cur = x_next;
@@ -1280,7 +1155,7 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
       };
       {
         PhaseScope scope(timer, kPhaseResidual, stream);
-        launch_zero(ws.pending.ptr, sizeof(int32_t), stream);
+        if (!flows) launch_zero(ws.pending.ptr, sizeof(int32_t), stream);
         residual(test_only ? nullptr : ws.r.ptr);
       }
       HG_HIP(hipGetLastError());
@@ -1295,6 +1170,12 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
       HG_HIP(hipStreamSynchronize(stream));
       if (timer) timer->resolve();
       if (!pending) break;
+      if (pending & kFlowAborted) {  // nothing the round wrote counts: start over level by level
+        ws.level_sweeps = true;
+        x_cur = x_home;
+        rounds = 0;
+        continue;
+      }
       if (test_only && rounds < max_rounds) {
         PhaseScope scope(timer, kPhaseResidual, stream);
         residual(ws.r.ptr);
