@@ -101,29 +101,32 @@ struct SweepArgs {
   int32_t gathers;   // the level's fronts have children (forward sweep): f gathers their updates
 };
 
-// The children's update rows that add into front-vector rows row[u] (u < 4), in two steps so a
+// The children's update rows that add into front-vector rows row[u] (u < N), in two steps so a
 // caller can issue other loads between them: gather_pairs loads each row's first two sources
 // (inline in gather_pair; -1: none; -2 in the second: more than two, the rest in the lists after
 // the first; live[u] false: none), gather_add loads every update row of column q[u] and then adds
-// them to v[u] in ascending child order. Two waits on memory for four entries, not two per entry.
+// them to v[u] in ascending child order. Two waits on memory for N entries, not two per entry.
 // Absent sources read row 0 and are not added.
-__device__ __forceinline__ void gather_pairs(const SweepArgs& a, const int64_t row[4],
-                                             const bool live[4], int2 p[4]) {
+template <int N>
+__device__ __forceinline__ void gather_pairs(const SweepArgs& a, const int64_t (&row)[N],
+                                             const bool (&live)[N], int2 (&p)[N]) {
   const int2* pairs = reinterpret_cast<const int2*>(a.gather_pair);
 #pragma unroll
-  for (int u = 0; u < 4; ++u) p[u] = live[u] ? pairs[row[u]] : make_int2(-1, -1);
+  for (int u = 0; u < N; ++u) p[u] = live[u] ? pairs[row[u]] : make_int2(-1, -1);
 }
 
-__device__ __forceinline__ void gather_add(const SweepArgs& a, const int64_t row[4],
-                                           const int q[4], const int2 p[4], double v[4]) {
-  double first[4], second[4];
+template <int N>
+__device__ __forceinline__ void gather_add(const SweepArgs& a, const int64_t (&row)[N],
+                                           const int (&q)[N], const int2 (&p)[N],
+                                           double (&v)[N]) {
+  double first[N], second[N];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < N; ++u) {
     first[u] = a.fvec[p[u].x >= 0 ? static_cast<int64_t>(p[u].x) * a.kk + q[u] : 0];
     second[u] = a.fvec[p[u].y >= 0 ? static_cast<int64_t>(p[u].y) * a.kk + q[u] : 0];
   }
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < N; ++u) {
     if (p[u].x >= 0) v[u] += first[u];
     if (p[u].y >= 0) {
       v[u] += second[u];
@@ -137,67 +140,26 @@ __device__ __forceinline__ void gather_add(const SweepArgs& a, const int64_t row
 // The tile products run on the FP64 matrix cores: v_mfma_f64_16x16x4 takes a 16 x 4 block of A
 // (lane l holds A[l % 16][l / 16]) and a 4 x 16 block of B (lane l holds B[l / 16][l % 16]) and
 // accumulates the 16 x 16 product, lane l holding rows l / 16 + 4v (v < 4) of column l % 16. A
-// tile's four waves each own 16 of its 64 rows and accumulate all 64 right-hand sides as four
-// 16-column blocks. Both operands are staged through LDS kInner inner indices at a time; the next
-// stage's global loads are issued before the current stage's products, so they overlap.
+// tile's four waves each own 16 of its 64 rows and accumulate NB blocks of 16 right-hand sides. The
+// vectors are staged through LDS, shared by the waves, kInner inner indices at a time; a wave's
+// part of the inverse factor is its own, so its lanes load it straight into the operand's layout.
+// The next stage's global loads are issued before the current stage's products, so they overlap.
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 constexpr int kInner = 16;
-// Staged rows are kTile + kPad doubles apart: the four inner rows an MFMA operand read spans start
-// 34 banks apart (mod 64), and the backward's transposed stores of sixteen inner rows at one
-// column land in distinct bank pairs.
+// Staged rows are kPad doubles more than their columns apart: the four inner rows an MFMA operand
+// read spans start 34 banks apart (mod 64) at 64 columns.
 constexpr int kPad = 17;
 
 __device__ __forceinline__ f64x4 mfma16x16x4(double a, double b, f64x4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// The 4-deep steps over one stage: A from As[k][16 * wave + l % 16] (the wave's 16 output rows),
-// B from Bs[k][16 n + l % 16] for each of the four 16-column blocks n of right-hand sides (columns
-// past the chunk's are staged as zeros, so every block is multiplied). kBatch steps' operands are
-// read before their products, so the reads overlap and the products issue back to back.
-template <int kDepth = kInner, int kBatch = 2>
-__device__ __forceinline__ void stage_products(const double (*As)[kTile + kPad],
-                                               const double (*Bs)[kCols + kPad], int wave, int lane,
-                                               f64x4 acc[4]) {
-  const int li = lane % 16, lk = lane / 16;
-#pragma unroll
-  for (int kb = 0; kb < kDepth; kb += 4 * kBatch) {
-    double av[kBatch], bv[kBatch][4];
-#pragma unroll
-    for (int h = 0; h < kBatch; ++h) {
-      av[h] = As[kb + 4 * h + lk][16 * wave + li];
-#pragma unroll
-      for (int n = 0; n < 4; ++n) bv[h][n] = Bs[kb + 4 * h + lk][16 * n + li];
-    }
-#pragma unroll
-    for (int h = 0; h < kBatch; ++h)
-#pragma unroll
-      for (int n = 0; n < 4; ++n) acc[n] = mfma16x16x4(av[h], bv[h][n], acc[n]);
-  }
+// The entry `bytes` past a wave-uniform base: one address register a lane for a run of loads.
+template <typename T>
+__device__ __forceinline__ T load_at(const T* base, uint32_t bytes) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + bytes);
 }
 
-// stage_products over the column blocks that hold right-hand sides only (blocks of them), a step
-// at a time: the backward's form, whose registers the unrolled form would spill.
-template <int kDepth>
-__device__ __forceinline__ void stage_products_blocks(const double (*As)[kTile + kPad],
-                                                      const double (*Bs)[kCols + kPad], int wave,
-                                                      int lane, int blocks, f64x4 acc[4]) {
-  const int li = lane % 16, lk = lane / 16;
-#pragma unroll 1
-  for (int kb = 0; kb < kDepth; kb += 4) {
-    const double av = As[kb + lk][16 * wave + li];
-#pragma unroll
-    for (int n = 0; n < 4; ++n)
-      if (n < blocks) acc[n] = mfma16x16x4(av, Bs[kb + lk][16 * n + li], acc[n]);
-  }
-}
-
-// Forward tile product for up to 64 right-hand sides: rows [r0, r0+64) of the front's inverse
-// factor times f over the inner range [k0, k1), f gathered as it is staged. slot < 0 applies the
-// product; otherwise it is stored as a partial for the reduction.
-// kGathers: the level's fronts have children whose update vectors f gathers (a.gathers); the
-// leaves' instance carries none of that code, and fits 80 registers: six waves a SIMD instead of
-// four.
 // A task's descriptor: {s, tile, k0, k1}, {slot, ncol, col_begin, m}, {a 64-bit offset of the
 // front's solve block, a 64-bit second offset}, read together.
 struct Task {
@@ -222,11 +184,16 @@ __device__ __forceinline__ Task load_task(const int4* __restrict__ desc, int32_t
   return t;
 }
 
-template <typename TW, bool kGathers>
-__global__ __launch_bounds__(256, kGathers ? 4 : 6) void fwd_tile_kernel(
+// Forward tile product for up to 16 NB right-hand sides: rows [r0, r0+64) of the front's inverse
+// factor times f over the inner range [k0, k1), f gathered as it is staged. slot < 0 applies the
+// product; otherwise it is stored as a partial for the reduction.
+// kGathers: the level's fronts have children whose update vectors f gathers (a.gathers); the
+// leaves' instance carries none of that code.
+template <typename TW, int NB, bool kGathers>
+__global__ __launch_bounds__(256, kGathers ? 4 : (NB == 4 ? 5 : 6)) void fwd_tile_kernel(
     const int4* __restrict__ desc, const TW* __restrict__ w, SweepArgs a) {
-  __shared__ double Ws[kInner][kTile + kPad];  // [inner][row]
-  __shared__ double Fs[kInner][kCols + kPad];  // [inner][right-hand side]
+  constexpr int kN = 16 * NB;
+  __shared__ double Fs[kInner][kN + kPad];  // [inner][right-hand side]
   const Task tk = load_task(desc, xcd_block());
   const int32_t r0 = tk.tile;
   const int32_t k0 = tk.k0, k1 = tk.k1;
@@ -236,7 +203,8 @@ __global__ __launch_bounds__(256, kGathers ? 4 : 6) void fwd_tile_kernel(
   const int32_t kk = a.kk;
   const TW* W = w + tk.w_off;
   const int64_t vbase = tk.other;
-  const int t = threadIdx.x, wave = t / 64, lane = t % 64;
+  const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t / 64), lane = t % 64;
+  const int li = lane % 16, lk = lane / 16;
   const bool rows_live = r0 + 16 * wave < m;  // wave-uniform
   // The epilogue's gather pairs (this lane's update rows lane / 16 + 4v), loaded before the stages.
   int2 epair[4];
@@ -245,69 +213,85 @@ __global__ __launch_bounds__(256, kGathers ? 4 : 6) void fwd_tile_kernel(
     bool elive[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int32_t i = r0 + 16 * wave + lane / 16 + 4 * v;
+      const int32_t i = r0 + 16 * wave + lk + 4 * v;
       erow[v] = vbase + i;
       elive[v] = kGathers && slot < 0 && i >= nc && i < m;
     }
-    gather_pairs(a, erow, elive, epair);
+    gather_pairs<4>(a, erow, elive, epair);
   }
-  // Staging: entry e = t + 256u of a stage is W row e % 64 / f column e % 64 at inner e / 64.
-  double wreg[4], freg[4];
+  // Operand step h of a stage: W row r0 + 16 wave + li at inner j0 + 4 h + lk (a row past the front
+  // reads its last, whose product nothing stores).
+  double wreg[4], freg[NB];
+  const uint32_t lane_w = (static_cast<uint32_t>(lk) * static_cast<uint32_t>(m) +
+                           static_cast<uint32_t>(min(r0 + 16 * wave + li, m - 1))) * sizeof(TW);
   // f = r(cols) plus the children's updates: a stage's gather pairs are loaded a stage ahead
-  // (load_pairs), so its W, r and update-row loads issue together.
-  int2 pair[4];
-  auto stage_rows = [&](int32_t j0, int64_t grow[4], int gq[4], bool glive[4]) {
+  // (load_pairs), so its W, r and update-row loads issue together. Entry e = t + 256u of a stage is
+  // f column e % kN at inner e / kN.
+  int2 pair[NB];
+  auto stage_rows = [&](int32_t j0, int64_t (&grow)[NB], int (&gq)[NB], bool (&glive)[NB]) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < NB; ++u) {
       const int e = t + 256 * u;
-      const int32_t j = j0 + e / kTile;
-      gq[u] = e % kCols;
+      const int32_t j = j0 + e / kN;
+      gq[u] = e % kN;
       glive[u] = gq[u] < kk && j < k1;
       grow[u] = vbase + j;
     }
   };
   auto load_pairs = [&](int32_t j0) {
     if (!kGathers) return;
-    int64_t grow[4];
-    int gq[4];
-    bool glive[4];
+    int64_t grow[NB];
+    int gq[NB];
+    bool glive[NB];
     stage_rows(j0, grow, gq, glive);
-    gather_pairs(a, grow, glive, pair);
+    gather_pairs<NB>(a, grow, glive, pair);
   };
   auto load = [&](int32_t j0) {
-    int64_t grow[4];
-    int gq[4];
-    bool glive[4];
+    int64_t grow[NB];
+    int gq[NB];
+    bool glive[NB];
     stage_rows(j0, grow, gq, glive);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int e = t + 256 * u;
-      const int ii = e % kTile, jj = e / kTile;
-      const int32_t i = r0 + ii, j = j0 + jj;
-      wreg[u] = (i < m && j < k1) ? widen(W[static_cast<int64_t>(j) * m + i]) : 0.0;
+    for (int h = 0; h < 4; ++h)
+      wreg[h] = rows_live && j0 + 4 * h + lk < k1
+                    ? widen(load_at(W + static_cast<int64_t>(j0 + 4 * h) * m, lane_w))
+                    : 0.0;
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const int32_t j = j0 + (t + 256 * u) / kN;
       freg[u] = glive[u] ? a.r[static_cast<int64_t>(c0 + j) * kk + gq[u]] : 0.0;
     }
-    if (kGathers) gather_add(a, grow, gq, pair, freg);
+    if (kGathers) gather_add<NB>(a, grow, gq, pair, freg);
   };
-  f64x4 acc[4];
+  f64x4 acc[NB];
 #pragma unroll
-  for (int n = 0; n < 4; ++n) acc[n] = f64x4{0.0, 0.0, 0.0, 0.0};
+  for (int n = 0; n < NB; ++n) acc[n] = f64x4{0.0, 0.0, 0.0, 0.0};
   load_pairs(k0);
   load(k0);
   if (k0 + kInner < k1) load_pairs(k0 + kInner);
   for (int32_t j0 = k0; j0 < k1; j0 += kInner) {
+    double av[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int h = 0; h < 4; ++h) av[h] = wreg[h];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
       const int e = t + 256 * u;
-      Ws[e / kTile][e % kTile] = wreg[u];
-      Fs[e / kCols][e % kCols] = freg[u];
+      Fs[e / kN][e % kN] = freg[u];
     }
     __syncthreads();
     if (j0 + kInner < k1) {
       load(j0 + kInner);
       if (j0 + 2 * kInner < k1) load_pairs(j0 + 2 * kInner);
     }
-    if (rows_live) stage_products(Ws, Fs, wave, lane, acc);
+    if (rows_live)
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        double bv[NB];
+#pragma unroll
+        for (int n = 0; n < NB; ++n) bv[n] = Fs[4 * h + lk][16 * n + li];
+#pragma unroll
+        for (int n = 0; n < NB; ++n) acc[n] = mfma16x16x4(av[h], bv[n], acc[n]);
+      }
     __syncthreads();
   }
   if (!rows_live) return;
@@ -315,28 +299,28 @@ __global__ __launch_bounds__(256, kGathers ? 4 : 6) void fwd_tile_kernel(
   // before any store, so the loads overlap instead of each waiting behind a store it might alias.
   // A lane's outputs are rows lane / 16 + 4v of its wave's block; the sums keep the gather's order
   // (0, then each child in ascending order, then the product).
-  double base[4][4] = {};
+  double base[NB][4] = {};
   if (kGathers && slot < 0) {
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      if (16 * n + lane % 16 >= kk) continue;
+    for (int n = 0; n < NB; ++n) {
+      if (16 * n + li >= kk) continue;
       int64_t erow[4];
       int gq[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        erow[v] = vbase + r0 + 16 * wave + lane / 16 + 4 * v;
-        gq[v] = 16 * n + lane % 16;
+        erow[v] = vbase + r0 + 16 * wave + lk + 4 * v;
+        gq[v] = 16 * n + li;
       }
-      gather_add(a, erow, gq, epair, base[n]);
+      gather_add<4>(a, erow, gq, epair, base[n]);
     }
   }
 #pragma unroll
-  for (int n = 0; n < 4; ++n) {
-    const int q = 16 * n + lane % 16;
+  for (int n = 0; n < NB; ++n) {
+    const int q = 16 * n + li;
     if (q >= kk) continue;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int32_t ii = 16 * wave + lane / 16 + 4 * v;
+      const int32_t ii = 16 * wave + lk + 4 * v;
       const int32_t i = r0 + ii;
       if (i >= m) continue;
       const double value = acc[n][v];
@@ -405,9 +389,9 @@ __global__ __launch_bounds__(256) void fwd_reduce_kernel(const int4* __restrict_
     glive[u] = live && r0 + ii >= nc;
   }
   int2 pair[4];
-  if (a.gathers) gather_pairs(a, grow, glive, pair);
+  if (a.gathers) gather_pairs<4>(a, grow, glive, pair);
   add_partials(a.partials, static_cast<int64_t>(kTile) * kk, first, count, off, sum);
-  if (a.gathers) gather_add(a, grow, gq, pair, base);
+  if (a.gathers) gather_add<4>(a, grow, gq, pair, base);
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int32_t e = threadIdx.x + 256 * u;
@@ -419,20 +403,39 @@ __global__ __launch_bounds__(256) void fwd_reduce_kernel(const int4* __restrict_
   }
 }
 
+// Four consecutive entries of an inverse-factor column, widened (8-byte aligned: two loads of two
+// doubles, or one of four floats).
+__device__ __forceinline__ void load_four(const double* p, double (&v)[4]) {
+  typedef double pair_t __attribute__((ext_vector_type(2), aligned(8)));
+  const pair_t a = *reinterpret_cast<const pair_t*>(p);
+  const pair_t b = *reinterpret_cast<const pair_t*>(p + 2);
+  v[0] = a.x;
+  v[1] = a.y;
+  v[2] = b.x;
+  v[3] = b.y;
+}
+
+__device__ __forceinline__ void load_four(const float* p, double (&v)[4]) {
+  typedef float quad_t __attribute__((ext_vector_type(4), aligned(4)));
+  const quad_t a = *reinterpret_cast<const quad_t*>(p);
+  v[0] = a.x;
+  v[1] = a.y;
+  v[2] = a.z;
+  v[3] = a.w;
+}
+
 // Backward tile product: inverse-factor columns [j0, j0+64) transposed, times
 // g = [y(cols); d(rows)] over the inner range [k0, k1); each wave owns 16 of the columns. Applied
 // results also give x_next = x + d when kIterate (a later round; the first round's d is the
 // iterate itself, and its instance holds no iterate registers).
-// The backward stage's depth. 32 (256 contiguous bytes of an inverse-factor column a stage) needs
-// 120 registers, four waves a SIMD, and measured slower than 16 at six waves.
-constexpr int kBwdInner = 16;
-
-template <typename TW, bool kIterate>
-__global__ __launch_bounds__(256, 6) void bwd_tile_kernel(
+// A lane loads four consecutive rows 4 lk .. 4 lk + 3 of its column a stage: its column's sixteen
+// rows of a stage are one 128-byte run, and operand step h contracts rows {4 g + h}, of both
+// operands alike.
+template <typename TW, int NB, bool kIterate>
+__global__ __launch_bounds__(256, NB == 4 ? 5 : 6) void bwd_tile_kernel(
     const int4* __restrict__ desc, const TW* __restrict__ w, SweepArgs a) {
-  constexpr int kD = kBwdInner, kPer = kD * kTile / 256;  // entries a thread stages per operand
-  __shared__ double Ws[kD][kTile + kPad];  // [inner][inverse-factor column]
-  __shared__ double Gs[kD][kCols + kPad];  // [inner][right-hand side]
+  constexpr int kN = 16 * NB;
+  __shared__ double Gs[kInner][kN + kPad];  // [inner][right-hand side]
   const Task tk = load_task(desc, xcd_block());
   const int32_t j0 = tk.tile;
   const int32_t k0 = tk.k0, k1 = tk.k1;
@@ -440,40 +443,42 @@ __global__ __launch_bounds__(256, 6) void bwd_tile_kernel(
   const int32_t nc = tk.nc, c0 = tk.c0;
   const int32_t m = tk.m;
   const int32_t kk = a.kk;
-  const TW* W = w + tk.w_off;
   const int32_t* srows = a.rows + tk.other;
-  const int t = threadIdx.x, wave = t / 64, lane = t % 64;
+  const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t / 64), lane = t % 64;
+  const int li = lane % 16, lk = lane / 16;
   const bool cols_live = j0 + 16 * wave < nc;  // wave-uniform
-  // Staging: entry e = t + 256u is inverse-factor column e / kD at inner e % kD (contiguous in
-  // memory), and g's right-hand side e % 64 at inner e / 64.
-  double wreg[kPer], greg[kPer];
+  // A column past the front's reads its last, whose product nothing stores.
+  const TW* W = w + tk.w_off;
+  const uint32_t column = static_cast<uint32_t>(min(j0 + 16 * wave + li, nc - 1)) *
+                              static_cast<uint32_t>(m) + 4 * lk;
+  double wreg[4], greg[NB];
   // A stage's structure-row indices are loaded a stage ahead (load_rows), so its W and g loads
-  // issue together.
-  int32_t srow[kPer];
+  // issue together. Entry e = t + 256u of a stage is g's right-hand side e % kN at inner e / kN.
+  int32_t srow[NB];
   auto load_rows = [&](int32_t i0) {
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int32_t ig = i0 + (t + 256 * u) / kCols;
+    for (int u = 0; u < NB; ++u) {
+      const int32_t ig = i0 + (t + 256 * u) / kN;
       srow[u] = (ig >= nc && ig < k1) ? srows[ig - nc] : 0;
     }
   };
   auto load = [&](int32_t i0) {
-    // 32-bit element offsets from wave-uniform bases (a front's block and a field both stay
-    // under 2^31 entries), one register an address.
+    if (cols_live) {
+      if (i0 + kInner <= k1) {  // uniform: the whole stage is inside the range
+        load_four(W + column + i0, wreg);
+      } else {
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int e = t + 256 * u;
-      const int ii = e % kD, jj = e / kD;
-      const int32_t i = i0 + ii, j = j0 + jj;
-      wreg[u] = (i < k1 && j < nc)
-                    ? widen(W[static_cast<uint32_t>(j) * static_cast<uint32_t>(m) + i])
-                    : 0.0;
+        for (int h = 0; h < 4; ++h)
+          wreg[h] = i0 + 4 * lk + h < k1 ? widen(W[column + i0 + h]) : 0.0;
+      }
     }
+    // 32-bit element offsets from wave-uniform bases (a field stays under 2^31 entries), one
+    // register an address.
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
+    for (int u = 0; u < NB; ++u) {
       const int e = t + 256 * u;
-      const int q = e % kCols;
-      const int32_t ig = i0 + e / kCols;
+      const int q = e % kN;
+      const int32_t ig = i0 + e / kN;
       double g = 0.0;
       if (q < kk && ig < k1) {
         if (ig < nc) g = a.y[static_cast<uint32_t>(c0 + ig) * static_cast<uint32_t>(kk) + q];
@@ -482,48 +487,58 @@ __global__ __launch_bounds__(256, 6) void bwd_tile_kernel(
       greg[u] = g;
     }
   };
-  f64x4 acc[4];
+  f64x4 acc[NB];
 #pragma unroll
-  for (int n = 0; n < 4; ++n) acc[n] = f64x4{0.0, 0.0, 0.0, 0.0};
+  for (int n = 0; n < NB; ++n) acc[n] = f64x4{0.0, 0.0, 0.0, 0.0};
   load_rows(k0);
   load(k0);
-  if (k0 + kD < k1) load_rows(k0 + kD);
-  for (int32_t i0 = k0; i0 < k1; i0 += kD) {
+  if (k0 + kInner < k1) load_rows(k0 + kInner);
+  for (int32_t i0 = k0; i0 < k1; i0 += kInner) {
+    double av[4];
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
+    for (int h = 0; h < 4; ++h) av[h] = wreg[h];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
       const int e = t + 256 * u;
-      Ws[e % kD][e / kD] = wreg[u];
-      Gs[e / kCols][e % kCols] = greg[u];
+      Gs[e / kN][e % kN] = greg[u];
     }
     __syncthreads();
-    if (i0 + kD < k1) {
-      load(i0 + kD);
-      if (i0 + 2 * kD < k1) load_rows(i0 + 2 * kD);
+    if (i0 + kInner < k1) {
+      load(i0 + kInner);
+      if (i0 + 2 * kInner < k1) load_rows(i0 + 2 * kInner);
     }
-    if (cols_live) stage_products_blocks<kD>(Ws, Gs, wave, lane, (kk + 15) / 16, acc);
+    if (cols_live)
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        double bv[NB];
+#pragma unroll
+        for (int n = 0; n < NB; ++n) bv[n] = Gs[4 * lk + h][16 * n + li];
+#pragma unroll
+        for (int n = 0; n < NB; ++n) acc[n] = mfma16x16x4(av[h], bv[n], acc[n]);
+      }
     __syncthreads();
   }
   if (!cols_live) return;
   // Epilogue: the iterate's entries are all loaded before any store (see the forward tile).
-  double xv[4][4] = {};
+  double xv[NB][4] = {};
   if (kIterate && slot < 0) {
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      const int q = 16 * n + lane % 16;
+    for (int n = 0; n < NB; ++n) {
+      const int q = 16 * n + li;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int32_t j = j0 + 16 * wave + lane / 16 + 4 * v;
+        const int32_t j = j0 + 16 * wave + lk + 4 * v;
         if (q < kk && j < nc) xv[n][v] = a.x[static_cast<int64_t>(c0 + j) * kk + q];
       }
     }
   }
 #pragma unroll
-  for (int n = 0; n < 4; ++n) {
-    const int q = 16 * n + lane % 16;
+  for (int n = 0; n < NB; ++n) {
+    const int q = 16 * n + li;
     if (q >= kk) continue;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int32_t jj = 16 * wave + lane / 16 + 4 * v;
+      const int32_t jj = 16 * wave + lk + 4 * v;
       const int32_t j = j0 + jj;
       if (j >= nc) continue;
       const double value = acc[n][v];
@@ -988,8 +1003,13 @@ __global__ __launch_bounds__(256) void rows_out_kernel(const double* __restrict_
 
 inline unsigned blocks_for(int64_t n) { return static_cast<unsigned>((n + 255) / 256); }
 
-template <typename TW>
-void sweep(const DevicePlan& plan, const TW* w, SweepArgs a, hipStream_t stream) {
+// The tile products' instances: the matrix cores take right-hand sides sixteen at a time, so a chunk
+// is padded to 16, 32 or 64. With 16, a stage's products, LDS reads and vector loads are a quarter
+// of the 64-column instance's: 5 columns on the 524,288-row torus took 898 us a sweep padded to 64
+// and take 636 padded to 16, 32 take 884 for 1,043, and 16 on icosphere(9) 2.58 ms for 3.75. Five
+// waves a SIMD for the 64-column instances (six spill: 1.32 -> 1.78 ms).
+template <typename TW, int NB>
+void sweep_blocks(const DevicePlan& plan, const TW* w, SweepArgs a, hipStream_t stream) {
   const DevicePlan::SweepTasks& F = plan.fwd;
   const DevicePlan::SweepTasks& B = plan.bwd;
   for (int32_t level = 0; level < plan.n_levels; ++level) {
@@ -997,7 +1017,7 @@ void sweep(const DevicePlan& plan, const TW* w, SweepArgs a, hipStream_t stream)
     const int32_t tasks = F.level_ptr[level + 1] - t0;
     if (tasks == 0) continue;
     a.gathers = plan.level_gathers[level];
-    auto tile = a.gathers ? fwd_tile_kernel<TW, true> : fwd_tile_kernel<TW, false>;
+    auto tile = a.gathers ? fwd_tile_kernel<TW, NB, true> : fwd_tile_kernel<TW, NB, false>;
     tile<<<tasks, 256, 0, stream>>>(F.desc.ptr + 3 * static_cast<int64_t>(t0), w, a);
     const int32_t r0 = F.reduce_ptr[level];
     const int32_t groups = F.reduce_ptr[level + 1] - r0;
@@ -1011,7 +1031,7 @@ void sweep(const DevicePlan& plan, const TW* w, SweepArgs a, hipStream_t stream)
     const int32_t t0 = B.level_ptr[level];
     const int32_t tasks = B.level_ptr[level + 1] - t0;
     if (tasks == 0) continue;
-    auto tile = a.x ? bwd_tile_kernel<TW, true> : bwd_tile_kernel<TW, false>;
+    auto tile = a.x ? bwd_tile_kernel<TW, NB, true> : bwd_tile_kernel<TW, NB, false>;
     tile<<<tasks, 256, 0, stream>>>(B.desc.ptr + 3 * static_cast<int64_t>(t0), w, a);
     const int32_t r0 = B.reduce_ptr[level];
     const int32_t groups = B.reduce_ptr[level + 1] - r0;
@@ -1021,6 +1041,13 @@ void sweep(const DevicePlan& plan, const TW* w, SweepArgs a, hipStream_t stream)
     }
   }
   HG_HIP(hipGetLastError());
+}
+
+template <typename TW>
+void sweep(const DevicePlan& plan, const TW* w, const SweepArgs& a, hipStream_t stream) {
+  if (a.kk <= 16) sweep_blocks<TW, 1>(plan, w, a, stream);
+  else if (a.kk <= 32) sweep_blocks<TW, 2>(plan, w, a, stream);
+  else sweep_blocks<TW, 4>(plan, w, a, stream);
 }
 
 }  // namespace
