@@ -39,11 +39,16 @@ struct DevicePlan {
     // {0, 0, vec_off (forward) as two words}.
     DeviceArray<int4> rdesc;
   };
-  SweepTasks fwd, bwd;
+  // Two task lists: [0] for up to 16 columns, whose tiles are one block each, and [1] for more, whose
+  // tiles' columns are dealt to up to four blocks (solve.hip) and so are split along the inner
+  // dimension towards a quarter as many tasks. A split costs its partials' round trip through
+  // memory: 64 columns took 3.86 ms a batch on the 524,288-row torus with one list for 1,024 tasks,
+  // 3.75 for 512, 3.70 for 256; 16 columns on icosphere(9) 8.37 for 1,024 and 8.44 for 512.
+  SweepTasks fwd[2], bwd[2];
   // The tasks of a sweep in one launch (flow.hip), three int4 each, the forward ones first.
   DeviceArray<int4> flow_desc;
   int32_t flow_forward = 0;
-  int32_t max_slots = 0;
+  int32_t max_slots[2] = {0, 0};
   int32_t split_target = kDefaultSplitTarget;
   // Forward gather lists: each front position's children contributions (absolute rows of the
   // front-vector arena), in ascending child order.

@@ -745,11 +745,14 @@ void upload_sweep(const Plan& plan, bool forward, const HostSweep& h,
 }  // namespace
 
 void DevicePlan::upload_sweeps(const Plan& plan, int32_t target_tasks, hipStream_t stream) {
-  const HostSweep hf = sweep_tasks(plan, true, target_tasks);
-  const HostSweep hb = sweep_tasks(plan, false, target_tasks);
-  max_slots = std::max(hf.max_slots, hb.max_slots);
-  upload_sweep(plan, true, hf, fwd, stream);
-  upload_sweep(plan, false, hb, bwd, stream);
+  for (int list = 0; list < 2; ++list) {
+    const int32_t target = list == 0 ? target_tasks : std::max(1, target_tasks / 4);
+    const HostSweep hf = sweep_tasks(plan, true, target);
+    const HostSweep hb = sweep_tasks(plan, false, target);
+    max_slots[list] = std::max(hf.max_slots, hb.max_slots);
+    upload_sweep(plan, true, hf, fwd[list], stream);
+    upload_sweep(plan, false, hb, bwd[list], stream);
+  }
   split_target = target_tasks;
   const HostFlow flow = flow_tasks(plan);
   flow_forward = flow.n_forward;
@@ -849,7 +852,8 @@ int64_t DevicePlan::bytes() const {
          row_ptr.bytes() + rows.bytes() + child_ptr.bytes() + children.bytes() + rel.bytes() +
          level_nodes.bytes() + front_off.bytes() + w_off.bytes() + vec_off.bytes() +
          entry_src.bytes() + entry_dst.bytes() + entry_row.bytes() + entry_col.bytes() +
-         fwd.desc.bytes() + fwd.rdesc.bytes() + bwd.desc.bytes() + bwd.rdesc.bytes() +
+         fwd[0].desc.bytes() + fwd[0].rdesc.bytes() + bwd[0].desc.bytes() + bwd[0].rdesc.bytes() +
+         fwd[1].desc.bytes() + fwd[1].rdesc.bytes() + bwd[1].desc.bytes() + bwd[1].rdesc.bytes() +
          gather_ptr.bytes() + gather_src.bytes() + gather_pair.bytes() +
          p_offsets.bytes() + p_columns.bytes() + p_src.bytes() + factor_tasks.bytes() +
          flow_desc.bytes();

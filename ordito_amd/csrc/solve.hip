@@ -101,12 +101,12 @@ struct SweepArgs {
   int32_t gathers;   // the level's fronts have children (forward sweep): f gathers their updates
 };
 
-// The children's update rows that add into front-vector rows row[u] (u < N), in two steps so a
-// caller can issue other loads between them: gather_pairs loads each row's first two sources
-// (inline in gather_pair; -1: none; -2 in the second: more than two, the rest in the lists after
-// the first; live[u] false: none), gather_add loads every update row of column q[u] and then adds
-// them to v[u] in ascending child order. Two waits on memory for N entries, not two per entry.
-// Absent sources read row 0 and are not added.
+// The children's update rows that add into front-vector rows, in three steps so that a caller can
+// issue other loads, and products, between them. gather_pairs: each row's first two sources (inline
+// in gather_pair; -1: none; -2 in the second: more than two, the rest in the lists after the first;
+// live[u] false: none). gather_issue: the two update rows' entries of column q[u] (an absent source
+// reads row 0). gather_add: the sum, in ascending child order. Nothing waits before gather_add.
+// q may run up to 63 past the chunk's columns: the update vectors end in as much padding.
 template <int N>
 __device__ __forceinline__ void gather_pairs(const SweepArgs& a, const int64_t (&row)[N],
                                              const bool (&live)[N], int2 (&p)[N]) {
@@ -115,26 +115,32 @@ __device__ __forceinline__ void gather_pairs(const SweepArgs& a, const int64_t (
   for (int u = 0; u < N; ++u) p[u] = live[u] ? pairs[row[u]] : make_int2(-1, -1);
 }
 
+__device__ __forceinline__ const double* update_row(const SweepArgs& a, int32_t row) {
+  return a.fvec + static_cast<int64_t>(max(row, 0)) * a.kk;
+}
+
 template <int N>
-__device__ __forceinline__ void gather_add(const SweepArgs& a, const int64_t (&row)[N],
-                                           const int (&q)[N], const int2 (&p)[N],
-                                           double (&v)[N]) {
-  double first[N], second[N];
+__device__ __forceinline__ void gather_issue(const SweepArgs& a, const int2 (&p)[N],
+                                             const int (&q)[N], double (&first)[N],
+                                             double (&second)[N]) {
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    first[u] = a.fvec[p[u].x >= 0 ? static_cast<int64_t>(p[u].x) * a.kk + q[u] : 0];
-    second[u] = a.fvec[p[u].y >= 0 ? static_cast<int64_t>(p[u].y) * a.kk + q[u] : 0];
+    first[u] = update_row(a, p[u].x)[q[u]];
+    second[u] = update_row(a, p[u].y)[q[u]];
   }
-#pragma unroll
-  for (int u = 0; u < N; ++u) {
-    if (p[u].x >= 0) v[u] += first[u];
-    if (p[u].y >= 0) {
-      v[u] += second[u];
-    } else if (p[u].y == -2) {
-      for (int32_t g = a.gather_ptr[row[u]] + 1; g < a.gather_ptr[row[u] + 1]; ++g)
-        v[u] += a.fvec[static_cast<int64_t>(a.gather_src[g]) * a.kk + q[u]];
-    }
+}
+
+// v plus row `row`'s gathered entries of column q, the first two already loaded.
+__device__ __forceinline__ double gather_add(const SweepArgs& a, int64_t row, int q, int2 p,
+                                             double first, double second, double v) {
+  if (p.x >= 0) v += first;
+  if (p.y >= 0) {
+    v += second;
+  } else if (p.y == -2) {
+    for (int32_t g = a.gather_ptr[row] + 1; g < a.gather_ptr[row + 1]; ++g)
+      v += a.fvec[static_cast<int64_t>(a.gather_src[g]) * a.kk + q];
   }
+  return v;
 }
 
 // The tile products run on the FP64 matrix cores: v_mfma_f64_16x16x4 takes a 16 x 4 block of A
@@ -191,10 +197,12 @@ __device__ __forceinline__ Task load_task(const int4* __restrict__ desc, int32_t
 // leaves' instance carries none of that code.
 template <typename TW, int NB, bool kGathers>
 __global__ __launch_bounds__(256, kGathers ? 4 : (NB == 4 ? 5 : 6)) void fwd_tile_kernel(
-    const int4* __restrict__ desc, const TW* __restrict__ w, SweepArgs a) {
+    const int4* __restrict__ desc, int32_t parts, const TW* __restrict__ w, SweepArgs a) {
   constexpr int kN = 16 * NB;
-  __shared__ double Fs[kInner][kN + kPad];  // [inner][right-hand side]
-  const Task tk = load_task(desc, xcd_block());
+  __shared__ double Fs[2][kInner][kN + kPad];  // [stage][inner][right-hand side]
+  const int32_t block = xcd_block();
+  const Task tk = load_task(desc, block / parts);
+  const int32_t q0 = block % parts * kN;  // the block's first right-hand side
   const int32_t r0 = tk.tile;
   const int32_t k0 = tk.k0, k1 = tk.k1;
   const int32_t slot = tk.slot;
@@ -206,131 +214,150 @@ __global__ __launch_bounds__(256, kGathers ? 4 : (NB == 4 ? 5 : 6)) void fwd_til
   const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t / 64), lane = t % 64;
   const int li = lane % 16, lk = lane / 16;
   const bool rows_live = r0 + 16 * wave < m;  // wave-uniform
+  // The wave's inner range: its rows of the leading block are zero past the diagonal.
+  const int32_t wave_k1 = !rows_live ? 0 : min(k1, r0 + 16 * wave + 16 <= nc ? r0 + 16 * wave + 16 : nc);
+  const bool applies = kGathers && slot < 0;  // the epilogue gathers too
   // The epilogue's gather pairs (this lane's update rows lane / 16 + 4v), loaded before the stages.
   int2 epair[4];
+  int64_t erow[4];
   {
-    int64_t erow[4];
     bool elive[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int32_t i = r0 + 16 * wave + lk + 4 * v;
       erow[v] = vbase + i;
-      elive[v] = kGathers && slot < 0 && i >= nc && i < m;
+      elive[v] = applies && i >= nc && i < m;
     }
     gather_pairs<4>(a, erow, elive, epair);
   }
   // Operand step h of a stage: W row r0 + 16 wave + li at inner j0 + 4 h + lk (a row past the front
   // reads its last, whose product nothing stores).
-  double wreg[4], freg[NB];
   const uint32_t lane_w = (static_cast<uint32_t>(lk) * static_cast<uint32_t>(m) +
                            static_cast<uint32_t>(min(r0 + 16 * wave + li, m - 1))) * sizeof(TW);
-  // f = r(cols) plus the children's updates: a stage's gather pairs are loaded a stage ahead
-  // (load_pairs), so its W, r and update-row loads issue together. Entry e = t + 256u of a stage is
-  // f column e % kN at inner e / kN.
-  int2 pair[NB];
-  auto stage_rows = [&](int32_t j0, int64_t (&grow)[NB], int (&gq)[NB], bool (&glive)[NB]) {
+  double wreg[4];
+  auto load_w = [&](int32_t j0) {
+    if (j0 >= wave_k1) return;
+    if (j0 + kInner <= k1) {
 #pragma unroll
-    for (int u = 0; u < NB; ++u) {
-      const int e = t + 256 * u;
-      const int32_t j = j0 + e / kN;
-      gq[u] = e % kN;
-      glive[u] = gq[u] < kk && j < k1;
-      grow[u] = vbase + j;
+      for (int h = 0; h < 4; ++h)
+        wreg[h] = widen(load_at(W + static_cast<int64_t>(j0 + 4 * h) * m, lane_w));
+    } else {
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+        wreg[h] = j0 + 4 * h + lk < k1
+                      ? widen(load_at(W + static_cast<int64_t>(j0 + 4 * h) * m, lane_w))
+                      : 0.0;
     }
   };
+  // f = r(cols) plus the children's updates: entry e = t + 256u of a stage is f column e % kN at
+  // inner e / kN (past the range, its last row again, which W multiplies by zero). A stage's gather
+  // pairs are loaded two stages ahead of its products, its entries one, and they are added and
+  // staged after the products in between: nothing waits for a load it has just issued.
+  int2 pair[NB];
+  double rreg[NB], first[NB], second[NB];
+  const int qe = q0 + t % kN, ql = min(qe, a.kk - 1);
+  auto inner_of = [&](int32_t j0, int u) { return min(j0 + (t + 256 * u) / kN, k1 - 1); };
   auto load_pairs = [&](int32_t j0) {
     if (!kGathers) return;
     int64_t grow[NB];
-    int gq[NB];
     bool glive[NB];
-    stage_rows(j0, grow, gq, glive);
-    gather_pairs<NB>(a, grow, glive, pair);
-  };
-  auto load = [&](int32_t j0) {
-    int64_t grow[NB];
-    int gq[NB];
-    bool glive[NB];
-    stage_rows(j0, grow, gq, glive);
-#pragma unroll
-    for (int h = 0; h < 4; ++h)
-      wreg[h] = rows_live && j0 + 4 * h + lk < k1
-                    ? widen(load_at(W + static_cast<int64_t>(j0 + 4 * h) * m, lane_w))
-                    : 0.0;
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
-      const int32_t j = j0 + (t + 256 * u) / kN;
-      freg[u] = glive[u] ? a.r[static_cast<int64_t>(c0 + j) * kk + gq[u]] : 0.0;
+      grow[u] = vbase + inner_of(j0, u);
+      glive[u] = true;
     }
-    if (kGathers) gather_add<NB>(a, grow, gq, pair, freg);
+    gather_pairs<NB>(a, grow, glive, pair);
+  };
+  int2 used[NB];  // the pairs of the entries in flight
+  auto load_f = [&](int32_t j0) {
+    int q[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      q[u] = qe;
+      rreg[u] = a.r[static_cast<int64_t>(c0 + inner_of(j0, u)) * kk + ql];
+    }
+    if constexpr (kGathers) {
+#pragma unroll
+      for (int u = 0; u < NB; ++u) used[u] = pair[u];
+      gather_issue<NB>(a, used, q, first, second);
+    }
+  };
+  auto stage = [&](int32_t j0, double (*F)[kN + kPad]) {
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      double v = rreg[u];
+      if constexpr (kGathers)
+        v = gather_add(a, vbase + inner_of(j0, u), ql, used[u], first[u], second[u], v);
+      F[(t + 256 * u) / kN][t % kN] = v;
+    }
   };
   f64x4 acc[NB];
 #pragma unroll
   for (int n = 0; n < NB; ++n) acc[n] = f64x4{0.0, 0.0, 0.0, 0.0};
   load_pairs(k0);
-  load(k0);
+  load_w(k0);
+  load_f(k0);
   if (k0 + kInner < k1) load_pairs(k0 + kInner);
-  for (int32_t j0 = k0; j0 < k1; j0 += kInner) {
+  stage(k0, Fs[0]);
+  __syncthreads();
+  int p = 0;
+  for (int32_t j0 = k0; j0 < k1; j0 += kInner, p ^= 1) {
     double av[4];
 #pragma unroll
     for (int h = 0; h < 4; ++h) av[h] = wreg[h];
-#pragma unroll
-    for (int u = 0; u < NB; ++u) {
-      const int e = t + 256 * u;
-      Fs[e / kN][e % kN] = freg[u];
-    }
-    __syncthreads();
-    if (j0 + kInner < k1) {
-      load(j0 + kInner);
+    const bool more = j0 + kInner < k1;
+    if (more) {
+      load_w(j0 + kInner);
+      load_f(j0 + kInner);
       if (j0 + 2 * kInner < k1) load_pairs(j0 + 2 * kInner);
     }
-    if (rows_live)
+    if (j0 < wave_k1)
 #pragma unroll
       for (int h = 0; h < 4; ++h) {
         double bv[NB];
 #pragma unroll
-        for (int n = 0; n < NB; ++n) bv[n] = Fs[4 * h + lk][16 * n + li];
+        for (int n = 0; n < NB; ++n) bv[n] = Fs[p][4 * h + lk][16 * n + li];
 #pragma unroll
         for (int n = 0; n < NB; ++n) acc[n] = mfma16x16x4(av[h], bv[n], acc[n]);
       }
-    __syncthreads();
+    if (more) {
+      stage(j0 + kInner, Fs[p ^ 1]);
+      __syncthreads();
+    }
   }
   if (!rows_live) return;
-  // Epilogue: every load (the children's update rows that add into this tile's update rows)
-  // before any store, so the loads overlap instead of each waiting behind a store it might alias.
-  // A lane's outputs are rows lane / 16 + 4v of its wave's block; the sums keep the gather's order
-  // (0, then each child in ascending order, then the product).
-  double base[NB][4] = {};
-  if (kGathers && slot < 0) {
+  // Epilogue: every load (the children's update rows that add into this tile's update rows) before
+  // any is added or stored. A lane's outputs are rows lane / 16 + 4v of its wave's block; the sums
+  // keep the gather's order (0, then each child in ascending order, then the product).
+  double efirst[NB][4], esecond[NB][4];
+  if (applies) {
 #pragma unroll
-    for (int n = 0; n < NB; ++n) {
-      if (16 * n + li >= kk) continue;
-      int64_t erow[4];
-      int gq[4];
+    for (int v = 0; v < 4; ++v) {
+      const double* one = update_row(a, epair[v].x) + q0 + li;
+      const double* two = update_row(a, epair[v].y) + q0 + li;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        erow[v] = vbase + r0 + 16 * wave + lk + 4 * v;
-        gq[v] = 16 * n + li;
+      for (int n = 0; n < NB; ++n) {
+        efirst[n][v] = one[16 * n];
+        esecond[n][v] = two[16 * n];
       }
-      gather_add<4>(a, erow, gq, epair, base[n]);
     }
   }
 #pragma unroll
-  for (int n = 0; n < NB; ++n) {
-    const int q = 16 * n + li;
-    if (q >= kk) continue;
+  for (int v = 0; v < 4; ++v) {
+    const int32_t ii = 16 * wave + lk + 4 * v;
+    const int32_t i = r0 + ii;
+    if (i >= m) continue;
+    double* out = slot >= 0 ? a.partials + (static_cast<int64_t>(slot) * kTile + ii) * kk
+                  : i < nc  ? a.y + static_cast<int64_t>(c0 + i) * kk
+                            : a.fvec + (vbase + i) * kk;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int32_t ii = 16 * wave + lk + 4 * v;
-      const int32_t i = r0 + ii;
-      if (i >= m) continue;
-      const double value = acc[n][v];
-      if (slot >= 0) {
-        a.partials[(static_cast<int64_t>(slot) * kTile + ii) * kk + q] = value;
-      } else if (i < nc) {
-        a.y[static_cast<int64_t>(c0 + i) * kk + q] = value;
-      } else {
-        a.fvec[(vbase + i) * kk + q] = base[n][v] + value;
-      }
+    for (int n = 0; n < NB; ++n) {
+      const int q = q0 + 16 * n + li;
+      if (q >= kk) continue;
+      double value = acc[n][v];
+      if (applies && i >= nc)
+        value += gather_add(a, erow[v], q, epair[v], efirst[n][v], esecond[n][v], 0.0);
+      out[q] = value;
     }
   }
 }
@@ -389,9 +416,16 @@ __global__ __launch_bounds__(256) void fwd_reduce_kernel(const int4* __restrict_
     glive[u] = live && r0 + ii >= nc;
   }
   int2 pair[4];
-  if (a.gathers) gather_pairs<4>(a, grow, glive, pair);
+  double first_row[4], second_row[4];
+  if (a.gathers) {
+    gather_pairs<4>(a, grow, glive, pair);
+    gather_issue<4>(a, pair, gq, first_row, second_row);
+  }
   add_partials(a.partials, static_cast<int64_t>(kTile) * kk, first, count, off, sum);
-  if (a.gathers) gather_add<4>(a, grow, gq, pair, base);
+  if (a.gathers)
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      base[u] = gather_add(a, grow[u], gq[u], pair[u], first_row[u], second_row[u], 0.0);
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int32_t e = threadIdx.x + 256 * u;
@@ -433,10 +467,12 @@ __device__ __forceinline__ void load_four(const float* p, double (&v)[4]) {
 // operands alike.
 template <typename TW, int NB, bool kIterate>
 __global__ __launch_bounds__(256, NB == 4 ? 5 : 6) void bwd_tile_kernel(
-    const int4* __restrict__ desc, const TW* __restrict__ w, SweepArgs a) {
+    const int4* __restrict__ desc, int32_t parts, const TW* __restrict__ w, SweepArgs a) {
   constexpr int kN = 16 * NB;
-  __shared__ double Gs[kInner][kN + kPad];  // [inner][right-hand side]
-  const Task tk = load_task(desc, xcd_block());
+  __shared__ double Gs[2][kInner][kN + kPad];  // [stage][inner][right-hand side]
+  const int32_t block = xcd_block();
+  const Task tk = load_task(desc, block / parts);
+  const int32_t q0 = block % parts * kN;  // the block's first right-hand side
   const int32_t j0 = tk.tile;
   const int32_t k0 = tk.k0, k1 = tk.k1;
   const int32_t slot = tk.slot;
@@ -447,6 +483,8 @@ __global__ __launch_bounds__(256, NB == 4 ? 5 : 6) void bwd_tile_kernel(
   const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t / 64), lane = t % 64;
   const int li = lane % 16, lk = lane / 16;
   const bool cols_live = j0 + 16 * wave < nc;  // wave-uniform
+  // The wave's inner range: its columns are zero above the diagonal.
+  const int32_t wave_k0 = cols_live ? j0 + 16 * wave : k1;
   // A column past the front's reads its last, whose product nothing stores.
   const TW* W = w + tk.w_off;
   const uint32_t column = static_cast<uint32_t>(min(j0 + 16 * wave + li, nc - 1)) *
@@ -463,7 +501,7 @@ __global__ __launch_bounds__(256, NB == 4 ? 5 : 6) void bwd_tile_kernel(
     }
   };
   auto load = [&](int32_t i0) {
-    if (cols_live) {
+    if (i0 + kInner > wave_k0) {
       if (i0 + kInner <= k1) {  // uniform: the whole stage is inside the range
         load_four(W + column + i0, wreg);
       } else {
@@ -477,7 +515,7 @@ __global__ __launch_bounds__(256, NB == 4 ? 5 : 6) void bwd_tile_kernel(
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
       const int e = t + 256 * u;
-      const int q = e % kN;
+      const int q = q0 + e % kN;
       const int32_t ig = i0 + e / kN;
       double g = 0.0;
       if (q < kk && ig < k1) {
@@ -490,33 +528,42 @@ __global__ __launch_bounds__(256, NB == 4 ? 5 : 6) void bwd_tile_kernel(
   f64x4 acc[NB];
 #pragma unroll
   for (int n = 0; n < NB; ++n) acc[n] = f64x4{0.0, 0.0, 0.0, 0.0};
-  load_rows(k0);
-  load(k0);
-  if (k0 + kInner < k1) load_rows(k0 + kInner);
-  for (int32_t i0 = k0; i0 < k1; i0 += kInner) {
-    double av[4];
-#pragma unroll
-    for (int h = 0; h < 4; ++h) av[h] = wreg[h];
+  auto stage = [&](double (*G)[kN + kPad]) {
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
       const int e = t + 256 * u;
-      Gs[e / kN][e % kN] = greg[u];
+      G[e / kN][e % kN] = greg[u];
     }
-    __syncthreads();
-    if (i0 + kInner < k1) {
+  };
+  const int32_t last = k0 + (k1 - 1 - k0) / kInner * kInner;
+  load_rows(k0);
+  load(k0);
+  if (last > k0) load_rows(k0 + kInner);
+  stage(Gs[0]);
+  __syncthreads();
+  int p = 0;
+  for (int32_t i0 = k0; i0 <= last; i0 += kInner, p ^= 1) {
+    double av[4];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) av[h] = wreg[h];
+    const bool more = i0 < last;
+    if (more) {
       load(i0 + kInner);
-      if (i0 + 2 * kInner < k1) load_rows(i0 + 2 * kInner);
+      if (i0 + kInner < last) load_rows(i0 + 2 * kInner);
     }
-    if (cols_live)
+    if (i0 + kInner > wave_k0)
 #pragma unroll
       for (int h = 0; h < 4; ++h) {
         double bv[NB];
 #pragma unroll
-        for (int n = 0; n < NB; ++n) bv[n] = Gs[4 * lk + h][16 * n + li];
+        for (int n = 0; n < NB; ++n) bv[n] = Gs[p][4 * lk + h][16 * n + li];
 #pragma unroll
         for (int n = 0; n < NB; ++n) acc[n] = mfma16x16x4(av[h], bv[n], acc[n]);
       }
-    __syncthreads();
+    if (more) {
+      stage(Gs[p ^ 1]);
+      __syncthreads();
+    }
   }
   if (!cols_live) return;
   // Epilogue: the iterate's entries are all loaded before any store (see the forward tile).
@@ -524,7 +571,7 @@ __global__ __launch_bounds__(256, NB == 4 ? 5 : 6) void bwd_tile_kernel(
   if (kIterate && slot < 0) {
 #pragma unroll
     for (int n = 0; n < NB; ++n) {
-      const int q = 16 * n + li;
+      const int q = q0 + 16 * n + li;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int32_t j = j0 + 16 * wave + lk + 4 * v;
@@ -534,7 +581,7 @@ __global__ __launch_bounds__(256, NB == 4 ? 5 : 6) void bwd_tile_kernel(
   }
 #pragma unroll
   for (int n = 0; n < NB; ++n) {
-    const int q = 16 * n + li;
+    const int q = q0 + 16 * n + li;
     if (q >= kk) continue;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -1003,22 +1050,62 @@ __global__ __launch_bounds__(256) void rows_out_kernel(const double* __restrict_
 
 inline unsigned blocks_for(int64_t n) { return static_cast<unsigned>((n + 255) / 256); }
 
-// The tile products' instances: the matrix cores take right-hand sides sixteen at a time, so a chunk
-// is padded to 16, 32 or 64. With 16, a stage's products, LDS reads and vector loads are a quarter
-// of the 64-column instance's: 5 columns on the 524,288-row torus took 898 us a sweep padded to 64
-// and take 636 padded to 16, 32 take 884 for 1,043, and 16 on icosphere(9) 2.58 ms for 3.75. Five
-// waves a SIMD for the 64-column instances (six spill: 1.32 -> 1.78 ms).
-template <typename TW, int NB>
-void sweep_blocks(const DevicePlan& plan, const TW* w, SweepArgs a, hipStream_t stream) {
-  const DevicePlan::SweepTasks& F = plan.fwd;
-  const DevicePlan::SweepTasks& B = plan.bwd;
+// A tile kernel for 16 NB right-hand sides a block, and the blocks a tile's columns take. The matrix
+// cores take right-hand sides sixteen at a time, so a chunk is padded to 16, 32 or 64: 5 columns on
+// the 524,288-row torus took 898 us a sweep padded to 64 and take 636 padded to 16, 32 took 1,043 and
+// take 884, 16 on icosphere(9) 3.75 ms and 2.58. Five waves a SIMD for the 64-column instances (six
+// spill: 1.32 -> 1.78 ms).
+template <typename Kernel>
+struct TileChoice {
+  Kernel kernel;
+  int32_t parts;
+};
+
+template <typename TW>
+using TileKernel = void (*)(const int4*, int32_t, const TW*, SweepArgs);
+
+template <typename TW>
+TileChoice<TileKernel<TW>> forward_tile(int32_t kk, int32_t blocks, bool gathers) {
+  const int32_t parts = (kk + 16 * blocks - 1) / (16 * blocks);
+  if (blocks == 1) return {gathers ? fwd_tile_kernel<TW, 1, true> : fwd_tile_kernel<TW, 1, false>, parts};
+  if (blocks == 2) return {gathers ? fwd_tile_kernel<TW, 2, true> : fwd_tile_kernel<TW, 2, false>, parts};
+  return {gathers ? fwd_tile_kernel<TW, 4, true> : fwd_tile_kernel<TW, 4, false>, parts};
+}
+
+template <typename TW>
+TileChoice<TileKernel<TW>> backward_tile(int32_t kk, int32_t blocks, bool iterate) {
+  const int32_t parts = (kk + 16 * blocks - 1) / (16 * blocks);
+  if (blocks == 1) return {iterate ? bwd_tile_kernel<TW, 1, true> : bwd_tile_kernel<TW, 1, false>, parts};
+  if (blocks == 2) return {iterate ? bwd_tile_kernel<TW, 2, true> : bwd_tile_kernel<TW, 2, false>, parts};
+  return {iterate ? bwd_tile_kernel<TW, 4, true> : bwd_tile_kernel<TW, 4, false>, parts};
+}
+
+// The leaves are bound by their bytes and take a tile's columns in one block (split in two, the
+// forward leaves took 25 us more of 235 on the 524,288-row torus). Past them a level is bound by its
+// tiles' chains of dependent loads, and splitting its columns over blocks shortens and multiplies
+// them: 32 columns a block, 16 in a level of few tiles (64 columns, a sweep, with whole tiles, with
+// halves, with quarters: torus 1,304, 1,274 and 1,314 us, icosphere(7) 562, 523 and 518).
+constexpr int32_t kNarrowTasks = 512;
+
+int32_t column_blocks(int32_t kk, int32_t tasks, bool leaves) {
+  const int32_t most = kk <= 16 ? 1 : kk <= 32 ? 2 : 4;
+  if (leaves) return most;
+  return tasks >= kNarrowTasks ? std::min(most, 2) : 1;
+}
+
+template <typename TW>
+void sweep(const DevicePlan& plan, const TW* w, SweepArgs a, hipStream_t stream) {
+  const int list = a.kk <= 16 ? 0 : 1;
+  const DevicePlan::SweepTasks& F = plan.fwd[list];
+  const DevicePlan::SweepTasks& B = plan.bwd[list];
   for (int32_t level = 0; level < plan.n_levels; ++level) {
     const int32_t t0 = F.level_ptr[level];
     const int32_t tasks = F.level_ptr[level + 1] - t0;
     if (tasks == 0) continue;
     a.gathers = plan.level_gathers[level];
-    auto tile = a.gathers ? fwd_tile_kernel<TW, NB, true> : fwd_tile_kernel<TW, NB, false>;
-    tile<<<tasks, 256, 0, stream>>>(F.desc.ptr + 3 * static_cast<int64_t>(t0), w, a);
+    const auto tile = forward_tile<TW>(a.kk, column_blocks(a.kk, tasks, !a.gathers), a.gathers);
+    tile.kernel<<<tasks * tile.parts, 256, 0, stream>>>(F.desc.ptr + 3 * static_cast<int64_t>(t0),
+                                                        tile.parts, w, a);
     const int32_t r0 = F.reduce_ptr[level];
     const int32_t groups = F.reduce_ptr[level + 1] - r0;
     if (groups > 0) {
@@ -1031,8 +1118,9 @@ void sweep_blocks(const DevicePlan& plan, const TW* w, SweepArgs a, hipStream_t 
     const int32_t t0 = B.level_ptr[level];
     const int32_t tasks = B.level_ptr[level + 1] - t0;
     if (tasks == 0) continue;
-    auto tile = a.x ? bwd_tile_kernel<TW, NB, true> : bwd_tile_kernel<TW, NB, false>;
-    tile<<<tasks, 256, 0, stream>>>(B.desc.ptr + 3 * static_cast<int64_t>(t0), w, a);
+    const auto tile = backward_tile<TW>(a.kk, column_blocks(a.kk, tasks, level == 0), a.x != nullptr);
+    tile.kernel<<<tasks * tile.parts, 256, 0, stream>>>(B.desc.ptr + 3 * static_cast<int64_t>(t0),
+                                                        tile.parts, w, a);
     const int32_t r0 = B.reduce_ptr[level];
     const int32_t groups = B.reduce_ptr[level + 1] - r0;
     if (groups > 0) {
@@ -1041,13 +1129,6 @@ void sweep_blocks(const DevicePlan& plan, const TW* w, SweepArgs a, hipStream_t 
     }
   }
   HG_HIP(hipGetLastError());
-}
-
-template <typename TW>
-void sweep(const DevicePlan& plan, const TW* w, const SweepArgs& a, hipStream_t stream) {
-  if (a.kk <= 16) sweep_blocks<TW, 1>(plan, w, a, stream);
-  else if (a.kk <= 32) sweep_blocks<TW, 2>(plan, w, a, stream);
-  else sweep_blocks<TW, 4>(plan, w, a, stream);
 }
 
 }  // namespace
@@ -1069,10 +1150,11 @@ void SolveWorkspace::reserve(const DevicePlan& plan, int64_t kk_needed) {
     capacity = entries;
   }
   if (fcap < plan.vec_size * kk) {
-    fvec.allocate(std::max<int64_t>(plan.vec_size * kk, 1));
+    fvec.allocate(plan.vec_size * kk + kCols);  // the gathers' padding
     fcap = plan.vec_size * kk;
   }
-  const int64_t pentries = static_cast<int64_t>(plan.max_slots) * kTile * kk;
+  const int64_t pentries = std::max(plan.max_slots[0] * std::min<int64_t>(kk, 16),
+                                    kk > 16 ? plan.max_slots[1] * kk : 0) * kTile;
   if (pcap < pentries) {
     partials.allocate(std::max<int64_t>(pentries, 1));
     pcap = pentries;
