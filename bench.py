@@ -18,7 +18,8 @@ path: seed, heat solve, unit-gradient divergence, Poisson solve, shift -- all on
   mixed-precision form), timed beside it, with its refinement rounds and its error against the
   served fields.
 - ``plain_fp64``: the reference's form, one query per call through the FP64 factors.
-- ``roofline``: the triangular sweep of the served path (forward + backward, the dominant kernel),
+- ``roofline``: the Poisson system's triangular sweep of the served path (forward + backward, the
+  dominant kernels; the heat system's covers, forward, only the fronts its sources reach),
   algorithmic bytes per sweep over its HIP-event-measured mean duration against the 8 TB/s HBM
   peak; ``traffic`` is the HBM bytes per sweep that rocprofv3's FETCH_SIZE / WRITE_SIZE passes
   measured (profiles/triangular_sweep_torus1024x512_traffic.json, scaled by a 1 GiB copy:
@@ -731,9 +732,24 @@ def extra_workloads(args, oracle_c2, c2_vertices, c2_faces, c2_sources) -> dict:
 
 
 # The served window of a profiled C2 run: every dispatch from the first to the last 64-column
-# sweep tile, whose sweep kernels (tiles and split-K reductions) make the triangular sweeps.
+# sweep tile, whose sweep kernels (tiles and split-K reductions) make the triangular sweeps. A sweep
+# is the Poisson system's from its call's divergence on (the heat system's covers, forward, only the
+# fronts its sources reach).
 _SWEEP_TILES = ("fwd_tile_kernel<double", "bwd_tile_kernel<double")
 _SWEEP_KERNELS = _SWEEP_TILES + ("fwd_reduce_kernel", "bwd_reduce_kernel")
+_SWEEP_FIRST = "fwd_tile_kernel<double, 4, false>"
+
+
+def _in_poisson(names: list[str]) -> list[bool]:
+    """Whether each dispatch, in order, belongs to a Poisson solve."""
+    flags, poisson = [], False
+    for name in names:
+        if name.startswith("divergence_"):
+            poisson = True
+        elif name.startswith("seed_kernel"):
+            poisson = False
+        flags.append(poisson)
+    return flags
 
 
 def _short_name(name: str) -> str:
@@ -785,12 +801,14 @@ def summarize_profiles(root: Path, traffic_out: Path | None = None,
     names = [_short_name(r["Kernel_Name"]) for r in trace]
     dur = [(int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3 for r in trace]
     lo, hi = _window(names)
-    sweeps = sum(1 for n in names[lo:hi] if n.startswith("fwd_tile_kernel<double, false>"))
-    sweep_us = sum(d for n, d in zip(names[lo:hi], dur[lo:hi]) if n.startswith(_SWEEP_KERNELS))
-    lines.append(f"- sweeps in the served window: {sweeps}")
+    poisson = _in_poisson(names)
+    sweeps = sum(1 for n, p in zip(names[lo:hi], poisson[lo:hi]) if p and n.startswith(_SWEEP_FIRST))
+    sweep_us = sum(d for n, d, p in zip(names[lo:hi], dur[lo:hi], poisson[lo:hi])
+                   if p and n.startswith(_SWEEP_KERNELS))
+    lines.append(f"- Poisson sweeps in the served window: {sweeps}")
     lines.append(f"- sweep kernels' time per sweep (rocprofv3): **{sweep_us / max(sweeps, 1) / 1e3:.4f} ms**")
     # The last sweep level by level.
-    starts = [i for i in range(lo, hi) if names[i].startswith("fwd_tile_kernel<double, false>")]
+    starts = [i for i in range(lo, hi) if poisson[i] and names[i].startswith(_SWEEP_FIRST)]
     if starts:
         lines += ["", "One sweep, launch by launch (the last of the window):", "",
                   "| launch | grid | µs |", "|---|---:|---:|"]
@@ -799,7 +817,7 @@ def summarize_profiles(root: Path, traffic_out: Path | None = None,
             grid = f"{trace[i].get('Grid_Size_X', trace[i].get('Grid_Size', '?'))}"
             lines.append(f"| `{names[i]}` | {grid} | {dur[i]:.2f} |")
             i += 1
-            if i < hi and names[i].startswith("fwd_tile_kernel<double, false>"):
+            if i < hi and names[i].startswith(_SWEEP_FIRST):
                 break
     agg = collections.defaultdict(lambda: [0, 0.0])
     for n, d in zip(names[lo:hi], dur[lo:hi]):
@@ -827,8 +845,10 @@ def summarize_profiles(root: Path, traffic_out: Path | None = None,
         ids = sorted(counters)
         nm = [counters[d]["name"] for d in ids]
         a, b = _window(nm)
-        n_sw = sum(1 for x in nm[a:b] if x.startswith("fwd_tile_kernel<double, false>"))
-        total = sum(counters[ids[j]].get(key, 0.0) for j in range(a, b) if nm[j].startswith(_SWEEP_KERNELS))
+        in_poisson = _in_poisson(nm)
+        n_sw = sum(1 for x, p in zip(nm[a:b], in_poisson[a:b]) if p and x.startswith(_SWEEP_FIRST))
+        total = sum(counters[ids[j]].get(key, 0.0) for j in range(a, b)
+                    if in_poisson[j] and nm[j].startswith(_SWEEP_KERNELS))
         per_sweep[label] = total * 1024 * scale / max(n_sw, 1)
         lines.append(f"- {label}: {per_sweep[label] / 1e9:.3f} GB per sweep "
                      f"({n_sw} sweeps in that run's window)")
@@ -852,7 +872,7 @@ def summarize_profiles(root: Path, traffic_out: Path | None = None,
                      f"{us if us else float('nan'):.1f} | {rate:.0f} |")
     if traffic_out is not None and per_sweep:
         record = {
-            "kernel": "triangular sweep (forward + backward)",
+            "kernel": "triangular sweep (forward + backward) of the Poisson system",
             "workload": "torus 1024x512 R=1 r=0.3 normal jitter 0.1h, 64 single-source queries per "
             "step as one batch, factors resident",
             "columns": 64,
@@ -1146,12 +1166,11 @@ def main() -> int:
     plain_value = args.plain_queries / (time.perf_counter() - t0)
     plain_stats = dict(solver.last_stats)
 
-    # Roofline of the dominant kernel: the served path's triangular sweeps (heat and Poisson).
-    sweep_ms = timing["heat_sweep"][0] + timing["poisson_sweep"][0]
-    sweep_count = timing["heat_sweep"][1] + timing["poisson_sweep"][1]
+    # Roofline of the dominant kernels: the served path's triangular sweep of the Poisson system.
+    sweep_ms, sweep_count = timing["poisson_sweep"]
     mean_sweep_s = sweep_ms / max(sweep_count, 1) / 1e3
-    # Each step's heat and Poisson solves start with a first-round sweep per 64-column chunk.
-    first_rounds = min(sweep_count, 2 * args.steps * -(-k // 64))
+    # Each step's Poisson solve starts with a first-round sweep per 64-column chunk.
+    first_rounds = min(sweep_count, args.steps * -(-k // 64))
     bytes_per_sweep = (
         first_rounds * sweep_bytes(stats, k, 8, True)
         + (sweep_count - first_rounds) * sweep_bytes(stats, k, 8, False)
@@ -1159,7 +1178,8 @@ def main() -> int:
     achieved = bytes_per_sweep / mean_sweep_s / 1e9 if mean_sweep_s > 0 else 0.0
     roofline = {
         "bound": "hbm",
-        "kernel": "triangular sweep (forward + backward level sweeps, FP64 inverse factors, 64 columns)",
+        "kernel": "triangular sweep (forward + backward level sweeps of the Poisson system, FP64 inverse "
+        "factors, 64 columns)",
         "achieved": round(achieved, 1),
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",

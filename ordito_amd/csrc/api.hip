@@ -143,6 +143,7 @@ struct hg_mesh {
   DeviceArray<int64_t> d_owner, d_offsets;
   PinnedArray<int64_t> h_stage;  // the owners and offsets of a call, staged for an async upload
   bool sources_on_device = false;  // d_offsets[k] holds this call's source count
+  int64_t host_sources = 0;        // the source count where it does not
   // The distance's destination per 64-column chunk, read by the finishing kernel (so a replayed
   // graph writes to each call's buffer), staged in pinned memory.
   DeviceArray<double*> d_slots;
@@ -666,10 +667,14 @@ bool backward_error_fails(hg_mesh& m, const double* values, const double* x, con
   return flag != 0;
 }
 
+// seeded: rhs holds the call's uploaded sources' seeds (or those off the rim), nothing else.
 int32_t diffuse_factored(hg_mesh& m, const HeatSystem& sys, double* rhs, double* x, int64_t k,
-                         int32_t precision, FieldLayout layout = FieldLayout::kColumns) {
+                         int32_t precision, FieldLayout layout = FieldLayout::kColumns,
+                         bool seeded = false) {
   const bool mixed = precision == HG_PRECISION_MIXED;
   factor_system(m, sys.code, mixed);
+  const SourceRows seeds{m.d_sources.ptr, m.sources_on_device ? m.d_offsets.ptr : nullptr,
+                         m.host_sources};
   int32_t* speculate =
       m.speculating ? m.h_speculate.ptr + (sys.code == HG_SYSTEM_PINNED ? m.spec_chunks : 0)
                     : nullptr;
@@ -678,7 +683,8 @@ int32_t diffuse_factored(hg_mesh& m, const HeatSystem& sys, double* rhs, double*
                        mixed ? kMixedRefineRounds : kRefineRounds,
                        m.has_heat_pins ? m.heat_pinned_new.ptr : nullptr,
                        m.on_side ? m.solve_side : m.solve, m.stream,
-                       &m.timer, kPhaseHeatSweep, layout, layout, speculate);
+                       &m.timer, kPhaseHeatSweep, layout, layout, speculate,
+                       seeded ? &seeds : nullptr);
 }
 
 // The settled iterate, verified, falling back to the factorization (solve_spd_settled,
@@ -687,7 +693,7 @@ int32_t diffuse_factored(hg_mesh& m, const HeatSystem& sys, double* rhs, double*
 // by rows (FieldLayout::kRows) go through the factors only.
 int32_t diffuse(hg_mesh& m, double* rhs, double* x, int64_t k, int32_t mode,
                 int32_t precision, FieldLayout layout = FieldLayout::kColumns,
-                bool pinned = false) {
+                bool pinned = false, bool seeded = false) {
   ensure_operators(m);
   const HeatSystem sys = heat_system(m, pinned);
   int32_t flags = 0;
@@ -702,7 +708,7 @@ int32_t diffuse(hg_mesh& m, double* rhs, double* x, int64_t k, int32_t mode,
   };
   if (mode == HG_MODE_FACTORED || sys.factor->held()) {
     try {
-      refinements = diffuse_factored(m, sys, rhs, x, k, precision, layout);
+      refinements = diffuse_factored(m, sys, rhs, x, k, precision, layout, seeded);
     } catch (const Error& e) {
       // Refused under the budget before anything was solved: marched instead.
       if (!is_budget_refusal(e) || layout != FieldLayout::kColumns) throw;
@@ -973,7 +979,8 @@ std::vector<uintptr_t> graph_signature(const hg_mesh& m, int64_t k) {
   std::memcpy(tol, m.refine_tolerance, sizeof(tol));
   return {static_cast<uintptr_t>(k), p(m.fields.ptr), p(w.bp.ptr), p(w.xa.ptr), p(w.xb.ptr),
           p(w.r.ptr), p(w.y.ptr), p(w.d.ptr), p(w.fvec.ptr), p(w.bmax.ptr), p(w.partials.ptr),
-          p(w.pending.ptr), static_cast<uintptr_t>(w.capacity),
+          p(w.pending.ptr), p(w.live.ptr), p(w.live_pairs.ptr), p(m.solve_side.live.ptr),
+          p(m.solve_side.live_pairs.ptr), static_cast<uintptr_t>(w.capacity),
           static_cast<uintptr_t>(w.level_sweeps), static_cast<uintptr_t>(m.solve_side.level_sweeps),
           p(m.d_sources.ptr),
           p(m.d_owner.ptr), static_cast<uintptr_t>(m.d_owner.size), p(m.d_offsets.ptr),
@@ -1162,14 +1169,15 @@ bool solve_columns(hg_mesh& m, const int64_t* offsets, int64_t k, double* phi, i
     HG_HIP(hipStreamWaitEvent(side.stream, side.fork, 0));
     {
       StreamSwap swap(m, side.stream, true);
-      flags |= diffuse(m, m.pinned_rhs.ptr, negdiv, k, HG_MODE_FACTORED, precision, layout, true);
+      flags |= diffuse(m, m.pinned_rhs.ptr, negdiv, k, HG_MODE_FACTORED, precision, layout, true,
+                       true);
     }
-    flags |= diffuse(m, u0, heat, k, mode, precision, layout);
+    flags |= diffuse(m, u0, heat, k, mode, precision, layout, false, true);
     HG_HIP(hipEventRecord(side.join, side.stream));
     HG_HIP(hipStreamWaitEvent(m.stream, side.join, 0));
     launch_average(heat, negdiv, n * k, m.stream);
   } else {
-    flags = diffuse(m, u0, heat, k, mode, precision, layout);
+    flags = diffuse(m, u0, heat, k, mode, precision, layout, false, true);
   }
   if (igl && !(layout == FieldLayout::kRows && m.speculating)) {
     // igl::heat_geodesics' boundary rule (heat.py:594-597): the Neumann heat averaged with the
@@ -1178,7 +1186,7 @@ bool solve_columns(hg_mesh& m, const int64_t* offsets, int64_t k, double* phi, i
     launch_off_rim(u0, u0, layout == FieldLayout::kRows ? m.d_rim_rows.ptr : m.d_rim.ptr, n, k,
                    layout, m.stream);
     flags |= diffuse(m, u0, negdiv, k, layout == FieldLayout::kRows ? HG_MODE_FACTORED : mode,
-                     precision, layout, true);
+                     precision, layout, true, true);
     launch_average(heat, negdiv, n * k, m.stream);
   }
   m.stats.backward_error_failed = flags & 1;
@@ -1875,6 +1883,7 @@ int hg_geodesic_packed(hg_mesh* mesh, const int32_t* d_sources, const int64_t* s
     }
     arm_speculation(m, width, precision == HG_PRECISION_FP64);
     m.sources_on_device = false;  // the seeds' count is the host's
+    m.host_sources = total;
     solve_columns(m, seed_offsets.data(), width, m.packed_phi.ptr, HG_MODE_FACTORED, precision);
     // A speculated first round that failed its test: solve again without speculating.
     HG_HIP(hipStreamSynchronize(m.stream));

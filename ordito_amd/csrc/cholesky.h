@@ -53,6 +53,9 @@ struct DevicePlan {
   // Forward gather lists: each front position's children contributions (absolute rows of the
   // front-vector arena), in ascending child order.
   DeviceArray<int32_t> gather_ptr, gather_src, gather_pair;
+  // The front of each row of the elimination order and of each front-vector row, and each front's
+  // parent (-1: a root).
+  DeviceArray<int32_t> row_front, vec_front, parent;
   // The operator's pattern in the elimination order (P A P^T) and each entry's original slot.
   DeviceArray<int32_t> p_offsets, p_columns, p_src;
   // The numeric factorization's tile launches (host list) and tasks (device, 4 int32 each).
@@ -85,9 +88,33 @@ struct Factor {
 // forward from r into y and the update words fvec, backward into d and, with x, x_next = x + d.
 // Clears *pending, and sets its kFlowAborted bit if the launch gave up waiting (y and d are then
 // undefined).
+// With live_fronts, the forward sweep covers those fronts only (see LiveFronts).
 void flow_sweep(const DevicePlan& plan, const Factor& factor, bool use_fp32, const double* r,
                 double* fvec, double* y, double* d, const double* x, double* x_next, int32_t kk,
-                int32_t* pending, int64_t patience, hipStream_t stream);
+                int32_t* pending, int64_t patience, const struct LiveFronts* live_fronts,
+                hipStream_t stream);
+
+// A right-hand side of a few nonzero rows reaches, forward, only the fronts on the paths from those
+// rows to the roots. The marked fronts (live[s] != 0) and the gather pairs of their front-vector rows
+// without the others' contributions. A front that is not live has y = 0 and no update vector:
+// neither is written, and the backward sweep reads its rows below the leading block only.
+struct LiveFronts {
+  const int32_t* live = nullptr;
+  const int32_t* pairs = nullptr;
+};
+
+// The rows a call's right-hand sides are nonzero on, on the device: column q on vertices
+// sources[offsets[q] .. offsets[q + 1]) in the caller's numbering, or, without offsets, every column
+// on some of sources[0 .. count). Entries out of range are skipped.
+struct SourceRows {
+  const int32_t* sources = nullptr;
+  const int64_t* offsets = nullptr;
+  int64_t count = 0;
+};
+
+// A plan of fewer fronts sweeps them all: marking takes three short launches (icosphere(4), 41
+// fronts: a query went from 192 to 201 us with it; icosphere(5), 164: 213 and 214).
+constexpr int32_t kSparseFronts = 256;
 
 // Polls of a one-launch sweep's waits before it gives up: about two seconds.
 constexpr int64_t kSweepPatience = int64_t{1} << 21;
@@ -97,15 +124,19 @@ struct SolveWorkspace {
   bool level_sweeps = false;  // a one-launch sweep gave up here: level by level from then on
   DeviceArray<double> bp, xa, xb, r, y, d, fvec, bmax, partials;
   DeviceArray<int32_t> pending;
+  DeviceArray<int32_t> live, live_pairs;  // a call's LiveFronts
   int64_t capacity = 0, fcap = 0, pcap = 0;
   void reserve(const DevicePlan& plan, int64_t kk);
   int64_t bytes() const {
     return bp.bytes() + xa.bytes() + xb.bytes() + r.bytes() + y.bytes() + d.bytes() +
-           fvec.bytes() + bmax.bytes() + partials.bytes() + pending.bytes();
+           fvec.bytes() + bmax.bytes() + partials.bytes() + pending.bytes() +
+           live.bytes() + live_pairs.bytes();
   }
   void release() {
     for (DeviceArray<double>* a : {&bp, &xa, &xb, &r, &y, &d, &fvec, &bmax, &partials}) a->reset();
     pending.reset();
+    live.reset();
+    live_pairs.reset();
     capacity = fcap = pcap = 0;
   }
 };
@@ -125,12 +156,14 @@ void factor_numeric(const DevicePlan& plan, const double* values, const int32_t*
 // run the first round alone and return without waiting for its test, whose verdict (nonzero: a
 // row still above tolerance) lands in speculate[chunk] with the stream's next synchronization. The
 // caller checks it there and solves again without speculating when any is set.
+// nonzero (b stored by rows only): the rows b is nonzero on, when the caller knows them to be few.
 int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp32,
                       double* b, double* x, int64_t k, double tolerance, bool componentwise,
                       int32_t max_rounds, const int32_t* pinned_new, SolveWorkspace& ws,
                       hipStream_t stream, PhaseTimer* timer = nullptr,
                       int sweep_phase = kPhaseHeatSweep, FieldLayout b_layout = FieldLayout::kColumns,
-                      FieldLayout x_layout = FieldLayout::kColumns, int32_t* speculate = nullptr);
+                      FieldLayout x_layout = FieldLayout::kColumns, int32_t* speculate = nullptr,
+                      const SourceRows* nonzero = nullptr);
 
 // The components' members cut into 256-member chunks, for the null-space projection's reductions.
 struct NullSpace {

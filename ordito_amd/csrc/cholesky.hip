@@ -714,6 +714,18 @@ void validate_factor_tasks(const Plan& plan, const HostFactorTasks& h) {
 
 namespace {
 
+// One block a front: its rows of the elimination order and of the front vectors name it.
+__global__ __launch_bounds__(64) void front_maps_kernel(
+    const int32_t* __restrict__ col_begin, const int32_t* __restrict__ ncol,
+    const int32_t* __restrict__ nrow, const int64_t* __restrict__ vec_off,
+    int32_t* __restrict__ row_front, int32_t* __restrict__ vec_front) {
+  const int32_t s = blockIdx.x, nc = ncol[s], m = nc + nrow[s];
+  for (int32_t i = threadIdx.x; i < m; i += 64) {
+    if (i < nc) row_front[col_begin[s] + i] = s;
+    vec_front[vec_off[s] + i] = s;
+  }
+}
+
 void upload_sweep(const Plan& plan, bool forward, const HostSweep& h,
                   DevicePlan::SweepTasks& out, hipStream_t stream) {
   std::vector<int4> desc(3 * h.s.size());
@@ -825,6 +837,7 @@ void DevicePlan::upload(const Plan& plan, const HostPattern& pattern, int32_t ta
   n_entries = static_cast<int64_t>(plan.entry_src.size());
   perm.upload(plan.perm, stream);
   iperm.upload(plan.iperm, stream);
+  parent.upload(plan.parent, stream);
   col_begin.upload(plan.col_begin, stream);
   ncol.upload(plan.ncol, stream);
   nrow.upload(plan.nrow, stream);
@@ -845,10 +858,17 @@ void DevicePlan::upload(const Plan& plan, const HostPattern& pattern, int32_t ta
   host_ncol = plan.ncol;
   host_front_off = plan.front_off;
   host_nrow = plan.nrow;
+  row_front.allocate(std::max<int64_t>(n, 1));
+  vec_front.allocate(std::max<int64_t>(vec_size, 1));
+  if (n_super > 0) {
+    front_maps_kernel<<<static_cast<unsigned>(n_super), 64, 0, stream>>>(
+        col_begin.ptr, ncol.ptr, nrow.ptr, vec_off.ptr, row_front.ptr, vec_front.ptr);
+    HG_HIP(hipGetLastError());
+  }
 }
 
 int64_t DevicePlan::bytes() const {
-  return perm.bytes() + iperm.bytes() + col_begin.bytes() + ncol.bytes() + nrow.bytes() +
+  return row_front.bytes() + vec_front.bytes() + parent.bytes() + perm.bytes() + iperm.bytes() + col_begin.bytes() + ncol.bytes() + nrow.bytes() +
          row_ptr.bytes() + rows.bytes() + child_ptr.bytes() + children.bytes() + rel.bytes() +
          level_nodes.bytes() + front_off.bytes() + w_off.bytes() + vec_off.bytes() +
          entry_src.bytes() + entry_dst.bytes() + entry_row.bytes() + entry_col.bytes() +

@@ -44,12 +44,14 @@ struct FlowArgs {
   const int32_t* gather_ptr;
   const int32_t* gather_src;
   const int32_t* rows;
+  const int32_t* live;       // null: every front is
+  const int32_t* vec_front;
   int32_t* pending;
   int64_t spin_limit;
 };
 
 struct FlowTask {
-  int32_t shape, tile, inner, gathers, nc, c0, m;
+  int32_t shape, tile, inner, gathers, nc, c0, m, s;
   int64_t w_off, other;
 };
 
@@ -63,6 +65,7 @@ __device__ __forceinline__ FlowTask load_flow(const int4* __restrict__ desc) {
   t.nc = d1.x;
   t.c0 = d1.y;
   t.m = d1.z;
+  t.s = d1.w;
   t.w_off = static_cast<int64_t>(static_cast<uint32_t>(d2.x)) | (static_cast<int64_t>(d2.y) << 32);
   t.other = static_cast<int64_t>(static_cast<uint32_t>(d2.z)) | (static_cast<int64_t>(d2.w) << 32);
   return t;
@@ -107,6 +110,7 @@ __device__ __forceinline__ void gather_words(const FlowArgs& a, Patience& wait,
       v[u] += wait.await(a.fvec + static_cast<int64_t>(pair[u].y) * a.kk + q[u], second[u]);
     } else if (pair[u].y == -2) {
       for (int32_t g = a.gather_ptr[row[u]] + 1; g < a.gather_ptr[row[u] + 1]; ++g) {
+        if (a.live && !a.live[a.vec_front[a.gather_src[g]]]) continue;
         const double* word = a.fvec + static_cast<int64_t>(a.gather_src[g]) * a.kk + q[u];
         v[u] += wait.await(word, peek(word));
       }
@@ -221,9 +225,10 @@ __device__ __forceinline__ void forward_task(const FlowArgs& a, const FlowTask& 
 }
 
 // Columns [tile, tile + 16 PASS) of a front's inverse factor, transposed, times [y(cols); d(rows)]
-// over rows [tile, m): d and, after the first round, x + d.
+// over rows [top, m): d and, after the first round, x + d. top is the tile, whose rows above are
+// zero, or the first row past the leading block of a front whose y is.
 template <typename TW, int KC, int PASS>
-__device__ __forceinline__ void backward_task(const FlowArgs& a, const FlowTask& tk,
+__device__ __forceinline__ void backward_task(const FlowArgs& a, const FlowTask& tk, int32_t top,
                                               const TW* __restrict__ w, double* staged) {
   constexpr int U = 16 / PASS;  // entries of a column a lane loads ahead
   constexpr int kChunk = kStage / KC;
@@ -231,11 +236,11 @@ __device__ __forceinline__ void backward_task(const FlowArgs& a, const FlowTask&
   const int32_t kk = a.kk, m = tk.m, nc = tk.nc, j0 = tk.tile;
   const int32_t* srows = a.rows + tk.other;
   const TW* W = w + tk.w_off;
-  // Entry (j0 + sub + 16 u, j0 + group + 16 p) is a lane's offset past (j0 + 16 u, j0 + 16 p), the
+  // Entry (top + sub + 16 u, j0 + group + 16 p) is a lane's offset past (top + 16 u, j0 + 16 p), the
   // group's column clamped to the front's last.
   uint32_t lane[PASS];
-  auto entry = [&](int p, int32_t i) {  // of row j0 + i + sub, i block-uniform
-    return load_at(W + static_cast<int64_t>(min(j0 + 16 * p, nc - 1)) * m + j0 + i, lane[p]);
+  auto entry = [&](int p, int32_t i) {  // of row top + i + sub, i block-uniform
+    return load_at(W + static_cast<int64_t>(min(j0 + 16 * p, nc - 1)) * m + top + i, lane[p]);
   };
   TW ahead[PASS][U];
 #pragma unroll
@@ -243,7 +248,7 @@ __device__ __forceinline__ void backward_task(const FlowArgs& a, const FlowTask&
     const int32_t last = max(0, nc - 1 - j0 - 16 * p);
     lane[p] = (static_cast<uint32_t>(min(group, last)) * static_cast<uint32_t>(m) + sub) * sizeof(TW);
 #pragma unroll
-    for (int u = 0; u < U; ++u) ahead[p][u] = j0 + sub + 16 * u < m ? entry(p, 16 * u) : TW(0);
+    for (int u = 0; u < U; ++u) ahead[p][u] = top + sub + 16 * u < m ? entry(p, 16 * u) : TW(0);
   }
   Patience wait{a};
   double acc[PASS][KC];
@@ -251,7 +256,7 @@ __device__ __forceinline__ void backward_task(const FlowArgs& a, const FlowTask&
   for (int p = 0; p < PASS; ++p)
 #pragma unroll
     for (int q = 0; q < KC; ++q) acc[p][q] = 0.0;
-  for (int32_t s0 = j0; s0 < m; s0 += kChunk) {
+  for (int32_t s0 = top; s0 < m; s0 += kChunk) {
     const int32_t se = min(kChunk, m - s0);
     {
       constexpr int N = kStage / kThreads;
@@ -277,7 +282,7 @@ __device__ __forceinline__ void backward_task(const FlowArgs& a, const FlowTask&
     }
     __syncthreads();
     int32_t i0 = 0;  // this lane's next row of the chunk, less sub
-    if (s0 == j0) {
+    if (s0 == top) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (16 * u < se) {  // block-uniform
@@ -299,7 +304,7 @@ __device__ __forceinline__ void backward_task(const FlowArgs& a, const FlowTask&
       for (int p = 0; p < PASS; ++p)
 #pragma unroll
         for (int u = 0; u < B; ++u)
-          next[p][u] = i0 + 16 * u + sub < se ? entry(p, s0 - j0 + i0 + 16 * u) : TW(0);
+          next[p][u] = i0 + 16 * u + sub < se ? entry(p, s0 - top + i0 + 16 * u) : TW(0);
 #pragma unroll
       for (int u = 0; u < B; ++u)
         if (i0 + 16 * u + sub < se) {
@@ -341,12 +346,14 @@ __global__ __launch_bounds__(kThreads, 4) void flow_kernel(const TW* __restrict_
   __shared__ double parts[kThreads * KC];
   const FlowTask tk = load_flow(a.desc + 3 * static_cast<int64_t>(blockIdx.x));
   if (static_cast<int32_t>(blockIdx.x) < a.n_forward) {
+    if (a.live && !a.live[tk.s]) return;  // y = 0 and no updates, which nobody waits for
     if (tk.shape == 1) forward_task<TW, KC, 1>(a, tk, w, staged, parts);
     else if (tk.shape == 4) forward_task<TW, KC, 4>(a, tk, w, staged, parts);
     else forward_task<TW, KC, 16>(a, tk, w, staged, parts);
   } else {
-    if (tk.shape == 4) backward_task<TW, KC, 4>(a, tk, w, staged);
-    else backward_task<TW, KC, 1>(a, tk, w, staged);
+    const int32_t top = a.live && !a.live[tk.s] ? tk.nc : tk.tile;
+    if (tk.shape == 4) backward_task<TW, KC, 4>(a, tk, top, w, staged);
+    else backward_task<TW, KC, 1>(a, tk, top, w, staged);
   }
 }
 
@@ -425,7 +432,8 @@ HostFlow flow_tasks(const Plan& plan) {
 
 void flow_sweep(const DevicePlan& plan, const Factor& factor, bool use_fp32, const double* r,
                 double* fvec, double* y, double* d, const double* x, double* x_next, int32_t kk,
-                int32_t* pending, int64_t patience, hipStream_t stream) {
+                int32_t* pending, int64_t patience, const LiveFronts* live_fronts,
+                hipStream_t stream) {
   FlowArgs a{};
   a.desc = plan.flow_desc.ptr;
   a.n_forward = plan.flow_forward;
@@ -436,7 +444,10 @@ void flow_sweep(const DevicePlan& plan, const Factor& factor, bool use_fp32, con
   a.d = d;
   a.x = x;
   a.x_next = x_next;
-  a.gather_pair = reinterpret_cast<const int2*>(plan.gather_pair.ptr);
+  a.gather_pair =
+      reinterpret_cast<const int2*>(live_fronts ? live_fronts->pairs : plan.gather_pair.ptr);
+  a.live = live_fronts ? live_fronts->live : nullptr;
+  a.vec_front = plan.vec_front.ptr;
   a.gather_ptr = plan.gather_ptr.ptr;
   a.gather_src = plan.gather_src.ptr;
   a.rows = plan.rows.ptr;

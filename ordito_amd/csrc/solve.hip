@@ -99,6 +99,8 @@ struct SweepArgs {
   double* partials;
   int32_t kk;
   int32_t gathers;   // the level's fronts have children (forward sweep): f gathers their updates
+  const int32_t* live;  // null, or the fronts the forward sweep reaches (LiveFronts)
+  const int32_t* vec_front;
 };
 
 // The children's update rows that add into front-vector rows, in three steps so that a caller can
@@ -138,7 +140,8 @@ __device__ __forceinline__ double gather_add(const SweepArgs& a, int64_t row, in
     v += second;
   } else if (p.y == -2) {
     for (int32_t g = a.gather_ptr[row] + 1; g < a.gather_ptr[row + 1]; ++g)
-      v += a.fvec[static_cast<int64_t>(a.gather_src[g]) * a.kk + q];
+      if (!a.live || a.live[a.vec_front[a.gather_src[g]]])
+        v += a.fvec[static_cast<int64_t>(a.gather_src[g]) * a.kk + q];
   }
   return v;
 }
@@ -203,6 +206,7 @@ __global__ __launch_bounds__(256, kGathers ? 4 : (NB == 4 ? 5 : 6)) void fwd_til
   const int32_t block = xcd_block();
   const Task tk = load_task(desc, block / parts);
   const int32_t q0 = block % parts * kN;  // the block's first right-hand side
+  if (a.live && !a.live[tk.s]) return;
   const int32_t r0 = tk.tile;
   const int32_t k0 = tk.k0, k1 = tk.k1;
   const int32_t slot = tk.slot;
@@ -391,6 +395,7 @@ __device__ __forceinline__ void add_partials(const double* __restrict__ partials
 __global__ __launch_bounds__(256) void fwd_reduce_kernel(const int4* __restrict__ rdesc,
                                                          SweepArgs a) {
   const Task g = load_task(rdesc, xcd_block());
+  if (a.live && !a.live[g.s]) return;
   const int32_t r0 = g.tile;
   const int32_t first = g.k0, count = g.k1;
   const int32_t nc = g.nc, m = g.m, c0 = g.c0;
@@ -474,9 +479,10 @@ __global__ __launch_bounds__(256, NB == 4 ? 5 : 6) void bwd_tile_kernel(
   const Task tk = load_task(desc, block / parts);
   const int32_t q0 = block % parts * kN;  // the block's first right-hand side
   const int32_t j0 = tk.tile;
-  const int32_t k0 = tk.k0, k1 = tk.k1;
   const int32_t slot = tk.slot;
   const int32_t nc = tk.nc, c0 = tk.c0;
+  // A front the forward sweep did not reach has y = 0: its range starts past the leading block.
+  const int32_t k0 = a.live && !a.live[tk.s] ? max(tk.k0, nc) : tk.k0, k1 = tk.k1;
   const int32_t m = tk.m;
   const int32_t kk = a.kk;
   const int32_t* srows = a.rows + tk.other;
@@ -535,11 +541,13 @@ __global__ __launch_bounds__(256, NB == 4 ? 5 : 6) void bwd_tile_kernel(
       G[e / kN][e % kN] = greg[u];
     }
   };
-  const int32_t last = k0 + (k1 - 1 - k0) / kInner * kInner;
-  load_rows(k0);
-  load(k0);
-  if (last > k0) load_rows(k0 + kInner);
-  stage(Gs[0]);
+  const int32_t last = k0 < k1 ? k0 + (k1 - 1 - k0) / kInner * kInner : k0 - 1;
+  if (k0 < k1) {
+    load_rows(k0);
+    load(k0);
+    if (last > k0) load_rows(k0 + kInner);
+    stage(Gs[0]);
+  }
   __syncthreads();
   int p = 0;
   for (int32_t i0 = k0; i0 <= last; i0 += kInner, p ^= 1) {
@@ -1048,6 +1056,45 @@ __global__ __launch_bounds__(256) void rows_out_kernel(const double* __restrict_
   for (int q = qq; q < kk; q += 4) out[static_cast<int64_t>(q) * n + v0 + lv] = tile[lv][q];
 }
 
+// Marks every front from each source's row's to its root. The heat step's right-hand side is 64
+// seeds on the 524,288-row torus, whose forward sweep reaches 2 % of the leaves: skipping the rest,
+// and in the backward sweep the leading blocks they would multiply by zero, takes that sweep from
+// 1,200 to 795 us (16 seeds on icosphere(9) 2,480 to 1,420, one on the torus 415 to 276).
+__global__ __launch_bounds__(256) void mark_fronts_kernel(
+    const int32_t* __restrict__ sources, const int64_t* __restrict__ offsets, int32_t kk,
+    int64_t count, int64_t n, const int32_t* __restrict__ iperm,
+    const int32_t* __restrict__ row_front, const int32_t* __restrict__ parent,
+    int32_t* __restrict__ live) {
+  const int64_t first = offsets ? offsets[0] : 0, last = offsets ? offsets[kk] : count;
+  for (int64_t e = first + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; e < last;
+       e += static_cast<int64_t>(gridDim.x) * 256) {
+    const int32_t v = sources[e];
+    if (v < 0 || v >= n) continue;  // out of range: the call fails once the stream is synced
+    // A front already marked has its ancestors marked, or being marked by whoever marked it.
+    for (int32_t s = row_front[iperm[v]]; s >= 0 && atomicExch(live + s, 1) == 0; s = parent[s]) {
+    }
+  }
+}
+
+// The gather pairs of the live fronts' rows, without the contributions of fronts that are not. A wave
+// a front.
+__global__ __launch_bounds__(256) void live_pairs_kernel(
+    const int32_t* __restrict__ live, const int32_t* __restrict__ ncol,
+    const int32_t* __restrict__ nrow, const int64_t* __restrict__ vec_off,
+    const int32_t* __restrict__ vec_front, const int2* __restrict__ pairs, int32_t n_super,
+    int2* __restrict__ out) {
+  const int32_t s = static_cast<int32_t>(blockIdx.x) * 4 + static_cast<int32_t>(threadIdx.x) / 64;
+  if (s >= n_super || !live[s]) return;
+  const int64_t base = vec_off[s];
+  const int32_t m = ncol[s] + nrow[s];
+  for (int32_t i = static_cast<int32_t>(threadIdx.x) % 64; i < m; i += 64) {
+    int2 p = pairs[base + i];
+    if (p.x >= 0 && !live[vec_front[p.x]]) p.x = -1;
+    if (p.y >= 0 && !live[vec_front[p.y]]) p.y = -1;
+    out[base + i] = p;
+  }
+}
+
 inline unsigned blocks_for(int64_t n) { return static_cast<unsigned>((n + 255) / 256); }
 
 // A tile kernel for 16 NB right-hand sides a block, and the blocks a tile's columns take. The matrix
@@ -1162,13 +1209,16 @@ void SolveWorkspace::reserve(const DevicePlan& plan, int64_t kk_needed) {
   const int64_t absmax = static_cast<int64_t>(blocks_for(plan.n)) * kCols + kCols;
   if (bmax.size < absmax) bmax.allocate(absmax);
   if (pending.size < 1) pending.allocate(1);
+  if (live.size < plan.n_super) live.allocate(plan.n_super);
+  if (live_pairs.size < 2 * plan.vec_size) live_pairs.allocate(2 * plan.vec_size);
 }
 
 int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp32,
                       double* b, double* x, int64_t k, double tolerance, bool componentwise,
                       int32_t max_rounds, const int32_t* pinned_new, SolveWorkspace& ws,
                       hipStream_t stream, PhaseTimer* timer, int sweep_phase,
-                      FieldLayout b_layout, FieldLayout x_layout, int32_t* speculate) {
+                      FieldLayout b_layout, FieldLayout x_layout, int32_t* speculate,
+                      const SourceRows* nonzero) {
   const int64_t n = plan.n;
   if (n == 0 || k == 0) return 0;
   int32_t max_used = 0;
@@ -1215,6 +1265,10 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
     a.y = ws.y.ptr;
     a.partials = ws.partials.ptr;
     a.kk = kk;
+    a.vec_front = plan.vec_front.ptr;
+    const bool sparse =
+        nonzero && b_layout == FieldLayout::kRows && plan.n_super >= kSparseFronts;
+    const LiveFronts reached{ws.live.ptr, ws.live_pairs.ptr};
     // The first round solves for the iterate itself from x = 0: its right-hand side is b and its
     // correction is written straight into the iterate. Later rounds correct it: d into ws.d and
     // x + d into the other iterate buffer. By rows the iterate lives in x itself (and ws.xa).
@@ -1238,9 +1292,23 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
       }
       {
         PhaseScope scope(timer, sweep_phase, stream);
+        // Only the first round's right-hand side is the caller's; a residual is dense.
+        const bool marked = sparse && rounds == 0;
+        if (marked) {
+          launch_zero(ws.live.ptr, static_cast<int64_t>(sizeof(int32_t)) * plan.n_super, stream);
+          mark_fronts_kernel<<<64, 256, 0, stream>>>(
+              nonzero->sources, nonzero->offsets ? nonzero->offsets + q0 : nullptr, kk,
+              nonzero->count, n, plan.iperm.ptr, plan.row_front.ptr, plan.parent.ptr, ws.live.ptr);
+          live_pairs_kernel<<<static_cast<unsigned>((plan.n_super + 3) / 4), 256, 0, stream>>>(
+              ws.live.ptr, plan.ncol.ptr, plan.nrow.ptr, plan.vec_off.ptr, plan.vec_front.ptr,
+              reinterpret_cast<const int2*>(plan.gather_pair.ptr), plan.n_super,
+              reinterpret_cast<int2*>(ws.live_pairs.ptr));
+        }
+        a.live = marked ? reached.live : nullptr;
+        a.gather_pair = marked ? reached.pairs : plan.gather_pair.ptr;
         if (flows)
           flow_sweep(plan, factor, use_fp32, a.r, a.fvec, a.y, a.d, a.x, a.x_next, kk,
-                     ws.pending.ptr, ws.patience, stream);
+                     ws.pending.ptr, ws.patience, marked ? &reached : nullptr, stream);
         else if (use_fp32) sweep<float>(plan, factor.w32.ptr, a, stream);
         else sweep<double>(plan, factor.w64.ptr, a, stream);
       }
