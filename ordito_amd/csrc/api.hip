@@ -99,9 +99,8 @@ struct hg_mesh {
   int32_t split_target = kDefaultSplitTarget;  // sweep tasks a level is split towards
   std::unique_ptr<Plan> host_plan;
   std::unique_ptr<DevicePlan> plan;
-  DeviceArray<int32_t> faces_rows;  // the faces' corners as rows of the elimination order
-  DeviceArray<int4> row_corners;    // each row's corners {corner id, its face's three rows}
-  DeviceArray<int32_t> row_corner_ptr;
+  CornerRecords corners;            // the divergence's records in the elimination order
+  bool corner_geometry = false;     // corners.geom is the assembled operators'
   Factor heat_factor, poisson_factor, pinned_factor, reg_factor;
   // The factorizations' memory budget in bytes (0: 90 % of the device memory free when a
   // factorization starts) and the systems refused under it (HG_SYSTEM_* bits).
@@ -214,7 +213,7 @@ int64_t mesh_device_bytes(const hg_mesh& m) {
        {&m.row_segment, &m.faces, &m.offsets, &m.columns, &m.corner_ptr, &m.corner_slots,
         &m.vertex_ptr, &m.vertex_corners, &m.d_rim, &m.d_rim_rows, &m.d_labels, &m.comp_ptr,
         &m.comp_members, &m.poisson_pinned_new, &m.poisson_dropped_old, &m.heat_pinned_new,
-        &m.heat_dropped_old, &m.faces_rows, &m.row_corner_ptr, &m.d_sources, &m.invalid,
+        &m.heat_dropped_old, &m.d_sources, &m.invalid,
         &m.q_local})
     total += a->bytes();
   for (const DeviceArray<float>* a : {&m.xyz, &m.cot, &m.normals, &m.areas, &m.heat32, &m.voronoi,
@@ -229,7 +228,7 @@ int64_t mesh_device_bytes(const hg_mesh& m) {
   for (const DeviceArray<int64_t>* a : {&m.d_owner, &m.d_offsets, &m.q_src_off, &m.q_dst_off,
                                         &m.q_len})
     total += a->bytes();
-  total += m.row_corners.bytes() + m.d_slots.bytes() + m.march.bytes();
+  total += m.corners.bytes() + m.d_slots.bytes() + m.march.bytes();
   if (m.poisson_mg) total += m.poisson_mg->bytes();
   total += m.heat_factor.bytes() + m.poisson_factor.bytes() + m.pinned_factor.bytes() +
            m.reg_factor.bytes();
@@ -388,6 +387,7 @@ void assemble(hg_mesh& m, double t_request, int32_t method, bool solver_default,
   for (int64_t s = 0; s < n_seg; ++s) m.seg_t[s] = host_scalars[4 * s + 3];
   m.t = m.seg_t[0];
   m.assembled = true;
+  m.corner_geometry = false;
   m.poisson_bound = -1.0;
   m.heat_factor.reset();
   m.poisson_factor.reset();
@@ -411,33 +411,9 @@ void ensure_plan(hg_mesh& m) {
   const Plan& plan = *m.host_plan;
   auto device = std::make_unique<DevicePlan>();
   device->upload(plan, m.pattern, m.split_target, m.stream);
-  {
-    std::vector<int32_t> rows(m.h_faces.size());
-    parallel_chunks(static_cast<int64_t>(rows.size()), 1 << 16, [&](int64_t b, int64_t e, int64_t) {
-      for (int64_t i = b; i < e; ++i) rows[i] = plan.iperm[m.h_faces[i]];
-    });
-    m.faces_rows.upload(rows, m.stream);
-    // Row r's corners are vertex perm[r]'s, in its ascending corner order: the row offsets in
-    // one pass, then each chunk of rows fills its own records.
-    std::vector<int32_t> ptr(static_cast<size_t>(m.n) + 1, 0);
-    for (int64_t r = 0; r < m.n; ++r) {
-      const int32_t v = plan.perm[r];
-      ptr[r + 1] = ptr[r] + (m.pattern.vertex_ptr[v + 1] - m.pattern.vertex_ptr[v]);
-    }
-    std::vector<int4> corners(m.pattern.vertex_corners.size());
-    parallel_chunks(m.n, 1 << 14, [&](int64_t b, int64_t e, int64_t) {
-      for (int64_t r = b; r < e; ++r) {
-        const int32_t v = plan.perm[r];
-        int32_t at = ptr[r];
-        for (int32_t k = m.pattern.vertex_ptr[v]; k < m.pattern.vertex_ptr[v + 1]; ++k) {
-          const int32_t c = m.pattern.vertex_corners[k], f = c / 3;
-          corners[at++] = make_int4(c, rows[3 * f], rows[3 * f + 1], rows[3 * f + 2]);
-        }
-      }
-    });
-    m.row_corners.upload(corners, m.stream);
-    m.row_corner_ptr.upload(ptr, m.stream);
-  }
+  build_corner_rows(m.faces.ptr, m.vertex_ptr.ptr, m.vertex_corners.ptr, device->perm.ptr,
+                    device->iperm.ptr, m.n, m.f, m.corners, m.stream);
+  m.corner_geometry = false;
   if (m.n_rim > 0) {
     std::vector<int32_t> rim_rows(static_cast<size_t>(m.n), 0);
     for (int64_t v = 0; v < m.n; ++v) rim_rows[plan.iperm[v]] = m.rim[v];
@@ -489,6 +465,17 @@ void ensure_plan(hg_mesh& m) {
   m.heat_dropped_old.upload(heat_dropped_old, m.stream);
   HG_HIP(hipStreamSynchronize(m.stream));
   m.plan = std::move(device);
+}
+
+// The divergence's per-corner geometry of the assembled operators, in the plan's order.
+void ensure_corner_geometry(hg_mesh& m) {
+  ensure_operators(m);
+  ensure_plan(m);
+  if (m.corner_geometry) return;
+  build_corner_geometry(m.normals.ptr, m.face_geom.ptr, m.vertex_ptr.ptr, m.vertex_corners.ptr,
+                        m.plan->perm.ptr, m.n, m.corners, m.stream);
+  m.corner_geometry = true;
+  invalidate_graphs(m);
 }
 
 // HG_METHOD_POTPOURRI3D's Poisson system -L + 1e-6 I over the Poisson pattern (built on first
@@ -922,10 +909,7 @@ void check_seeds(const hg_mesh& m) {
 void divergence(hg_mesh& m, const double* heat, double* out, int64_t k,
                 FieldLayout layout = FieldLayout::kColumns) {
   PhaseScope scope(&m.timer, kPhaseDivergence, m.stream);
-  const bool rows = layout == FieldLayout::kRows;
-  launch_divergence(rows ? m.faces_rows.ptr : m.faces.ptr, rows ? m.plan->iperm.ptr : nullptr,
-                    m.face_geom.ptr, m.vertex_ptr.ptr, m.vertex_corners.ptr,
-                    rows ? m.row_corners.ptr : nullptr, rows ? m.row_corner_ptr.ptr : nullptr,
+  launch_divergence(m.faces.ptr, m.face_geom.ptr, m.vertex_ptr.ptr, m.vertex_corners.ptr, &m.corners,
                     heat, m.n, k, out, layout, m.stream);
 }
 
@@ -1002,7 +986,7 @@ std::vector<uintptr_t> graph_signature(const hg_mesh& m, int64_t k) {
 // the fused finish, no phase timing, a single mesh.
 bool graphable(const hg_mesh& m, int32_t mode, int32_t precision) {
   return m.use_graphs && !m.graphs_broken && precision == HG_PRECISION_FP64 &&
-         !m.timer.enabled && m.segments() == 1 && m.plan && m.rows_by_component &&
+         !m.timer.enabled && m.segments() == 1 && m.plan && m.corner_geometry && m.rows_by_component &&
          (mode == HG_MODE_FACTORED || m.heat_factor.held()) && m.heat_factor.held() &&
          (m.method == HG_METHOD_POTPOURRI3D ? m.reg_factor.held() : m.poisson_factor.held()) &&
          (m.method != HG_METHOD_IGL || m.n_rim == 0 || m.pinned_factor.held());
@@ -1142,6 +1126,7 @@ bool solve_columns(hg_mesh& m, const int64_t* offsets, int64_t k, double* phi, i
       factor_system(m, HG_SYSTEM_HEAT, mixed);
       factor_system(m, regularized ? HG_SYSTEM_REGULARIZED : HG_SYSTEM_POISSON, mixed);
       if (m.method == HG_METHOD_IGL && m.n_rim > 0) factor_system(m, HG_SYSTEM_PINNED, mixed);
+      ensure_corner_geometry(m);
     } catch (const Error& e) {
       if (!is_budget_refusal(e) || m.segments() > 1) throw;
       factored = false;
@@ -1446,6 +1431,7 @@ int hg_factor(hg_mesh* mesh, int32_t systems, int32_t precision, int32_t* out_fa
         if (!is_budget_refusal(e)) throw;
       }
     }
+    if (mesh->heat_factor.held()) ensure_corner_geometry(*mesh);
     if (out_factored) {
       bool ok = (!(systems & HG_SYSTEM_HEAT) || mesh->heat_factor.held()) &&
                 (!(systems & HG_SYSTEM_POISSON) || mesh->poisson_factor.held()) &&

@@ -12,6 +12,8 @@
 #include <cmath>
 #include <vector>
 
+#include <hipcub/hipcub.hpp>
+
 #include "kernels.h"
 
 namespace hg {
@@ -532,43 +534,29 @@ __device__ __forceinline__ double corner_term(const double* __restrict__ geom, i
 
 // -b at vertex i and column q: the terms of i's corners for that column summed in ascending corner
 // order (kernels/heat.py:626-687, heat.py:3218-3232), each term recomputed from the face's heat
-// values (no per-corner intermediate in memory). heat and out share a layout: entry (row r,
-// column q) at r * vstride + q * qstride, vertex i at row row_of[i] (row i when row_of is null),
-// and `faces` name rows. Corners go four at a time: their corner ids, then their faces' vertices,
-// then the other two heat values and the face data, each step's loads issued together (a vertex
-// has about six corners).
-//
-// kWaveVertex: one wave a vertex, its lanes the columns (kk <= 64 columns stored by rows, so the
-// heat rows it reads and the row it writes are contiguous); the vertex, its corners and their face
-// data are wave-uniform. Blocks are numbered so that each XCD's share of the grid is one
-// contiguous range of vertices (xcd_block), whose neighbours' heat rows then stay in that XCD's
-// L2. Otherwise one thread per (vertex, column), the contiguous index fastest.
-template <bool kWaveVertex>
+// values (no per-corner intermediate in memory). heat and out share a layout: entry (vertex i,
+// column q) at i * vstride + q * qstride. Corners go four at a time: their corner ids, then their
+// faces' vertices, then the other two heat values and the face data, each step's loads issued
+// together (a vertex has about six corners). One thread per (vertex, column), the contiguous index
+// fastest.
 __global__ __launch_bounds__(256) void divergence_kernel(
     const int32_t* __restrict__ faces, const double* __restrict__ geom,
     const int32_t* __restrict__ vertex_ptr, const int32_t* __restrict__ vertex_corners,
-    const int32_t* __restrict__ row_of, const double* __restrict__ heat, int64_t n, int64_t kk,
-    int64_t vstride, int64_t qstride, double* __restrict__ out) {
+    const double* __restrict__ heat, int64_t n, int64_t kk, int64_t vstride, int64_t qstride,
+    double* __restrict__ out) {
+  // Whichever index is contiguous in memory runs fastest across the threads.
+  const int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (e >= n * kk) return;
   int64_t i, q;
-  if (kWaveVertex) {
-    i = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(xcd_block() * 4 + threadIdx.x / 64));
-    q = threadIdx.x % 64;
-    if (i >= n || q >= kk) return;
+  if (vstride == 1) {
+    q = e / n;
+    i = e - q * n;
   } else {
-    // Whichever index is contiguous in memory runs fastest across the threads.
-    const int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (e >= n * kk) return;
-    if (vstride == 1) {
-      q = e / n;
-      i = e - q * n;
-    } else {
-      i = e / kk;
-      q = e - i * kk;
-    }
+    i = e / kk;
+    q = e - i * kk;
   }
   const double* u = heat + q * qstride;
-  const int64_t row = row_of ? row_of[i] : i;
-  const double ui = u[row * vstride];
+  const double ui = u[i * vstride];
   double sum = 0.0;
   const int32_t kbeg = vertex_ptr[i], kend = vertex_ptr[i + 1];
   for (int32_t kb = kbeg; kb < kend; kb += 4) {
@@ -597,44 +585,138 @@ __global__ __launch_bounds__(256) void divergence_kernel(
       if (kb + w < kend) sum += term;
     }
   }
-  out[row * vstride + q * qstride] = sum;
+  out[i * vstride + q * qstride] = sum;
 }
 
-// The same -b for a chunk of kk columns stored by rows, one wave a row r of the elimination order
-// (its lanes the columns): row r's corners are corners[corner_ptr[r] ..], each {corner id 3f + c,
-// rows of face f's vertices 0, 1, 2}, in the vertex's ascending corner order. A wave reads eight
-// corner records, then every heat value and face datum they name, then adds the terms of the
-// corners that exist (a uniform branch: a vertex's last batch computes no padding); the result row
-// is written contiguously. Same terms, same order as divergence_kernel.
+// ---- the divergence of fields stored by rows ---------------------------------------------------
+//
+// A query evaluates every corner of every face, so what a corner needs is laid out for it once per
+// mesh, in the order the rows read it: for row r of the elimination order and its vertex's corners
+// in ascending order, the rows of the face's next and previous vertices, and kCornerGeom doubles.
+// With the corner's own vertex as the face's origin the gradient is d1 A1 + d2 A2, d1 and d2 the
+// heat at the next and the previous vertex less its own, A1 and A2 their basis vectors (the three
+// sum to zero); all of it lies in the face's plane, so in an orthonormal frame of that plane with
+// A1 on its first axis the corner needs A1 = (x1, 0), A2 = (x2, y2) and its integration vector
+// (gx, gy): five doubles in one run where the face's nine of fifteen were gathered, three products
+// for the gradient where there were six, and two neighbours' heat where there were three
+// vertices'. Both kernels wait on the neighbours' rows, which the caches serve but for about twice
+// the field (595 MB fetched for a field of 262 MB at 524,288 rows by 64 columns).
+
+// Row r's corner count, for the records' offsets.
+__global__ void corner_counts_kernel(const int32_t* __restrict__ vertex_ptr,
+                                     const int32_t* __restrict__ perm, int64_t n,
+                                     int32_t* __restrict__ counts) {
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (r > n) return;
+  const int32_t v = r < n ? perm[r] : 0;
+  counts[r] = r < n ? vertex_ptr[v + 1] - vertex_ptr[v] : 0;
+}
+
+__global__ void corner_rows_kernel(const int32_t* __restrict__ faces,
+                                   const int32_t* __restrict__ vertex_ptr,
+                                   const int32_t* __restrict__ vertex_corners,
+                                   const int32_t* __restrict__ perm,
+                                   const int32_t* __restrict__ iperm,
+                                   const int32_t* __restrict__ corner_ptr, int64_t n,
+                                   int2* __restrict__ corner_rows) {
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (r >= n) return;
+  const int32_t v = perm[r], first = vertex_ptr[v], last = vertex_ptr[v + 1];
+  for (int32_t k = first; k < last; ++k) {
+    const int32_t c = vertex_corners[k], f = c / 3, l = c - 3 * f;
+    corner_rows[corner_ptr[r] + k - first] =
+        make_int2(iperm[faces[3 * static_cast<int64_t>(f) + (l + 1) % 3]],
+                  iperm[faces[3 * static_cast<int64_t>(f) + (l + 2) % 3]]);
+  }
+}
+
+__global__ void corner_geometry_kernel(const float* __restrict__ normals,
+                                       const double* __restrict__ face_geom,
+                                       const int32_t* __restrict__ vertex_ptr,
+                                       const int32_t* __restrict__ vertex_corners,
+                                       const int32_t* __restrict__ perm,
+                                       const int32_t* __restrict__ corner_ptr, int64_t n,
+                                       double* __restrict__ geom) {
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (r >= n) return;
+  const int32_t v = perm[r], first = vertex_ptr[v], last = vertex_ptr[v + 1];
+  for (int32_t k = first; k < last; ++k) {
+    const int32_t c = vertex_corners[k], f = c / 3, l = c - 3 * f;
+    const double* face = face_geom + kFaceGeom * static_cast<int64_t>(f);
+    const D3 a0{face[0], face[1], face[2]}, a1{face[3], face[4], face[5]};
+    const D3 a2{-(a0.x + a1.x), -(a0.y + a1.y), -(a0.z + a1.z)};
+    const D3 next = l == 0 ? a1 : l == 1 ? a2 : a0, prev = l == 0 ? a2 : l == 1 ? a0 : a1;
+    const D3 g{face[6 + 3 * l], face[7 + 3 * l], face[8 + 3 * l]};
+    // The frame: along A1 (along A2 where A1 vanishes), and the unit normal's turn of it.
+    const D3 nrm = widen(load3(normals, f));
+    const double along = sqrt(dot(next, next)), other = sqrt(dot(prev, prev));
+    const D3 axis = along > 0.0   ? scale(1.0 / along, next)
+                    : other > 0.0 ? scale(1.0 / other, prev)
+                                  : D3{0.0, 0.0, 0.0};
+    const double length = sqrt(dot(nrm, nrm));
+    const D3 turn = length > 0.0 ? scale(1.0 / length, cross(nrm, axis)) : D3{0.0, 0.0, 0.0};
+    double* out = geom + kCornerGeom * static_cast<int64_t>(corner_ptr[r] + k - first);
+    out[0] = along;
+    out[1] = dot(prev, axis);
+    out[2] = dot(prev, turn);
+    out[3] = dot(g, axis);
+    out[4] = dot(g, turn);
+  }
+}
+
+// corner_term in the corner's frame, for heat differences d1 and d2. Where the squared length is
+// far from both ends of the range the direction is normalized as it is: the scaling to its largest
+// component is by a power of two, which changes no bit of the result there, and it is a third of
+// the term's instructions. The rest (the far field of a large mesh, flat heat) is scaled.
+__device__ __forceinline__ double corner_term_2d(double x1, double x2, double y2, double gx,
+                                                 double gy, double d1, double d2) {
+#pragma clang fp contract(fast)
+  const double sx = d1 * x1 + d2 * x2;
+  const double sy = d2 * y2;
+  const double square = sx * sx + sy * sy;
+  double term = (gx * sx + gy * sy) * rsqrt(square);
+  if (!(square >= 0x1p-800 && square <= 0x1p800)) {
+    const double largest = fmax(fabs(sx), fabs(sy));
+    int e;
+    (void)frexp(largest, &e);
+    const double wx = ldexp(sx, -e), wy = ldexp(sy, -e);
+    term = largest == 0.0 ? 0.0 : (gx * wx + gy * wy) * rsqrt(wx * wx + wy * wy);
+  }
+  return term;
+}
+
+// -b for a chunk of kk columns stored by rows, one wave a row of the elimination order (its lanes the
+// columns), its corners' records read as wave-uniform data, six at a time (a whole interior row of a
+// regular mesh): all the heat rows they name, then their terms in ascending corner order. The result
+// row is written contiguously. 64 columns on the 524,288-row torus: 359 us, 384 eight at a time, 512
+// from the faces' own arrays.
 __global__ __launch_bounds__(256) void divergence_rows_kernel(
-    const int4* __restrict__ corners, const int32_t* __restrict__ corner_ptr,
+    const int2* __restrict__ corner_rows, const int32_t* __restrict__ corner_ptr,
     const double* __restrict__ geom, const double* __restrict__ heat, int64_t n, int64_t kk,
     double* __restrict__ out) {
+  constexpr int B = 6;
   const int64_t r =
       __builtin_amdgcn_readfirstlane(static_cast<int32_t>(xcd_block() * 4 + threadIdx.x / 64));
   const int64_t q = threadIdx.x % 64;
   if (r >= n || q >= kk) return;
   const int32_t kbeg = corner_ptr[r], kend = corner_ptr[r + 1];
+  // A row's base is wave-uniform and the column the lane's offset.
+  const uint32_t lane = static_cast<uint32_t>(q);
+  const double own = (heat + r * kk)[lane];
   double sum = 0.0;
-  for (int32_t kb = kbeg; kb < kend; kb += 8) {
-    int4 c[8];
+  for (int32_t kb = kbeg; kb < kend; kb += B) {
+    double h1[B], h2[B];
 #pragma unroll
-    for (int w = 0; w < 8; ++w) c[w] = corners[min(kb + w, kend - 1)];  // past the end: unused
-    // A row's base is wave-uniform and the column the lane's offset.
-    const uint32_t lane = static_cast<uint32_t>(q);
-    double h[8][3];
-#pragma unroll
-    for (int w = 0; w < 8; ++w) {
-      h[w][0] = (heat + static_cast<int64_t>(c[w].y) * kk)[lane];
-      h[w][1] = (heat + static_cast<int64_t>(c[w].z) * kk)[lane];
-      h[w][2] = (heat + static_cast<int64_t>(c[w].w) * kk)[lane];
+    for (int w = 0; w < B; ++w) {
+      const int2 c = corner_rows[min(kb + w, kend - 1)];  // past the end: unused
+      h1[w] = (heat + static_cast<int64_t>(c.x) * kk)[lane];
+      h2[w] = (heat + static_cast<int64_t>(c.y) * kk)[lane];
     }
 #pragma unroll
-    for (int w = 0; w < 8; ++w) {
+    for (int w = 0; w < B; ++w) {
       if (kb + w >= kend) break;
-      const int32_t f = c[w].x / 3;
-      sum += corner_term(geom + kFaceGeom * static_cast<int64_t>(f), c[w].x - 3 * f, h[w][0],
-                         h[w][1], h[w][2]);
+      const double* g = geom + kCornerGeom * static_cast<int64_t>(kb + w);
+      sum += corner_term_2d(g[0], g[1], g[2], g[3], g[4], h1[w] - own, h2[w] - own);
     }
   }
   out[r * kk + q] = sum;
@@ -642,10 +724,13 @@ __global__ __launch_bounds__(256) void divergence_rows_kernel(
 
 // divergence_rows_kernel for kk <= 32 columns: 64 / kk rows a wave, lane l holding column l % kk
 // of row l / kk (lanes past the last whole row idle), so narrow batches keep their lanes busy.
-// Each lane walks its own row's corners four at a time (loads first, then the terms in ascending
-// corner order): the same terms in the same order as divergence_rows_kernel.
+// Each lane walks its own row's corners B at a time: the same terms in the same order. Six (a whole
+// interior row) from 8 columns on, four below, where a lane's records are its own run of memory. One
+// column on the 524,288-row torus: 51 us (six at a time 90, the faces' own arrays 72); 16 on
+// icosphere(9): 915 us (four at a time 1,110, the faces' own arrays 1,482).
+template <int B>
 __global__ __launch_bounds__(256) void divergence_rows_packed_kernel(
-    const int4* __restrict__ corners, const int32_t* __restrict__ corner_ptr,
+    const int2* __restrict__ corner_rows, const int32_t* __restrict__ corner_ptr,
     const double* __restrict__ geom, const double* __restrict__ heat, int64_t n, int32_t kk,
     double* __restrict__ out) {
   const int32_t per_wave = 64 / kk;
@@ -657,24 +742,29 @@ __global__ __launch_bounds__(256) void divergence_rows_packed_kernel(
   const int32_t q = lane % kk;
   if (sub >= per_wave || r >= n) return;
   const int32_t kbeg = corner_ptr[r], kend = corner_ptr[r + 1];
+  const double own = heat[r * kk + q];
   double sum = 0.0;
-  for (int32_t kb = kbeg; kb < kend; kb += 4) {
-    int4 c[4];
+  for (int32_t kb = kbeg; kb < kend; kb += B) {
+    double h1[B], h2[B], g[B][5];
+    int2 c[B];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) c[w] = corners[min(kb + w, kend - 1)];  // past the end: unused
-    double h[4][3];
+    for (int w = 0; w < B; ++w) c[w] = corner_rows[min(kb + w, kend - 1)];  // past the end: unused
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      h[w][0] = heat[static_cast<int64_t>(c[w].y) * kk + q];
-      h[w][1] = heat[static_cast<int64_t>(c[w].z) * kk + q];
-      h[w][2] = heat[static_cast<int64_t>(c[w].w) * kk + q];
+    for (int w = 0; w < B; ++w) {
+      const double* from = geom + kCornerGeom * static_cast<int64_t>(min(kb + w, kend - 1));
+#pragma unroll
+      for (int k = 0; k < 5; ++k) g[w][k] = from[k];
     }
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      if (kb + w >= kend) break;
-      const int32_t f = c[w].x / 3;
-      sum += corner_term(geom + kFaceGeom * static_cast<int64_t>(f), c[w].x - 3 * f, h[w][0],
-                         h[w][1], h[w][2]);
+    for (int w = 0; w < B; ++w) {
+      h1[w] = heat[static_cast<int64_t>(c[w].x) * kk + q];
+      h2[w] = heat[static_cast<int64_t>(c[w].y) * kk + q];
+    }
+#pragma unroll
+    for (int w = 0; w < B; ++w) {
+      const double term = corner_term_2d(g[w][0], g[w][1], g[w][2], g[w][3], g[w][4], h1[w] - own,
+                                         h2[w] - own);
+      if (kb + w < kend) sum += term;
     }
   }
   out[r * kk + q] = sum;
@@ -921,9 +1011,39 @@ void launch_face_geometry(const float* xyz, const int32_t* faces, const float* n
   HG_HIP(hipGetLastError());
 }
 
-void launch_divergence(const int32_t* faces, const int32_t* row_of, const double* geom,
-                       const int32_t* vertex_ptr, const int32_t* vertex_corners,
-                       const int4* row_corners, const int32_t* row_corner_ptr,
+void build_corner_rows(const int32_t* faces, const int32_t* vertex_ptr,
+                       const int32_t* vertex_corners, const int32_t* perm, const int32_t* iperm,
+                       int64_t n, int64_t n_faces, CornerRecords& out, hipStream_t stream) {
+  out.ptr.allocate(n + 1);
+  out.rows.allocate(std::max<int64_t>(3 * n_faces, 1));
+  DeviceArray<int32_t> counts(n + 1);
+  corner_counts_kernel<<<blocks_for(n + 1), kBlock, 0, stream>>>(vertex_ptr, perm, n, counts.ptr);
+  size_t bytes = 0;
+  HG_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, counts.ptr, out.ptr.ptr,
+                                          static_cast<int>(n + 1), stream));
+  DeviceArray<uint8_t> temp(static_cast<int64_t>(bytes));
+  HG_HIP(hipcub::DeviceScan::ExclusiveSum(temp.ptr, bytes, counts.ptr, out.ptr.ptr,
+                                          static_cast<int>(n + 1), stream));
+  if (n > 0)
+    corner_rows_kernel<<<blocks_for(n), kBlock, 0, stream>>>(faces, vertex_ptr, vertex_corners, perm,
+                                                             iperm, out.ptr.ptr, n, out.rows.ptr);
+  HG_HIP(hipGetLastError());
+  HG_HIP(hipStreamSynchronize(stream));  // the temporaries are freed on return
+}
+
+void build_corner_geometry(const float* normals, const double* face_geom,
+                           const int32_t* vertex_ptr, const int32_t* vertex_corners,
+                           const int32_t* perm, int64_t n, CornerRecords& out,
+                           hipStream_t stream) {
+  if (out.geom.size < kCornerGeom * out.rows.size) out.geom.allocate(kCornerGeom * out.rows.size);
+  if (n > 0)
+    corner_geometry_kernel<<<blocks_for(n), kBlock, 0, stream>>>(
+        normals, face_geom, vertex_ptr, vertex_corners, perm, out.ptr.ptr, n, out.geom.ptr);
+  HG_HIP(hipGetLastError());
+}
+
+void launch_divergence(const int32_t* faces, const double* geom, const int32_t* vertex_ptr,
+                       const int32_t* vertex_corners, const CornerRecords* records,
                        const double* heat, int64_t n, int64_t n_columns, double* out,
                        FieldLayout layout, hipStream_t stream) {
   if (n == 0 || n_columns == 0) return;
@@ -933,20 +1053,20 @@ void launch_divergence(const int32_t* faces, const int32_t* row_of, const double
       // A wave a row while at least half its lanes hold columns; 64 / kk rows a wave below.
       if (kk > kFieldChunk / 2) {
         divergence_rows_kernel<<<static_cast<unsigned>((n + 3) / 4), kBlock, 0, stream>>>(
-            row_corners, row_corner_ptr, geom, heat + c0 * n, n, kk, out + c0 * n);
+            records->rows.ptr, records->ptr.ptr, records->geom.ptr, heat + c0 * n, n, kk,
+            out + c0 * n);
       } else {
         const int64_t rows_per_block = 4 * (kFieldChunk / kk);
-        divergence_rows_packed_kernel<<<static_cast<unsigned>((n + rows_per_block - 1) /
-                                                              rows_per_block),
-                                        kBlock, 0, stream>>>(row_corners, row_corner_ptr, geom,
-                                                             heat + c0 * n, n,
-                                                             static_cast<int32_t>(kk),
-                                                             out + c0 * n);
+        auto kernel =
+            kk >= 8 ? divergence_rows_packed_kernel<6> : divergence_rows_packed_kernel<4>;
+        kernel<<<static_cast<unsigned>((n + rows_per_block - 1) / rows_per_block), kBlock, 0, stream>>>(
+            records->rows.ptr, records->ptr.ptr, records->geom.ptr, heat + c0 * n, n,
+            static_cast<int32_t>(kk), out + c0 * n);
       }
     }
   } else {
-    divergence_kernel<false><<<blocks_for(n * n_columns), kBlock, 0, stream>>>(
-        faces, geom, vertex_ptr, vertex_corners, nullptr, heat, n, n_columns, 1, n, out);
+    divergence_kernel<<<blocks_for(n * n_columns), kBlock, 0, stream>>>(
+        faces, geom, vertex_ptr, vertex_corners, heat, n, n_columns, 1, n, out);
   }
   HG_HIP(hipGetLastError());
 }

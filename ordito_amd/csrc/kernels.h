@@ -156,13 +156,28 @@ constexpr int64_t kFaceGeom = 15;
 void launch_face_geometry(const float* xyz, const int32_t* faces, const float* normals,
                           const float* areas, const float* cot, int64_t n_faces, double* geom,
                           hipStream_t stream);
-// -b per vertex and column from the heat (both in `layout`), gathered over each vertex's corners.
-// kRows: vertex v's row is row_of[v], `faces` name rows (row_of applied to every corner), and
-// row_corners[row_corner_ptr[r] ..] are row r's corners in ascending corner order, each
-// {corner id 3f + c, rows of face f's vertices 0, 1, 2}.
-void launch_divergence(const int32_t* faces, const int32_t* row_of, const double* geom,
-                       const int32_t* vertex_ptr, const int32_t* vertex_corners,
-                       const int4* row_corners, const int32_t* row_corner_ptr,
+// What the divergence of fields stored by rows reads (assembly.hip): row r's corners are records
+// ptr[r] .. ptr[r + 1], each the rows of its face's next and previous vertices and kCornerGeom
+// doubles. The rows follow the elimination order, the geometry the operators.
+constexpr int64_t kCornerGeom = 5;
+struct CornerRecords {
+  DeviceArray<int32_t> ptr;
+  DeviceArray<int2> rows;
+  DeviceArray<double> geom;
+  int64_t bytes() const { return ptr.bytes() + rows.bytes() + geom.bytes(); }
+};
+// Synchronizes the stream.
+void build_corner_rows(const int32_t* faces, const int32_t* vertex_ptr,
+                       const int32_t* vertex_corners, const int32_t* perm, const int32_t* iperm,
+                       int64_t n, int64_t n_faces, CornerRecords& out, hipStream_t stream);
+void build_corner_geometry(const float* normals, const double* face_geom,
+                           const int32_t* vertex_ptr, const int32_t* vertex_corners,
+                           const int32_t* perm, int64_t n, CornerRecords& out,
+                           hipStream_t stream);
+// -b per vertex and column from the heat (both in `layout`), gathered over each vertex's corners;
+// records: kRows only.
+void launch_divergence(const int32_t* faces, const double* geom, const int32_t* vertex_ptr,
+                       const int32_t* vertex_corners, const CornerRecords* records,
                        const double* heat, int64_t n, int64_t n_columns, double* out,
                        FieldLayout layout, hipStream_t stream);
 int32_t shift_partial_blocks(int64_t n);
