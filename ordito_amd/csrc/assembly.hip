@@ -599,8 +599,7 @@ __global__ __launch_bounds__(256) void divergence_kernel(
 // A1 on its first axis the corner needs A1 = (x1, 0), A2 = (x2, y2) and its integration vector
 // (gx, gy): five doubles in one run where the face's nine of fifteen were gathered, three products
 // for the gradient where there were six, and two neighbours' heat where there were three
-// vertices'. Both kernels wait on the neighbours' rows, which the caches serve but for about twice
-// the field (595 MB fetched for a field of 262 MB at 524,288 rows by 64 columns).
+// vertices'.
 
 // Row r's corner count, for the records' offsets.
 __global__ void corner_counts_kernel(const int32_t* __restrict__ vertex_ptr,
@@ -656,83 +655,74 @@ __global__ void corner_geometry_kernel(const float* __restrict__ normals,
     const double length = sqrt(dot(nrm, nrm));
     const D3 turn = length > 0.0 ? scale(1.0 / length, cross(nrm, axis)) : D3{0.0, 0.0, 0.0};
     double* out = geom + kCornerGeom * static_cast<int64_t>(corner_ptr[r] + k - first);
-    out[0] = along;
-    out[1] = dot(prev, axis);
-    out[2] = dot(prev, turn);
+    // Only the direction of the gradient counts: its basis is scaled by a power of two so that
+    // squares of heat differences from 2^-950 to 2^50 are normal numbers (a mesh a thousand edges
+    // across takes heat to 1e-300).
+    int power = 0;
+    (void)frexp(fmax(along, other), &power);
+    out[0] = ldexp(along, 450 - power);
+    out[1] = ldexp(dot(prev, axis), 450 - power);
+    out[2] = ldexp(dot(prev, turn), 450 - power);
     out[3] = dot(g, axis);
     out[4] = dot(g, turn);
   }
 }
 
-// corner_term in the corner's frame, for heat differences d1 and d2. Where the squared length is
-// far from both ends of the range the direction is normalized as it is: the scaling to its largest
-// component is by a power of two, which changes no bit of the result there, and it is a third of
-// the term's instructions. The rest (the far field of a large mesh, flat heat) is scaled.
-__device__ __forceinline__ double corner_term_2d(double x1, double x2, double y2, double gx,
-                                                 double gy, double d1, double d2) {
+// A corner's record in its plane's frame: x1, x2, y2, gx, gy.
+struct Corner {
+  double x1, x2, y2, gx, gy;
+};
+
+__device__ __forceinline__ Corner load_corner(const double* __restrict__ g) {
+  return Corner{g[0], g[1], g[2], g[3], g[4]};
+}
+
+// corner_term in the corner's frame, for heat differences d1 and d2, where the direction's squared
+// length is a normal number; normal says whether it is. The inverse length is the unit's estimate
+// and Householder's third-order step (no case of rsqrt's besides normal squares comes here).
+__device__ __forceinline__ double corner_term_fast(const Corner& c, double d1, double d2,
+                                                   bool& normal) {
 #pragma clang fp contract(fast)
-  const double sx = d1 * x1 + d2 * x2;
-  const double sy = d2 * y2;
+  const double sx = d1 * c.x1 + d2 * c.x2;
+  const double sy = d2 * c.y2;
   const double square = sx * sx + sy * sy;
-  double term = (gx * sx + gy * sy) * rsqrt(square);
-  if (!(square >= 0x1p-800 && square <= 0x1p800)) {
-    const double largest = fmax(fabs(sx), fabs(sy));
-    int e;
-    (void)frexp(largest, &e);
-    const double wx = ldexp(sx, -e), wy = ldexp(sy, -e);
-    term = largest == 0.0 ? 0.0 : (gx * wx + gy * wy) * rsqrt(wx * wx + wy * wy);
-  }
+  normal = __builtin_amdgcn_class(square, 0x100);
+  const double y = __builtin_amdgcn_rsq(square);
+  const double e = 1.0 - (square * y) * y;
+  return (c.gx * sx + c.gy * sy) * (y + (y * e) * (0.5 + 0.375 * e));
+}
+
+// The same for any direction, scaled first to its largest component (by a power of two: exact): flat
+// heat, and heat at the ends of the exponent's range.
+__device__ __forceinline__ double corner_term_scaled(const Corner& c, double d1, double d2) {
+#pragma clang fp contract(fast)
+  const double sx = d1 * c.x1 + d2 * c.x2;
+  const double sy = d2 * c.y2;
+  const double largest = fmax(fabs(sx), fabs(sy));
+  if (largest == 0.0) return 0.0;
+  int power;
+  (void)frexp(largest, &power);
+  const double wx = ldexp(sx, -power), wy = ldexp(sy, -power);
+  return (c.gx * wx + c.gy * wy) * rsqrt(wx * wx + wy * wy);
+}
+
+__device__ __forceinline__ double corner_term_2d(const Corner& c, double d1, double d2) {
+  bool normal;
+  double term = corner_term_fast(c, d1, d2, normal);
+  if (!normal) term = corner_term_scaled(c, d1, d2);
   return term;
 }
 
-// -b for a chunk of kk columns stored by rows, one wave a row of the elimination order (its lanes the
-// columns), its corners' records read as wave-uniform data, six at a time (a whole interior row of a
-// regular mesh): all the heat rows they name, then their terms in ascending corner order. The result
-// row is written contiguously. 64 columns on the 524,288-row torus: 359 us, 384 eight at a time, 512
-// from the faces' own arrays.
+// -b for up to three columns stored by rows: 64 / kk rows a wave, lane l holding column l % kk of row
+// l / kk (lanes past the last whole row idle). Each lane walks its row's corners in ascending order,
+// four at a time: their records, then the heat rows they name. A lane's records are its own run of
+// memory, which larger batches read apart (one column on the 524,288-row torus: 51 us, six at a time
+// 90, the faces' own arrays 72).
 __global__ __launch_bounds__(256) void divergence_rows_kernel(
-    const int2* __restrict__ corner_rows, const int32_t* __restrict__ corner_ptr,
-    const double* __restrict__ geom, const double* __restrict__ heat, int64_t n, int64_t kk,
-    double* __restrict__ out) {
-  constexpr int B = 6;
-  const int64_t r =
-      __builtin_amdgcn_readfirstlane(static_cast<int32_t>(xcd_block() * 4 + threadIdx.x / 64));
-  const int64_t q = threadIdx.x % 64;
-  if (r >= n || q >= kk) return;
-  const int32_t kbeg = corner_ptr[r], kend = corner_ptr[r + 1];
-  // A row's base is wave-uniform and the column the lane's offset.
-  const uint32_t lane = static_cast<uint32_t>(q);
-  const double own = (heat + r * kk)[lane];
-  double sum = 0.0;
-  for (int32_t kb = kbeg; kb < kend; kb += B) {
-    double h1[B], h2[B];
-#pragma unroll
-    for (int w = 0; w < B; ++w) {
-      const int2 c = corner_rows[min(kb + w, kend - 1)];  // past the end: unused
-      h1[w] = (heat + static_cast<int64_t>(c.x) * kk)[lane];
-      h2[w] = (heat + static_cast<int64_t>(c.y) * kk)[lane];
-    }
-#pragma unroll
-    for (int w = 0; w < B; ++w) {
-      if (kb + w >= kend) break;
-      const double* g = geom + kCornerGeom * static_cast<int64_t>(kb + w);
-      sum += corner_term_2d(g[0], g[1], g[2], g[3], g[4], h1[w] - own, h2[w] - own);
-    }
-  }
-  out[r * kk + q] = sum;
-}
-
-// divergence_rows_kernel for kk <= 32 columns: 64 / kk rows a wave, lane l holding column l % kk
-// of row l / kk (lanes past the last whole row idle), so narrow batches keep their lanes busy.
-// Each lane walks its own row's corners B at a time: the same terms in the same order. Six (a whole
-// interior row) from 8 columns on, four below, where a lane's records are its own run of memory. One
-// column on the 524,288-row torus: 51 us (six at a time 90, the faces' own arrays 72); 16 on
-// icosphere(9): 915 us (four at a time 1,110, the faces' own arrays 1,482).
-template <int B>
-__global__ __launch_bounds__(256) void divergence_rows_packed_kernel(
     const int2* __restrict__ corner_rows, const int32_t* __restrict__ corner_ptr,
     const double* __restrict__ geom, const double* __restrict__ heat, int64_t n, int32_t kk,
     double* __restrict__ out) {
+  constexpr int B = 4;
   const int32_t per_wave = 64 / kk;
   const int32_t lane = static_cast<int32_t>(threadIdx.x % 64);
   const int32_t sub = lane / kk;
@@ -762,12 +752,89 @@ __global__ __launch_bounds__(256) void divergence_rows_packed_kernel(
     }
 #pragma unroll
     for (int w = 0; w < B; ++w) {
-      const double term = corner_term_2d(g[w][0], g[w][1], g[w][2], g[w][3], g[w][4], h1[w] - own,
-                                         h2[w] - own);
+      const double term =
+          corner_term_2d(Corner{g[w][0], g[w][1], g[w][2], g[w][3], g[w][4]}, h1[w] - own, h2[w] - own);
       if (kb + w < kend) sum += term;
     }
   }
   out[r * kk + q] = sum;
+}
+
+// -b for four columns and more stored by rows: a lane holds two columns of a row (the last lane of an
+// odd number repeats one), a block the rows of pair_rows, whose corner records it first brings into LDS
+// (they lie in one run): loads of 16 bytes a lane for the heat rows and none of the records'. A block
+// of rows with more corners than it can hold reads the records where they lie. Six corners at a time (a
+// whole interior row), their heat rows all loaded before the first is used. Five blocks a unit: the
+// registers for six spill (842 us against 455 at 16 columns on icosphere(9)), four wait longer (543). 524,288-row
+// torus at 64 columns: 246 us (a lane a column, records through the scalar units: 359; the faces' own
+// arrays 512), of which the terms' arithmetic is about 150; 16 columns on icosphere(9): 455 (915,
+// 1,482).
+constexpr int kPairCorners = 480;
+
+__global__ __launch_bounds__(256, 5) void divergence_pairs_kernel(
+    const int2* __restrict__ corner_rows, const int32_t* __restrict__ corner_ptr,
+    const double* __restrict__ geom, const double* __restrict__ heat, int64_t n, int32_t kk,
+    int32_t rows, double* __restrict__ out) {
+  __shared__ int32_t ptr[kPairRows + 1];
+  __shared__ int2 named[kPairCorners];
+  __shared__ double staged[kCornerGeom * kPairCorners];
+  constexpr int B = 6;
+  const int32_t tid = static_cast<int32_t>(threadIdx.x);
+  const int64_t first = static_cast<int64_t>(xcd_block()) * rows;
+  const int32_t here = static_cast<int32_t>(min(static_cast<int64_t>(rows), n - first));
+  if (tid <= here) ptr[tid] = corner_ptr[first + tid];
+  const int32_t lanes = (kk + 1) / 2, per = 256 / lanes, s0 = tid / lanes;
+  const int32_t q = min(2 * (tid % lanes), kk - 2);
+  const bool takes = s0 < min(per, here);
+  Pair own0 = {0.0, 0.0};
+  if (takes) own0 = *reinterpret_cast<const Pair*>(heat + (first + s0) * kk + q);
+  __syncthreads();
+  const int32_t base = ptr[0], count = ptr[here] - base;
+  const bool fits = count <= kPairCorners;
+  if (fits) {
+    for (int32_t e = tid; e < count; e += 256) named[e] = corner_rows[base + e];
+    for (int32_t e = tid; e < kCornerGeom * count; e += 256)
+      staged[e] = geom[kCornerGeom * static_cast<int64_t>(base) + e];
+  }
+  __syncthreads();
+  auto row = [&](int32_t s, const int2* names, const double* g) {
+    const int64_t at = (first + s) * kk + q;
+    const Pair own = s == s0 ? own0 : *reinterpret_cast<const Pair*>(heat + at);
+    double sum0 = 0.0, sum1 = 0.0;
+    const int32_t kend = ptr[s + 1] - base;
+    for (int32_t kb = ptr[s] - base; kb < kend; kb += B) {
+      Pair h1[B], h2[B];
+#pragma unroll
+      for (int w = 0; w < B; ++w) {
+        const int2 c = names[min(kb + w, kend - 1)];  // past the end: unused
+        h1[w] = *reinterpret_cast<const Pair*>(heat + static_cast<int64_t>(c.x) * kk + q);
+        h2[w] = *reinterpret_cast<const Pair*>(heat + static_cast<int64_t>(c.y) * kk + q);
+      }
+#pragma unroll
+      for (int w = 0; w < B; ++w) {
+        if (kb + w >= kend) break;
+        const Corner c = load_corner(g + kCornerGeom * (kb + w));
+        bool normal0, normal1;
+        const double d1 = h1[w].x - own.x, d2 = h2[w].x - own.x;
+        const double e1 = h1[w].y - own.y, e2 = h2[w].y - own.y;
+        double t0 = corner_term_fast(c, d1, d2, normal0);
+        double t1 = corner_term_fast(c, e1, e2, normal1);
+        if (!(normal0 && normal1)) {
+          t0 = corner_term_scaled(c, d1, d2);
+          t1 = corner_term_scaled(c, e1, e2);
+        }
+        sum0 += t0;
+        sum1 += t1;
+      }
+    }
+    *reinterpret_cast<Pair*>(out + at) = Pair{sum0, sum1};
+  };
+  if (!takes) return;
+  if (fits)
+    for (int32_t s = s0; s < here; s += per) row(s, named, staged);
+  else
+    for (int32_t s = s0; s < here; s += per)
+      row(s, corner_rows + base, geom + kCornerGeom * static_cast<int64_t>(base));
 }
 
 // Columns of the shift: column q starts at col_off[q] and holds col_len[q] entries (packed meshes'
@@ -1050,16 +1117,17 @@ void launch_divergence(const int32_t* faces, const double* geom, const int32_t* 
   if (layout == FieldLayout::kRows) {
     for (int64_t c0 = 0; c0 < n_columns; c0 += kFieldChunk) {
       const int64_t kk = std::min<int64_t>(kFieldChunk, n_columns - c0);
-      // A wave a row while at least half its lanes hold columns; 64 / kk rows a wave below.
-      if (kk > kFieldChunk / 2) {
-        divergence_rows_kernel<<<static_cast<unsigned>((n + 3) / 4), kBlock, 0, stream>>>(
-            records->rows.ptr, records->ptr.ptr, records->geom.ptr, heat + c0 * n, n, kk,
-            out + c0 * n);
+      // Pairs from four columns on (on the 524,288-row torus 63 us against 72 there, 71 against 97 at
+      // 8; equal at three).
+      if (kk >= 4) {
+        const int32_t rows = pair_rows(static_cast<int32_t>(kk));
+        divergence_pairs_kernel<<<static_cast<unsigned>((n + rows - 1) / rows), kBlock, 0, stream>>>(
+            records->rows.ptr, records->ptr.ptr, records->geom.ptr, heat + c0 * n, n,
+            static_cast<int32_t>(kk), rows, out + c0 * n);
       } else {
         const int64_t rows_per_block = 4 * (kFieldChunk / kk);
-        auto kernel =
-            kk >= 8 ? divergence_rows_packed_kernel<6> : divergence_rows_packed_kernel<4>;
-        kernel<<<static_cast<unsigned>((n + rows_per_block - 1) / rows_per_block), kBlock, 0, stream>>>(
+        divergence_rows_kernel<<<static_cast<unsigned>((n + rows_per_block - 1) / rows_per_block),
+                                 kBlock, 0, stream>>>(
             records->rows.ptr, records->ptr.ptr, records->geom.ptr, heat + c0 * n, n,
             static_cast<int32_t>(kk), out + c0 * n);
       }

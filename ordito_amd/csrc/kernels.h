@@ -25,6 +25,21 @@ __device__ __forceinline__ int32_t xcd_block() {
   return xcd * per + min(xcd, extra) + b / 8;
 }
 
+// Two neighbouring columns of a field stored by rows (a row of an odd number of columns starts on a
+// multiple of 8 bytes only; gfx950 loads 16 from any multiple of 4). The passes that gather whole rows
+// of a field (the residual, the divergence) are held back by the rate at which the texture units take
+// loads, which is by four lanes a cycle whatever their size up to 16 bytes, so a lane loads a pair.
+typedef double Pair __attribute__((ext_vector_type(2), aligned(8)));
+
+// The rows a block of 256 threads takes there, for kk >= 3 columns: one a group of (kk + 1) / 2 lanes,
+// and at least 32 in turn, so that what the rows name is staged in LDS by runs worth a load of every
+// thread (64 columns, the divergence of 524,288 rows: 246 us; eight rows a block 275).
+constexpr int32_t kPairRows = 128;
+inline int32_t pair_rows(int32_t kk) {
+  const int32_t at_once = 256 / ((kk + 1) / 2);
+  return at_once * std::max(1, (31 + at_once) / at_once);
+}
+
 // Device time of the phases of a solve, from HIP events on the stream the work is issued on.
 enum Phase : int {
   kPhaseFactor = 0,

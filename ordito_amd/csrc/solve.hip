@@ -644,14 +644,6 @@ __global__ __launch_bounds__(256) void bwd_reduce_kernel(const int4* __restrict_
 // Raises *flag once per block that fails, and not at all once the flag reads set: with every row
 // failing in a solve's first rounds, an atomic a wave on one word serializes the whole launch.
 // Block-collective.
-// Lane `lane`'s double, as a wave-uniform value.
-__device__ __forceinline__ double readlane_f64(double v, int lane) {
-  const uint64_t bits = __builtin_bit_cast(uint64_t, v);
-  const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(bits), lane);
-  const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(bits >> 32), lane);
-  return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
-}
-
 __device__ __forceinline__ void raise_flag(bool fail, int32_t* flag) {
   const int any = __syncthreads_or(fail ? 1 : 0);
   if (any && threadIdx.x == 0 &&
@@ -662,10 +654,7 @@ __device__ __forceinline__ void raise_flag(bool fail, int32_t* flag) {
 // r = b - A x in the elimination order and whether any row is still above tolerance
 // (componentwise against (|A||x| + |b|)_i, normwise against the larger of that and the column's
 // largest |b|; kernels/cholesky.py:1393-1440). Pinned rows are dropped. One thread a (row,
-// right-hand side); the row's operator entries are shared by its kk threads.
-// kWaveRow: kk is the full 64, so each wave holds one row and the row's offsets, columns and
-// values are wave-uniform (read once per wave through the scalar unit).
-template <bool kWaveRow>
+// right-hand side), for one and two right-hand sides.
 __global__ void residual_kernel(const int32_t* __restrict__ offsets,
                                 const int32_t* __restrict__ columns,
                                 const double* __restrict__ values, const double* __restrict__ b,
@@ -676,8 +665,7 @@ __global__ void residual_kernel(const int32_t* __restrict__ offsets,
   int64_t t = static_cast<int64_t>(xcd_block()) * blockDim.x + threadIdx.x;
   bool fail = false;
   if (t < n * kk) {
-    const int64_t i =
-        kWaveRow ? __builtin_amdgcn_readfirstlane(static_cast<int32_t>(t / kCols)) : t / kk;
+    const int64_t i = t / kk;
     const int64_t q = t % kk;
     const double bi = b[t];
     const bool dropped = pinned && pinned[i];
@@ -685,28 +673,16 @@ __global__ void residual_kernel(const int32_t* __restrict__ offsets,
     double total = bi, scale = fabs(bi);
     // Eight entries at a time (a row of a triangle mesh has about seven): their column and value
     // loads, then their iterate loads, issue together; entries past the row's end repeat its last
-    // one and are not added, and the sums stay in entry order. A wave on one row loads the eight
-    // columns and values in its first lanes at once and reads them out lane by lane.
+    // one and are not added, and the sums stay in entry order.
     const int32_t e0 = offsets[i], e1 = offsets[i + 1];
     for (int32_t e = e0; e < e1; e += 8) {
       int32_t c[8];
       double v[8], xv[8];
-      if (kWaveRow) {
-        const int32_t at = min(e + static_cast<int32_t>(threadIdx.x % 8), e1 - 1);
-        const int32_t lane_c = columns[at];
-        const double lane_v = values[at];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          c[u] = __builtin_amdgcn_readlane(lane_c, u);
-          v[u] = readlane_f64(lane_v, u);
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int32_t at = min(e + u, e1 - 1);
-          c[u] = columns[at];
-          v[u] = values[at];
-        }
+      for (int u = 0; u < 8; ++u) {
+        const int32_t at = min(e + u, e1 - 1);
+        c[u] = columns[at];
+        v[u] = values[at];
       }
 #pragma unroll
       for (int u = 0; u < 8; ++u) xv[u] = x[static_cast<int64_t>(c[u]) * kk + q];
@@ -724,78 +700,81 @@ __global__ void residual_kernel(const int32_t* __restrict__ offsets,
   raise_flag(fail, pending);
 }
 
-// The residual of residual_kernel for 64 right-hand sides, kRowsPerWave rows a wave: a lane is a
-// right-hand side of each of its wave's rows. Every round of loads covers all the wave's rows
-// (their offsets; then eight entries of each, columns and values loaded lane-parallel and read out
-// lane by lane; then every iterate entry they name), so a wave keeps several rows' loads in flight
-// where one row would wait on three dependent rounds alone. Sums keep entry order.
-constexpr int kRowsPerWave = 4;
-
-__global__ __launch_bounds__(256) void residual_rows_kernel(
+// The residual of residual_kernel for three right-hand sides and more: a lane holds two columns of a
+// row (the last lane of an odd number repeats one), a block the rows of pair_rows, whose entries it
+// first brings into LDS (they lie in one run); a block of rows with more entries than it can hold reads
+// them where they lie. A thread's first row of the right-hand side and of the iterate are loaded before
+// the entries are (the iterate's for the caches alone: its row is some row's entry), which hides part of
+// the chain offsets, entries, iterate (icosphere(9) at 16 columns: 267 us against 286). Sums keep entry
+// order. 524,288-row torus: 32 columns 105 us (a lane a column 204), 64 columns 197 (214), where the
+// rows fetched twice from beyond L2 hold it (850 MB at 4.4 TB/s; 570 are needed).
+constexpr int32_t kPairEntries = 1024;
+__global__ __launch_bounds__(256) void residual_pairs_kernel(
     const int32_t* __restrict__ offsets, const int32_t* __restrict__ columns,
     const double* __restrict__ values, const double* __restrict__ b,
     const double* __restrict__ x, const int32_t* __restrict__ pinned,
-    const double* __restrict__ bmax, int64_t n, double tolerance, int32_t componentwise,
-    double* __restrict__ r, int32_t* __restrict__ pending) {
-  constexpr int R = kRowsPerWave;
-  const int32_t lane = static_cast<int32_t>(threadIdx.x % 64);
-  const int64_t first = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(
-                            static_cast<int32_t>(xcd_block() * 4 + threadIdx.x / 64))) * R;
-  const double bscale = componentwise ? 0.0 : bmax[lane];
-  int32_t e0[R], e1[R];
-  double bi[R], total[R], scale[R];
-  bool dropped[R];
-#pragma unroll
-  for (int u = 0; u < R; ++u) {
-    const int64_t i = first + u;
-    const bool live = i < n;
-    e0[u] = live ? offsets[i] : 0;
-    e1[u] = live ? offsets[i + 1] : 0;
-    bi[u] = live ? b[i * kCols + lane] : 0.0;
-    dropped[u] = !live || (pinned && pinned[i]);
-    total[u] = bi[u];
-    scale[u] = fabs(bi[u]);
+    const double* __restrict__ bmax, int64_t n, int32_t kk, int32_t rows, double tolerance,
+    int32_t componentwise, double* __restrict__ r, int32_t* __restrict__ pending) {
+  __shared__ int32_t ptr[kPairRows + 1];
+  __shared__ int32_t named[kPairEntries];
+  __shared__ double staged[kPairEntries];
+  constexpr int B = 8;
+  const int32_t tid = static_cast<int32_t>(threadIdx.x);
+  const int64_t first = static_cast<int64_t>(xcd_block()) * rows;
+  const int32_t here = static_cast<int32_t>(min(static_cast<int64_t>(rows), n - first));
+  if (tid <= here) ptr[tid] = offsets[first + tid];
+  const int32_t lanes = (kk + 1) / 2, per = 256 / lanes, s0 = tid / lanes;
+  const int32_t q = min(2 * (tid % lanes), kk - 2);
+  const bool takes = s0 < min(per, here);
+  Pair b0 = {0.0, 0.0}, x0 = {0.0, 0.0};
+  if (takes) {
+    b0 = __builtin_nontemporal_load(reinterpret_cast<const Pair*>(b + (first + s0) * kk + q));
+    x0 = *reinterpret_cast<const Pair*>(x + (first + s0) * kk + q);
   }
-  for (int32_t base = 0;; base += 8) {
-    bool more = false;
-#pragma unroll
-    for (int u = 0; u < R; ++u) more |= e0[u] + base < e1[u];
-    if (!more) break;  // wave-uniform
-    // Lane 8u + j loads entry base + j of row u (an entry past the row's end, or of an empty
-    // row, reads one in range and is not added).
-    const int u_lane = min(lane / 8, R - 1);
-    int32_t at = e0[0];
-#pragma unroll
-    for (int u = 0; u < R; ++u)
-      if (u == u_lane) at = e1[u] > e0[u] ? min(e0[u] + base + lane % 8, e1[u] - 1) : 0;
-    const int32_t lane_c = columns[at];
-    const double lane_v = values[at];
-    double xv[R][8];
-#pragma unroll
-    for (int u = 0; u < R; ++u)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int32_t c = __builtin_amdgcn_readlane(lane_c, 8 * u + j);
-        xv[u][j] = x[static_cast<int64_t>(c) * kCols + lane];
-      }
-#pragma unroll
-    for (int u = 0; u < R; ++u)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const double v = readlane_f64(lane_v, 8 * u + j);
-        const double term = e0[u] + base + j < e1[u] ? v * xv[u][j] : 0.0;
-        total[u] -= term;
-        scale[u] += fabs(term);
-      }
-  }
+  __syncthreads();
+  const int32_t base = ptr[0], count = ptr[here] - base;
+  const bool fits = count <= kPairEntries;
+  if (fits)
+    for (int32_t e = tid; e < count; e += 256) {
+      named[e] = columns[base + e];
+      staged[e] = values[base + e];
+    }
+  __syncthreads();
+  asm volatile("" ::"v"(x0));  // loaded, though nothing takes its value
+  const Pair bscale = componentwise ? Pair{0.0, 0.0} : *reinterpret_cast<const Pair*>(bmax + q);
   bool fail = false;
+  auto row = [&](int32_t s, const int32_t* names, const double* v) {
+    const int64_t i = first + s, at = i * kk + q;
+    Pair total = s == s0 ? b0 : __builtin_nontemporal_load(reinterpret_cast<const Pair*>(b + at));
+    Pair scale = {fabs(total.x), fabs(total.y)};
+    const bool dropped = pinned && pinned[i];
+    const int32_t e1 = ptr[s + 1] - base;
+    for (int32_t e = ptr[s] - base; e < e1; e += B) {
+      Pair xv[B];
 #pragma unroll
-  for (int u = 0; u < R; ++u) {
-    const int64_t i = first + u;
-    if (i >= n) continue;
-    if (r) r[i * kCols + lane] = dropped[u] ? 0.0 : total[u];
-    const double sc = componentwise ? scale[u] : fmax(scale[u], bscale);
-    fail |= !dropped[u] && !(fabs(total[u]) <= tolerance * sc);
+      for (int u = 0; u < B; ++u)
+        xv[u] = *reinterpret_cast<const Pair*>(
+            x + static_cast<int64_t>(names[min(e + u, e1 - 1)]) * kk + q);
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        if (e + u >= e1) break;
+        const double a = v[e + u];
+        const double t0 = a * xv[u].x, t1 = a * xv[u].y;
+        total.x -= t0;
+        total.y -= t1;
+        scale.x += fabs(t0);
+        scale.y += fabs(t1);
+      }
+    }
+    if (r) *reinterpret_cast<Pair*>(r + at) = dropped ? Pair{0.0, 0.0} : total;
+    fail |= !dropped && !(fabs(total.x) <= tolerance * fmax(scale.x, bscale.x) &&
+                          fabs(total.y) <= tolerance * fmax(scale.y, bscale.y));
+  };
+  if (takes) {
+    if (fits)
+      for (int32_t s = s0; s < here; s += per) row(s, named, staged);
+    else
+      for (int32_t s = s0; s < here; s += per) row(s, columns + base, values + base);
   }
   raise_flag(fail, pending);
 }
@@ -1318,17 +1297,18 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
       // the test alone and written (a second pass) only when another round follows.
       const bool test_only = !use_fp32 && rounds == 1;
       auto residual = [&](double* r_out) {
-        if (kk == kCols)
-          residual_rows_kernel<<<static_cast<unsigned>((n + 4 * kRowsPerWave - 1) /
-                                                       (4 * kRowsPerWave)),
-                                 256, 0, stream>>>(plan.p_offsets.ptr, plan.p_columns.ptr,
-                                                   factor.pvalues.ptr, bp, x_cur, pinned_new,
-                                                   bmax, n, tolerance, componentwise ? 1 : 0,
-                                                   r_out, ws.pending.ptr);
-        else
-          residual_kernel<false><<<grid, 256, 0, stream>>>(
+        // Pairs from three columns on (on the 524,288-row torus 46 us for two against 63, 47 against 67
+        // at four; the rows' entries read once a column below).
+        if (kk >= 3) {
+          const int32_t rows = pair_rows(kk);
+          residual_pairs_kernel<<<static_cast<unsigned>((n + rows - 1) / rows), 256, 0, stream>>>(
+              plan.p_offsets.ptr, plan.p_columns.ptr, factor.pvalues.ptr, bp, x_cur, pinned_new,
+              bmax, n, kk, rows, tolerance, componentwise ? 1 : 0, r_out, ws.pending.ptr);
+        } else {
+          residual_kernel<<<grid, 256, 0, stream>>>(
               plan.p_offsets.ptr, plan.p_columns.ptr, factor.pvalues.ptr, bp, x_cur, pinned_new,
               bmax, n, kk, tolerance, componentwise ? 1 : 0, r_out, ws.pending.ptr);
+        }
       };
       {
         PhaseScope scope(timer, kPhaseResidual, stream);
