@@ -905,56 +905,81 @@ __global__ void component_shift_kernel(const int32_t* __restrict__ chunk_comp,
 // its own and numbered in component order), so the null-space chunks (256 members of one
 // component) are row ranges too: chunk k covers rows [chunk_first[k], min(+256, comp end)).
 
-// Column sums over each chunk: thread (q, part) adds rows part, part + 4, ... (four loads issued
-// before their adds), then the four parts add in order. partials[q * n_chunks + k], the layout
-// component_mean_kernel reads.
+// Column sums over each chunk: a lane holds two columns of a row (one column: one row a thread), whose
+// rows are added in turn, then over the block. partials[q * n_chunks + k], the layout
+// component_mean_kernel reads. 16 columns on icosphere(9): 55 us (a lane a column of 64: 116).
 __global__ __launch_bounds__(256) void rows_partial_kernel(const int32_t* __restrict__ chunk_comp,
                                                            const int32_t* __restrict__ chunk_first,
                                                            const int32_t* __restrict__ comp_ptr,
                                                            const double* __restrict__ x,
                                                            int32_t kk,
                                                            double* __restrict__ partials) {
-  __shared__ double part_sum[4][kCols];
-  const int32_t chunk = blockIdx.x;
+  __shared__ Pair part[256];
+  const int32_t chunk = blockIdx.x, tid = static_cast<int32_t>(threadIdx.x);
   const int32_t first = chunk_first[chunk];
   const int32_t end = min(first + 256, comp_ptr[chunk_comp[chunk] + 1]);
-  const int q = threadIdx.x % kCols, part = threadIdx.x / kCols;
-  double sum = 0.0;
-  if (q < kk) {
-    int32_t r = first + part;
-    for (; r + 12 < end; r += 16) {
-      double v[4];
+  const int32_t lanes = (kk + 1) / 2, per = 256 / lanes, s = tid / lanes;
+  const int32_t q = max(min(2 * (tid % lanes), kk - 2), 0);
+  Pair sum = {0.0, 0.0};
+  if (kk == 1) {
+    if (first + s < end) sum.x = x[first + s];
+  } else if (s < per) {
+    for (int32_t r = first + s; r < end; r += 8 * per) {
+      Pair v[8];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = x[static_cast<int64_t>(r + 4 * u) * kk + q];
+      for (int u = 0; u < 8; ++u)
+        v[u] = *reinterpret_cast<const Pair*>(
+            x + static_cast<int64_t>(min(r + u * per, end - 1)) * kk + q);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) sum += v[u];
+      for (int u = 0; u < 8; ++u)
+        if (r + u * per < end) sum += v[u];
     }
-    for (; r < end; r += 4) sum += x[static_cast<int64_t>(r) * kk + q];
   }
-  part_sum[part][q] = sum;
-  __syncthreads();
-  if (part == 0)
-    partials[static_cast<int64_t>(q) * gridDim.x + chunk] =
-        ((part_sum[0][q] + part_sum[1][q]) + part_sum[2][q]) + part_sum[3][q];
+  part[tid] = sum;
+  for (int32_t c = per; c > 1;) {
+    const int32_t half = (c + 1) / 2;
+    __syncthreads();
+    if (s < c - half) part[tid] += part[tid + half * lanes];
+    c = half;
+  }
+  if (s > 0) return;
+  partials[static_cast<int64_t>(q) * gridDim.x + chunk] = part[tid].x;
+  if (kk > 1) partials[static_cast<int64_t>(q + 1) * gridDim.x + chunk] = part[tid].y;
 }
 
 // One block per column q, after each component's mean (component_mean_kernel,
 // kernels/cholesky.py:1467-1660): the shift of the mean-removed field (kernels/heat.py:3383-3424),
 // offset = its mean over the column's sources (vertex v at row iperm[v]), negated when its mean
 // over every vertex (the chunks' sums less their share of the means) is below the offset.
-// shift[2q] = offset, shift[2q + 1] = 1 to negate.
+// shift[2q] = offset, shift[2q + 1] = 1 to negate. own_mean: the one component's mean is formed here
+// too (a launch less: 4.7 us of a small call), and left in means.
 __global__ __launch_bounds__(256) void rows_decide_kernel(
     const int32_t* __restrict__ comp_ptr, const int32_t* __restrict__ chunk_comp,
     const int32_t* __restrict__ chunk_first, int32_t n_comp, int32_t n_chunks,
-    const double* __restrict__ partials, const double* __restrict__ means,
+    const double* __restrict__ partials, double* means, bool own_mean,
     const double* __restrict__ x, int32_t kk, int64_t n, const int32_t* __restrict__ iperm,
     const int32_t* __restrict__ labels, const int32_t* __restrict__ sources,
     const int64_t* __restrict__ source_offsets, double* __restrict__ shift) {
   __shared__ double s_total[256];
   __shared__ double s_src[256];
   const int q = blockIdx.x, t = threadIdx.x;
-  const double* mean = means + static_cast<int64_t>(q) * n_comp;
+  double* mean = means + static_cast<int64_t>(q) * n_comp;
+  if (own_mean) {
+    double sum = 0.0;
+#pragma unroll 8
+    for (int32_t k = t; k < n_chunks; k += 256)
+      sum += partials[static_cast<int64_t>(q) * n_chunks + k];
+    s_total[t] = sum;
+    __syncthreads();
+    for (int stride = 128; stride > 0; stride >>= 1) {
+      if (t < stride) s_total[t] += s_total[t + stride];
+      __syncthreads();
+    }
+    if (t == 0) mean[0] = s_total[0] / static_cast<double>(comp_ptr[1] - comp_ptr[0]);
+    __syncthreads();
+  }
   double total = 0.0;
+#pragma unroll 4
   for (int32_t k = t; k < n_chunks; k += 256) {
     const int32_t c = chunk_comp[k];
     const int32_t len = min(256, comp_ptr[c + 1] - chunk_first[k]);
@@ -988,7 +1013,10 @@ __global__ __launch_bounds__(256) void rows_decide_kernel(
 
 // The distance in the caller's layout (column q at q * n): vertex v's entry is the mean-removed
 // value at row iperm[v], shifted and oriented. 64 vertices a block, transposed through LDS so the
-// row reads and the column writes are both contiguous.
+// row reads and the column writes are both contiguous: a lane reads two columns of each of its rows,
+// all of them before any is used, and the tile is W columns wide (16, 32 or 64: a wider one than the
+// chunk keeps blocks off the unit). 16 columns on icosphere(9): 131 us (64 wide, an element a lane: 275).
+template <int W>
 __global__ __launch_bounds__(256) void rows_out_kernel(const double* __restrict__ x, int32_t kk,
                                                        int64_t n, const int32_t* __restrict__ iperm,
                                                        const int32_t* __restrict__ labels,
@@ -996,37 +1024,40 @@ __global__ __launch_bounds__(256) void rows_out_kernel(const double* __restrict_
                                                        const double* __restrict__ means,
                                                        const double* __restrict__ shift,
                                                        double* const* __restrict__ out_slot) {
-  __shared__ double tile[kTile][kCols + 1];
+  constexpr int kTurns = W / 8;  // rows a thread takes: 64 over the 256 / (W / 2) read at once
+  __shared__ double tile[kTile][W + 1];
   double* __restrict__ out = *out_slot;
   const int64_t v0 = static_cast<int64_t>(blockIdx.x) * kTile;
   const int32_t rows = static_cast<int32_t>(min<int64_t>(kTile, n - v0));
-  if (kk == kCols) {
-    // A lane is a column q; wave w reads rows w, w + 4, ... (each a contiguous row of x), all
-    // sixteen rows' loads issued before any is used.
-    const int q = threadIdx.x % kCols, w = threadIdx.x / kCols;
-    const double offset = shift[2 * q];
-    const bool flip = shift[2 * q + 1] != 0.0;
-    double xv[kTile / 4], mv[kTile / 4];
+  const int32_t tid = static_cast<int32_t>(threadIdx.x);
+  if (kk == 1) {
+    if (tid < rows) {
+      const double value = x[iperm[v0 + tid]] - means[n_comp > 1 ? labels[v0 + tid] : 0];
+      out[v0 + tid] = shift[1] != 0.0 ? shift[0] - value : value - shift[0];
+    }
+    return;
+  }
+  const int32_t lanes = (kk + 1) / 2, per = 256 / lanes, s = tid / lanes;
+  const int32_t q = min(2 * (tid % lanes), kk - 2);
+  if (s < per) {
+    const double offset0 = shift[2 * q], offset1 = shift[2 * q + 2];
+    const bool flip0 = shift[2 * q + 1] != 0.0, flip1 = shift[2 * q + 3] != 0.0;
+    Pair xv[kTurns], mv[kTurns];
 #pragma unroll
-    for (int j = 0; j < kTile / 4; ++j) {
-      const int lv = w + 4 * j;
-      const int64_t v = v0 + min(lv, rows - 1);
-      xv[j] = x[static_cast<int64_t>(iperm[v]) * kCols + q];
-      mv[j] = means[static_cast<int64_t>(q) * n_comp + labels[v]];
+    for (int j = 0; j < kTurns; ++j) {
+      const int64_t v = v0 + min(s + j * per, rows - 1);
+      xv[j] = *reinterpret_cast<const Pair*>(x + static_cast<int64_t>(iperm[v]) * kk + q);
+      const int32_t c = n_comp > 1 ? labels[v] : 0;
+      mv[j] = Pair{means[static_cast<int64_t>(q) * n_comp + c],
+                   means[static_cast<int64_t>(q + 1) * n_comp + c]};
     }
 #pragma unroll
-    for (int j = 0; j < kTile / 4; ++j) {
-      const double value = xv[j] - mv[j];
-      tile[w + 4 * j][q] = flip ? offset - value : value - offset;
-    }
-  } else {
-    for (int e = threadIdx.x; e < rows * kk; e += 256) {
-      const int lv = e / kk, q = e % kk;
-      const int64_t v = v0 + lv;
-      const double value = x[static_cast<int64_t>(iperm[v]) * kk + q] -
-                           means[static_cast<int64_t>(q) * n_comp + labels[v]];
-      const double offset = shift[2 * q];
-      tile[lv][q] = shift[2 * q + 1] != 0.0 ? offset - value : value - offset;
+    for (int j = 0; j < kTurns; ++j) {
+      const int32_t lv = s + j * per;
+      if (lv >= rows) break;
+      const Pair value = xv[j] - mv[j];
+      tile[lv][q] = flip0 ? offset0 - value.x : value.x - offset0;
+      tile[lv][q + 1] = flip1 ? offset1 - value.y : value.y - offset1;
     }
   }
   __syncthreads();
@@ -1056,7 +1087,8 @@ __global__ __launch_bounds__(256) void mark_fronts_kernel(
 }
 
 // The gather pairs of the live fronts' rows, without the contributions of fronts that are not. A wave
-// a front.
+// a front, eight of each lane's rows at a time: the largest fronts, a thousand rows and more, are
+// the launch's length (one source on icosphere(7): 21.5 us a row a lane at a time, 10.4 so; 16 on icosphere(9) 84 and 40).
 __global__ __launch_bounds__(256) void live_pairs_kernel(
     const int32_t* __restrict__ live, const int32_t* __restrict__ ncol,
     const int32_t* __restrict__ nrow, const int64_t* __restrict__ vec_off,
@@ -1066,11 +1098,26 @@ __global__ __launch_bounds__(256) void live_pairs_kernel(
   if (s >= n_super || !live[s]) return;
   const int64_t base = vec_off[s];
   const int32_t m = ncol[s] + nrow[s];
-  for (int32_t i = static_cast<int32_t>(threadIdx.x) % 64; i < m; i += 64) {
-    int2 p = pairs[base + i];
-    if (p.x >= 0 && !live[vec_front[p.x]]) p.x = -1;
-    if (p.y >= 0 && !live[vec_front[p.y]]) p.y = -1;
-    out[base + i] = p;
+  constexpr int U = 8;
+  for (int32_t i = static_cast<int32_t>(threadIdx.x) % 64; i < m; i += 64 * U) {
+    int2 p[U];
+    int32_t fx[U], fy[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) p[u] = pairs[base + min(i + 64 * u, m - 1)];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      fx[u] = p[u].x >= 0 ? vec_front[p[u].x] : s;  // the front itself is live
+      fy[u] = p[u].y >= 0 ? vec_front[p[u].y] : s;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      fx[u] = live[fx[u]];
+      fy[u] = live[fy[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i + 64 * u < m)
+        out[base + i + 64 * u] = make_int2(fx[u] ? p[u].x : -1, fy[u] ? p[u].y : -1);
   }
 }
 
@@ -1400,16 +1447,18 @@ void finish_rows(const DevicePlan& plan, const NullSpace& ns, const int32_t* com
     const double* xq = x + q0 * n;
     rows_partial_kernel<<<static_cast<unsigned>(ns.n_chunks), 256, 0, stream>>>(
         ns.chunk_comp.ptr, ns.chunk_first.ptr, comp_ptr, xq, kk, partials);
-    if (remove_means)
+    const bool own_mean = remove_means && ns.n_comp == 1;
+    if (remove_means && !own_mean)
       component_mean_kernel<<<dim3(static_cast<unsigned>(ns.n_comp), static_cast<unsigned>(kk)),
                               256, 0, stream>>>(ns.comp_chunk_ptr.ptr, comp_ptr, ns.n_chunks,
                                                 partials, means);
-    else
+    else if (!remove_means)
       launch_zero(means, static_cast<int64_t>(sizeof(double)) * ns.n_comp * kk, stream);
     rows_decide_kernel<<<static_cast<unsigned>(kk), 256, 0, stream>>>(
         comp_ptr, ns.chunk_comp.ptr, ns.chunk_first.ptr, ns.n_comp, ns.n_chunks, partials, means,
-        xq, kk, n, plan.iperm.ptr, labels, sources, source_offsets + q0, shift);
-    rows_out_kernel<<<static_cast<unsigned>((n + kTile - 1) / kTile), 256, 0, stream>>>(
+        own_mean, xq, kk, n, plan.iperm.ptr, labels, sources, source_offsets + q0, shift);
+    auto out = kk <= 16 ? rows_out_kernel<16> : kk <= 32 ? rows_out_kernel<32> : rows_out_kernel<64>;
+    out<<<static_cast<unsigned>((n + kTile - 1) / kTile), 256, 0, stream>>>(
         xq, kk, n, plan.iperm.ptr, labels, ns.n_comp, means, shift, out_slots + q0 / kCols);
   }
   HG_HIP(hipGetLastError());
