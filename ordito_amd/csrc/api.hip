@@ -135,7 +135,7 @@ struct hg_mesh {
   SolveWorkspace solve;
   SolveWorkspace solve_side;  // the rim-pinned heat solve's, when it runs beside the Neumann one
   bool on_side = false;       // the solves being enqueued use solve_side
-  DeviceArray<double> fields, shift_partials, shift_values, null_partials;
+  DeviceArray<double> fields, shift_partials, shift_values, null_partials, maxima;
   NullSpace null_space;
   DeviceArray<int32_t> d_sources, invalid;
   PinnedArray<int32_t> h_invalid;  // the seeds' range flag, read back with the call's last sync
@@ -223,7 +223,7 @@ int64_t mesh_device_bytes(const hg_mesh& m) {
        {&m.mass, &m.lap, &m.heat, &m.poisson, &m.heat_inv, &m.poisson_inv, &m.scalars,
         &m.edge_partials, &m.face_geom, &m.pinned, &m.pinned_inv, &m.pinned_rhs, &m.reg,
         &m.reg_inv, &m.fields,
-        &m.shift_partials, &m.shift_values, &m.null_partials, &m.packed_phi})
+        &m.shift_partials, &m.shift_values, &m.null_partials, &m.maxima, &m.packed_phi})
     total += a->bytes();
   for (const DeviceArray<int64_t>* a : {&m.d_owner, &m.d_offsets, &m.q_src_off, &m.q_dst_off,
                                         &m.q_len})
@@ -255,6 +255,7 @@ void release_workspaces(hg_mesh& m) {
   m.shift_partials.reset();
   m.shift_values.reset();
   m.null_partials.reset();
+  m.maxima.reset();
 }
 
 // ---- operators --------------------------------------------------------------------------------
@@ -750,6 +751,12 @@ double dominance_bound(hg_mesh& m, const double* values, double& cached) {
   return cached;
 }
 
+// The Poisson system's pinned rows in the elimination order (null: none).
+const int32_t* poisson_pins(const hg_mesh& m, bool regularized) {
+  if (!regularized) return m.poisson_pinned_new.ptr;
+  return m.has_heat_pins ? m.heat_pinned_new.ptr : nullptr;
+}
+
 // The right-hand side and the solution may be stored by rows (factored only). A solution stored by
 // columns has each component's mean removed here; one stored by rows is left for finish_rows.
 // `regularized` solves HG_METHOD_POTPOURRI3D's -L + 1e-6 I instead of -L: no null space, its
@@ -764,8 +771,7 @@ void solve_poisson(hg_mesh& m, double* rhs, double* x, int64_t k, int32_t mode,
   Factor& factor = regularized ? m.reg_factor : m.poisson_factor;
   const double* values = regularized ? m.reg.ptr : m.poisson.ptr;
   const double* inv_diag = regularized ? m.reg_inv.ptr : m.poisson_inv.ptr;
-  const int32_t* pins = regularized ? (m.has_heat_pins ? m.heat_pinned_new.ptr : nullptr)
-                                    : m.poisson_pinned_new.ptr;
+  const int32_t* pins = poisson_pins(m, regularized);
   bool factored = mode == HG_MODE_FACTORED || factor.held() || m.heat_factor.held();
   if (factored && rhs_layout == FieldLayout::kColumns && x_layout == FieldLayout::kColumns) {
     // By columns a refusal under the budget leaves the solve to the iteration.
@@ -782,7 +788,7 @@ void solve_poisson(hg_mesh& m, double* rhs, double* x, int64_t k, int32_t mode,
         *m.plan, factor, mixed, rhs, x, k, m.refine_tolerance[mixed ? 1 : 0][1], false,
         mixed ? kMixedRefineRounds : kRefineRounds, pins, m.solve, m.stream, &m.timer,
         kPhasePoissonSweep, rhs_layout, x_layout,
-        m.speculating ? m.h_speculate.ptr + 2 * m.spec_chunks : nullptr);
+        m.speculating ? m.h_speculate.ptr + 2 * m.spec_chunks : nullptr, nullptr, m.maxima.ptr);
     m.stats.poisson_rounds = 0;
   } else {
     HG_REQUIRE(rhs_layout == FieldLayout::kColumns && x_layout == FieldLayout::kColumns,
@@ -906,11 +912,13 @@ void check_seeds(const hg_mesh& m) {
              "every entry of sources must be a vertex index in [0, " + std::to_string(m.n) + ")");
 }
 
+// By rows, as the right-hand side of the Poisson system with these pins (null: none).
 void divergence(hg_mesh& m, const double* heat, double* out, int64_t k,
-                FieldLayout layout = FieldLayout::kColumns) {
+                FieldLayout layout = FieldLayout::kColumns, const int32_t* pins = nullptr) {
+  if (layout == FieldLayout::kRows) reserve(m.maxima, divergence_maxima(m.n, k));
   PhaseScope scope(&m.timer, kPhaseDivergence, m.stream);
   launch_divergence(m.faces.ptr, m.face_geom.ptr, m.vertex_ptr.ptr, m.vertex_corners.ptr, &m.corners,
-                    heat, m.n, k, out, layout, m.stream);
+                    heat, m.n, k, out, layout, pins, m.maxima.ptr, m.stream);
 }
 
 // The call's three fields, sized for the next power of two of columns (see SolveWorkspace).
@@ -969,7 +977,7 @@ std::vector<uintptr_t> graph_signature(const hg_mesh& m, int64_t k) {
           p(m.d_sources.ptr),
           p(m.d_owner.ptr), static_cast<uintptr_t>(m.d_owner.size), p(m.d_offsets.ptr),
           p(m.invalid.ptr), p(m.h_invalid.ptr), p(m.h_speculate.ptr), p(m.d_slots.ptr),
-          p(m.h_slots.ptr), p(m.null_partials.ptr), p(m.heat_factor.w64.ptr),
+          p(m.h_slots.ptr), p(m.null_partials.ptr), p(m.maxima.ptr), p(m.heat_factor.w64.ptr),
           p(m.heat_factor.pvalues.ptr), p(m.poisson_factor.w64.ptr),
           p(m.poisson_factor.pvalues.ptr), p(m.pinned_factor.w64.ptr),
           p(m.pinned_factor.pvalues.ptr), p(m.reg_factor.w64.ptr), p(m.reg_factor.pvalues.ptr),
@@ -1175,7 +1183,8 @@ bool solve_columns(hg_mesh& m, const int64_t* offsets, int64_t k, double* phi, i
     launch_average(heat, negdiv, n * k, m.stream);
   }
   m.stats.backward_error_failed = flags & 1;
-  divergence(m, heat, negdiv, k, layout);
+  divergence(m, heat, negdiv, k, layout,
+             layout == FieldLayout::kRows ? poisson_pins(m, regularized) : nullptr);
   if (finish && layout == FieldLayout::kRows && m.rows_by_component) {
     // The heat field is spent once the divergence has read it: its buffer takes the Poisson
     // solution, which one pass turns into the distance in the caller's layout.

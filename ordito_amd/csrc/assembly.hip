@@ -713,16 +713,21 @@ __device__ __forceinline__ double corner_term_2d(const Corner& c, double d1, dou
   return term;
 }
 
-// -b for up to three columns stored by rows: 64 / kk rows a wave, lane l holding column l % kk of row
+// -b for up to four columns stored by rows: 64 / kk rows a wave, lane l holding column l % kk of row
 // l / kk (lanes past the last whole row idle). Each lane walks its row's corners in ascending order,
 // four at a time: their records, then the heat rows they name. A lane's records are its own run of
 // memory, which larger batches read apart (one column on the 524,288-row torus: 51 us, six at a time
-// 90, the faces' own arrays 72).
+// 90, the faces' own arrays 72). The pinned rows of the Poisson system that takes the result are
+// left zero and each block's largest |b| is kept, before that (passes of their own took 9.6 us of one
+// source on icosphere(7)).
 __global__ __launch_bounds__(256) void divergence_rows_kernel(
     const int2* __restrict__ corner_rows, const int32_t* __restrict__ corner_ptr,
     const double* __restrict__ geom, const double* __restrict__ heat, int64_t n, int32_t kk,
-    double* __restrict__ out) {
+    const int32_t* __restrict__ pinned, double* __restrict__ out, double* __restrict__ maxima) {
   constexpr int B = 4;
+  __shared__ unsigned long long best[4];
+  if (threadIdx.x < 4) best[threadIdx.x] = 0ull;
+  __syncthreads();
   const int32_t per_wave = 64 / kk;
   const int32_t lane = static_cast<int32_t>(threadIdx.x % 64);
   const int32_t sub = lane / kk;
@@ -730,9 +735,9 @@ __global__ __launch_bounds__(256) void divergence_rows_kernel(
       static_cast<int64_t>(xcd_block() * 4 + static_cast<int32_t>(threadIdx.x / 64)) * per_wave +
       sub;
   const int32_t q = lane % kk;
-  if (sub >= per_wave || r >= n) return;
-  const int32_t kbeg = corner_ptr[r], kend = corner_ptr[r + 1];
-  const double own = heat[r * kk + q];
+  const bool live = sub < per_wave && r < n;
+  const int32_t kbeg = live ? corner_ptr[r] : 0, kend = live ? corner_ptr[r + 1] : 0;
+  const double own = live ? heat[r * kk + q] : 0.0;
   double sum = 0.0;
   for (int32_t kb = kbeg; kb < kend; kb += B) {
     double h1[B], h2[B], g[B][5];
@@ -757,10 +762,18 @@ __global__ __launch_bounds__(256) void divergence_rows_kernel(
       if (kb + w < kend) sum += term;
     }
   }
-  out[r * kk + q] = sum;
+  // The block's largest of each column by its bits, whose order is that of non-negative values.
+  if (live) {
+    out[r * kk + q] = pinned && pinned[r] ? 0.0 : sum;
+    atomicMax(&best[q], static_cast<unsigned long long>(__builtin_bit_cast(uint64_t, fabs(sum))));
+  }
+  __syncthreads();
+  if (threadIdx.x < kk)
+    maxima[static_cast<int64_t>(threadIdx.x) * gridDim.x + xcd_block()] =
+        __builtin_bit_cast(double, static_cast<uint64_t>(best[threadIdx.x]));
 }
 
-// -b for four columns and more stored by rows: a lane holds two columns of a row (the last lane of an
+// -b for five columns and more stored by rows: a lane holds two columns of a row (the last lane of an
 // odd number repeats one), a block the rows of pair_rows, whose corner records it first brings into LDS
 // (they lie in one run): loads of 16 bytes a lane for the heat rows and none of the records'. A block
 // of rows with more corners than it can hold reads the records where they lie. Six corners at a time (a
@@ -770,6 +783,7 @@ __global__ __launch_bounds__(256) void divergence_rows_kernel(
 // arrays 512), of which the terms' arithmetic is about 150; 16 columns on icosphere(9): 455 (915,
 // 1,482).
 constexpr int kPairCorners = 480;
+constexpr int32_t kMaximaRows = 256;
 
 __global__ __launch_bounds__(256, 5) void divergence_pairs_kernel(
     const int2* __restrict__ corner_rows, const int32_t* __restrict__ corner_ptr,
@@ -835,6 +849,47 @@ __global__ __launch_bounds__(256, 5) void divergence_pairs_kernel(
   else
     for (int32_t s = s0; s < here; s += per)
       row(s, corner_rows + base, geom + kCornerGeom * static_cast<int64_t>(base));
+}
+
+// A chunk's largest |b| of each column in every 256 rows, two columns a lane, and its pinned rows zeroed
+// once they are read. A pass of its own for five columns and more: folded into divergence_pairs_kernel
+// its registers spill (icosphere(9) at 16 columns 452 to 647 us, this pass 62, one loading an element a lane 166).
+__global__ __launch_bounds__(256) void column_maxima_kernel(double* __restrict__ b, int64_t n,
+                                                            int32_t kk,
+                                                            const int32_t* __restrict__ pinned,
+                                                            double* __restrict__ maxima) {
+  __shared__ Pair most[256];
+  const int32_t tid = static_cast<int32_t>(threadIdx.x);
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * kMaximaRows;
+  const int64_t end = min(first + kMaximaRows, n);
+  const int32_t lanes = (kk + 1) / 2, per = 256 / lanes, s = tid / lanes;
+  const int32_t q = min(2 * (tid % lanes), kk - 2);
+  Pair v = {0.0, 0.0};
+  if (s < per)
+    for (int64_t r = first + s; r < end; r += 8 * per) {
+      Pair x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        x[u] = *reinterpret_cast<const Pair*>(b + min(r + u * per, end - 1) * kk + q);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v = Pair{fmax(v.x, fabs(x[u].x)), fmax(v.y, fabs(x[u].y))};
+    }
+  most[tid] = v;
+  __syncthreads();  // the rows are read
+  if (pinned && first + tid < end && pinned[first + tid])
+    for (int32_t c = 0; c < kk; ++c) b[(first + tid) * kk + c] = 0.0;
+  for (int32_t c = per; c > 1;) {
+    const int32_t half = (c + 1) / 2;
+    if (s < c - half) {
+      const Pair o = most[tid + half * lanes];
+      most[tid] = Pair{fmax(most[tid].x, o.x), fmax(most[tid].y, o.y)};
+    }
+    __syncthreads();
+    c = half;
+  }
+  if (s > 0) return;
+  maxima[static_cast<int64_t>(q) * gridDim.x + blockIdx.x] = most[tid].x;
+  maxima[static_cast<int64_t>(q + 1) * gridDim.x + blockIdx.x] = most[tid].y;
 }
 
 // Columns of the shift: column q starts at col_off[q] and holds col_len[q] entries (packed meshes'
@@ -1109,27 +1164,42 @@ void build_corner_geometry(const float* normals, const double* face_geom,
   HG_HIP(hipGetLastError());
 }
 
+// Pairs from five columns on (with their pass for the maxima 82 us against 97 at 8 on the 524,288-row
+// torus; 73 against 72 at four).
+constexpr int64_t kDivergencePairs = 5;
+
+int64_t divergence_blocks(int64_t n, int64_t kk) {
+  const int64_t rows = kk >= kDivergencePairs ? kMaximaRows : 4 * (kFieldChunk / kk);
+  return (n + rows - 1) / rows;
+}
+
+int64_t divergence_maxima(int64_t n, int64_t n_columns) {
+  const int64_t whole = n_columns / kFieldChunk * kFieldChunk, rest = n_columns - whole;
+  return whole * divergence_blocks(n, kFieldChunk) + (rest > 0 ? rest * divergence_blocks(n, rest) : 0);
+}
+
 void launch_divergence(const int32_t* faces, const double* geom, const int32_t* vertex_ptr,
                        const int32_t* vertex_corners, const CornerRecords* records,
                        const double* heat, int64_t n, int64_t n_columns, double* out,
-                       FieldLayout layout, hipStream_t stream) {
+                       FieldLayout layout, const int32_t* pinned, double* maxima,
+                       hipStream_t stream) {
   if (n == 0 || n_columns == 0) return;
   if (layout == FieldLayout::kRows) {
     for (int64_t c0 = 0; c0 < n_columns; c0 += kFieldChunk) {
       const int64_t kk = std::min<int64_t>(kFieldChunk, n_columns - c0);
-      // Pairs from four columns on (on the 524,288-row torus 63 us against 72 there, 71 against 97 at
-      // 8; equal at three).
-      if (kk >= 4) {
+      const unsigned blocks = static_cast<unsigned>(divergence_blocks(n, kk));  // as many maxima
+      double* most = maxima + c0 * divergence_blocks(n, kFieldChunk);
+      if (kk >= kDivergencePairs) {
         const int32_t rows = pair_rows(static_cast<int32_t>(kk));
         divergence_pairs_kernel<<<static_cast<unsigned>((n + rows - 1) / rows), kBlock, 0, stream>>>(
             records->rows.ptr, records->ptr.ptr, records->geom.ptr, heat + c0 * n, n,
             static_cast<int32_t>(kk), rows, out + c0 * n);
+        column_maxima_kernel<<<blocks, kBlock, 0, stream>>>(out + c0 * n, n, static_cast<int32_t>(kk),
+                                                            pinned, most);
       } else {
-        const int64_t rows_per_block = 4 * (kFieldChunk / kk);
-        divergence_rows_kernel<<<static_cast<unsigned>((n + rows_per_block - 1) / rows_per_block),
-                                 kBlock, 0, stream>>>(
+        divergence_rows_kernel<<<blocks, kBlock, 0, stream>>>(
             records->rows.ptr, records->ptr.ptr, records->geom.ptr, heat + c0 * n, n,
-            static_cast<int32_t>(kk), out + c0 * n);
+            static_cast<int32_t>(kk), pinned, out + c0 * n, most);
       }
     }
   } else {

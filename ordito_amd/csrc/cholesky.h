@@ -91,7 +91,7 @@ struct Factor {
 // With live_fronts, the forward sweep covers those fronts only (see LiveFronts).
 void flow_sweep(const DevicePlan& plan, const Factor& factor, bool use_fp32, const double* r,
                 double* fvec, double* y, double* d, const double* x, double* x_next, int32_t kk,
-                int32_t* pending, int64_t patience, const struct LiveFronts* live_fronts,
+                const ColumnMaxima& maxima, int32_t* pending, int64_t patience, const struct LiveFronts* live_fronts,
                 hipStream_t stream);
 
 // A right-hand side of a few nonzero rows reaches, forward, only the fronts on the paths from those
@@ -151,7 +151,8 @@ void factor_numeric(const DevicePlan& plan, const double* values, const int32_t*
 // factor's permuted values) until every row passes the test (componentwise or normwise) or
 // max_rounds sweeps ran; returns the most sweeps any 64-column chunk took. Pinned rows are
 // dropped. b stored by columns is only read; b stored by rows is the solve's own right-hand side,
-// its pinned rows zeroed in place.
+// its pinned rows zeroed in place, or for a normwise test by the divergence that wrote it, which left
+// the blocks' maxima too (launch_divergence).
 // speculate (host memory from hipHostMalloc, one int a 64-column chunk; FP64 solve blocks only):
 // run the first round alone and return without waiting for its test, whose verdict (nonzero: a
 // row still above tolerance) lands in speculate[chunk] with the stream's next synchronization. The
@@ -163,7 +164,7 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
                       hipStream_t stream, PhaseTimer* timer = nullptr,
                       int sweep_phase = kPhaseHeatSweep, FieldLayout b_layout = FieldLayout::kColumns,
                       FieldLayout x_layout = FieldLayout::kColumns, int32_t* speculate = nullptr,
-                      const SourceRows* nonzero = nullptr);
+                      const SourceRows* nonzero = nullptr, const double* maxima = nullptr);
 
 // The components' members cut into 256-member chunks, for the null-space projection's reductions.
 struct NullSpace {

@@ -357,13 +357,20 @@ __global__ __launch_bounds__(kThreads, 4) void flow_kernel(const TW* __restrict_
   }
 }
 
-// Every word the sweep hands over emptied, and the solve's verdict cleared.
+// Every word the sweep hands over emptied, the solve's verdict cleared, and (partials not null) the
+// columns' largest values folded by its first blocks.
 __global__ __launch_bounds__(256) void flow_empty_kernel(uint64_t* __restrict__ y,
                                                          uint64_t* __restrict__ d,
                                                          int64_t entries,
                                                          uint64_t* __restrict__ fvec,
                                                          int64_t updates,
-                                                         int32_t* __restrict__ pending) {
+                                                         int32_t* __restrict__ pending,
+                                                         ColumnMaxima maxima, int32_t kk) {
+  if (maxima.partials)
+    for (int32_t q = static_cast<int32_t>(blockIdx.x); q < kk; q += static_cast<int32_t>(gridDim.x)) {
+      fold_maxima(maxima, q);
+      __syncthreads();
+    }
   const int64_t first = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
   if (first == 0) *pending = 0;
@@ -432,7 +439,7 @@ HostFlow flow_tasks(const Plan& plan) {
 
 void flow_sweep(const DevicePlan& plan, const Factor& factor, bool use_fp32, const double* r,
                 double* fvec, double* y, double* d, const double* x, double* x_next, int32_t kk,
-                int32_t* pending, int64_t patience, const LiveFronts* live_fronts,
+                const ColumnMaxima& maxima, int32_t* pending, int64_t patience, const LiveFronts* live_fronts,
                 hipStream_t stream) {
   FlowArgs a{};
   a.desc = plan.flow_desc.ptr;
@@ -457,7 +464,7 @@ void flow_sweep(const DevicePlan& plan, const Factor& factor, bool use_fp32, con
   flow_empty_kernel<<<static_cast<unsigned>(std::min<int64_t>((updates + entries + 255) / 256, 2048)),
                       256, 0, stream>>>(reinterpret_cast<uint64_t*>(y),
                                         reinterpret_cast<uint64_t*>(d), entries,
-                                        reinterpret_cast<uint64_t*>(fvec), updates, pending);
+                                        reinterpret_cast<uint64_t*>(fvec), updates, pending, maxima, kk);
   const unsigned tasks = static_cast<unsigned>(plan.flow_desc.size / 3);
   if (use_fp32) launch_flow<float>(factor.w32.ptr, a, tasks, stream);
   else launch_flow<double>(factor.w64.ptr, a, tasks, stream);

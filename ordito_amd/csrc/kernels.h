@@ -189,12 +189,42 @@ void build_corner_geometry(const float* normals, const double* face_geom,
                            const int32_t* vertex_ptr, const int32_t* vertex_corners,
                            const int32_t* perm, int64_t n, CornerRecords& out,
                            hipStream_t stream);
-// -b per vertex and column from the heat (both in `layout`), gathered over each vertex's corners;
-// records: kRows only.
+// -b per vertex and column from the heat (both in `layout`), gathered over each vertex's corners.
+// By rows, from the records: rows flagged in `pinned` (the elimination order; may be null) are left
+// zero, and blocks of rows leave their largest |b| of every column, pinned rows' included, in
+// `maxima` (divergence_maxima entries): chunk c's at c * 64 * divergence_blocks(n, 64), column by
+// column, divergence_blocks(n, kk) each.
+int64_t divergence_blocks(int64_t n, int64_t kk);
+int64_t divergence_maxima(int64_t n, int64_t n_columns);
 void launch_divergence(const int32_t* faces, const double* geom, const int32_t* vertex_ptr,
                        const int32_t* vertex_corners, const CornerRecords* records,
                        const double* heat, int64_t n, int64_t n_columns, double* out,
-                       FieldLayout layout, hipStream_t stream);
+                       FieldLayout layout, const int32_t* pinned, double* maxima,
+                       hipStream_t stream);
+
+// Blocks' largest values of each column, to be folded into `out` (column by column, `blocks` each).
+struct ColumnMaxima {
+  const double* partials = nullptr;
+  int32_t blocks = 0;
+  double* out = nullptr;
+};
+
+// Column q's fold, by a block of 256 threads. A maximum does not depend on the order it is taken in.
+__device__ __forceinline__ void fold_maxima(const ColumnMaxima& m, int64_t q) {
+  __shared__ double scratch[256];
+  double v = 0.0;
+#pragma unroll 8
+  for (int32_t b = static_cast<int32_t>(threadIdx.x); b < m.blocks; b += 256)
+    v = fmax(v, m.partials[q * m.blocks + b]);
+  scratch[threadIdx.x] = v;
+  __syncthreads();
+  for (int stride = 128; stride > 0; stride >>= 1) {
+    if (threadIdx.x < stride)
+      scratch[threadIdx.x] = fmax(scratch[threadIdx.x], scratch[threadIdx.x + stride]);
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) m.out[q] = scratch[0];
+}
 int32_t shift_partial_blocks(int64_t n);
 // Columns start at col_off[q] with col_len[q] entries (device; both null: q * n and n), n the
 // longest.

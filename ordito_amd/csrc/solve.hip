@@ -794,55 +794,11 @@ __global__ void absmax_partial_kernel(const double* __restrict__ b, int64_t n,
   if (threadIdx.x == 0) partials[q * gridDim.x + blockIdx.x] = scratch[0];
 }
 
-// The same partial maxima for a chunk stored by rows: block b covers rows [256 b, 256 b + 256);
-// thread (q, part) = (t % 64, t / 64) folds every fourth of them for column q. A maximum does not
-// depend on the order it is taken in.
-__global__ void absmax_rows_partial_kernel(const double* __restrict__ b, int64_t n, int32_t kk,
-                                           double* __restrict__ partials) {
-  __shared__ double scratch[4][64];
-  __shared__ unsigned long long best[kCols];
-  const int q = threadIdx.x % 64, part = threadIdx.x / 64;
-  const int64_t i0 = static_cast<int64_t>(blockIdx.x) * 256;
-  if (kk < kCols / 4) {
-    // Few columns: the block's rows are read as one contiguous run, every lane busy, and each
-    // column's maximum kept by an LDS atomic on the bits (for non-negative doubles their order is
-    // the values' order, and a maximum does not depend on the order it is taken in).
-    if (threadIdx.x < kCols) best[threadIdx.x] = 0ull;
-    __syncthreads();
-    const int64_t count = min<int64_t>(n - i0, 256) * kk;
-    const double* run = b + i0 * kk;
-    for (int64_t e = threadIdx.x; e < count; e += 256)
-      atomicMax(&best[e % kk], static_cast<unsigned long long>(
-                                   __builtin_bit_cast(uint64_t, fabs(run[e]))));
-    __syncthreads();
-    if (threadIdx.x < kk)
-      partials[static_cast<int64_t>(threadIdx.x) * gridDim.x + blockIdx.x] =
-          __builtin_bit_cast(double, static_cast<uint64_t>(best[threadIdx.x]));
-    return;
-  }
-  double v = 0.0;
-  if (q < kk)
-    for (int64_t i = i0 + part; i < min<int64_t>(n, i0 + 256); i += 4) v = fmax(v, fabs(b[i * kk + q]));
-  scratch[part][q] = v;
-  __syncthreads();
-  if (part == 0 && q < kk)
-    partials[static_cast<int64_t>(q) * gridDim.x + blockIdx.x] =
-        fmax(fmax(scratch[0][q], scratch[1][q]), fmax(scratch[2][q], scratch[3][q]));
-}
-
-__global__ void absmax_final_kernel(const double* __restrict__ partials, int32_t blocks,
-                                    double* __restrict__ out) {
-  __shared__ double scratch[256];
-  const int64_t q = blockIdx.x;
-  double v = 0.0;
-  for (int32_t b = threadIdx.x; b < blocks; b += 256) v = fmax(v, partials[q * blocks + b]);
-  scratch[threadIdx.x] = v;
-  __syncthreads();
-  for (int stride = 128; stride > 0; stride >>= 1) {
-    if (threadIdx.x < stride) scratch[threadIdx.x] = fmax(scratch[threadIdx.x], scratch[threadIdx.x + stride]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[q] = scratch[0];
+// The columns' largest values, and a solve's verdict cleared for its first round.
+__global__ __launch_bounds__(256) void absmax_final_kernel(ColumnMaxima maxima,
+                                                           int32_t* __restrict__ pending) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *pending = 0;
+  fold_maxima(maxima, blockIdx.x);
 }
 
 // Component sums for the null-space projection: block partials per (component chunk, column).
@@ -1244,8 +1200,10 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
                       int32_t max_rounds, const int32_t* pinned_new, SolveWorkspace& ws,
                       hipStream_t stream, PhaseTimer* timer, int sweep_phase,
                       FieldLayout b_layout, FieldLayout x_layout, int32_t* speculate,
-                      const SourceRows* nonzero) {
+                      const SourceRows* nonzero, const double* maxima) {
   const int64_t n = plan.n;
+  HG_REQUIRE(b_layout == FieldLayout::kColumns || componentwise || maxima, HG_ERR_RUNTIME,
+             "a normwise solve of a right-hand side stored by rows takes its blocks' maxima");
   if (n == 0 || k == 0) return 0;
   int32_t max_used = 0;
   if (use_fp32) speculate = nullptr;
@@ -1261,20 +1219,26 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
     const unsigned grid = blocks_for(n * kk);
     const unsigned row_tiles = static_cast<unsigned>((n + kTile - 1) / kTile);
     // The right-hand side in the elimination order with its pinned rows zero: b itself by rows
-    // (zeroed in place below, after the normwise scale has read it), else permuted into ws.bp.
+    // (zeroed in place below, or by what wrote a normwise solve's), else permuted into ws.bp.
     double* bp = b_layout == FieldLayout::kRows ? bq : ws.bp.ptr;
     if (b_layout == FieldLayout::kColumns)
       perm_in_kernel<<<row_tiles, 256, 0, stream>>>(bq, plan.perm.ptr, pinned_new, n, kk, bp);
     double* bmax = ws.bmax.ptr + static_cast<int64_t>(blocks_for(n)) * kCols;
+    // The normwise scale: folded from blocks' maxima, which b stored by rows comes with, in the launch
+    // that readies the first sweep.
+    ColumnMaxima fold{};
     if (!componentwise) {
-      const unsigned blocks = blocks_for(n);
-      if (b_layout == FieldLayout::kRows)
-        absmax_rows_partial_kernel<<<blocks, 256, 0, stream>>>(bq, n, kk, ws.bmax.ptr);
-      else
-        absmax_partial_kernel<<<dim3(blocks, kk), 256, 0, stream>>>(bq, n, ws.bmax.ptr);
-      absmax_final_kernel<<<kk, 256, 0, stream>>>(ws.bmax.ptr, static_cast<int32_t>(blocks), bmax);
+      const int64_t blocks =
+          b_layout == FieldLayout::kRows ? divergence_blocks(n, kk) : blocks_for(n);
+      if (b_layout == FieldLayout::kColumns)
+        absmax_partial_kernel<<<dim3(static_cast<unsigned>(blocks), kk), 256, 0, stream>>>(
+            bq, n, ws.bmax.ptr);
+      fold = ColumnMaxima{b_layout == FieldLayout::kRows
+                              ? maxima + q0 * divergence_blocks(n, kCols)
+                              : ws.bmax.ptr,
+                          static_cast<int32_t>(blocks), bmax};
     }
-    if (b_layout == FieldLayout::kRows && pinned_new)
+    if (b_layout == FieldLayout::kRows && componentwise && pinned_new)
       zero_pinned_rows_kernel<<<blocks_for(n), 256, 0, stream>>>(pinned_new, n, kk, bp);
     SweepArgs a{};
     a.col_begin = plan.col_begin.ptr;
@@ -1332,12 +1296,19 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
         }
         a.live = marked ? reached.live : nullptr;
         a.gather_pair = marked ? reached.pairs : plan.gather_pair.ptr;
+        if (!flows) {
+          if (fold.partials)
+            absmax_final_kernel<<<kk, 256, 0, stream>>>(fold, ws.pending.ptr);
+          else
+            launch_zero(ws.pending.ptr, sizeof(int32_t), stream);
+        }
         if (flows)
-          flow_sweep(plan, factor, use_fp32, a.r, a.fvec, a.y, a.d, a.x, a.x_next, kk,
+          flow_sweep(plan, factor, use_fp32, a.r, a.fvec, a.y, a.d, a.x, a.x_next, kk, fold,
                      ws.pending.ptr, ws.patience, marked ? &reached : nullptr, stream);
         else if (use_fp32) sweep<float>(plan, factor.w32.ptr, a, stream);
         else sweep<double>(plan, factor.w64.ptr, a, stream);
       }
+      fold.partials = nullptr;  // once
       if (rounds > 0) x_cur = x_next;
       ++rounds;
       // Through FP64 factors the first round almost always passes, so its residual is formed for
@@ -1359,7 +1330,6 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
       };
       {
         PhaseScope scope(timer, kPhaseResidual, stream);
-        if (!flows) launch_zero(ws.pending.ptr, sizeof(int32_t), stream);
         residual(test_only ? nullptr : ws.r.ptr);
       }
       HG_HIP(hipGetLastError());
