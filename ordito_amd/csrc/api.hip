@@ -118,7 +118,10 @@ struct hg_mesh {
   int32_t settle_window = 0;
   // Speculative refinement (FP64 factors): the verdicts of the first rounds of the heat, pinned and
   // Poisson solves of a call, [system][chunk], read at the call's last synchronization.
-  PinnedArray<int32_t> h_speculate;
+  // A call's flags, on the device and read back by its last copy: [0] a source out of range, then the
+  // speculated verdicts of the heat, rim-pinned and Poisson solves, spec_chunks each.
+  DeviceArray<int32_t> d_flags;
+  PinnedArray<int32_t> h_flags;
   bool speculating = false;
   int64_t spec_chunks = 0;
   // Refinement targets of the factored solves, [precision][0 heat (componentwise), 1 Poisson
@@ -138,15 +141,19 @@ struct hg_mesh {
   DeviceArray<double> fields, shift_partials, shift_values, null_partials, maxima;
   NullSpace null_space;
   DeviceArray<int32_t> d_sources, invalid;
-  PinnedArray<int32_t> h_invalid;  // the seeds' range flag, read back with the call's last sync
   DeviceArray<int64_t> d_owner, d_offsets;
-  PinnedArray<int64_t> h_stage;  // the owners and offsets of a call, staged for an async upload
-  bool sources_on_device = false;  // d_offsets[k] holds this call's source count
+  // A call's offsets, output slots (a pointer a 64-column chunk) and source owners, staged for one
+  // asynchronous upload.
+  PinnedArray<int64_t> h_stage;
+  DeviceArray<int64_t> d_stage;
+  const int64_t* query_offsets = nullptr;  // into d_stage, or d_offsets of packed meshes
+  double* const* out_slots = nullptr;
+  const int64_t* owners = nullptr;  // into d_stage, or d_owner of packed meshes
+  int64_t owner_capacity = 0;
+  bool sources_on_device = false;  // query_offsets[k] holds this call's source count
   int64_t host_sources = 0;        // the source count where it does not
   // The distance's destination per 64-column chunk, read by the finishing kernel (so a replayed
   // graph writes to each call's buffer), staged in pinned memory.
-  DeviceArray<double*> d_slots;
-  PinnedArray<double*> h_slots;
   // Replay of the factored FP64 path: one instantiated graph per column count, valid while every
   // buffer it names is the one it was captured with (signature) and no state change intervened.
   struct Graph {
@@ -213,7 +220,7 @@ int64_t mesh_device_bytes(const hg_mesh& m) {
        {&m.row_segment, &m.faces, &m.offsets, &m.columns, &m.corner_ptr, &m.corner_slots,
         &m.vertex_ptr, &m.vertex_corners, &m.d_rim, &m.d_rim_rows, &m.d_labels, &m.comp_ptr,
         &m.comp_members, &m.poisson_pinned_new, &m.poisson_dropped_old, &m.heat_pinned_new,
-        &m.heat_dropped_old, &m.d_sources, &m.invalid,
+        &m.heat_dropped_old, &m.d_sources, &m.invalid, &m.d_flags,
         &m.q_local})
     total += a->bytes();
   for (const DeviceArray<float>* a : {&m.xyz, &m.cot, &m.normals, &m.areas, &m.heat32, &m.voronoi,
@@ -225,10 +232,10 @@ int64_t mesh_device_bytes(const hg_mesh& m) {
         &m.reg_inv, &m.fields,
         &m.shift_partials, &m.shift_values, &m.null_partials, &m.maxima, &m.packed_phi})
     total += a->bytes();
-  for (const DeviceArray<int64_t>* a : {&m.d_owner, &m.d_offsets, &m.q_src_off, &m.q_dst_off,
+  for (const DeviceArray<int64_t>* a : {&m.d_owner, &m.d_offsets, &m.d_stage, &m.q_src_off, &m.q_dst_off,
                                         &m.q_len})
     total += a->bytes();
-  total += m.corners.bytes() + m.d_slots.bytes() + m.march.bytes();
+  total += m.corners.bytes() + m.march.bytes();
   if (m.poisson_mg) total += m.poisson_mg->bytes();
   total += m.heat_factor.bytes() + m.poisson_factor.bytes() + m.pinned_factor.bytes() +
            m.reg_factor.bytes();
@@ -661,10 +668,10 @@ int32_t diffuse_factored(hg_mesh& m, const HeatSystem& sys, double* rhs, double*
                          bool seeded = false) {
   const bool mixed = precision == HG_PRECISION_MIXED;
   factor_system(m, sys.code, mixed);
-  const SourceRows seeds{m.d_sources.ptr, m.sources_on_device ? m.d_offsets.ptr : nullptr,
+  const SourceRows seeds{m.d_sources.ptr, m.sources_on_device ? m.query_offsets : nullptr,
                          m.host_sources};
   int32_t* speculate =
-      m.speculating ? m.h_speculate.ptr + (sys.code == HG_SYSTEM_PINNED ? m.spec_chunks : 0)
+      m.speculating ? m.d_flags.ptr + 1 + (sys.code == HG_SYSTEM_PINNED ? m.spec_chunks : 0)
                     : nullptr;
   return refined_solve(*m.plan, *sys.factor, mixed, rhs, x, k,
                        m.refine_tolerance[mixed ? 1 : 0][0], true,
@@ -788,7 +795,7 @@ void solve_poisson(hg_mesh& m, double* rhs, double* x, int64_t k, int32_t mode,
         *m.plan, factor, mixed, rhs, x, k, m.refine_tolerance[mixed ? 1 : 0][1], false,
         mixed ? kMixedRefineRounds : kRefineRounds, pins, m.solve, m.stream, &m.timer,
         kPhasePoissonSweep, rhs_layout, x_layout,
-        m.speculating ? m.h_speculate.ptr + 2 * m.spec_chunks : nullptr, nullptr, m.maxima.ptr);
+        m.speculating ? m.d_flags.ptr + 1 + 2 * m.spec_chunks : nullptr, nullptr, m.maxima.ptr);
     m.stats.poisson_rounds = 0;
   } else {
     HG_REQUIRE(rhs_layout == FieldLayout::kColumns && x_layout == FieldLayout::kColumns,
@@ -863,52 +870,64 @@ void reserve(Array& a, int64_t need) {
   if (a.size < need) a.allocate(std::max<int64_t>({need, 2 * a.size, 1024}));
 }
 
-// Each source entry's query and the queries' offsets, staged in pinned memory so both uploads stay
-// asynchronous (the stage is rewritten only by the next call, after this one's synchronization).
-void upload_sources(hg_mesh& m, const int32_t* d_sources, const int64_t* offsets, int64_t k) {
+// The queries' offsets, the slots of the output (k columns; may be null) and each source entry's query,
+// staged in pinned memory so that one asynchronous copy takes them (the stage is rewritten only by the
+// next call, after this one's synchronization). Each copy of a call costs it about 4 us.
+void upload_sources(hg_mesh& m, const int32_t* d_sources, const int64_t* offsets, int64_t k,
+                    double* out = nullptr) {
   const int64_t total = offsets[k] - offsets[0];
-  const int64_t owners = std::max<int64_t>(total, 1);
-  reserve(m.h_stage, owners + k + 1);
-  int64_t* owner = m.h_stage.ptr;
-  int64_t* rel_offsets = m.h_stage.ptr + owners;
-  owner[0] = 0;
+  const int64_t chunks = (k + kFieldChunk - 1) / kFieldChunk;
+  const int64_t head = k + 1 + chunks, count = head + std::max<int64_t>(total, 1);
+  reserve(m.h_stage, count);
+  reserve(m.d_stage, count);
+  int64_t* stage = m.h_stage.ptr;
+  for (int64_t q = 0; q <= k; ++q) stage[q] = offsets[q] - offsets[0];
+  for (int64_t c = 0; c < chunks; ++c)
+    stage[k + 1 + c] = reinterpret_cast<int64_t>(out ? out + c * kFieldChunk * m.n : nullptr);
+  stage[head] = 0;
   for (int64_t q = 0; q < k; ++q)
-    for (int64_t e = offsets[q]; e < offsets[q + 1]; ++e) owner[e - offsets[0]] = q;
-  for (int64_t q = 0; q <= k; ++q) rel_offsets[q] = offsets[q] - offsets[0];
-  reserve(m.d_owner, owners);
-  reserve(m.d_offsets, k + 1);
-  m.d_owner.upload(owner, owners, m.stream);
-  m.d_offsets.upload(rel_offsets, k + 1, m.stream);
+    for (int64_t e = offsets[q]; e < offsets[q + 1]; ++e) stage[head + e - offsets[0]] = q;
+  m.d_stage.upload(stage, count, m.stream);
+  m.query_offsets = m.d_stage.ptr;
+  m.out_slots = reinterpret_cast<double* const*>(m.d_stage.ptr + k + 1);
+  m.owners = m.d_stage.ptr + head;
+  m.owner_capacity = m.d_stage.size - head;
   m.sources_on_device = true;
-  reserve(m.d_sources, owners);
+  reserve(m.d_sources, std::max<int64_t>(total, 1));
   if (total > 0)
     HG_HIP(hipMemcpyAsync(m.d_sources.ptr, d_sources + offsets[0], sizeof(int32_t) * total,
                           hipMemcpyDefault, m.stream));
 }
 
+int64_t flag_count(int64_t k) { return 1 + 3 * ((k + kFieldChunk - 1) / kFieldChunk); }
+
 void seed(hg_mesh& m, const int64_t* offsets, int64_t k, double* u0,
           FieldLayout layout = FieldLayout::kColumns) {
   const int64_t total = offsets[k] - offsets[0];
-  launch_zero(u0, static_cast<int64_t>(sizeof(double)) * m.n * k, m.stream);
-  if (m.invalid.size < 1) m.invalid.allocate(1);
-  launch_zero(m.invalid.ptr, sizeof(int32_t), m.stream);
+  reserve(m.d_flags, flag_count(k));
+  launch_zero(u0, static_cast<int64_t>(sizeof(double)) * m.n * k, m.stream, m.d_flags.ptr,
+              static_cast<int64_t>(sizeof(int32_t)) * flag_count(k));
   const bool rows = layout == FieldLayout::kRows;
   // With the offsets on the device the kernel reads the count there (a replay's own count).
   const bool on_device = m.sources_on_device;
-  launch_seed(m.d_sources.ptr, m.d_owner.ptr, on_device ? m.d_owner.size : total,
-              on_device ? m.d_offsets.ptr + k : nullptr, m.n, rows ? k : 0,
-              rows ? m.plan->iperm.ptr : nullptr, u0, m.invalid.ptr, m.stream);
-  // The range flag comes back with the call's next synchronization (check_seeds); until then the
-  // solve runs on, every kernel that reads the sources skipping the ones out of range.
-  if (!m.h_invalid.ptr) m.h_invalid.allocate(1);
-  HG_HIP(hipMemcpyAsync(m.h_invalid.ptr, m.invalid.ptr, sizeof(int32_t), hipMemcpyDeviceToHost,
-                        m.stream));
+  launch_seed(m.d_sources.ptr, m.owners, on_device ? m.owner_capacity : total,
+              on_device ? m.query_offsets + k : nullptr, m.n, rows ? k : 0,
+              rows ? m.plan->iperm.ptr : nullptr, u0, m.d_flags.ptr, m.stream);
+}
+
+// The call's flags, read back behind everything else it issued: until its last synchronization the
+// solve runs on, every kernel that reads the sources skipping the ones out of range (check_seeds), and
+// every speculated verdict unread (speculation_failed).
+void collect_flags(hg_mesh& m, int64_t k) {
+  reserve(m.h_flags, flag_count(k));
+  HG_HIP(hipMemcpyAsync(m.h_flags.ptr, m.d_flags.ptr, sizeof(int32_t) * flag_count(k),
+                        hipMemcpyDeviceToHost, m.stream));
 }
 
 // After a synchronization of the mesh's stream: fail the call if a seed was out of range
 // (kernels/heat.py:599-623, heat.py:5488-5503).
 void check_seeds(const hg_mesh& m) {
-  HG_REQUIRE(!m.h_invalid.ptr || *m.h_invalid.ptr == 0, HG_ERR_VALUE,
+  HG_REQUIRE(!m.h_flags.ptr || m.h_flags.ptr[0] == 0, HG_ERR_VALUE,
              "every entry of sources must be a vertex index in [0, " + std::to_string(m.n) + ")");
 }
 
@@ -937,7 +956,7 @@ void shift(hg_mesh& m, double* phi, int64_t k) {
   reserve(m.shift_partials, blocks * k);
   reserve(m.shift_values, 2 * k);
   PhaseScope scope(&m.timer, kPhaseShift, m.stream);
-  launch_shift(phi, m.d_sources.ptr, m.d_offsets.ptr, m.n, k, nullptr, nullptr,
+  launch_shift(phi, m.d_sources.ptr, m.query_offsets, m.n, k, nullptr, nullptr,
                m.shift_partials.ptr, m.shift_values.ptr, m.stream);
 }
 
@@ -949,8 +968,9 @@ void arm_speculation(hg_mesh& m, int64_t k, bool on) {
   m.speculating = on;
   if (!on) return;
   m.spec_chunks = (k + kFieldChunk - 1) / kFieldChunk;
-  if (m.h_speculate.size < 3 * m.spec_chunks) m.h_speculate.allocate(3 * m.spec_chunks);
-  std::fill(m.h_speculate.ptr, m.h_speculate.ptr + 3 * m.spec_chunks, 0);
+  reserve(m.d_flags, flag_count(k));
+  reserve(m.h_flags, flag_count(k));
+  std::fill(m.h_flags.ptr, m.h_flags.ptr + flag_count(k), 0);
 }
 
 // After the stream's synchronization: whether a speculated first round failed its test.
@@ -958,7 +978,7 @@ bool speculation_failed(hg_mesh& m) {
   const bool was = m.speculating;
   m.speculating = false;
   if (!was) return false;
-  return std::any_of(m.h_speculate.ptr, m.h_speculate.ptr + 3 * m.spec_chunks,
+  return std::any_of(m.h_flags.ptr + 1, m.h_flags.ptr + 1 + 3 * m.spec_chunks,
                      [](int32_t v) { return v != 0; });
 }
 
@@ -975,9 +995,8 @@ std::vector<uintptr_t> graph_signature(const hg_mesh& m, int64_t k) {
           p(m.solve_side.live_pairs.ptr), static_cast<uintptr_t>(w.capacity),
           static_cast<uintptr_t>(w.level_sweeps), static_cast<uintptr_t>(m.solve_side.level_sweeps),
           p(m.d_sources.ptr),
-          p(m.d_owner.ptr), static_cast<uintptr_t>(m.d_owner.size), p(m.d_offsets.ptr),
-          p(m.invalid.ptr), p(m.h_invalid.ptr), p(m.h_speculate.ptr), p(m.d_slots.ptr),
-          p(m.h_slots.ptr), p(m.null_partials.ptr), p(m.maxima.ptr), p(m.heat_factor.w64.ptr),
+          p(m.d_stage.ptr), static_cast<uintptr_t>(m.d_stage.size), p(m.d_flags.ptr),
+          p(m.h_flags.ptr), p(m.null_partials.ptr), p(m.maxima.ptr), p(m.heat_factor.w64.ptr),
           p(m.heat_factor.pvalues.ptr), p(m.poisson_factor.w64.ptr),
           p(m.poisson_factor.pvalues.ptr), p(m.pinned_factor.w64.ptr),
           p(m.pinned_factor.pvalues.ptr), p(m.reg_factor.w64.ptr), p(m.reg_factor.pvalues.ptr),
@@ -1099,8 +1118,6 @@ bool run_graph(hg_mesh& m, const int64_t* offsets, int64_t k, double* d_out, int
     g = std::move(graph);
   }
   arm_speculation(m, k, true);
-  const int64_t chunks = (k + kFieldChunk - 1) / kFieldChunk;
-  for (int64_t c = 0; c < chunks; ++c) m.h_slots.ptr[c] = d_out + c * kFieldChunk * m.n;
   m.stats = g->stats;
   HG_HIP(hipGraphLaunch(g->exec, gs.stream));
   HG_HIP(hipStreamSynchronize(gs.stream));
@@ -1109,7 +1126,8 @@ bool run_graph(hg_mesh& m, const int64_t* offsets, int64_t k, double* d_out, int
 
 // Seed, heat step, divergence and Poisson step over k columns of the whole (possibly packed)
 // system into phi (the caller's layout). The sources must be uploaded. With `finish` and the
-// fields stored by rows, phi is the finished distance (null space removed, shifted, oriented) and
+// fields stored by rows, phi (where the uploaded slots point) is the finished distance (null space
+// removed, shifted, oriented) and
 // the call returns true; otherwise phi is the unshifted distance with each component's mean
 // removed.
 bool solve_columns(hg_mesh& m, const int64_t* offsets, int64_t k, double* phi, int32_t mode,
@@ -1190,16 +1208,13 @@ bool solve_columns(hg_mesh& m, const int64_t* offsets, int64_t k, double* phi, i
     // solution, which one pass turns into the distance in the caller's layout.
     solve_poisson(m, negdiv, heat, k, mode, precision, layout, FieldLayout::kRows, regularized);
     PhaseScope scope(&m.timer, kPhaseShift, m.stream);
-    const int64_t chunks = (k + kFieldChunk - 1) / kFieldChunk;
-    reserve(m.d_slots, chunks);
-    reserve(m.h_slots, chunks);
-    for (int64_t c = 0; c < chunks; ++c) m.h_slots.ptr[c] = phi + c * kFieldChunk * n;
-    m.d_slots.upload(m.h_slots.ptr, chunks, m.stream);
     finish_rows(*m.plan, m.null_space, m.comp_ptr.ptr, m.d_labels.ptr, heat, k, m.d_sources.ptr,
-                m.d_offsets.ptr, m.d_slots.ptr, m.null_partials, m.stream, !regularized);
+                m.query_offsets, m.out_slots, m.null_partials, m.stream, !regularized);
+    collect_flags(m, k);
     return true;
   }
   solve_poisson(m, negdiv, phi, k, mode, precision, layout, FieldLayout::kColumns, regularized);
+  collect_flags(m, k);
   return false;
 }
 
@@ -1664,6 +1679,7 @@ int hg_seed_sources(hg_mesh* mesh, const int32_t* d_sources, const int64_t* sour
     require_mesh(mesh);
     upload_sources(*mesh, d_sources, source_offsets, n_columns);
     seed(*mesh, source_offsets, n_columns, d_u0);
+    collect_flags(*mesh, n_columns);
     HG_HIP(hipStreamSynchronize(mesh->stream));
     check_seeds(*mesh);
   });
@@ -1786,7 +1802,7 @@ int hg_geodesic(hg_mesh* mesh, const int32_t* d_sources, const int64_t* source_o
       return;
     }
     ensure_operators(m);
-    upload_sources(m, d_sources, source_offsets, k);
+    upload_sources(m, d_sources, source_offsets, k, d_out);
     bool done = false;
     if (graphable(m, mode, precision)) done = run_graph(m, source_offsets, k, d_out, precision);
     if (!done) {
@@ -1870,6 +1886,8 @@ int hg_geodesic_packed(hg_mesh* mesh, const int32_t* d_sources, const int64_t* s
     // The seed reads the packed sources with their slot owners; the offsets are unused there.
     m.d_sources.assign(packed, m.stream);
     m.d_owner.assign(owner, m.stream);
+    m.owners = m.d_owner.ptr;
+    m.query_offsets = nullptr;
     std::vector<int64_t> seed_offsets(width + 1, 0);
     seed_offsets[width] = total;
     if (m.packed_capacity < m.n * width) {

@@ -459,12 +459,13 @@ __global__ void seed_kernel(const int32_t* __restrict__ sources, const int64_t* 
   }
 }
 
-// Zeroes `words` 32-bit words: the clears of a solve, as kernels so a captured graph holds no
-// memset node.
-__global__ void zero_words_kernel(uint32_t* __restrict__ p, int64_t words) {
-  for (int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; e < words;
-       e += static_cast<int64_t>(gridDim.x) * blockDim.x)
-    p[e] = 0u;
+// Zeroes 32-bit words: the clears of a solve, as kernels so a captured graph holds no memset node.
+__global__ void zero_words_kernel(uint32_t* __restrict__ p, int64_t words, uint32_t* __restrict__ q,
+                                  int64_t q_words) {
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t step = static_cast<int64_t>(gridDim.x) * blockDim.x;
+  for (int64_t e = first; e < words; e += step) p[e] = 0u;
+  for (int64_t e = first; e < q_words; e += step) q[e] = 0u;
 }
 
 // Per face, the float64 quantities every query's divergence reuses (kernels/triangles.py:834-894,
@@ -1115,12 +1116,14 @@ void launch_seed(const int32_t* sources, const int64_t* owner, int64_t n_entries
   HG_HIP(hipGetLastError());
 }
 
-void launch_zero(void* p, int64_t bytes, hipStream_t stream) {
-  if (bytes <= 0) return;
-  HG_REQUIRE(bytes % 4 == 0, HG_ERR_RUNTIME, "a cleared range is whole 32-bit words");
-  const int64_t words = bytes / 4;
-  const unsigned blocks = std::min<unsigned>(blocks_for(words), 2048u);
-  zero_words_kernel<<<blocks, kBlock, 0, stream>>>(static_cast<uint32_t*>(p), words);
+void launch_zero(void* p, int64_t bytes, hipStream_t stream, void* q, int64_t q_bytes) {
+  if (bytes <= 0 && q_bytes <= 0) return;
+  HG_REQUIRE(bytes % 4 == 0 && q_bytes % 4 == 0, HG_ERR_RUNTIME,
+             "a cleared range is whole 32-bit words");
+  const int64_t words = bytes / 4, q_words = q_bytes / 4;
+  const unsigned blocks = std::min<unsigned>(blocks_for(std::max(words, q_words)), 2048u);
+  zero_words_kernel<<<blocks, kBlock, 0, stream>>>(static_cast<uint32_t*>(p), words,
+                                                   static_cast<uint32_t*>(q), q_words);
   HG_HIP(hipGetLastError());
 }
 

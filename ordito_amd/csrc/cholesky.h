@@ -153,10 +153,10 @@ void factor_numeric(const DevicePlan& plan, const double* values, const int32_t*
 // dropped. b stored by columns is only read; b stored by rows is the solve's own right-hand side,
 // its pinned rows zeroed in place, or for a normwise test by the divergence that wrote it, which left
 // the blocks' maxima too (launch_divergence).
-// speculate (host memory from hipHostMalloc, one int a 64-column chunk; FP64 solve blocks only):
-// run the first round alone and return without waiting for its test, whose verdict (nonzero: a
-// row still above tolerance) lands in speculate[chunk] with the stream's next synchronization. The
-// caller checks it there and solves again without speculating when any is set.
+// speculate (device memory, one int a 64-column chunk; FP64 solve blocks only): run the first round
+// alone and return without waiting for its test, whose verdict (nonzero: a row still above
+// tolerance) the stream leaves in speculate[chunk]. The caller reads it back and solves again
+// without speculating when any is set.
 // nonzero (b stored by rows only): the rows b is nonzero on, when the caller knows them to be few.
 int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp32,
                       double* b, double* x, int64_t k, double tolerance, bool componentwise,

@@ -1214,6 +1214,7 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
                "a solve chunk of " + std::to_string(n) + " rows x " + std::to_string(kk) +
                    " columns exceeds 2^31 entries; solve fewer columns per call");
     ws.reserve(plan, kk);
+    int32_t* const verdict = speculate ? speculate + q0 / kCols : ws.pending.ptr;
     double* bq = b + q0 * n;
     double* xq = x + q0 * n;
     const unsigned grid = blocks_for(n * kk);
@@ -1298,13 +1299,13 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
         a.gather_pair = marked ? reached.pairs : plan.gather_pair.ptr;
         if (!flows) {
           if (fold.partials)
-            absmax_final_kernel<<<kk, 256, 0, stream>>>(fold, ws.pending.ptr);
+            absmax_final_kernel<<<kk, 256, 0, stream>>>(fold, verdict);
           else
-            launch_zero(ws.pending.ptr, sizeof(int32_t), stream);
+            launch_zero(verdict, sizeof(int32_t), stream);
         }
         if (flows)
           flow_sweep(plan, factor, use_fp32, a.r, a.fvec, a.y, a.d, a.x, a.x_next, kk, fold,
-                     ws.pending.ptr, ws.patience, marked ? &reached : nullptr, stream);
+                     verdict, ws.patience, marked ? &reached : nullptr, stream);
         else if (use_fp32) sweep<float>(plan, factor.w32.ptr, a, stream);
         else sweep<double>(plan, factor.w64.ptr, a, stream);
       }
@@ -1321,11 +1322,11 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
           const int32_t rows = pair_rows(kk);
           residual_pairs_kernel<<<static_cast<unsigned>((n + rows - 1) / rows), 256, 0, stream>>>(
               plan.p_offsets.ptr, plan.p_columns.ptr, factor.pvalues.ptr, bp, x_cur, pinned_new,
-              bmax, n, kk, rows, tolerance, componentwise ? 1 : 0, r_out, ws.pending.ptr);
+              bmax, n, kk, rows, tolerance, componentwise ? 1 : 0, r_out, verdict);
         } else {
           residual_kernel<<<grid, 256, 0, stream>>>(
               plan.p_offsets.ptr, plan.p_columns.ptr, factor.pvalues.ptr, bp, x_cur, pinned_new,
-              bmax, n, kk, tolerance, componentwise ? 1 : 0, r_out, ws.pending.ptr);
+              bmax, n, kk, tolerance, componentwise ? 1 : 0, r_out, verdict);
         }
       };
       {
@@ -1333,13 +1334,9 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
         residual(test_only ? nullptr : ws.r.ptr);
       }
       HG_HIP(hipGetLastError());
-      if (speculate) {
-        HG_HIP(hipMemcpyAsync(speculate + q0 / kCols, ws.pending.ptr, sizeof(int32_t),
-                              hipMemcpyDeviceToHost, stream));
-        break;
-      }
+      if (speculate) break;
       int32_t pending = 0;
-      HG_HIP(hipMemcpyAsync(&pending, ws.pending.ptr, sizeof(int32_t), hipMemcpyDeviceToHost,
+      HG_HIP(hipMemcpyAsync(&pending, verdict, sizeof(int32_t), hipMemcpyDeviceToHost,
                             stream));
       HG_HIP(hipStreamSynchronize(stream));
       if (timer) timer->resolve();
