@@ -150,14 +150,17 @@ __device__ __forceinline__ double gather_add(const SweepArgs& a, int64_t row, in
 // (lane l holds A[l % 16][l / 16]) and a 4 x 16 block of B (lane l holds B[l / 16][l % 16]) and
 // accumulates the 16 x 16 product, lane l holding rows l / 16 + 4v (v < 4) of column l % 16. A
 // tile's four waves each own 16 of its 64 rows and accumulate NB blocks of 16 right-hand sides. The
-// vectors are staged through LDS, shared by the waves, kInner inner indices at a time; a wave's
+// vectors are staged through LDS, shared by the waves, kDepth inner indices at a time; a wave's
 // part of the inverse factor is its own, so its lanes load it straight into the operand's layout.
 // The next stage's global loads are issued before the current stage's products, so they overlap.
 typedef double f64x4 __attribute__((ext_vector_type(4)));
-constexpr int kInner = 16;
-// Staged rows are kPad doubles more than their columns apart: the four inner rows an MFMA operand
-// read spans start 34 banks apart (mod 64) at 64 columns.
-constexpr int kPad = 17;
+// A stage is 16 inner indices of 32 or 64 right-hand sides, 32 of 16: a block of few columns waits on
+// its loads' round trips (16 columns on icosphere(7): 303 us a heat sweep 16 deep, 285 at 32; 64
+// deep 298, and on icosphere(9) 1.60 ms against 1.36).
+template <int NB>
+constexpr int kStages = NB == 1 ? 2 : 1;
+// Staged rows are kPad doubles more than their columns apart, which puts the two inner rows that half a
+// wave's operand read spans (neighbours forward, four apart backward) 32 banks apart.
 
 __device__ __forceinline__ f64x4 mfma16x16x4(double a, double b, f64x4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
@@ -201,8 +204,9 @@ __device__ __forceinline__ Task load_task(const int4* __restrict__ desc, int32_t
 template <typename TW, int NB, bool kGathers>
 __global__ __launch_bounds__(256, kGathers ? 4 : (NB == 4 ? 5 : 6)) void fwd_tile_kernel(
     const int4* __restrict__ desc, int32_t parts, const TW* __restrict__ w, SweepArgs a) {
-  constexpr int kN = 16 * NB;
-  __shared__ double Fs[2][kInner][kN + kPad];  // [stage][inner][right-hand side]
+  constexpr int D = kStages<NB>, kN = 16 * NB, kDepth = 16 * D, U = NB * D;
+  constexpr int kPad = NB == 1 ? 0 : 16;
+  __shared__ double Fs[2][kDepth][kN + kPad];  // [stage][inner][right-hand side]
   const int32_t block = xcd_block();
   const Task tk = load_task(desc, block / parts);
   const int32_t q0 = block % parts * kN;  // the block's first right-hand side
@@ -238,16 +242,16 @@ __global__ __launch_bounds__(256, kGathers ? 4 : (NB == 4 ? 5 : 6)) void fwd_til
   // reads its last, whose product nothing stores).
   const uint32_t lane_w = (static_cast<uint32_t>(lk) * static_cast<uint32_t>(m) +
                            static_cast<uint32_t>(min(r0 + 16 * wave + li, m - 1))) * sizeof(TW);
-  double wreg[4];
+  double wreg[4 * D];
   auto load_w = [&](int32_t j0) {
     if (j0 >= wave_k1) return;
-    if (j0 + kInner <= k1) {
+    if (j0 + kDepth <= k1) {
 #pragma unroll
-      for (int h = 0; h < 4; ++h)
+      for (int h = 0; h < 4 * D; ++h)
         wreg[h] = widen(load_at(W + static_cast<int64_t>(j0 + 4 * h) * m, lane_w));
     } else {
 #pragma unroll
-      for (int h = 0; h < 4; ++h)
+      for (int h = 0; h < 4 * D; ++h)
         wreg[h] = j0 + 4 * h + lk < k1
                       ? widen(load_at(W + static_cast<int64_t>(j0 + 4 * h) * m, lane_w))
                       : 0.0;
@@ -257,38 +261,38 @@ __global__ __launch_bounds__(256, kGathers ? 4 : (NB == 4 ? 5 : 6)) void fwd_til
   // inner e / kN (past the range, its last row again, which W multiplies by zero). A stage's gather
   // pairs are loaded two stages ahead of its products, its entries one, and they are added and
   // staged after the products in between: nothing waits for a load it has just issued.
-  int2 pair[NB];
-  double rreg[NB], first[NB], second[NB];
+  int2 pair[U];
+  double rreg[U], first[U], second[U];
   const int qe = q0 + t % kN, ql = min(qe, a.kk - 1);
   auto inner_of = [&](int32_t j0, int u) { return min(j0 + (t + 256 * u) / kN, k1 - 1); };
   auto load_pairs = [&](int32_t j0) {
     if (!kGathers) return;
-    int64_t grow[NB];
-    bool glive[NB];
+    int64_t grow[U];
+    bool glive[U];
 #pragma unroll
-    for (int u = 0; u < NB; ++u) {
+    for (int u = 0; u < U; ++u) {
       grow[u] = vbase + inner_of(j0, u);
       glive[u] = true;
     }
-    gather_pairs<NB>(a, grow, glive, pair);
+    gather_pairs<U>(a, grow, glive, pair);
   };
-  int2 used[NB];  // the pairs of the entries in flight
+  int2 used[U];  // the pairs of the entries in flight
   auto load_f = [&](int32_t j0) {
-    int q[NB];
+    int q[U];
 #pragma unroll
-    for (int u = 0; u < NB; ++u) {
+    for (int u = 0; u < U; ++u) {
       q[u] = qe;
       rreg[u] = a.r[static_cast<int64_t>(c0 + inner_of(j0, u)) * kk + ql];
     }
     if constexpr (kGathers) {
 #pragma unroll
-      for (int u = 0; u < NB; ++u) used[u] = pair[u];
-      gather_issue<NB>(a, used, q, first, second);
+      for (int u = 0; u < U; ++u) used[u] = pair[u];
+      gather_issue<U>(a, used, q, first, second);
     }
   };
   auto stage = [&](int32_t j0, double (*F)[kN + kPad]) {
 #pragma unroll
-    for (int u = 0; u < NB; ++u) {
+    for (int u = 0; u < U; ++u) {
       double v = rreg[u];
       if constexpr (kGathers)
         v = gather_add(a, vbase + inner_of(j0, u), ql, used[u], first[u], second[u], v);
@@ -301,23 +305,23 @@ __global__ __launch_bounds__(256, kGathers ? 4 : (NB == 4 ? 5 : 6)) void fwd_til
   load_pairs(k0);
   load_w(k0);
   load_f(k0);
-  if (k0 + kInner < k1) load_pairs(k0 + kInner);
+  if (k0 + kDepth < k1) load_pairs(k0 + kDepth);
   stage(k0, Fs[0]);
   __syncthreads();
   int p = 0;
-  for (int32_t j0 = k0; j0 < k1; j0 += kInner, p ^= 1) {
-    double av[4];
+  for (int32_t j0 = k0; j0 < k1; j0 += kDepth, p ^= 1) {
+    double av[4 * D];
 #pragma unroll
-    for (int h = 0; h < 4; ++h) av[h] = wreg[h];
-    const bool more = j0 + kInner < k1;
+    for (int h = 0; h < 4 * D; ++h) av[h] = wreg[h];
+    const bool more = j0 + kDepth < k1;
     if (more) {
-      load_w(j0 + kInner);
-      load_f(j0 + kInner);
-      if (j0 + 2 * kInner < k1) load_pairs(j0 + 2 * kInner);
+      load_w(j0 + kDepth);
+      load_f(j0 + kDepth);
+      if (j0 + 2 * kDepth < k1) load_pairs(j0 + 2 * kDepth);
     }
     if (j0 < wave_k1)
 #pragma unroll
-      for (int h = 0; h < 4; ++h) {
+      for (int h = 0; h < 4 * D; ++h) {
         double bv[NB];
 #pragma unroll
         for (int n = 0; n < NB; ++n) bv[n] = Fs[p][4 * h + lk][16 * n + li];
@@ -325,7 +329,7 @@ __global__ __launch_bounds__(256, kGathers ? 4 : (NB == 4 ? 5 : 6)) void fwd_til
         for (int n = 0; n < NB; ++n) acc[n] = mfma16x16x4(av[h], bv[n], acc[n]);
       }
     if (more) {
-      stage(j0 + kInner, Fs[p ^ 1]);
+      stage(j0 + kDepth, Fs[p ^ 1]);
       __syncthreads();
     }
   }
@@ -473,8 +477,9 @@ __device__ __forceinline__ void load_four(const float* p, double (&v)[4]) {
 template <typename TW, int NB, bool kIterate>
 __global__ __launch_bounds__(256, NB == 4 ? 5 : 6) void bwd_tile_kernel(
     const int4* __restrict__ desc, int32_t parts, const TW* __restrict__ w, SweepArgs a) {
-  constexpr int kN = 16 * NB;
-  __shared__ double Gs[2][kInner][kN + kPad];  // [stage][inner][right-hand side]
+  constexpr int D = kStages<NB>, kN = 16 * NB, kDepth = 16 * D, U = NB * D;
+  constexpr int kPad = 4;
+  __shared__ double Gs[2][kDepth][kN + kPad];  // [stage][inner][right-hand side]
   const int32_t block = xcd_block();
   const Task tk = load_task(desc, block / parts);
   const int32_t q0 = block % parts * kN;  // the block's first right-hand side
@@ -495,31 +500,35 @@ __global__ __launch_bounds__(256, NB == 4 ? 5 : 6) void bwd_tile_kernel(
   const TW* W = w + tk.w_off;
   const uint32_t column = static_cast<uint32_t>(min(j0 + 16 * wave + li, nc - 1)) *
                               static_cast<uint32_t>(m) + 4 * lk;
-  double wreg[4], greg[NB];
+  double wreg[D][4], greg[U];
   // A stage's structure-row indices are loaded a stage ahead (load_rows), so its W and g loads
   // issue together. Entry e = t + 256u of a stage is g's right-hand side e % kN at inner e / kN.
-  int32_t srow[NB];
+  int32_t srow[U];
   auto load_rows = [&](int32_t i0) {
 #pragma unroll
-    for (int u = 0; u < NB; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int32_t ig = i0 + (t + 256 * u) / kN;
       srow[u] = (ig >= nc && ig < k1) ? srows[ig - nc] : 0;
     }
   };
   auto load = [&](int32_t i0) {
-    if (i0 + kInner > wave_k0) {
-      if (i0 + kInner <= k1) {  // uniform: the whole stage is inside the range
-        load_four(W + column + i0, wreg);
+    if (i0 + kDepth > wave_k0) {
+      if (i0 + kDepth <= k1) {  // uniform: the whole stage is inside the range
+#pragma unroll
+        for (int g = 0; g < D; ++g) load_four(W + column + i0 + 16 * g, wreg[g]);
       } else {
 #pragma unroll
-        for (int h = 0; h < 4; ++h)
-          wreg[h] = i0 + 4 * lk + h < k1 ? widen(W[column + i0 + h]) : 0.0;
+        for (int g = 0; g < D; ++g)
+#pragma unroll
+          for (int h = 0; h < 4; ++h)
+            wreg[g][h] =
+                i0 + 16 * g + 4 * lk + h < k1 ? widen(W[column + i0 + 16 * g + h]) : 0.0;
       }
     }
     // 32-bit element offsets from wave-uniform bases (a field stays under 2^31 entries), one
     // register an address.
 #pragma unroll
-    for (int u = 0; u < NB; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int e = t + 256 * u;
       const int q = q0 + e % kN;
       const int32_t ig = i0 + e / kN;
@@ -536,38 +545,42 @@ __global__ __launch_bounds__(256, NB == 4 ? 5 : 6) void bwd_tile_kernel(
   for (int n = 0; n < NB; ++n) acc[n] = f64x4{0.0, 0.0, 0.0, 0.0};
   auto stage = [&](double (*G)[kN + kPad]) {
 #pragma unroll
-    for (int u = 0; u < NB; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int e = t + 256 * u;
       G[e / kN][e % kN] = greg[u];
     }
   };
-  const int32_t last = k0 < k1 ? k0 + (k1 - 1 - k0) / kInner * kInner : k0 - 1;
+  const int32_t last = k0 < k1 ? k0 + (k1 - 1 - k0) / kDepth * kDepth : k0 - 1;
   if (k0 < k1) {
     load_rows(k0);
     load(k0);
-    if (last > k0) load_rows(k0 + kInner);
+    if (last > k0) load_rows(k0 + kDepth);
     stage(Gs[0]);
   }
   __syncthreads();
   int p = 0;
-  for (int32_t i0 = k0; i0 <= last; i0 += kInner, p ^= 1) {
-    double av[4];
+  for (int32_t i0 = k0; i0 <= last; i0 += kDepth, p ^= 1) {
+    double av[D][4];
 #pragma unroll
-    for (int h = 0; h < 4; ++h) av[h] = wreg[h];
+    for (int g = 0; g < D; ++g)
+#pragma unroll
+      for (int h = 0; h < 4; ++h) av[g][h] = wreg[g][h];
     const bool more = i0 < last;
     if (more) {
-      load(i0 + kInner);
-      if (i0 + kInner < last) load_rows(i0 + 2 * kInner);
+      load(i0 + kDepth);
+      if (i0 + kDepth < last) load_rows(i0 + 2 * kDepth);
     }
-    if (i0 + kInner > wave_k0)
+    if (i0 + kDepth > wave_k0)
 #pragma unroll
-      for (int h = 0; h < 4; ++h) {
-        double bv[NB];
+      for (int g = 0; g < D; ++g)
 #pragma unroll
-        for (int n = 0; n < NB; ++n) bv[n] = Gs[p][4 * lk + h][16 * n + li];
+        for (int h = 0; h < 4; ++h) {
+          double bv[NB];
 #pragma unroll
-        for (int n = 0; n < NB; ++n) acc[n] = mfma16x16x4(av[h], bv[n], acc[n]);
-      }
+          for (int n = 0; n < NB; ++n) bv[n] = Gs[p][16 * g + 4 * lk + h][16 * n + li];
+#pragma unroll
+          for (int n = 0; n < NB; ++n) acc[n] = mfma16x16x4(av[g][h], bv[n], acc[n]);
+        }
     if (more) {
       stage(Gs[p ^ 1]);
       __syncthreads();
