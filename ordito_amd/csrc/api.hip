@@ -1,6 +1,7 @@
 // The C ABI of libheatgeo (include/heatgeo.h): mesh state, operator assembly, the heat and Poisson
 // solves in both modes, the divergence, the shift and the fused geodesic path.
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
 #include <limits>
@@ -96,6 +97,7 @@ struct hg_mesh {
   bool has_heat_pins = false;
   // Cholesky.
   AnalysisOptions options;                  // nested-dissection leaf and top-merge sizes
+  std::unique_ptr<std::array<int64_t, 3>> unmerged_sizes;  // planned_peak_bytes'
   int32_t split_target = kDefaultSplitTarget;  // sweep tasks a level is split towards
   std::unique_ptr<Plan> host_plan;
   std::unique_ptr<DevicePlan> plan;
@@ -415,7 +417,10 @@ void ensure_operators(hg_mesh& m) {
 
 void ensure_plan(hg_mesh& m) {
   if (m.plan) return;
-  m.host_plan = std::make_unique<Plan>(analyse(m.pattern, m.h_xyz.data(), m.options));
+  // Under a budget the plan keeps every separator its own front (planned_peak_bytes).
+  AnalysisOptions options = m.options;
+  if (m.budget > 0) options.merge_rows = 0;
+  m.host_plan = std::make_unique<Plan>(analyse(m.pattern, m.h_xyz.data(), options));
   const Plan& plan = *m.host_plan;
   auto device = std::make_unique<DevicePlan>();
   device->upload(plan, m.pattern, m.split_target, m.stream);
@@ -520,11 +525,26 @@ int64_t factor_peak_bytes(const DevicePlan& plan, bool keep_fp32) {
   return 8 * plan.arena_size + (keep_fp32 ? 12 : 8) * plan.w_size + 8 * plan.nnz_w;
 }
 
+// The peak a budget is held against: that of the plan with every separator its own front, which is the
+// mesh's own plan unless the budget was set when a factor was held.
+int64_t planned_peak_bytes(hg_mesh& m, bool keep_fp32) {
+  if (m.budget <= 0 || !m.host_plan->merged) return factor_peak_bytes(*m.plan, keep_fp32);
+  if (!m.unmerged_sizes) {
+    AnalysisOptions options = m.options;
+    options.merge_rows = 0;
+    const Plan plan = analyse(m.pattern, m.h_xyz.data(), options);
+    m.unmerged_sizes = std::make_unique<std::array<int64_t, 3>>(
+        std::array<int64_t, 3>{plan.arena_size, plan.w_size, plan.nnz_w});
+  }
+  const std::array<int64_t, 3>& s = *m.unmerged_sizes;
+  return 8 * s[0] + (keep_fp32 ? 12 : 8) * s[1] + 8 * s[2];
+}
+
 // Refuse (HG_ERR_BUDGET) a factorization whose peak exceeds the budget, as sparse_cholesky refuses
 // one past CHOLESKY_MEMORY_BUDGET (cholesky.py:72, linalg.py:2393-2420); the system is then solved
 // by iteration. With no budget set the limit is 90 % of the device memory free now.
 void require_budget(hg_mesh& m, int32_t system, bool keep_fp32) {
-  const int64_t need = factor_peak_bytes(*m.plan, keep_fp32);
+  const int64_t need = planned_peak_bytes(m, keep_fp32);
   int64_t limit = m.budget;
   if (limit <= 0) {
     size_t free_bytes = 0, total_bytes = 0;
@@ -546,7 +566,7 @@ bool exceeds_budget(hg_mesh& m, int32_t system) {
   if (m.refused & system) return true;
   if (m.budget <= 0 || !m.budget_probe) return false;
   ensure_plan(m);
-  if (factor_peak_bytes(*m.plan, false) <= m.budget) return false;
+  if (planned_peak_bytes(m, false) <= m.budget) return false;
   m.refused |= system;
   return true;
 }
@@ -1497,6 +1517,7 @@ int hg_set_plan_options(hg_mesh* mesh, int32_t leaf_rows, int32_t top_rows,
       m.reg_factor.reset();
       m.plan.reset();
       m.host_plan.reset();
+      m.unmerged_sizes.reset();
       m.options.leaf_rows = leaf;
       m.options.top_rows = top;
       m.split_target = split;
@@ -1635,9 +1656,17 @@ int hg_set_memory_budget(hg_mesh* mesh, int64_t bytes) {
   return guarded([&] {
     require_mesh(mesh);
     HG_REQUIRE(bytes >= 0, HG_ERR_VALUE, "the memory budget must not be negative");
-    mesh->budget = bytes;
-    mesh->refused = 0;
-    invalidate_graphs(*mesh);
+    hg_mesh& m = *mesh;
+    m.budget = bytes;
+    m.refused = 0;
+    invalidate_graphs(m);
+    // A merged plan that no factor needs yet gives way to the one the budget is held against.
+    if (bytes > 0 && m.host_plan && m.host_plan->merged && !m.heat_factor.held() &&
+        !m.poisson_factor.held() && !m.pinned_factor.held() && !m.reg_factor.held()) {
+      HG_HIP(hipStreamSynchronize(m.stream));
+      m.plan.reset();
+      m.host_plan.reset();
+    }
   });
 }
 

@@ -176,6 +176,7 @@ struct Plan {
   double flops = 0.0;               // dense partial-factorization flops
   int64_t nnz_w = 0;                // stored solve-block entries
   int32_t max_front = 0;
+  bool merged = false;  // separators were merged upwards
 };
 
 // Leaf 128: on the 1024 x 512 torus with 64 right-hand sides, leaves of 96-192 rows serve fastest
@@ -183,6 +184,7 @@ struct Plan {
 struct AnalysisOptions {
   int32_t leaf_rows = 128;
   int32_t top_rows = 512;
+  int32_t merge_rows = -1;  // small separators merged upwards (0: none; -1: by the rows, analyse)
 };
 
 Plan analyse(const HostPattern& pattern, const float* coordinates, const AnalysisOptions& options);
