@@ -121,7 +121,8 @@ struct hg_mesh {
   // Speculative refinement (FP64 factors): the verdicts of the first rounds of the heat, pinned and
   // Poisson solves of a call, [system][chunk], read at the call's last synchronization.
   // A call's flags, on the device and read back by its last copy: [0] a source out of range, then the
-  // speculated verdicts of the heat, rim-pinned and Poisson solves, spec_chunks each.
+  // speculated verdicts of the heat, rim-pinned and Poisson solves, spec_chunks each. Behind them the
+  // bitmap of the rows with a source (launch_seed).
   DeviceArray<int32_t> d_flags;
   PinnedArray<int32_t> h_flags;
   bool speculating = false;
@@ -682,6 +683,9 @@ bool backward_error_fails(hg_mesh& m, const double* values, const double* x, con
   return flag != 0;
 }
 
+// The flags of a call of k columns (hg_mesh::d_flags).
+int64_t flag_count(int64_t k) { return 1 + 3 * ((k + kFieldChunk - 1) / kFieldChunk); }
+
 // seeded: rhs holds the call's uploaded sources' seeds (or those off the rim), nothing else.
 int32_t diffuse_factored(hg_mesh& m, const HeatSystem& sys, double* rhs, double* x, int64_t k,
                          int32_t precision, FieldLayout layout = FieldLayout::kColumns,
@@ -689,7 +693,8 @@ int32_t diffuse_factored(hg_mesh& m, const HeatSystem& sys, double* rhs, double*
   const bool mixed = precision == HG_PRECISION_MIXED;
   factor_system(m, sys.code, mixed);
   const SourceRows seeds{m.d_sources.ptr, m.sources_on_device ? m.query_offsets : nullptr,
-                         m.host_sources};
+                         m.host_sources,
+                         reinterpret_cast<const uint32_t*>(m.d_flags.ptr + flag_count(k))};
   int32_t* speculate =
       m.speculating ? m.d_flags.ptr + 1 + (sys.code == HG_SYSTEM_PINNED ? m.spec_chunks : 0)
                     : nullptr;
@@ -919,20 +924,16 @@ void upload_sources(hg_mesh& m, const int32_t* d_sources, const int64_t* offsets
                           hipMemcpyDefault, m.stream));
 }
 
-int64_t flag_count(int64_t k) { return 1 + 3 * ((k + kFieldChunk - 1) / kFieldChunk); }
-
 void seed(hg_mesh& m, const int64_t* offsets, int64_t k, double* u0,
           FieldLayout layout = FieldLayout::kColumns) {
   const int64_t total = offsets[k] - offsets[0];
-  reserve(m.d_flags, flag_count(k));
-  launch_zero(u0, static_cast<int64_t>(sizeof(double)) * m.n * k, m.stream, m.d_flags.ptr,
-              static_cast<int64_t>(sizeof(int32_t)) * flag_count(k));
+  reserve(m.d_flags, flag_count(k) + seed_words(m.n));
   const bool rows = layout == FieldLayout::kRows;
   // With the offsets on the device the kernel reads the count there (a replay's own count).
   const bool on_device = m.sources_on_device;
   launch_seed(m.d_sources.ptr, m.owners, on_device ? m.owner_capacity : total,
-              on_device ? m.query_offsets + k : nullptr, m.n, rows ? k : 0,
-              rows ? m.plan->iperm.ptr : nullptr, u0, m.d_flags.ptr, m.stream);
+              on_device ? m.query_offsets + k : nullptr, m.n, k,
+              rows ? m.plan->iperm.ptr : nullptr, u0, m.d_flags.ptr, flag_count(k), m.stream);
 }
 
 // The call's flags, read back behind everything else it issued: until its last synchronization the
@@ -988,7 +989,7 @@ void arm_speculation(hg_mesh& m, int64_t k, bool on) {
   m.speculating = on;
   if (!on) return;
   m.spec_chunks = (k + kFieldChunk - 1) / kFieldChunk;
-  reserve(m.d_flags, flag_count(k));
+  reserve(m.d_flags, flag_count(k) + seed_words(m.n));
   reserve(m.h_flags, flag_count(k));
   std::fill(m.h_flags.ptr, m.h_flags.ptr + flag_count(k), 0);
 }

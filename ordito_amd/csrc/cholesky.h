@@ -110,6 +110,7 @@ struct SourceRows {
   const int32_t* sources = nullptr;
   const int64_t* offsets = nullptr;
   int64_t count = 0;
+  const uint32_t* seeded = nullptr;  // the bitmap of their rows in the elimination order
 };
 
 // A plan of fewer fronts sweeps them all: marking takes three short launches (icosphere(4), 41

@@ -157,12 +157,14 @@ void launch_operator_rows(const int32_t* offsets, const int32_t* columns,
                           const double* mass, const double* scalars, const int32_t* row_segment,
                           int64_t n, double* lap, double* heat, double* poisson, float* heat32,
                           double* heat_inv_diag, double* poisson_inv_diag, hipStream_t stream);
-// rows_k > 0: u0 stored by rows (FieldLayout::kRows) over rows_k columns, vertex v at row
-// row_of[v]; 0: by columns.
+// u0 = the indicator of each of k columns' sources, flags[0 .. n_flags) cleared and flags[0] raised by a
+// source out of range. row_of not null: u0 stored by rows (FieldLayout::kRows), vertex v at row
+// row_of[v], and the seed_words(n) words behind the flags become the bitmap of the rows with a source.
 // count_at (device, nullable): read the entry count there, at most n_entries.
+inline int64_t seed_words(int64_t n) { return (n + 31) / 32; }
 void launch_seed(const int32_t* sources, const int64_t* owner, int64_t n_entries,
-                 const int64_t* count_at, int64_t n, int64_t rows_k, const int32_t* row_of,
-                 double* u0, int32_t* invalid, hipStream_t stream);
+                 const int64_t* count_at, int64_t n, int64_t k, const int32_t* row_of, double* u0,
+                 int32_t* flags, int64_t n_flags, hipStream_t stream);
 // Zeroes `bytes` (whole 32-bit words) with a kernel (graph-capturable, unlike a memset node).
 // Zeroes p's bytes, and q's (multiples of 4).
 void launch_zero(void* p, int64_t bytes, hipStream_t stream, void* q = nullptr, int64_t q_bytes = 0);

@@ -720,14 +720,16 @@ __global__ void residual_kernel(const int32_t* __restrict__ offsets,
 // the entries are (the iterate's for the caches alone: its row is some row's entry), which hides part of
 // the chain offsets, entries, iterate (icosphere(9) at 16 columns: 267 us against 286). Sums keep entry
 // order. 524,288-row torus: 32 columns 105 us (a lane a column 204), 64 columns 197 (214), where the
-// rows fetched twice from beyond L2 hold it (850 MB at 4.4 TB/s; 570 are needed).
+// rows fetched twice from beyond L2 hold it (850 MB at 4.4 TB/s; 570 are needed). The heat step's
+// right-hand side is read where the bitmap of seeded rows has one (197 to 163).
 constexpr int32_t kPairEntries = 1024;
 __global__ __launch_bounds__(256) void residual_pairs_kernel(
     const int32_t* __restrict__ offsets, const int32_t* __restrict__ columns,
     const double* __restrict__ values, const double* __restrict__ b,
     const double* __restrict__ x, const int32_t* __restrict__ pinned,
-    const double* __restrict__ bmax, int64_t n, int32_t kk, int32_t rows, double tolerance,
-    int32_t componentwise, double* __restrict__ r, int32_t* __restrict__ pending) {
+    const double* __restrict__ bmax, const uint32_t* __restrict__ seeded, int64_t n, int32_t kk,
+    int32_t rows, double tolerance, int32_t componentwise, double* __restrict__ r,
+    int32_t* __restrict__ pending) {
   __shared__ int32_t ptr[kPairRows + 1];
   __shared__ int32_t named[kPairEntries];
   __shared__ double staged[kPairEntries];
@@ -739,9 +741,15 @@ __global__ __launch_bounds__(256) void residual_pairs_kernel(
   const int32_t lanes = (kk + 1) / 2, per = 256 / lanes, s0 = tid / lanes;
   const int32_t q = min(2 * (tid % lanes), kk - 2);
   const bool takes = s0 < min(per, here);
+  // b's entries of row s; seeded (nullable): only rows flagged there have any.
+  auto right_hand_side = [&](int32_t s) {
+    const int64_t i = first + s;
+    if (seeded && !(seeded[i / 32] >> (i % 32) & 1)) return Pair{0.0, 0.0};
+    return __builtin_nontemporal_load(reinterpret_cast<const Pair*>(b + i * kk + q));
+  };
   Pair b0 = {0.0, 0.0}, x0 = {0.0, 0.0};
   if (takes) {
-    b0 = __builtin_nontemporal_load(reinterpret_cast<const Pair*>(b + (first + s0) * kk + q));
+    b0 = right_hand_side(s0);
     x0 = *reinterpret_cast<const Pair*>(x + (first + s0) * kk + q);
   }
   __syncthreads();
@@ -758,7 +766,7 @@ __global__ __launch_bounds__(256) void residual_pairs_kernel(
   bool fail = false;
   auto row = [&](int32_t s, const int32_t* names, const double* v) {
     const int64_t i = first + s, at = i * kk + q;
-    Pair total = s == s0 ? b0 : __builtin_nontemporal_load(reinterpret_cast<const Pair*>(b + at));
+    Pair total = s == s0 ? b0 : right_hand_side(s);
     Pair scale = {fabs(total.x), fabs(total.y)};
     const bool dropped = pinned && pinned[i];
     const int32_t e1 = ptr[s + 1] - base;
@@ -1272,6 +1280,8 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
     a.vec_front = plan.vec_front.ptr;
     const bool sparse =
         nonzero && b_layout == FieldLayout::kRows && plan.n_super >= kSparseFronts;
+    const uint32_t* seeded =
+        nonzero && b_layout == FieldLayout::kRows ? nonzero->seeded : nullptr;
     const LiveFronts reached{ws.live.ptr, ws.live_pairs.ptr};
     // The first round solves for the iterate itself from x = 0: its right-hand side is b and its
     // correction is written straight into the iterate. Later rounds correct it: d into ws.d and
@@ -1335,7 +1345,8 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
           const int32_t rows = pair_rows(kk);
           residual_pairs_kernel<<<static_cast<unsigned>((n + rows - 1) / rows), 256, 0, stream>>>(
               plan.p_offsets.ptr, plan.p_columns.ptr, factor.pvalues.ptr, bp, x_cur, pinned_new,
-              bmax, n, kk, rows, tolerance, componentwise ? 1 : 0, r_out, verdict);
+              bmax, seeded, n, kk, rows, tolerance,
+              componentwise ? 1 : 0, r_out, verdict);
         } else {
           residual_kernel<<<grid, 256, 0, stream>>>(
               plan.p_offsets.ptr, plan.p_columns.ptr, factor.pvalues.ptr, bp, x_cur, pinned_new,
