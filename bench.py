@@ -746,7 +746,7 @@ def _in_poisson(names: list[str]) -> list[bool]:
     for name in names:
         if name.startswith("divergence_"):
             poisson = True
-        elif name.startswith("seed_kernel"):
+        elif name.startswith("seed_"):
             poisson = False
         flags.append(poisson)
     return flags
