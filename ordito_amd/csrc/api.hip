@@ -1014,7 +1014,7 @@ std::vector<uintptr_t> graph_signature(const hg_mesh& m, int64_t k) {
           p(w.r.ptr), p(w.y.ptr), p(w.d.ptr), p(w.fvec.ptr), p(w.bmax.ptr), p(w.partials.ptr),
           p(w.pending.ptr), p(w.live.ptr), p(w.live_pairs.ptr), p(m.solve_side.live.ptr),
           p(m.solve_side.live_pairs.ptr), static_cast<uintptr_t>(w.capacity),
-          static_cast<uintptr_t>(w.level_sweeps), static_cast<uintptr_t>(m.solve_side.level_sweeps),
+          static_cast<uintptr_t>(w.level_sweeps), static_cast<uintptr_t>(w.flows), static_cast<uintptr_t>(m.solve_side.level_sweeps),
           p(m.d_sources.ptr),
           p(m.d_stage.ptr), static_cast<uintptr_t>(m.d_stage.size), p(m.d_flags.ptr),
           p(m.h_flags.ptr), p(m.null_partials.ptr), p(m.maxima.ptr), p(m.heat_factor.w64.ptr),
@@ -1093,6 +1093,23 @@ struct SideStream {
   hipEvent_t fork = nullptr, join = nullptr;
 };
 thread_local SideStream t_side_stream;
+
+// The WaitClaim of a call of k columns, if its last chunk is narrow enough to sweep in one launch, and the
+// main workspace's leave to (the side one never has it: its sweeps run beside these).
+struct FlowScope {
+  hg_mesh& m;
+  const bool wanted;
+  WaitClaim claim;
+  FlowScope(hg_mesh& mesh, int64_t k)
+      : m(mesh),
+        wanted((k + kFieldChunk - 1) % kFieldChunk < kFlowColumns && k > 0),
+        claim(wanted, false) {
+    m.solve.flows = claim.held();
+  }
+  ~FlowScope() { m.solve.flows = false; }
+  // A captured call sweeps as the claim allows.
+  bool as_captured() const { return !wanted || claim.held(); }
+};
 
 bool run_graph(hg_mesh& m, const int64_t* offsets, int64_t k, double* d_out, int32_t precision) {
   GraphStream& gs = t_graph_stream;
@@ -1561,6 +1578,7 @@ int hg_diffuse(hg_mesh* mesh, const double* d_rhs, double* d_solution, int64_t n
     require_single_or_factored(*mesh, mode);
     SpeculationDisarm disarm(*mesh);
     mesh->stats = hg_solve_stats{};
+    FlowScope flow(*mesh, n_columns);
     // By columns (the caller's layout) the solve only reads its right-hand side.
     int32_t flags = diffuse(*mesh, const_cast<double*>(d_rhs), d_solution, n_columns, mode,
                             precision);
@@ -1579,6 +1597,7 @@ int hg_diffuse_pinned(hg_mesh* mesh, const double* d_rhs, double* d_solution, in
     hg_mesh& m = *mesh;
     SpeculationDisarm disarm(m);
     m.stats = hg_solve_stats{};
+    FlowScope flow(m, n_columns);
     ensure_operators(m);
     int32_t flags = 0;
     if (m.n_rim > 0 && n_columns > 0) {
@@ -1687,6 +1706,7 @@ int hg_solve_poisson(hg_mesh* mesh, const double* d_rhs, double* d_solution, int
     require_single_or_factored(*mesh, mode);
     SpeculationDisarm disarm(*mesh);
     mesh->stats = hg_solve_stats{};
+    FlowScope flow(*mesh, n_columns);
     // By columns (the caller's layout) the solve only reads its right-hand side.
     solve_poisson(*mesh, const_cast<double*>(d_rhs), d_solution, n_columns, mode, precision);
     HG_HIP(hipStreamSynchronize(mesh->stream));
@@ -1832,9 +1852,10 @@ int hg_geodesic(hg_mesh* mesh, const int32_t* d_sources, const int64_t* source_o
       return;
     }
     ensure_operators(m);
+    FlowScope flow(m, k);
     upload_sources(m, d_sources, source_offsets, k, d_out);
     bool done = false;
-    if (graphable(m, mode, precision)) done = run_graph(m, source_offsets, k, d_out, precision);
+    if (graphable(m, mode, precision) && flow.as_captured()) done = run_graph(m, source_offsets, k, d_out, precision);
     if (!done) {
       for (bool speculate : {precision == HG_PRECISION_FP64, false}) {
         m.stats = hg_solve_stats{};
@@ -1924,6 +1945,7 @@ int hg_geodesic_packed(hg_mesh* mesh, const int32_t* d_sources, const int64_t* s
       m.packed_phi.allocate(m.n * width);
       m.packed_capacity = m.n * width;
     }
+    FlowScope flow(m, width);
     arm_speculation(m, width, precision == HG_PRECISION_FP64);
     m.sources_on_device = false;  // the seeds' count is the host's
     m.host_sources = total;

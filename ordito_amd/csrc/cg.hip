@@ -1080,6 +1080,7 @@ int32_t run_cg(const CgProblem& problem, CgWorkspace& ws, hipStream_t stream) {
   const int64_t k = problem.n_columns;
   HG_REQUIRE(k >= 1 && k <= kMaxColumns, HG_ERR_VALUE, "conjugate gradient takes 1-64 columns");
   if (n == 0) return 0;
+  const WaitClaim claim(true, true);
   if (ws.counters.size < 4 + kBarrierGroups) ws.counters.allocate(4 + kBarrierGroups);
   CgArgs a{};
   a.n = n;

@@ -21,6 +21,9 @@
 // A forward task is 256 / LN rows of a front, LN threads a row splitting the inner range; a
 // backward task is 16 * PASS columns, sixteen lanes a column along its rows. Every output is one
 // task's: no partial products cross blocks, and each sum has one fixed order.
+#include <exception>
+#include <mutex>
+
 #include "cholesky.h"
 #include "words.h"
 
@@ -435,6 +438,32 @@ HostFlow flow_tasks(const Plan& plan) {
     }
   }
   return out;
+}
+
+namespace {
+constexpr int kClaimDevices = 64;
+std::mutex g_wait_claims[kClaimDevices];
+thread_local bool t_holds_claim[kClaimDevices] = {};
+}  // namespace
+
+WaitClaim::WaitClaim(bool wanted, bool wait) {
+  if (!wanted) return;
+  HG_HIP(hipGetDevice(&device_));
+  if (device_ >= kClaimDevices) return;
+  held_ = t_holds_claim[device_];
+  if (held_) return;
+  if (wait) g_wait_claims[device_].lock();
+  else if (!g_wait_claims[device_].try_lock()) return;
+  unwinding_ = std::uncaught_exceptions();
+  held_ = owner_ = t_holds_claim[device_] = true;
+}
+
+WaitClaim::~WaitClaim() {
+  if (!owner_) return;
+  // A call that throws leaves work running.
+  if (std::uncaught_exceptions() > unwinding_) (void)hipDeviceSynchronize();
+  t_holds_claim[device_] = false;
+  g_wait_claims[device_].unlock();
 }
 
 void flow_sweep(const DevicePlan& plan, const Factor& factor, bool use_fp32, const double* r,

@@ -40,6 +40,27 @@ inline int32_t pair_rows(int32_t kk) {
   return at_once * std::max(1, (31 + at_once) / at_once);
 }
 
+// A process's claim, while it lives, on the device's kernels whose blocks wait for words that others of
+// their launch write (flow.hip's sweeps, the conjugate gradients): one holder at a time. The hardware
+// hands each XCD its blocks in order, but not the XCDs theirs in step, so two such launches on two
+// streams can each fill one XCD's compute units with blocks that wait for what the other XCD's queue
+// holds behind the other launch's; both then wait out their patience. With 64 meshes served by four
+// threads that made a query's median 176 ms, against 1.6 with the sweeps level by level.
+// `wait`: until another thread's claim ends; else the claim is not held if there is one. A thread that
+// holds one already holds it here too. The holder's work is to have run when the claim ends.
+class WaitClaim {
+ public:
+  WaitClaim(bool wanted, bool wait);
+  ~WaitClaim();
+  WaitClaim(const WaitClaim&) = delete;
+  WaitClaim& operator=(const WaitClaim&) = delete;
+  bool held() const { return held_; }
+
+ private:
+  int device_ = 0, unwinding_ = 0;
+  bool held_ = false, owner_ = false;
+};
+
 // Device time of the phases of a solve, from HIP events on the stream the work is issued on.
 enum Phase : int {
   kPhaseFactor = 0,

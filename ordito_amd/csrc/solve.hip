@@ -1290,8 +1290,9 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
     double* x_cur = x_home;
     int32_t rounds = 0;
     while (rounds < max_rounds) {
-      // A few columns sweep in one launch (flow.hip), unless one such launch has given up here.
-      const bool flows = kk <= kFlowColumns && !ws.level_sweeps;
+      // A few columns sweep in one launch (flow.hip), if the call may and no such launch has given up
+      // here.
+      const bool flows = kk <= kFlowColumns && ws.flows && !ws.level_sweeps;
       double* x_next = x_cur == x_home ? ws.xa.ptr : x_home;
       if (rounds == 0) {
         a.r = bp;
