@@ -1201,7 +1201,12 @@ bool solve_columns(hg_mesh& m, const int64_t* offsets, int64_t k, double* phi, i
   seed(m, offsets, k, u0, layout);
   const bool igl = m.method == HG_METHOD_IGL && m.n_rim > 0;
   int32_t flags = 0;
-  if (igl && layout == FieldLayout::kRows && m.speculating) {
+  // Side by side, unless both solves can sweep in one launch each, which go one after the other
+  // (WaitClaim): one source on a grid of 131,044 430 us a call, with the second level by level beside the
+  // first 519; four on 524,176 1,192 and 1,207.
+  const bool beside = igl && layout == FieldLayout::kRows && m.speculating &&
+                      !(m.solve.flows && !m.solve.level_sweeps && k <= kFlowColumns);
+  if (beside) {
     // igl::heat_geodesics' boundary rule (heat.py:594-597) with the two heat solves side by side:
     // the rim-pinned one, from the seeds zeroed on the rim, runs on a second stream with its own
     // workspace and first-round verdict while the Neumann one runs here; neither waits on the host
@@ -1228,7 +1233,7 @@ bool solve_columns(hg_mesh& m, const int64_t* offsets, int64_t k, double* phi, i
   } else {
     flags = diffuse(m, u0, heat, k, mode, precision, layout, false, true);
   }
-  if (igl && !(layout == FieldLayout::kRows && m.speculating)) {
+  if (igl && !beside) {
     // igl::heat_geodesics' boundary rule (heat.py:594-597): the Neumann heat averaged with the
     // heat pinned to zero on the rim, solved from the seeds zeroed there. The divergence's buffer
     // holds the pinned heat until the average has read it.
