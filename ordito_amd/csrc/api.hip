@@ -966,6 +966,7 @@ double* reserve_fields(hg_mesh& m, int64_t k) {
   if (m.field_capacity < 3 * m.n * k) {
     int64_t columns = 1;
     while (columns < k) columns *= 2;
+    m.field_capacity = 0;
     m.fields.allocate(std::max<int64_t>(3 * m.n * columns, 1));
     m.field_capacity = 3 * m.n * columns;
   }
@@ -1947,6 +1948,7 @@ int hg_geodesic_packed(hg_mesh* mesh, const int32_t* d_sources, const int64_t* s
     std::vector<int64_t> seed_offsets(width + 1, 0);
     seed_offsets[width] = total;
     if (m.packed_capacity < m.n * width) {
+      m.packed_capacity = 0;
       m.packed_phi.allocate(m.n * width);
       m.packed_capacity = m.n * width;
     }

@@ -1136,6 +1136,7 @@ int32_t run_cg(const CgProblem& problem, CgWorkspace& ws, hipStream_t stream) {
   const int32_t G = single ? 1 : cooperative_grid(n);
   const int64_t entries = n * k;
   if (ws.capacity_entries < entries) {
+    ws.capacity_entries = 0;
     ws.vectors.allocate(9 * entries);
     ws.capacity_entries = entries;
   }

@@ -55,10 +55,11 @@ struct DeviceArray {
     return *this;
   }
   ~DeviceArray() { reset(); }
+  // An allocation that fails leaves the array empty: callers grow it by its size.
   void allocate(int64_t n) {
     reset();
-    size = n;
     if (n > 0) HG_HIP(hipMalloc(&ptr, sizeof(T) * static_cast<size_t>(n)));
+    size = n;
   }
   void reset() {
     if (ptr) (void)hipFree(ptr);

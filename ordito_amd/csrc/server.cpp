@@ -180,8 +180,10 @@ void run_batch(hg_server* s, Worker& worker, Mesh* mesh, std::vector<Request>& b
       HG_HIP(hipStreamSynchronize(worker.stream));
       if (worker.d_sources) (void)hipFree(worker.d_sources);
       worker.d_sources = nullptr;
-      worker.sources_capacity = std::max<int64_t>(total, 2 * worker.sources_capacity);
-      HG_HIP(hipMalloc(&worker.d_sources, sizeof(int32_t) * worker.sources_capacity));
+      const int64_t grown = std::max<int64_t>(total, 2 * worker.sources_capacity);
+      worker.sources_capacity = 0;
+      HG_HIP(hipMalloc(&worker.d_sources, sizeof(int32_t) * grown));
+      worker.sources_capacity = grown;
     }
     std::vector<int32_t> flat(static_cast<size_t>(total), 0);
     for (size_t q = 0; q < batch.size(); ++q)
@@ -193,8 +195,10 @@ void run_batch(hg_server* s, Worker& worker, Mesh* mesh, std::vector<Request>& b
       HG_HIP(hipStreamSynchronize(worker.stream));
       if (worker.d_fields) (void)hipFree(worker.d_fields);
       worker.d_fields = nullptr;
-      worker.fields_capacity = std::max<int64_t>(k * mesh->n, 2 * worker.fields_capacity);
-      HG_HIP(hipMalloc(&worker.d_fields, sizeof(double) * worker.fields_capacity));
+      const int64_t grown = std::max<int64_t>(k * mesh->n, 2 * worker.fields_capacity);
+      worker.fields_capacity = 0;
+      HG_HIP(hipMalloc(&worker.d_fields, sizeof(double) * grown));
+      worker.fields_capacity = grown;
     }
     check(hg_geodesic(mesh->handle, worker.d_sources, offsets.data(), k, worker.d_fields,
                       HG_MODE_FACTORED, s->precision, nullptr));

@@ -1191,6 +1191,7 @@ void SolveWorkspace::reserve(const DevicePlan& plan, int64_t kk_needed) {
   kk = std::min<int64_t>(kk, kCols);
   const int64_t entries = plan.n * kk;
   if (capacity < entries) {
+    capacity = 0;  // while any of them may be missing
     bp.allocate(entries);
     xa.allocate(entries);
     xb.allocate(entries);
@@ -1200,12 +1201,14 @@ void SolveWorkspace::reserve(const DevicePlan& plan, int64_t kk_needed) {
     capacity = entries;
   }
   if (fcap < plan.vec_size * kk) {
+    fcap = 0;
     fvec.allocate(plan.vec_size * kk + kCols);  // the gathers' padding
     fcap = plan.vec_size * kk;
   }
   const int64_t pentries = std::max(plan.max_slots[0] * std::min<int64_t>(kk, 16),
                                     kk > 16 ? plan.max_slots[1] * kk : 0) * kTile;
   if (pcap < pentries) {
+    pcap = 0;
     partials.allocate(std::max<int64_t>(pentries, 1));
     pcap = pentries;
   }

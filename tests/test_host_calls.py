@@ -1,0 +1,170 @@
+"""
+The library's host code with a HIP runtime that only keeps memory and a log of launches
+(``tests/fake_hip.cpp``): what a call allocates and launches, in what order and beside which other
+calls, where no GPU is needed to tell. Kernels do nothing there, so device memory stays zero and a
+mesh's pattern is empty; the solves' sequences of launches are the real ones.
+
+Each test runs in a process of its own, which binds the library to that runtime.
+"""
+
+from __future__ import annotations
+
+import ctypes
+import subprocess
+import sys
+from pathlib import Path
+
+import numpy as np
+
+ROOT = Path(__file__).resolve().parents[1]
+HEAT, POISSON = 1, 2
+ITERATE, FACTORED = 0, 1
+
+
+class Library:
+    """libheatgeo over the fake runtime; a call that fails raises its message."""
+
+    def __init__(self, fake: str) -> None:
+        self.fake = ctypes.CDLL(fake, mode=ctypes.RTLD_GLOBAL)
+        self.lib = ctypes.CDLL(str(ROOT / "ordito_amd" / "libheatgeo.so"))
+        self.lib.hg_last_error.restype = ctypes.c_char_p
+        for name in ("fake_live_bytes", "fake_launches", "fake_thread_launches"):
+            getattr(self.fake, name).restype = ctypes.c_long
+
+    def call(self, name: str, *args) -> None:
+        values = [a.ctypes.data_as(ctypes.c_void_p) if isinstance(a, np.ndarray)
+                  else ctypes.c_int64(a) if isinstance(a, int) else a for a in args]
+        if getattr(self.lib, name)(*values):
+            raise RuntimeError(self.lib.hg_last_error().decode())
+
+    def launches(self, part: str) -> int:
+        return self.fake.fake_launches(part.encode())
+
+    def mesh(self, n: int) -> ctypes.c_void_p:
+        xyz = np.random.default_rng(n).random((n, 3), dtype=np.float32)
+        faces = (np.arange(3 * n, dtype=np.int32) % n)
+        handle = ctypes.c_void_p()
+        self.call("hg_mesh_create", xyz, n, faces, n, None, ctypes.byref(handle))
+        return handle
+
+    def geodesic(self, mesh, n: int, columns: int, mode: int = FACTORED) -> None:
+        sources = np.zeros(columns, np.int32)
+        out = np.zeros((columns, n))
+        self.call("hg_geodesic", mesh, sources, np.arange(columns + 1), columns, out, mode, 0, None)
+
+    def diffuse(self, mesh, n: int, columns: int) -> None:
+        fields = np.zeros((2, columns, n))
+        self.call("hg_diffuse", mesh, fields[0], fields[1], columns, ITERATE, 0, None)
+
+    def solve_poisson(self, mesh, n: int, columns: int) -> None:
+        fields = np.zeros((2, columns, n))
+        self.call("hg_solve_poisson", mesh, fields[0], fields[1], columns, ITERATE, 0)
+
+    def device_bytes(self, mesh) -> int:
+        out = ctypes.c_int64()
+        self.call("hg_device_bytes", mesh, ctypes.byref(out))
+        return out.value
+
+
+def _alone(name: str, tmp_path) -> None:
+    fake = tmp_path / "fake_hip.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", str(ROOT / "tests" / "fake_hip.cpp"), "-o", str(fake)],
+                   check=True)
+    run = subprocess.run([sys.executable, __file__, name, str(fake)], capture_output=True, text=True,
+                         timeout=100)
+    assert run.returncode == 0, run.stdout + run.stderr
+
+
+def _failing(lib: Library, attempt) -> None:
+    """`attempt` with each of its allocations failing in turn: `attempt(None)` is one that may fail,
+    `attempt(error)` what must hold after it did."""
+    for n in range(1, 1000):
+        state = attempt(None)
+        lib.fake.fake_fail_allocation(n)
+        try:
+            state()
+            error = None
+        except RuntimeError as raised:
+            error = str(raised)
+        if lib.fake.fake_failure_pending():
+            assert error is None and n > 1
+            return
+        # (A capture that runs out of memory falls back to an eager solve.)
+        assert error is None or "out of memory" in error, (n, error)
+        attempt(n)
+    raise AssertionError("the call never ran out of allocations")
+
+
+def workspaces_after_a_failed_allocation(lib: Library) -> None:
+    """A call that could not allocate says so, holds no more than the mesh counts, and leaves
+    workspaces that a narrower call can trust: none of theirs is missing."""
+    n = 300
+    held = {}
+
+    def attempt(failed):
+        if failed is None:
+            held["mesh"] = lib.mesh(n)
+            lib.geodesic(held["mesh"], n, 1)
+            lib.diffuse(held["mesh"], n, 2)
+            held["bytes"] = lib.device_bytes(held["mesh"])
+
+            def wide():
+                lib.geodesic(held["mesh"], n, 4)
+                lib.call("hg_release", held["mesh"])
+                lib.diffuse(held["mesh"], n, 3)
+
+            return wide
+        assert lib.device_bytes(held["mesh"]) <= lib.fake.fake_live_bytes(), failed
+        lib.geodesic(held["mesh"], n, 1)
+        lib.call("hg_release", held["mesh"])
+        lib.diffuse(held["mesh"], n, 2)
+        lib.geodesic(held["mesh"], n, 1)
+        assert lib.device_bytes(held["mesh"]) >= held["bytes"], failed
+        lib.call("hg_mesh_destroy", held["mesh"])
+        return None
+
+    _failing(lib, attempt)
+
+
+def server_after_a_failed_allocation(lib: Library) -> None:
+    """A query that a worker's buffers could not grow for fails alone: the next one is answered."""
+    n = 300
+    xyz = np.random.default_rng(n).random((n, 3), dtype=np.float32)
+    faces = np.arange(3 * n, dtype=np.int32) % n
+    out = np.zeros(n)
+    held = {}
+
+    def query():
+        ticket, done = ctypes.c_int64(), ctypes.c_int32()
+        sources = np.zeros(2000, np.int32)
+        lib.call("hg_server_submit", held["server"], held["id"].value, sources, len(sources), out,
+                 ctypes.byref(ticket))
+        lib.call("hg_server_wait", held["server"], ticket.value, ctypes.c_double(20000.0),
+                 ctypes.byref(done))
+        assert done.value
+
+    def attempt(failed):
+        if failed is None:
+            server, held["id"] = ctypes.c_void_p(), ctypes.c_int64()
+            lib.call("hg_server_create", 1 << 40, 1, 8, 0, ctypes.byref(server))
+            held["server"] = server
+            lib.call("hg_server_add_mesh", server, xyz, n, faces, n, ctypes.byref(held["id"]))
+            return query
+        query()
+        lib.call("hg_server_destroy", held["server"])
+        return None
+
+    _failing(lib, attempt)
+
+
+def test_workspaces_after_a_failed_allocation(tmp_path):
+    _alone("workspaces_after_a_failed_allocation", tmp_path)
+
+
+def test_server_after_a_failed_allocation(tmp_path):
+    _alone("server_after_a_failed_allocation", tmp_path)
+
+
+if __name__ == "__main__":
+    globals()[sys.argv[1]](Library(sys.argv[2]))
