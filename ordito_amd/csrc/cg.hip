@@ -10,6 +10,8 @@
 // with grid-wide barriers, so nothing returns to the host until the solve ends. Every block folds
 // the per-block partials in the same fixed order, so all blocks agree on alpha, beta and the stop
 // decision bit for bit (the redundant fold ordito uses instead of a barrier, here beside one).
+#include <utility>
+
 #include <hipcub/hipcub.hpp>
 
 #include "kernels.h"
@@ -1048,15 +1050,20 @@ bool wants_spatial_order(int64_t n, int64_t n_columns) {
 
 void spatial_order(const float* xyz, int64_t n, SpatialOrder& out, CgWorkspace& ws,
                    hipStream_t stream) {
-  out.order.allocate(std::max<int64_t>(n, 1));
-  out.inverse.allocate(std::max<int64_t>(n, 1));
-  if (n == 0) return;
+  // `out` takes the order once it is complete: one that could not be built is built by a later call.
+  SpatialOrder built;
+  built.order.allocate(std::max<int64_t>(n, 1));
+  built.inverse.allocate(std::max<int64_t>(n, 1));
+  if (n == 0) {
+    out = std::move(built);
+    return;
+  }
   // Keys, sorted keys, indices, bounds and the sort's storage, in the exchange of the solve that
   // follows.
   size_t bytes = 0;
   uint32_t* keys = nullptr;
   int32_t* ids = nullptr;
-  HG_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, keys, keys, ids, out.order.ptr,
+  HG_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, keys, keys, ids, built.order.ptr,
                                             static_cast<int>(n), 0, 30, stream));
   const int64_t head = (4 * (3 * n + 6) + 255) / 256 * 256;
   reserve_exchange(ws, std::max(exchange_words(n), (head + static_cast<int64_t>(bytes) + 7) / 8));
@@ -1069,10 +1076,11 @@ void spatial_order(const float* xyz, int64_t n, SpatialOrder& out, CgWorkspace& 
   bounds_kernel<<<std::min(blocks, 256u), kBlock, 0, stream>>>(xyz, n, bounds);
   morton_kernel<<<blocks, kBlock, 0, stream>>>(xyz, n, bounds, keys, ids);
   HG_HIP(hipGetLastError());
-  HG_HIP(hipcub::DeviceRadixSort::SortPairs(temp, bytes, keys, keys + n, ids, out.order.ptr,
+  HG_HIP(hipcub::DeviceRadixSort::SortPairs(temp, bytes, keys, keys + n, ids, built.order.ptr,
                                             static_cast<int>(n), 0, 30, stream));
-  invert_kernel<<<blocks, kBlock, 0, stream>>>(out.order.ptr, n, out.inverse.ptr);
+  invert_kernel<<<blocks, kBlock, 0, stream>>>(built.order.ptr, n, built.inverse.ptr);
   HG_HIP(hipGetLastError());
+  out = std::move(built);
 }
 
 int32_t run_cg(const CgProblem& problem, CgWorkspace& ws, hipStream_t stream) {

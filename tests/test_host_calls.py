@@ -158,12 +158,36 @@ def server_after_a_failed_allocation(lib: Library) -> None:
     _failing(lib, attempt)
 
 
+def row_order_after_a_failed_allocation(lib: Library) -> None:
+    """A solve whose state stays on the chip indexes by the rows' order, which must have been built."""
+    n = 2000
+    held = {}
+
+    def attempt(failed):
+        if failed is None:
+            held["mesh"] = lib.mesh(n)
+            held["inverted"] = lib.launches("invert_kernel")
+            return lambda: lib.solve_poisson(held["mesh"], n, 1)
+        solves = lib.launches("cg_resident_kernel")
+        lib.solve_poisson(held["mesh"], n, 1)
+        assert lib.launches("cg_resident_kernel") == solves + 1, failed
+        assert lib.launches("invert_kernel") > held["inverted"], failed
+        lib.call("hg_mesh_destroy", held["mesh"])
+        return None
+
+    _failing(lib, attempt)
+
+
 def test_workspaces_after_a_failed_allocation(tmp_path):
     _alone("workspaces_after_a_failed_allocation", tmp_path)
 
 
 def test_server_after_a_failed_allocation(tmp_path):
     _alone("server_after_a_failed_allocation", tmp_path)
+
+
+def test_row_order_after_a_failed_allocation(tmp_path):
+    _alone("row_order_after_a_failed_allocation", tmp_path)
 
 
 if __name__ == "__main__":
