@@ -196,8 +196,8 @@ int hg_set_budget_probe(hg_mesh* mesh, int32_t probe);
 /*
  * How often a one-launch sweep's waits poll before it gives up and its solve starts over level by
  * level, as this mesh's solves then do from then on (default 2^21, about two seconds; 0 gives up at
- * the first value not there yet). Setting it returns the mesh to one-launch sweeps. No counterpart
- * in the reference.
+ * the first value not there yet; at most 2^31 - 2). Setting it returns the mesh to one-launch sweeps.
+ * No counterpart in the reference.
  */
 int hg_set_sweep_patience(hg_mesh* mesh, int64_t polls);
 

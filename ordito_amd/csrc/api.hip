@@ -10,6 +10,7 @@
 
 #include "cholesky.h"
 #include "multigrid.h"
+#include "words.h"
 
 namespace hg {
 
@@ -1655,7 +1656,8 @@ int hg_set_budget_probe(hg_mesh* mesh, int32_t probe) {
 int hg_set_sweep_patience(hg_mesh* mesh, int64_t polls) {
   return guarded([&] {
     require_mesh(mesh);
-    HG_REQUIRE(polls >= 0, HG_ERR_VALUE, "a negative number of polls");
+    HG_REQUIRE(polls >= 0 && polls <= kMostPolls, HG_ERR_VALUE,
+               "the polls of a wait must lie in [0, " + std::to_string(kMostPolls) + "]");
     invalidate_graphs(*mesh);
     for (SolveWorkspace* ws : {&mesh->solve, &mesh->solve_side}) {
       ws->patience = polls;

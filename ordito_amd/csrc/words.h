@@ -40,8 +40,11 @@ __device__ __forceinline__ uint64_t peek(const double* word) {
 // This wave's stores have reached the point of coherence.
 __device__ __forceinline__ void drain_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// A wait's patience: false once it has polled past `limit` or another wait has given up, which it
-// then tells everyone by setting `bit` of *flag.
+// The most polls a wait may be told to make: its count of them goes one further.
+constexpr int64_t kMostPolls = (int64_t{1} << 31) - 2;
+
+// A wait's patience: false once it has polled past `limit` (at most kMostPolls) or another wait has
+// given up, which it then tells everyone by setting `bit` of *flag.
 __device__ __forceinline__ bool wait_on(int32_t* flag, int32_t bit, int64_t limit, int32_t& polls,
                                         bool& aborted) {
   if (aborted) return false;

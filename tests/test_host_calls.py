@@ -178,6 +178,20 @@ def row_order_after_a_failed_allocation(lib: Library) -> None:
     _failing(lib, attempt)
 
 
+def a_wait_is_bounded(lib: Library) -> None:
+    """The waits count their polls in 32 bits: a patience such a count cannot pass is refused."""
+    mesh = lib.mesh(300)
+    for polls in (0, 1 << 21, 2**31 - 2):
+        lib.call("hg_set_sweep_patience", mesh, polls)
+    for polls in (-1, 2**31 - 1, 2**31, 1 << 40, 2**63 - 1):
+        try:
+            lib.call("hg_set_sweep_patience", mesh, polls)
+        except RuntimeError as error:
+            assert "2147483646" in str(error)
+        else:
+            raise AssertionError(f"{polls} polls accepted")
+
+
 def test_workspaces_after_a_failed_allocation(tmp_path):
     _alone("workspaces_after_a_failed_allocation", tmp_path)
 
@@ -188,6 +202,10 @@ def test_server_after_a_failed_allocation(tmp_path):
 
 def test_row_order_after_a_failed_allocation(tmp_path):
     _alone("row_order_after_a_failed_allocation", tmp_path)
+
+
+def test_a_wait_is_bounded(tmp_path):
+    _alone("a_wait_is_bounded", tmp_path)
 
 
 if __name__ == "__main__":
