@@ -98,7 +98,7 @@ struct hg_mesh {
   bool has_heat_pins = false;
   // Cholesky.
   AnalysisOptions options;                  // nested-dissection leaf and top-merge sizes
-  std::unique_ptr<std::array<int64_t, 3>> unmerged_sizes;  // planned_peak_bytes'
+  std::unique_ptr<std::array<int64_t, 3>> unmerged_sizes;  // unmerged_peak_bytes'
   int32_t split_target = kDefaultSplitTarget;  // sweep tasks a level is split towards
   std::unique_ptr<Plan> host_plan;
   std::unique_ptr<DevicePlan> plan;
@@ -419,7 +419,7 @@ void ensure_operators(hg_mesh& m) {
 
 void ensure_plan(hg_mesh& m) {
   if (m.plan) return;
-  // Under a budget the plan keeps every separator its own front (planned_peak_bytes).
+  // Under a budget the plan keeps every separator its own front (unmerged_peak_bytes).
   AnalysisOptions options = m.options;
   if (m.budget > 0) options.merge_rows = 0;
   m.host_plan = std::make_unique<Plan>(analyse(m.pattern, m.h_xyz.data(), options));
@@ -522,15 +522,20 @@ void ensure_pinned_system(hg_mesh& m) {
   invalidate_graphs(m);
 }
 
-// A factorization's peak device memory: the transient front arena plus the blocks it keeps.
+// The peak a factorization's budget is held against: the transient front arena plus the blocks it
+// keeps, their structural nonzeros counted beside what is stored.
 int64_t factor_peak_bytes(const DevicePlan& plan, bool keep_fp32) {
   return 8 * plan.arena_size + (keep_fp32 ? 12 : 8) * plan.w_size + 8 * plan.nnz_w;
 }
 
-// The peak a budget is held against: that of the plan with every separator its own front, which is the
-// mesh's own plan unless the budget was set when a factor was held.
-int64_t planned_peak_bytes(hg_mesh& m, bool keep_fp32) {
-  if (m.budget <= 0 || !m.host_plan->merged) return factor_peak_bytes(*m.plan, keep_fp32);
+// What factor_numeric has allocated at its peak: the arena, the blocks and the operator's values.
+int64_t factor_allocated_bytes(const DevicePlan& plan, bool keep_fp32) {
+  return 8 * plan.arena_size + (keep_fp32 ? 12 : 8) * plan.w_size + 8 * plan.nnz;
+}
+
+// factor_peak_bytes of the plan with every separator its own front.
+int64_t unmerged_peak_bytes(hg_mesh& m, bool keep_fp32) {
+  if (!m.host_plan->merged) return factor_peak_bytes(*m.plan, keep_fp32);
   if (!m.unmerged_sizes) {
     AnalysisOptions options = m.options;
     options.merge_rows = 0;
@@ -542,16 +547,66 @@ int64_t planned_peak_bytes(hg_mesh& m, bool keep_fp32) {
   return 8 * s[0] + (keep_fp32 ? 12 : 8) * s[1] + 8 * s[2];
 }
 
+Factor& factor_of(hg_mesh& m, int32_t system) {
+  return system == HG_SYSTEM_HEAT      ? m.heat_factor
+         : system == HG_SYSTEM_POISSON ? m.poisson_factor
+         : system == HG_SYSTEM_PINNED  ? m.pinned_factor
+                                       : m.reg_factor;
+}
+
+// The numeric factorization of a system through the mesh's plan.
+void factor_values(hg_mesh& m, int32_t system, bool keep_fp32) {
+  invalidate_graphs(m);
+  Factor& target = factor_of(m, system);
+  if (system == HG_SYSTEM_POISSON) {
+    factor_numeric(*m.plan, m.poisson.ptr, m.poisson_pinned_new.ptr, m.poisson_pin_slots, target,
+                   keep_fp32, m.stream);
+    return;
+  }
+  const double* values = system == HG_SYSTEM_HEAT     ? m.heat.ptr
+                         : system == HG_SYSTEM_PINNED ? m.pinned.ptr
+                                                      : m.reg.ptr;
+  factor_numeric(*m.plan, values, m.has_heat_pins ? m.heat_pinned_new.ptr : nullptr,
+                 m.heat_pin_slots, target, keep_fp32, m.stream);
+}
+
+// The unmerged plan in a merged one's place, and the factors held on that one formed again on it.
+void replace_merged_plan(hg_mesh& m) {
+  constexpr int32_t kSystems[] = {HG_SYSTEM_HEAT, HG_SYSTEM_POISSON, HG_SYSTEM_PINNED,
+                                  HG_SYSTEM_REGULARIZED};
+  int32_t held = 0, held_fp32 = 0;
+  HG_HIP(hipStreamSynchronize(m.stream));
+  invalidate_graphs(m);
+  for (int32_t system : kSystems) {
+    Factor& factor = factor_of(m, system);
+    if (factor.held()) held |= system;
+    if (factor.w32.ptr) held_fp32 |= system;
+    factor.reset();
+  }
+  m.plan.reset();
+  m.host_plan.reset();
+  m.options.merge_rows = 0;
+  ensure_plan(m);
+  for (int32_t system : kSystems)
+    if (held & system) factor_values(m, system, (held_fp32 & system) != 0);
+}
+
 // Refuse (HG_ERR_BUDGET) a factorization whose peak exceeds the budget, as sparse_cholesky refuses
 // one past CHOLESKY_MEMORY_BUDGET (cholesky.py:72, linalg.py:2393-2420); the system is then solved
-// by iteration. With no budget set the limit is 90 % of the device memory free now.
+// by iteration. With no budget set the limit is 90 % of the device memory free now. A budget is held
+// against the unmerged plan's peak; where only that plan keeps within the limit, it takes the merged
+// one's place.
 void require_budget(hg_mesh& m, int32_t system, bool keep_fp32) {
-  const int64_t need = planned_peak_bytes(m, keep_fp32);
   int64_t limit = m.budget;
   if (limit <= 0) {
     size_t free_bytes = 0, total_bytes = 0;
     HG_HIP(hipMemGetInfo(&free_bytes, &total_bytes));
     limit = static_cast<int64_t>(0.9 * static_cast<double>(free_bytes));
+  }
+  int64_t need = factor_peak_bytes(*m.plan, keep_fp32);
+  if (m.host_plan->merged && (m.budget > 0 || need > limit)) {
+    need = unmerged_peak_bytes(m, keep_fp32);
+    if (need <= limit && factor_allocated_bytes(*m.plan, keep_fp32) > limit) replace_merged_plan(m);
   }
   if (need > limit) m.refused |= system;
   HG_REQUIRE(need <= limit, HG_ERR_BUDGET,
@@ -568,7 +623,7 @@ bool exceeds_budget(hg_mesh& m, int32_t system) {
   if (m.refused & system) return true;
   if (m.budget <= 0 || !m.budget_probe) return false;
   ensure_plan(m);
-  if (planned_peak_bytes(m, false) <= m.budget) return false;
+  if (unmerged_peak_bytes(m, false) <= m.budget) return false;
   m.refused |= system;
   return true;
 }
@@ -582,9 +637,7 @@ void factor_system(hg_mesh& m, int32_t system, bool keep_fp32) {
     PhaseScope scope(&m.timer, kPhaseFactor, m.stream);
     if (!m.pinned_factor.held() || (keep_fp32 && !m.pinned_factor.w32.ptr)) {
       require_budget(m, system, keep_fp32);
-      invalidate_graphs(m);
-      factor_numeric(*m.plan, m.pinned.ptr, m.has_heat_pins ? m.heat_pinned_new.ptr : nullptr,
-                     m.heat_pin_slots, m.pinned_factor, keep_fp32, m.stream);
+      factor_values(m, system, keep_fp32);
     }
     return;
   }
@@ -593,30 +646,15 @@ void factor_system(hg_mesh& m, int32_t system, bool keep_fp32) {
     PhaseScope scope(&m.timer, kPhaseFactor, m.stream);
     if (!m.reg_factor.held() || (keep_fp32 && !m.reg_factor.w32.ptr)) {
       require_budget(m, system, keep_fp32);
-      invalidate_graphs(m);
-      factor_numeric(*m.plan, m.reg.ptr, m.has_heat_pins ? m.heat_pinned_new.ptr : nullptr,
-                     m.heat_pin_slots, m.reg_factor, keep_fp32, m.stream);
+      factor_values(m, system, keep_fp32);
     }
     return;
   }
-  Factor& target = system == HG_SYSTEM_HEAT ? m.heat_factor : m.poisson_factor;
-  if (!target.held() || (keep_fp32 && !target.w32.ptr)) {
-    require_budget(m, system, keep_fp32);
-    invalidate_graphs(m);
-  }
+  const Factor& target = factor_of(m, system);
+  const bool wanted = !target.held() || (keep_fp32 && !target.w32.ptr);
+  if (wanted) require_budget(m, system, keep_fp32);
   PhaseScope scope(&m.timer, kPhaseFactor, m.stream);
-  if (system == HG_SYSTEM_HEAT) {
-    if (!m.heat_factor.held())
-      factor_numeric(*m.plan, m.heat.ptr, m.has_heat_pins ? m.heat_pinned_new.ptr : nullptr,
-                     m.heat_pin_slots, m.heat_factor, keep_fp32, m.stream);
-    else if (keep_fp32 && !m.heat_factor.w32.ptr)
-      factor_numeric(*m.plan, m.heat.ptr, m.has_heat_pins ? m.heat_pinned_new.ptr : nullptr,
-                     m.heat_pin_slots, m.heat_factor, true, m.stream);
-  } else {
-    if (!m.poisson_factor.held() || (keep_fp32 && !m.poisson_factor.w32.ptr))
-      factor_numeric(*m.plan, m.poisson.ptr, m.poisson_pinned_new.ptr, m.poisson_pin_slots,
-                     m.poisson_factor, keep_fp32, m.stream);
-  }
+  if (wanted) factor_values(m, system, keep_fp32);
 }
 
 // ---- solves -----------------------------------------------------------------------------------
@@ -804,7 +842,6 @@ void solve_poisson(hg_mesh& m, double* rhs, double* x, int64_t k, int32_t mode,
   Factor& factor = regularized ? m.reg_factor : m.poisson_factor;
   const double* values = regularized ? m.reg.ptr : m.poisson.ptr;
   const double* inv_diag = regularized ? m.reg_inv.ptr : m.poisson_inv.ptr;
-  const int32_t* pins = poisson_pins(m, regularized);
   bool factored = mode == HG_MODE_FACTORED || factor.held() || m.heat_factor.held();
   if (factored && rhs_layout == FieldLayout::kColumns && x_layout == FieldLayout::kColumns) {
     // By columns a refusal under the budget leaves the solve to the iteration.
@@ -819,8 +856,8 @@ void solve_poisson(hg_mesh& m, double* rhs, double* x, int64_t k, int32_t mode,
     factor_system(m, system, mixed);
     m.stats.poisson_refinements = refined_solve(
         *m.plan, factor, mixed, rhs, x, k, m.refine_tolerance[mixed ? 1 : 0][1], false,
-        mixed ? kMixedRefineRounds : kRefineRounds, pins, m.solve, m.stream, &m.timer,
-        kPhasePoissonSweep, rhs_layout, x_layout,
+        mixed ? kMixedRefineRounds : kRefineRounds, poisson_pins(m, regularized), m.solve,
+        m.stream, &m.timer, kPhasePoissonSweep, rhs_layout, x_layout,
         m.speculating ? m.d_flags.ptr + 1 + 2 * m.spec_chunks : nullptr, nullptr, m.maxima.ptr);
     m.stats.poisson_rounds = 0;
   } else {
@@ -1543,6 +1580,7 @@ int hg_set_plan_options(hg_mesh* mesh, int32_t leaf_rows, int32_t top_rows,
       m.plan.reset();
       m.host_plan.reset();
       m.unmerged_sizes.reset();
+      m.options.merge_rows = defaults.merge_rows;
       m.options.leaf_rows = leaf;
       m.options.top_rows = top;
       m.split_target = split;
