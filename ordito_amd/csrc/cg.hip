@@ -1088,7 +1088,6 @@ int32_t run_cg(const CgProblem& problem, CgWorkspace& ws, hipStream_t stream) {
   const int64_t k = problem.n_columns;
   HG_REQUIRE(k >= 1 && k <= kMaxColumns, HG_ERR_VALUE, "conjugate gradient takes 1-64 columns");
   if (n == 0) return 0;
-  const WaitClaim claim(true, true);
   if (ws.counters.size < 4 + kBarrierGroups) ws.counters.allocate(4 + kBarrierGroups);
   CgArgs a{};
   a.n = n;
@@ -1133,6 +1132,7 @@ int32_t run_cg(const CgProblem& problem, CgWorkspace& ws, hipStream_t stream) {
                         kBlock, 0, stream>>>(reinterpret_cast<uint64_t*>(ws.exchange.ptr), words);
     HG_HIP(hipGetLastError());
     // Cooperative: every block waits for words of the others, so all must be resident.
+    const WaitClaim claim(true, true);
     HG_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(choice.kernel),
                                       dim3(static_cast<unsigned>(G)), dim3(choice.threads), args,
                                       0, stream));
@@ -1161,6 +1161,7 @@ int32_t run_cg(const CgProblem& problem, CgWorkspace& ws, hipStream_t stream) {
   a.da = base + 7 * entries;
   a.db = base + 8 * entries;
   a.partials = ws.partials.ptr;
+  const WaitClaim claim(!single, true);
   if (single) {
     hipLaunchKernelGGL((cg_kernel<1024, true>), dim3(1), dim3(1024), 0, stream, a);
     HG_HIP(hipGetLastError());

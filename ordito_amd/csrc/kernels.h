@@ -41,7 +41,7 @@ inline int32_t pair_rows(int32_t kk) {
 }
 
 // A process's claim, while it lives, on the device's kernels whose blocks wait for words that others of
-// their launch write (flow.hip's sweeps, the conjugate gradients): one holder at a time. The hardware
+// their launch write (flow.hip's sweeps, conjugate gradients of several blocks): one holder at a time. The hardware
 // hands each XCD its blocks in order, but not the XCDs theirs in step, so two such launches on two
 // streams can each fill one XCD's compute units with blocks that wait for what the other XCD's queue
 // holds behind the other launch's; both then wait out their patience. With 64 meshes served by four

@@ -9,9 +9,11 @@ Each test runs in a process of its own, which binds the library to that runtime.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import subprocess
 import sys
+import threading
 from pathlib import Path
 
 import numpy as np
@@ -94,6 +96,63 @@ def _failing(lib: Library, attempt) -> None:
         assert error is None or "out of memory" in error, (n, error)
         attempt(n)
     raise AssertionError("the call never ran out of allocations")
+
+
+@contextlib.contextmanager
+def _held(lib: Library, kernel: str, call):
+    """`call` running on another thread, held where it launches `kernel` until the block ends."""
+    failures = []
+
+    def work():
+        try:
+            call()
+        except Exception as error:  # reported by the test's thread
+            failures.append(error)
+
+    lib.fake.fake_gate(kernel.encode())
+    thread = threading.Thread(target=work)
+    thread.start()
+    try:
+        assert lib.fake.fake_held(), f"{kernel} was not launched {failures}"
+        yield
+        assert thread.is_alive()
+    finally:
+        lib.fake.fake_open()
+        thread.join(20)
+    assert not thread.is_alive() and not failures, failures
+
+
+def _beside(call, seconds: float = 20.0) -> dict:
+    """`call` on a thread of its own: what it returned, or that it did not end in time."""
+    out = {}
+
+    def work():
+        try:
+            out["value"] = call()
+        except Exception as error:  # reported by the test's thread
+            out["error"] = error
+
+    thread = threading.Thread(target=work, daemon=True)
+    thread.start()
+    thread.join(seconds)
+    out["ended"] = not thread.is_alive()
+    out["thread"] = thread
+    assert "error" not in out, out["error"]
+    return out
+
+
+def iterations_of_one_block_run_beside_others(lib: Library) -> None:
+    """Conjugate gradients of one block wait for no other block, so they run whatever else does; two
+    of several blocks take turns."""
+    large, other, small, middle = (lib.mesh(n) for n in (2000, 2100, 300, 3000))
+    with _held(lib, "cg_resident_kernel", lambda: lib.solve_poisson(large, 2000, 1)):
+        assert _beside(lambda: lib.diffuse(small, 300, 1))["ended"]
+        assert _beside(lambda: lib.solve_poisson(small, 300, 1))["ended"]
+        assert _beside(lambda: lib.diffuse(middle, 3000, 4))["ended"]
+        waits = _beside(lambda: lib.solve_poisson(other, 2100, 1), 0.3)
+        assert not waits["ended"]
+    waits["thread"].join(20)
+    assert not waits["thread"].is_alive()
 
 
 def workspaces_after_a_failed_allocation(lib: Library) -> None:
@@ -206,6 +265,10 @@ def test_row_order_after_a_failed_allocation(tmp_path):
 
 def test_a_wait_is_bounded(tmp_path):
     _alone("a_wait_is_bounded", tmp_path)
+
+
+def test_iterations_of_one_block_run_beside_others(tmp_path):
+    _alone("iterations_of_one_block_run_beside_others", tmp_path)
 
 
 if __name__ == "__main__":
