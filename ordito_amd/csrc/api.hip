@@ -1079,7 +1079,7 @@ bool graphable(const hg_mesh& m, int32_t mode, int32_t precision) {
          (m.method != HG_METHOD_IGL || m.n_rim == 0 || m.pinned_factor.held());
 }
 
-bool solve_columns(hg_mesh& m, const int64_t* offsets, int64_t k, double* phi, int32_t mode,
+bool solve_columns(hg_mesh& m, const int64_t* offsets, int64_t k, double* phi, bool factored,
                    int32_t precision, bool finish);
 
 // The factored FP64 path of hg_geodesic replayed as one graph: captured on the first such call at
@@ -1133,15 +1133,18 @@ struct SideStream {
 };
 thread_local SideStream t_side_stream;
 
-// The WaitClaim of a call of k columns, if its last chunk is narrow enough to sweep in one launch, and the
-// main workspace's leave to (the side one never has it: its sweeps run beside these).
+// The WaitClaim of a call that solves k columns by speculation, up to its last synchronization, if its
+// last chunk is narrow enough to sweep in one launch, and the main workspace's leave to (the side one
+// never has it: its sweeps run beside these). Other solves wait for their verdicts, and claim the
+// device for themselves (refined_solve).
 struct FlowScope {
   hg_mesh& m;
   const bool wanted;
   WaitClaim claim;
-  FlowScope(hg_mesh& mesh, int64_t k)
+  FlowScope(hg_mesh& mesh, bool speculates, int64_t k)
       : m(mesh),
-        wanted((k + kFieldChunk - 1) % kFieldChunk < kFlowColumns && k > 0),
+        wanted(speculates && k > 0 && (k + kFieldChunk - 1) % kFieldChunk < kFlowColumns &&
+               !mesh.solve.level_sweeps),
         claim(wanted, false) {
     m.solve.flows = claim.held();
   }
@@ -1174,7 +1177,7 @@ bool run_graph(hg_mesh& m, const int64_t* offsets, int64_t k, double* d_out, int
       ok = hipStreamBeginCapture(gs.stream, hipStreamCaptureModeRelaxed) == hipSuccess;
       if (ok) {
         try {
-          solve_columns(m, offsets, k, d_out, HG_MODE_FACTORED, precision, true);
+          solve_columns(m, offsets, k, d_out, true, precision, true);
         } catch (...) {
           ok = false;
         }
@@ -1201,13 +1204,34 @@ bool run_graph(hg_mesh& m, const int64_t* offsets, int64_t k, double* d_out, int
   return !speculation_failed(m);
 }
 
+// Whether a geodesic call solves through the factors: every system its path solves is factored here,
+// and the divergence's records formed. One refused under the memory budget sends the whole call down
+// the iterated path (packed meshes have none: the refusal stands).
+bool ready_factors(hg_mesh& m, int32_t mode, int32_t precision) {
+  if (mode != HG_MODE_FACTORED && !m.heat_factor.held()) return false;
+  ensure_operators(m);
+  const bool mixed = precision == HG_PRECISION_MIXED;
+  try {
+    factor_system(m, HG_SYSTEM_HEAT, mixed);
+    factor_system(m, m.method == HG_METHOD_POTPOURRI3D ? HG_SYSTEM_REGULARIZED : HG_SYSTEM_POISSON,
+                  mixed);
+    if (m.method == HG_METHOD_IGL && m.n_rim > 0) factor_system(m, HG_SYSTEM_PINNED, mixed);
+    ensure_corner_geometry(m);
+  } catch (const Error& e) {
+    if (!is_budget_refusal(e) || m.segments() > 1) throw;
+    return false;
+  }
+  return true;
+}
+
 // Seed, heat step, divergence and Poisson step over k columns of the whole (possibly packed)
-// system into phi (the caller's layout). The sources must be uploaded. With `finish` and the
+// system into phi (the caller's layout), through the factors (ready_factors) or iterated. The sources
+// must be uploaded. With `finish` and the
 // fields stored by rows, phi (where the uploaded slots point) is the finished distance (null space
 // removed, shifted, oriented) and
 // the call returns true; otherwise phi is the unshifted distance with each component's mean
 // removed.
-bool solve_columns(hg_mesh& m, const int64_t* offsets, int64_t k, double* phi, int32_t mode,
+bool solve_columns(hg_mesh& m, const int64_t* offsets, int64_t k, double* phi, bool factored,
                    int32_t precision, bool finish = false) {
   const int64_t n = m.n;
   double* fields = reserve_fields(m, k);
@@ -1216,26 +1240,10 @@ bool solve_columns(hg_mesh& m, const int64_t* offsets, int64_t k, double* phi, i
   double* negdiv = fields + 2 * n * k;
   // Through the factors the intermediate fields stay in the solves' row layout, in the elimination
   // order: the seeds land there, the heat step's solution stays there for the divergence, which
-  // writes the Poisson step's right-hand side there; only the distance is permuted out. Every
-  // system the path solves is factored first; one refused under the memory budget sends the whole
-  // call down the iterated path (packed meshes have none: the refusal stands).
-  bool factored = mode == HG_MODE_FACTORED || m.heat_factor.held();
+  // writes the Poisson step's right-hand side there; only the distance is permuted out.
   // geometry-central's Poisson step at HG_METHOD_POTPOURRI3D (heat.py:3121-3128).
   const bool regularized = m.method == HG_METHOD_POTPOURRI3D;
-  if (factored) {
-    ensure_operators(m);
-    const bool mixed = precision == HG_PRECISION_MIXED;
-    try {
-      factor_system(m, HG_SYSTEM_HEAT, mixed);
-      factor_system(m, regularized ? HG_SYSTEM_REGULARIZED : HG_SYSTEM_POISSON, mixed);
-      if (m.method == HG_METHOD_IGL && m.n_rim > 0) factor_system(m, HG_SYSTEM_PINNED, mixed);
-      ensure_corner_geometry(m);
-    } catch (const Error& e) {
-      if (!is_budget_refusal(e) || m.segments() > 1) throw;
-      factored = false;
-    }
-  }
-  mode = factored ? HG_MODE_FACTORED : HG_MODE_ITERATE;
+  const int32_t mode = factored ? HG_MODE_FACTORED : HG_MODE_ITERATE;
   const FieldLayout layout = factored ? FieldLayout::kRows : FieldLayout::kColumns;
   seed(m, offsets, k, u0, layout);
   const bool igl = m.method == HG_METHOD_IGL && m.n_rim > 0;
@@ -1623,7 +1631,6 @@ int hg_diffuse(hg_mesh* mesh, const double* d_rhs, double* d_solution, int64_t n
     require_single_or_factored(*mesh, mode);
     SpeculationDisarm disarm(*mesh);
     mesh->stats = hg_solve_stats{};
-    FlowScope flow(*mesh, n_columns);
     // By columns (the caller's layout) the solve only reads its right-hand side.
     int32_t flags = diffuse(*mesh, const_cast<double*>(d_rhs), d_solution, n_columns, mode,
                             precision);
@@ -1642,7 +1649,6 @@ int hg_diffuse_pinned(hg_mesh* mesh, const double* d_rhs, double* d_solution, in
     hg_mesh& m = *mesh;
     SpeculationDisarm disarm(m);
     m.stats = hg_solve_stats{};
-    FlowScope flow(m, n_columns);
     ensure_operators(m);
     int32_t flags = 0;
     if (m.n_rim > 0 && n_columns > 0) {
@@ -1752,7 +1758,6 @@ int hg_solve_poisson(hg_mesh* mesh, const double* d_rhs, double* d_solution, int
     require_single_or_factored(*mesh, mode);
     SpeculationDisarm disarm(*mesh);
     mesh->stats = hg_solve_stats{};
-    FlowScope flow(*mesh, n_columns);
     // By columns (the caller's layout) the solve only reads its right-hand side.
     solve_poisson(*mesh, const_cast<double*>(d_rhs), d_solution, n_columns, mode, precision);
     HG_HIP(hipStreamSynchronize(mesh->stream));
@@ -1898,15 +1903,19 @@ int hg_geodesic(hg_mesh* mesh, const int32_t* d_sources, const int64_t* source_o
       return;
     }
     ensure_operators(m);
-    FlowScope flow(m, k);
     upload_sources(m, d_sources, source_offsets, k, d_out);
+    const bool replays = graphable(m, mode, precision);  // factors formed here are first used eagerly
+    reserve_fields(m, k);
+    const bool factored = ready_factors(m, mode, precision);
+    FlowScope flow(m, factored && precision == HG_PRECISION_FP64, k);
     bool done = false;
-    if (graphable(m, mode, precision) && flow.as_captured()) done = run_graph(m, source_offsets, k, d_out, precision);
+    if (replays && flow.as_captured()) done = run_graph(m, source_offsets, k, d_out, precision);
     if (!done) {
       for (bool speculate : {precision == HG_PRECISION_FP64, false}) {
         m.stats = hg_solve_stats{};
         arm_speculation(m, k, speculate);
-        if (!solve_columns(m, source_offsets, k, d_out, mode, precision, true)) shift(m, d_out, k);
+        if (!solve_columns(m, source_offsets, k, d_out, factored, precision, true))
+          shift(m, d_out, k);
         HG_HIP(hipStreamSynchronize(m.stream));
         if (!speculation_failed(m)) break;
       }
@@ -1992,16 +2001,18 @@ int hg_geodesic_packed(hg_mesh* mesh, const int32_t* d_sources, const int64_t* s
       m.packed_phi.allocate(m.n * width);
       m.packed_capacity = m.n * width;
     }
-    FlowScope flow(m, width);
+    reserve_fields(m, width);
+    ready_factors(m, HG_MODE_FACTORED, precision);
+    FlowScope flow(m, precision == HG_PRECISION_FP64, width);
     arm_speculation(m, width, precision == HG_PRECISION_FP64);
     m.sources_on_device = false;  // the seeds' count is the host's
     m.host_sources = total;
-    solve_columns(m, seed_offsets.data(), width, m.packed_phi.ptr, HG_MODE_FACTORED, precision);
+    solve_columns(m, seed_offsets.data(), width, m.packed_phi.ptr, true, precision);
     // A speculated first round that failed its test: solve again without speculating.
     HG_HIP(hipStreamSynchronize(m.stream));
     if (speculation_failed(m)) {
       m.stats = hg_solve_stats{};
-      solve_columns(m, seed_offsets.data(), width, m.packed_phi.ptr, HG_MODE_FACTORED, precision);
+      solve_columns(m, seed_offsets.data(), width, m.packed_phi.ptr, true, precision);
     }
     // Each query's segment of its slot's column, then its shift against its own sources.
     m.q_src_off.assign(src_off, m.stream);

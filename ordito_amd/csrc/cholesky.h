@@ -122,7 +122,7 @@ constexpr int64_t kSweepPatience = int64_t{1} << 21;
 
 struct SolveWorkspace {
   int64_t patience = kSweepPatience;
-  bool flows = false;  // the call holds the device's WaitClaim: it may sweep in one launch
+  bool flows = false;  // the call holds the device's WaitClaim: its speculated solves may sweep in one launch
   bool level_sweeps = false;  // a one-launch sweep gave up here: level by level from then on
   DeviceArray<double> bp, xa, xb, r, y, d, fvec, bmax, partials;
   DeviceArray<int32_t> pending;

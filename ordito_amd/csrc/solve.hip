@@ -1292,10 +1292,14 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
     double* const x_home = x_layout == FieldLayout::kRows ? xq : ws.xb.ptr;
     double* x_cur = x_home;
     int32_t rounds = 0;
+    // A few columns sweep in one launch (flow.hip) while no such launch has given up here and the
+    // device is claimed for it: by the call where the solve only enqueues, else by the solve, which
+    // waits for every round.
+    const bool narrow = kk <= kFlowColumns && !ws.level_sweeps;
+    const WaitClaim claim(narrow && !speculate, false);
+    const bool claimed = narrow && (speculate ? ws.flows : claim.held());
     while (rounds < max_rounds) {
-      // A few columns sweep in one launch (flow.hip), if the call may and no such launch has given up
-      // here.
-      const bool flows = kk <= kFlowColumns && ws.flows && !ws.level_sweeps;
+      const bool flows = claimed && !ws.level_sweeps;
       double* x_next = x_cur == x_home ? ws.xa.ptr : x_home;
       if (rounds == 0) {
         a.r = bp;

@@ -155,6 +155,34 @@ def iterations_of_one_block_run_beside_others(lib: Library) -> None:
     assert not waits["thread"].is_alive()
 
 
+def preparation_leaves_the_device_unclaimed(lib: Library) -> None:
+    """Only solves keep others from sweeping in one launch: not a call that is still factoring, nor
+    one that iterates."""
+    small, large, fresh = lib.mesh(300), lib.mesh(2000), lib.mesh(400)
+
+    def swept() -> int:
+        before = lib.fake.fake_thread_launches(b"flow_kernel")
+        fields = np.zeros((2, 1, 300))
+        lib.call("hg_diffuse", small, fields[0], fields[1], 1, FACTORED, 0, None)
+        return lib.fake.fake_thread_launches(b"flow_kernel") - before
+
+    def iterates():
+        lib.solve_poisson(large, 2000, 1)
+
+    assert swept() == 1
+    for kernel, call in (("panel_diag", lambda: lib.geodesic(fresh, 400, 1)),
+                         ("cg_resident_kernel", lambda: lib.geodesic(lib.mesh(500), 500, 1, ITERATE))):
+        with _held(lib, kernel, call):
+            assert _beside(swept)["value"] == 1, kernel
+            assert _beside(iterates)["ended"], kernel
+    # One that does hold the claim: a sweep in one launch, and a solve of several blocks.
+    for kernel, call in (("flow_kernel", lambda: lib.geodesic(fresh, 400, 2)),
+                         ("cg_resident_kernel", iterates)):
+        with _held(lib, kernel, call):
+            assert _beside(swept)["value"] == 0, kernel
+    assert swept() == 1
+
+
 def workspaces_after_a_failed_allocation(lib: Library) -> None:
     """A call that could not allocate says so, holds no more than the mesh counts, and leaves
     workspaces that a narrower call can trust: none of theirs is missing."""
@@ -269,6 +297,10 @@ def test_a_wait_is_bounded(tmp_path):
 
 def test_iterations_of_one_block_run_beside_others(tmp_path):
     _alone("iterations_of_one_block_run_beside_others", tmp_path)
+
+
+def test_preparation_leaves_the_device_unclaimed(tmp_path):
+    _alone("preparation_leaves_the_device_unclaimed", tmp_path)
 
 
 if __name__ == "__main__":
