@@ -203,6 +203,13 @@ int hg_set_budget_probe(hg_mesh* mesh, int32_t probe);
 int hg_set_sweep_patience(hg_mesh* mesh, int64_t polls);
 
 /*
+ * How the mesh's refinement rounds were swept since it was bound: out3 = {rounds enqueued as one
+ * launch, rounds enqueued level by level, one-launch sweeps seen to have given up}. A captured
+ * graph's rounds count once, when it is captured. No counterpart in the reference.
+ */
+int hg_sweep_counts(hg_mesh* mesh, int64_t* out3);
+
+/*
  * The settle rule of the heat solves' iteration (solve_spd_settled's check_rounds,
  * change_tolerance and settle_rounds, linalg.py:2490-2560): every check_rounds rounds the iterate
  * stops once each entry changed by less than change_tolerance of itself since the last check, or

@@ -51,6 +51,7 @@ EXPORTED = (
     "hg_set_memory_budget",
     "hg_set_budget_probe",
     "hg_set_sweep_patience",
+    "hg_sweep_counts",
     "hg_set_settle_rule",
     "hg_inverse_factor_entries",
     "hg_set_refinement",
@@ -177,6 +178,7 @@ _SIGNATURES = {
     "hg_set_memory_budget": ([_P, _I64], ctypes.c_int),
     "hg_set_budget_probe": ([_P, _I32], ctypes.c_int),
     "hg_set_sweep_patience": ([_P, _I64], ctypes.c_int),
+    "hg_sweep_counts": ([_P, _PI64], ctypes.c_int),
     "hg_set_settle_rule": ([_P, _I32, ctypes.c_double, _I32], ctypes.c_int),
     "hg_inverse_factor_entries": ([_P, _PI64], ctypes.c_int),
     "hg_set_graphs": ([_P, _I32], ctypes.c_int),

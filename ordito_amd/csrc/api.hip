@@ -1040,8 +1040,10 @@ bool speculation_failed(hg_mesh& m) {
   const bool was = m.speculating;
   m.speculating = false;
   if (!was) return false;
-  return std::any_of(m.h_flags.ptr + 1, m.h_flags.ptr + 1 + 3 * m.spec_chunks,
-                     [](int32_t v) { return v != 0; });
+  int32_t seen = 0;
+  for (int64_t e = 1; e <= 3 * m.spec_chunks; ++e) seen |= m.h_flags.ptr[e];
+  if (seen & kFlowAborted) m.solve.gave_up();  // the solve that follows waits for no such launch again
+  return seen != 0;
 }
 
 // Every buffer and setting a captured geodesic graph names: a replay is valid while all are the
@@ -1706,6 +1708,16 @@ int hg_set_sweep_patience(hg_mesh* mesh, int64_t polls) {
       ws->patience = polls;
       ws->level_sweeps = false;
     }
+  });
+}
+
+int hg_sweep_counts(hg_mesh* mesh, int64_t* out) {
+  return guarded([&] {
+    require_mesh(mesh);
+    HG_REQUIRE(out != nullptr, HG_ERR_VALUE, "out3 is null");
+    out[0] = mesh->solve.flow_count;
+    out[1] = mesh->solve.level_count + mesh->solve_side.level_count;
+    out[2] = mesh->solve.given_up;
   });
 }
 

@@ -124,6 +124,11 @@ struct SolveWorkspace {
   int64_t patience = kSweepPatience;
   bool flows = false;  // the call holds the device's WaitClaim: its speculated solves may sweep in one launch
   bool level_sweeps = false;  // a one-launch sweep gave up here: level by level from then on
+  int64_t flow_count = 0, level_count = 0, given_up = 0;  // hg_sweep_counts
+  void gave_up() {
+    level_sweeps = true;
+    ++given_up;
+  }
   DeviceArray<double> bp, xa, xb, r, y, d, fvec, bmax, partials;
   DeviceArray<int32_t> pending;
   DeviceArray<int32_t> live, live_pairs;  // a call's LiveFronts

@@ -1328,6 +1328,7 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
         }
         a.live = marked ? reached.live : nullptr;
         a.gather_pair = marked ? reached.pairs : plan.gather_pair.ptr;
+        ++(flows ? ws.flow_count : ws.level_count);
         if (!flows) {
           if (fold.partials)
             absmax_final_kernel<<<kk, 256, 0, stream>>>(fold, verdict);
@@ -1374,7 +1375,7 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
       if (timer) timer->resolve();
       if (!pending) break;
       if (pending & kFlowAborted) {  // nothing the round wrote counts: start over level by level
-        ws.level_sweeps = true;
+        ws.gave_up();
         x_cur = x_home;
         rounds = 0;
         continue;
