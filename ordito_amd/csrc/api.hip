@@ -136,6 +136,7 @@ struct hg_mesh {
   // Workspaces.
   CgWorkspace cg;
   SpatialOrder cg_order;  // the iterated solves' row order, built on the first that wants it
+  int32_t longest_row = -1;  // the pattern's, known then
   MarchWorkspace march;  // the band march of a system refused under the budget
   // The Poisson system's multigrid hierarchy, built on its first solve past the budget.
   std::unique_ptr<Multigrid> poisson_mg;
@@ -684,6 +685,12 @@ void order_rows(hg_mesh& m, CgProblem& p) {
   if (!m.cg_order.order.ptr) spatial_order(m.xyz.ptr, m.n, m.cg_order, m.cg, m.stream);
   p.order = m.cg_order.order.ptr;
   p.inverse = m.cg_order.inverse.ptr;
+  if (m.longest_row < 0) {
+    m.longest_row = 0;
+    for (int64_t v = 0; v < m.n; ++v)
+      m.longest_row = std::max(m.longest_row, m.pattern.offsets[v + 1] - m.pattern.offsets[v]);
+  }
+  p.longest_row = m.longest_row;
 }
 
 int32_t diffuse_iterated(hg_mesh& m, const HeatSystem& sys, const double* rhs, double* x,

@@ -442,6 +442,13 @@ __global__ __launch_bounds__(kThreads) void cg_kernel(CgArgs a) {
 // solve repeats bit for bit. Every wait is bounded as the grid barrier's are.
 constexpr int kPhases = 4, kSlotPhases = 3, kSlotWidth = 4;
 
+// A row's thread reads up to so many entries past those in registers, each a chain of three loads. A
+// longer row's are dealt over its wave (kLong), 64 chains at a time: a one-shot call on a cone whose
+// apex has 400 neighbours (8,001 rows) takes 9.0 ms so, 40 with the thread reading them all and 27
+// with the state in memory; 8,000 neighbours (64,001 rows) 73, 670 and 266 ms. Instances of their own,
+// for systems that have such a row: the four rows a thread of the largest have no registers to spare.
+constexpr int32_t kOwnExtra = 16;
+
 // A thread's value of a vector for each of its rows, in registers or in LDS (l = the thread's
 // first entry, entries kStride apart).
 template <int R, int kStride, bool kLds>
@@ -460,9 +467,9 @@ struct RowVector {
 
 // T threads a block, R rows a thread, E operator entries of a row in registers, TV the operator's
 // values (float: the narrowed heat operator), kCheb the polynomial preconditioner, kGrid more than
-// one block. Instances with double values keep x, p, s and r in LDS: they are touched once a round,
+// one block, kLong some rows of more than E + kOwnExtra entries. Instances with double values keep x, p, s and r in LDS: they are touched once a round,
 // and the registers are the operator's.
-template <int T, int R, int E, typename TV, bool kCheb, bool kGrid>
+template <int T, int R, int E, typename TV, bool kCheb, bool kGrid, bool kLong>
 __global__ __launch_bounds__(T) void cg_resident_kernel(CgArgs a) {
   constexpr int L = R * T, kWaves = T / 64;
   static_assert((kWaves & (kWaves - 1)) == 0, "the waves' sums fold in a butterfly");
@@ -530,8 +537,16 @@ __global__ __launch_bounds__(T) void cg_resident_kernel(CgArgs a) {
     }
     if (kGrid)
 #pragma unroll 1
-      for (int32_t e = E; e < degree; ++e)
+      for (int32_t e = E; e < (kLong && extra[j] > kOwnExtra ? 0 : degree); ++e)
         if (locate(a.columns[begin[j] + e]) < 0) outer |= 1u << j;
+    if constexpr (kGrid && kLong)
+      for (uint64_t rows = __ballot(extra[j] > kOwnExtra); rows; rows &= rows - 1) {
+        const int owner = __ffsll(static_cast<unsigned long long>(rows)) - 1;
+        const int32_t from = __shfl(begin[j], owner, 64) + E, more = __shfl(extra[j], owner, 64);
+        bool any = false;
+        for (int32_t e = lane; e < more; e += 64) any |= locate(a.columns[from + e]) < 0;
+        if (__any(any) && lane == owner) outer |= 1u << j;
+      }
   }
 
   // Phase k of the exchange: this thread's rows' values, into LDS and, for rows with a neighbour
@@ -593,7 +608,8 @@ __global__ __launch_bounds__(T) void cg_resident_kernel(CgArgs a) {
         sum += static_cast<double>(val[j][e]) * __builtin_bit_cast(double, raw[e]);
       }
 #pragma unroll 1
-      for (int32_t e = 0; e < extra[j]; ++e) {  // the rest of a long row
+      for (int32_t e = 0; e < (kLong && extra[j] > kOwnExtra ? 0 : extra[j]); ++e) {
+        // The rest of a row longer than E.
         const int32_t c = locate(a.columns[begin[j] + E + e]);
         uint64_t bits;
         if (kGrid && c < 0) {
@@ -605,6 +621,28 @@ __global__ __launch_bounds__(T) void cg_resident_kernel(CgArgs a) {
         }
         sum += static_cast<double>(values[begin[j] + E + e]) * __builtin_bit_cast(double, bits);
       }
+      if constexpr (kLong)
+        for (uint64_t rows = __ballot(extra[j] > kOwnExtra); rows; rows &= rows - 1) {
+          const int owner = __ffsll(static_cast<unsigned long long>(rows)) - 1;
+          const int32_t from = __shfl(begin[j], owner, 64) + E, more = __shfl(extra[j], owner, 64);
+          double part = 0.0;
+#pragma unroll 1
+          for (int32_t e = lane; e < more; e += 64) {
+            const int32_t c = locate(a.columns[from + e]);
+            uint64_t bits;
+            if (kGrid && c < 0) {
+              int32_t polls = 0;
+              while ((bits = at_remote(c)) == kEmpty && wait_on(a.counters + 1, 1, a.spin_limit, polls, aborted)) {
+              }
+            } else {
+              bits = at_local(c);
+            }
+            part += static_cast<double>(values[from + e]) * __builtin_bit_cast(double, bits);
+          }
+#pragma unroll
+          for (int offset = 32; offset > 0; offset >>= 1) part += __shfl_xor(part, offset, 64);
+          if (lane == owner) sum += part;
+        }
       out[j] = sum;
     }
   };
@@ -999,30 +1037,38 @@ struct ResidentChoice {
   int32_t threads = 0, rows = 0;  // rows a block
 };
 
-template <int T, int R, int E, bool kGrid>
-ResidentChoice resident_choice(bool cheb, bool narrow) {
+template <int T, int R, int E, bool kGrid, bool kLong>
+ResidentChoice resident_instance(bool cheb, bool narrow) {
   ResidentChoice c;
   c.threads = T;
   c.rows = T * R;
-  if (cheb) c.kernel = cg_resident_kernel<T, R, E, double, true, kGrid>;
-  else if (narrow) c.kernel = cg_resident_kernel<T, R, E, float, false, kGrid>;
-  else if constexpr (!kGrid) c.kernel = cg_resident_kernel<T, R, E, double, false, kGrid>;
+  if (cheb) c.kernel = cg_resident_kernel<T, R, E, double, true, kGrid, kLong>;
+  else if (narrow) c.kernel = cg_resident_kernel<T, R, E, float, false, kGrid, kLong>;
+  else if constexpr (!kGrid) c.kernel = cg_resident_kernel<T, R, E, double, false, kGrid, kLong>;
   return c;
+}
+
+template <int T, int R, int E, bool kGrid>
+ResidentChoice resident_choice(const CgProblem& p, bool cheb, bool narrow) {
+  // One block's vectors are all in its LDS, where a thread reads a long row quickly enough.
+  if constexpr (kGrid)
+    if (p.longest_row > E + kOwnExtra) return resident_instance<T, R, E, kGrid, true>(cheb, narrow);
+  return resident_instance<T, R, E, kGrid, false>(cheb, narrow);
 }
 
 ResidentChoice choose_resident(const CgProblem& p) {
   const bool cheb = p.chebyshev_steps > 0, narrow = p.values32 != nullptr;
   if (p.n_columns != 1 || (cheb && narrow)) return {};
-  if (p.n <= 1024) return resident_choice<1024, 1, 9, false>(cheb, narrow);
+  if (p.n <= 1024) return resident_choice<1024, 1, 9, false>(p, cheb, narrow);
   if (!p.order || !p.inverse) {
-    if (p.n <= 2048) return resident_choice<1024, 2, 9, false>(cheb, narrow);
-    if (p.n <= 3072) return resident_choice<1024, 3, 5, false>(cheb, narrow);
+    if (p.n <= 2048) return resident_choice<1024, 2, 9, false>(p, cheb, narrow);
+    if (p.n <= 3072) return resident_choice<1024, 3, 5, false>(p, cheb, narrow);
     return {};
   }
   const int64_t units = resident_units();
-  if (p.n <= 256 * units) return resident_choice<256, 1, 9, true>(cheb, narrow);
-  if (p.n <= 1024 * units) return resident_choice<512, 2, 9, true>(cheb, narrow);
-  if (p.n <= 2048 * units) return resident_choice<512, 4, 7, true>(cheb, narrow);
+  if (p.n <= 256 * units) return resident_choice<256, 1, 9, true>(p, cheb, narrow);
+  if (p.n <= 1024 * units) return resident_choice<512, 2, 9, true>(p, cheb, narrow);
+  if (p.n <= 2048 * units) return resident_choice<512, 4, 7, true>(p, cheb, narrow);
   return {};
 }
 

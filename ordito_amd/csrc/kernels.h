@@ -275,6 +275,7 @@ struct CgProblem {
   // pattern.
   const int32_t* order = nullptr;
   const int32_t* inverse = nullptr;
+  int32_t longest_row = 0;  // the most entries of a row, where the caller knows
   // Stop rule: settle (the heat step) or relative residual tol (the Poisson step).
   int32_t settle = 1;
   int32_t check_rounds = 16;
