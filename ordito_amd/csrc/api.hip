@@ -490,8 +490,8 @@ void ensure_corner_geometry(hg_mesh& m) {
   ensure_operators(m);
   ensure_plan(m);
   if (m.corner_geometry) return;
-  build_corner_geometry(m.normals.ptr, m.face_geom.ptr, m.vertex_ptr.ptr, m.vertex_corners.ptr,
-                        m.plan->perm.ptr, m.n, m.corners, m.stream);
+  build_corner_geometry(m.faces.ptr, m.normals.ptr, m.face_geom.ptr, m.vertex_ptr.ptr,
+                        m.vertex_corners.ptr, m.plan->iperm.ptr, m.f, m.corners, m.stream);
   m.corner_geometry = true;
   invalidate_graphs(m);
 }

@@ -209,9 +209,9 @@ struct CornerRecords {
 void build_corner_rows(const int32_t* faces, const int32_t* vertex_ptr,
                        const int32_t* vertex_corners, const int32_t* perm, const int32_t* iperm,
                        int64_t n, int64_t n_faces, CornerRecords& out, hipStream_t stream);
-void build_corner_geometry(const float* normals, const double* face_geom,
+void build_corner_geometry(const int32_t* faces, const float* normals, const double* face_geom,
                            const int32_t* vertex_ptr, const int32_t* vertex_corners,
-                           const int32_t* perm, int64_t n, CornerRecords& out,
+                           const int32_t* iperm, int64_t n_faces, CornerRecords& out,
                            hipStream_t stream);
 // -b per vertex and column from the heat (both in `layout`), gathered over each vertex's corners.
 // By rows, from the records: rows flagged in `pinned` (the elimination order; may be null) are left

@@ -1,11 +1,14 @@
 """
 Meshes with vertices of very many neighbours: the conjugate gradient deals a long row's entries over
-its wave (``csrc/cg.hip``, ``kLong``). Rows about the length where it starts to, of a wave's width and
-past it, several in a wave, at each of the instances' sizes.
+its wave (``csrc/cg.hip``, ``kLong``), the residual of three columns and more over its block
+(``csrc/solve.hip``), and the divergence's records are formed a thread a corner. Rows about the lengths
+where those start, of a wave's width and past it, several in a wave and a block, more than a block
+stages, at each of the instances' sizes.
 
 Bars, as for every iterate: a heat iterate that is accepted passes the solver's own test, a componentwise
 backward error of 1e-6 in float64; a Poisson iterate's true residual is within twice the stopping
-tolerance 1e-8 of its right-hand side; a repeated solve gives the same bits.
+tolerance 1e-8 of its right-hand side; a repeated solve gives the same bits. Refined factored solves meet their targets, computed here (twice them, for the rounding of
+sums of thousands of terms).
 """
 
 from __future__ import annotations
@@ -90,3 +93,62 @@ def test_iterates_meet_their_stopping_rules(cuda, name):
         fields.append(out.cpu().numpy())
     assert np.array_equal(fields[0], fields[1])
     assert np.linalg.norm(b - L @ fields[0]) <= 2e-8 * np.linalg.norm(b)
+
+
+FACTORED = {
+    "63": lambda: cone(63, 9),  # a row of 64 entries
+    "64": lambda: cone(64, 9),  # 65: dealt
+    "70": lambda: _cones(40, 70),  # several in a block
+    "1500": lambda: cone(1500, 3),  # more than a block stages
+}
+
+
+@pytest.mark.parametrize("columns", [3, 4, 5, 20, 63, 64])
+@pytest.mark.parametrize("name", sorted(FACTORED))
+def test_refined_solves_meet_their_targets(cuda, name, columns):
+    """From FP32 blocks, so that every round but the last multiplies a residual."""
+    from ordito_amd import heat
+
+    v, f = FACTORED[name]()
+    n = len(v)
+    mesh = heat.Trimesh(v, f)
+    solver = mesh.heat_solver(method="meshlab", precision="mixed")
+    assert solver.factor()
+    solver.set_refinement(heat=1e-11, poisson=1e-11)
+    A, L = solver.operators[0].to_scipy(), solver.operators[3].to_scipy()
+    rng = np.random.default_rng(columns)
+    b = np.zeros((columns, n))
+    b[np.arange(columns), rng.integers(0, n, columns)] = 1.0
+    b[0] = 0.0
+    b[0, np.diff(A.indptr) > 64] = 1.0  # the hubs themselves
+    rhs = cuda.from_numpy(b).cuda()
+    out = cuda.empty_like(rhs)
+    solver.diffuse(rhs, out)
+    assert solver.last_stats["heat_refinements"] > 1
+    for x, source in zip(out.cpu().numpy(), b):
+        assert np.all(np.abs(source - A @ x) <= 2e-11 * (abs(A) @ np.abs(x) + np.abs(source)))
+
+    b = (L @ rng.standard_normal((n, columns))).T.copy()
+    rhs = cuda.from_numpy(b).cuda()
+    solver.solve_poisson(rhs, out)
+    for x, source in zip(out.cpu().numpy(), b):
+        bar = np.maximum(abs(L) @ np.abs(x) + np.abs(source), np.abs(source).max())
+        assert np.all(np.abs(source - L @ x) <= 2e-11 * bar)
+
+
+@pytest.mark.parametrize("name", sorted(FACTORED))
+def test_distances_match_the_oracle(cuda, name):
+    from oracle import heat_oracle as oracle
+    from ordito_amd import heat
+
+    v, f = FACTORED[name]()
+    mesh = heat.Trimesh(v, f)
+    solver = mesh.heat_solver(method="meshlab")
+    assert solver.factor()
+    want = oracle.geodesic(v, f.reshape(-1), [1]).distance
+    reached = want != 0.0  # other components hold no distance from this source
+    reached[1] = True
+    for columns in (1, 3, 8):
+        sets = [cuda.tensor([1], dtype=cuda.int32, device="cuda")] * columns
+        for got in solver.geodesic(sets).cpu().numpy().reshape(columns, -1):
+            assert oracle.relative_error(got[reached], want[reached])[0] <= 1e-9
