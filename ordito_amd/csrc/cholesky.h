@@ -9,6 +9,7 @@ namespace hg {
 struct DevicePlan {
   int64_t n = 0;
   int64_t nnz = 0;
+  int32_t longest_row = 0;  // the most entries of a row of the operator
   int32_t n_super = 0;
   int32_t n_levels = 0;
   std::vector<int32_t> level_ptr;  // host copies: the launches are per level

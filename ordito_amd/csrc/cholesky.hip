@@ -792,9 +792,12 @@ void DevicePlan::upload(const Plan& plan, const HostPattern& pattern, int32_t ta
   {
     const int64_t nn = plan.n;
     std::vector<int32_t> offs(nn + 1, 0);
+    longest_row = 0;
     for (int64_t i = 0; i < nn; ++i) {
       const int32_t old = plan.perm[i];
-      offs[i + 1] = offs[i] + (pattern.offsets[old + 1] - pattern.offsets[old]);
+      const int32_t entries = pattern.offsets[old + 1] - pattern.offsets[old];
+      longest_row = std::max(longest_row, entries);
+      offs[i + 1] = offs[i] + entries;
     }
     std::vector<int32_t> cols(static_cast<size_t>(offs[nn])), src(static_cast<size_t>(offs[nn]));
     parallel_chunks(nn, 1 << 14, [&](int64_t b, int64_t e_end, int64_t) {

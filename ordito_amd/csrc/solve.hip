@@ -722,7 +722,12 @@ __global__ void residual_kernel(const int32_t* __restrict__ offsets,
 // order. 524,288-row torus: 32 columns 105 us (a lane a column 204), 64 columns 197 (214), where the
 // rows fetched twice from beyond L2 hold it (850 MB at 4.4 TB/s; 570 are needed). The heat step's
 // right-hand side is read where the bitmap of seeded rows has one (197 to 163).
+// kLong: the plan has rows of more than kLongRow entries, which are dealt over the block's groups of
+// lanes, a row at a time (a vertex of 8,000 neighbours, 20 columns: 1.6 ms with a wave a row, 2.5 with
+// one group reading them all, 0.05 so; an instance of its own, since it takes 82 registers to 58).
 constexpr int32_t kPairEntries = 1024;
+constexpr int32_t kLongRow = 64;
+template <bool kLong>
 __global__ __launch_bounds__(256) void residual_pairs_kernel(
     const int32_t* __restrict__ offsets, const int32_t* __restrict__ columns,
     const double* __restrict__ values, const double* __restrict__ b,
@@ -764,7 +769,12 @@ __global__ __launch_bounds__(256) void residual_pairs_kernel(
   asm volatile("" ::"v"(x0));  // loaded, though nothing takes its value
   const Pair bscale = componentwise ? Pair{0.0, 0.0} : *reinterpret_cast<const Pair*>(bmax + q);
   bool fail = false;
+  auto within = [&](Pair total, Pair scale) {
+    return fabs(total.x) <= tolerance * fmax(scale.x, bscale.x) &&
+           fabs(total.y) <= tolerance * fmax(scale.y, bscale.y);
+  };
   auto row = [&](int32_t s, const int32_t* names, const double* v) {
+    if (kLong && ptr[s + 1] - ptr[s] > kLongRow) return;
     const int64_t i = first + s, at = i * kk + q;
     Pair total = s == s0 ? b0 : right_hand_side(s);
     Pair scale = {fabs(total.x), fabs(total.y)};
@@ -788,14 +798,57 @@ __global__ __launch_bounds__(256) void residual_pairs_kernel(
       }
     }
     if (r) *reinterpret_cast<Pair*>(r + at) = dropped ? Pair{0.0, 0.0} : total;
-    fail |= !dropped && !(fabs(total.x) <= tolerance * fmax(scale.x, bscale.x) &&
-                          fabs(total.y) <= tolerance * fmax(scale.y, bscale.y));
+    fail |= !dropped && !within(total, scale);
   };
   if (takes) {
     if (fits)
       for (int32_t s = s0; s < here; s += per) row(s, named, staged);
     else
       for (int32_t s = s0; s < here; s += per) row(s, columns + base, values + base);
+  }
+  if (kLong && count > kLongRow) {
+    Pair* parts = reinterpret_cast<Pair*>(staged);  // [256] of the sums, [256] of the scales
+    __syncthreads();
+    for (int32_t s = 0; s < here; ++s) {
+      const int32_t e1 = ptr[s + 1];
+      if (e1 - ptr[s] <= kLongRow) continue;
+      Pair sum = {0.0, 0.0}, size = {0.0, 0.0};
+      if (s0 < per)
+        for (int32_t e = ptr[s] + B * s0; e < e1; e += B * per) {
+          int32_t c[B];
+          double a[B];
+#pragma unroll
+          for (int u = 0; u < B; ++u) {
+            c[u] = columns[min(e + u, e1 - 1)];
+            a[u] = e + u < e1 ? values[e + u] : 0.0;
+          }
+#pragma unroll
+          for (int u = 0; u < B; ++u) {
+            const Pair xv = *reinterpret_cast<const Pair*>(x + static_cast<int64_t>(c[u]) * kk + q);
+            const double t0 = e + u < e1 ? a[u] * xv.x : 0.0, t1 = e + u < e1 ? a[u] * xv.y : 0.0;
+            sum.x += t0;
+            sum.y += t1;
+            size.x += fabs(t0);
+            size.y += fabs(t1);
+          }
+        }
+      parts[tid] = sum;
+      parts[256 + tid] = size;
+      __syncthreads();
+      if (s0 == 0) {
+        const int64_t i = first + s;
+        Pair total = right_hand_side(s);
+        Pair scale = {fabs(total.x), fabs(total.y)};
+        for (int32_t g = 0; g < per; ++g) {
+          total -= parts[tid + g * lanes];
+          scale += parts[256 + tid + g * lanes];
+        }
+        const bool dropped = pinned && pinned[i];
+        if (r) *reinterpret_cast<Pair*>(r + i * kk + q) = dropped ? Pair{0.0, 0.0} : total;
+        fail |= !dropped && !within(total, scale);
+      }
+      __syncthreads();
+    }
   }
   raise_flag(fail, pending);
 }
@@ -1352,7 +1405,9 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
         // at four; the rows' entries read once a column below).
         if (kk >= 3) {
           const int32_t rows = pair_rows(kk);
-          residual_pairs_kernel<<<static_cast<unsigned>((n + rows - 1) / rows), 256, 0, stream>>>(
+          auto kernel = plan.longest_row > kLongRow ? residual_pairs_kernel<true>
+                                                    : residual_pairs_kernel<false>;
+          kernel<<<static_cast<unsigned>((n + rows - 1) / rows), 256, 0, stream>>>(
               plan.p_offsets.ptr, plan.p_columns.ptr, factor.pvalues.ptr, bp, x_cur, pinned_new,
               bmax, seeded, n, kk, rows, tolerance,
               componentwise ? 1 : 0, r_out, verdict);
