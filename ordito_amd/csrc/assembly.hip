@@ -436,11 +436,22 @@ __global__ void average_kernel(double* __restrict__ a, const double* __restrict_
 // row_of[v].
 // count_at (device, nullable): the entry count is min(*count_at, n_entries) (a replayed launch
 // reads each call's count); the grid strides over the entries.
+// Many sources on few rows would wait for each other at the few words of the bitmap, so a block gathers
+// its bits in LDS where the words are kNearWords at most.
+constexpr int32_t kNearWords = 256;
+
 __global__ void seed_kernel(const int32_t* __restrict__ sources, const int64_t* __restrict__ owner,
                             int64_t n_entries, const int64_t* __restrict__ count_at, int64_t n,
                             int64_t rows_k, const int32_t* __restrict__ row_of,
                             double* __restrict__ u0, int32_t* __restrict__ invalid,
                             uint32_t* __restrict__ seeded) {
+  __shared__ uint32_t near[kNearWords];
+  const int32_t words = static_cast<int32_t>(rows_k > 0 ? min((n + 31) / 32, int64_t{kNearWords + 1}) : 0);
+  const bool local = words <= kNearWords;
+  if (local) {
+    for (int32_t w = threadIdx.x; w < words; w += blockDim.x) near[w] = 0u;
+    __syncthreads();
+  }
   const int64_t count = count_at ? min(*count_at, n_entries) : n_entries;
   for (int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; e < count;
        e += static_cast<int64_t>(gridDim.x) * blockDim.x) {
@@ -455,22 +466,31 @@ __global__ void seed_kernel(const int32_t* __restrict__ sources, const int64_t* 
       const int64_t kk = min(kFieldChunk, rows_k - chunk * kFieldChunk);
       const int32_t row = row_of[v];
       u0[chunk * kFieldChunk * n + static_cast<int64_t>(row) * kk + q % kFieldChunk] = 1.0;
-      atomicOr(seeded + row / 32, 1u << (row % 32));
+      if (local) atomicOr(&near[row / 32], 1u << (row % 32));
+      else atomicOr(seeded + row / 32, 1u << (row % 32));
     } else {
       u0[q * n + v] = 1.0;
     }
   }
+  if (!local) return;
+  __syncthreads();
+  for (int32_t w = threadIdx.x; w < words; w += blockDim.x)
+    if (near[w]) atomicOr(seeded + w, near[w]);
 }
 
-// The same by rows for a few sources, clears included: a block clears its rows of every chunk, their
-// words of the bitmap and (block 0) the flags, then looks through all the sources for its own. One
-// launch for two (icosphere(4), one source: 148 us a call, 145 so).
+// The same by rows for a few sources, clears included: a block clears its rows (32 kNearWords at most)
+// of every chunk and (block 0) the flags, then looks through all the sources for its own, four a thread
+// at a time, and writes its words of the bitmap. One launch for two (icosphere(4), one source: 148 us a
+// call, 145 so).
 __global__ __launch_bounds__(256) void seed_rows_kernel(
     const int32_t* __restrict__ sources, const int64_t* __restrict__ owner, int64_t n_entries,
     const int64_t* __restrict__ count_at, int64_t n, int64_t k, int32_t rows,
     const int32_t* __restrict__ row_of, double* __restrict__ u0, int32_t* __restrict__ flags,
     int64_t n_flags, uint32_t* __restrict__ seeded) {
+  constexpr int B = 4;
+  __shared__ uint32_t near[kNearWords];
   const int64_t r0 = static_cast<int64_t>(blockIdx.x) * rows, r1 = min(r0 + rows, n);
+  const int32_t words = static_cast<int32_t>((r1 + 31) / 32 - r0 / 32);
   const int32_t tid = static_cast<int32_t>(threadIdx.x);
   for (int64_t c0 = 0; c0 < k; c0 += kFieldChunk) {
     const int64_t kk = min(kFieldChunk, k - c0), count = (r1 - r0) * kk;
@@ -479,23 +499,31 @@ __global__ __launch_bounds__(256) void seed_rows_kernel(
       *reinterpret_cast<Pair*>(part + e) = Pair{0.0, 0.0};
     if (tid == 0 && count % 2) part[count - 1] = 0.0;
   }
-  for (int64_t e = r0 / 32 + tid; e < (r1 + 31) / 32; e += 256) seeded[e] = 0u;
+  if (tid < words) near[tid] = 0u;
   if (blockIdx.x == 0)
     for (int64_t e = tid; e < n_flags; e += 256) flags[e] = 0;
   __syncthreads();
   const int64_t count = count_at ? min(*count_at, n_entries) : n_entries;
-  for (int64_t e = tid; e < count; e += 256) {
-    const int32_t v = sources[e];
-    if (v < 0 || v >= n) {
-      if (blockIdx.x == 0) atomicOr(flags, 1);
-      continue;
+  for (int64_t e0 = tid; e0 < count; e0 += 256 * B) {
+    int32_t v[B], row[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) v[u] = sources[min(e0 + 256 * u, count - 1)];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const bool bad = v[u] < 0 || v[u] >= n;
+      if (bad && blockIdx.x == 0) atomicOr(flags, 1);
+      row[u] = bad ? -1 : row_of[v[u]];
     }
-    const int32_t row = row_of[v];
-    if (row < r0 || row >= r1) continue;
-    const int64_t q = owner[e], c0 = q / kFieldChunk * kFieldChunk;
-    u0[c0 * n + row * min(kFieldChunk, k - c0) + q - c0] = 1.0;
-    atomicOr(seeded + row / 32, 1u << (row % 32));
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      if (row[u] < r0 || row[u] >= r1 || e0 + 256 * u >= count) continue;
+      const int64_t q = owner[e0 + 256 * u], c0 = q / kFieldChunk * kFieldChunk;
+      u0[c0 * n + row[u] * min(kFieldChunk, k - c0) + q - c0] = 1.0;
+      atomicOr(&near[(row[u] - r0) / 32], 1u << (row[u] % 32));
+    }
   }
+  __syncthreads();
+  if (tid < words) seeded[r0 / 32 + tid] = near[tid];
 }
 
 // Zeroes 32-bit words: the clears of a solve, as kernels so a captured graph holds no memset node.
@@ -1163,8 +1191,8 @@ void launch_seed(const int32_t* sources, const int64_t* owner, int64_t n_entries
                  const int64_t* count_at, int64_t n, int64_t k, const int32_t* row_of, double* u0,
                  int32_t* flags, int64_t n_flags, hipStream_t stream) {
   uint32_t* seeded = reinterpret_cast<uint32_t*>(flags + n_flags);
-  if (row_of && n > 0 && n_entries <= kFewSeeds) {
-    const int64_t rows = 32 * ((n + 32 * 2048 - 1) / (32 * 2048));
+  const int64_t rows = 32 * ((n + 32 * 2048 - 1) / (32 * 2048));
+  if (row_of && n > 0 && n_entries <= kFewSeeds && rows <= 32 * kNearWords) {
     seed_rows_kernel<<<static_cast<unsigned>((n + rows - 1) / rows), 256, 0, stream>>>(
         sources, owner, n_entries, count_at, n, k, static_cast<int32_t>(rows), row_of, u0, flags,
         n_flags, seeded);
