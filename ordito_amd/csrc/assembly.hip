@@ -1286,7 +1286,7 @@ void launch_divergence(const int32_t* faces, const double* geom, const int32_t* 
       const unsigned blocks = static_cast<unsigned>(divergence_blocks(n, kk));  // as many maxima
       double* most = maxima + c0 * divergence_blocks(n, kFieldChunk);
       if (kk >= kDivergencePairs) {
-        const int32_t rows = pair_rows(static_cast<int32_t>(kk));
+        const int32_t rows = pair_rows(static_cast<int32_t>(kk), n);
         divergence_pairs_kernel<<<static_cast<unsigned>((n + rows - 1) / rows), kBlock, 0, stream>>>(
             records->rows.ptr, records->ptr.ptr, records->geom.ptr, heat + c0 * n, n,
             static_cast<int32_t>(kk), rows, out + c0 * n);

@@ -1404,7 +1404,7 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
         // Pairs from three columns on (on the 524,288-row torus 46 us for two against 63, 47 against 67
         // at four; the rows' entries read once a column below).
         if (kk >= 3) {
-          const int32_t rows = pair_rows(kk);
+          const int32_t rows = pair_rows(kk, n);
           auto kernel = plan.longest_row > kLongRow ? residual_pairs_kernel<true>
                                                     : residual_pairs_kernel<false>;
           kernel<<<static_cast<unsigned>((n + rows - 1) / rows), 256, 0, stream>>>(
