@@ -1013,16 +1013,6 @@ int32_t cooperative_grid(int64_t n) {
 
 using CgKernel = void (*)(CgArgs);
 
-// The resident kernel for a one-column problem: its threads, rows a thread and function, by size.
-// Up to 1,024 rows one block, which exchanges nothing (and up to 3,072 where there is no spatial
-// order; with one, 2,562 rows took 1.04 ms for both solves of a one-shot call in one block, which
-// reads three rows' entries out of one compute unit's LDS, and 0.88 ms in eleven of 256 threads).
-// Up to 65,536 rows a row a thread in blocks of 256, as few blocks as hold them (icosphere(6),
-// 40,962 rows: 3.51 ms; blocks of 512, 3.56; of 1024, 4.73). Past that every compute unit gets a
-// block of 512 threads with two rows each (icosphere(7), 163,842 rows: 11.7 ms; as few blocks as
-// hold them 12.0, 1024 threads with one row 12.1, 256 with four 15.2), or four with seven entries
-// in registers (torus of 524,288 rows, the heat solve: 10.8 ms; nine entries spill, 13.4 ms; 1024
-// threads with two rows 13.6 and 18.8 ms).
 // Blocks of a resident solve at most: one a compute unit, and no more than a block has threads to
 // read the sums of.
 int64_t resident_units() {
@@ -1056,9 +1046,23 @@ ResidentChoice resident_choice(const CgProblem& p, bool cheb, bool narrow) {
   return resident_instance<T, R, E, kGrid, false>(cheb, narrow);
 }
 
+// The resident kernel for a one-column problem: its threads, rows a thread and function, by size.
+// Up to 1,024 rows one block, which exchanges nothing, of 256, 512 or 1024 threads: a round waits for all
+// its waves, idle ones too (the heat solve of 162 rows 136 us in 256 threads, 246 in 1024; of 258 rows 233
+// in 512, 363 in 1024). Up to 3,072 too where there is no spatial order; with one, 2,562 rows took
+// 1.04 ms for both solves of a one-shot call in one block, which reads three rows' entries out of one
+// compute unit's LDS, and 0.88 ms in eleven of 256 threads.
+// Up to 65,536 rows a row a thread in blocks of 256, as few blocks as hold them (icosphere(6),
+// 40,962 rows: 3.51 ms; blocks of 512, 3.56; of 1024, 4.73). Past that every compute unit gets a
+// block of 512 threads with two rows each (icosphere(7), 163,842 rows: 11.7 ms; as few blocks as
+// hold them 12.0, 1024 threads with one row 12.1, 256 with four 15.2), or four with seven entries
+// in registers (torus of 524,288 rows, the heat solve: 10.8 ms; nine entries spill, 13.4 ms; 1024
+// threads with two rows 13.6 and 18.8 ms).
 ResidentChoice choose_resident(const CgProblem& p) {
   const bool cheb = p.chebyshev_steps > 0, narrow = p.values32 != nullptr;
   if (p.n_columns != 1 || (cheb && narrow)) return {};
+  if (p.n <= 256) return resident_choice<256, 1, 9, false>(p, cheb, narrow);
+  if (p.n <= 512) return resident_choice<512, 1, 9, false>(p, cheb, narrow);
   if (p.n <= 1024) return resident_choice<1024, 1, 9, false>(p, cheb, narrow);
   if (!p.order || !p.inverse) {
     if (p.n <= 2048) return resident_choice<1024, 2, 9, false>(p, cheb, narrow);
