@@ -228,6 +228,12 @@ struct HostFlow {
 // and 2.14 ms against 3.58 on icosphere(9); of 8, 360 against 411, 927 against 900 and 4.22 ms
 // against 3.62.
 constexpr int32_t kFlowColumns = 4;
+// The most stored entries of FP32 blocks such a sweep takes. Its loads bring half the bytes then, and the
+// level sweeps' tiles catch up where the blocks outgrow the last-level cache: refined diffusions of one
+// column and of four took 671 and 777 us in one launch a sweep and 821 and 829 level by level with 27.5
+// million entries (a grid of 160,000), 953 and 1,067 against 907 and 932 with 38.3 (a torus of 160,000),
+// 2,377 and 2,606 against 1,721 and 1,789 with 108 (the 524,288-row torus).
+constexpr int64_t kFlowFp32Entries = int64_t{1} << 25;
 // A level of this many 64-wide tiles keeps them (icosphere(7): 160 us a sweep; from 128 on 164, from
 // 2,048 on 161, never 187).
 constexpr int64_t kFlowWideTiles = 512;

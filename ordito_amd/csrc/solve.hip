@@ -1348,7 +1348,8 @@ int32_t refined_solve(const DevicePlan& plan, const Factor& factor, bool use_fp3
     // A few columns sweep in one launch (flow.hip) while no such launch has given up here and the
     // device is claimed for it: by the call where the solve only enqueues, else by the solve, which
     // waits for every round.
-    const bool narrow = kk <= kFlowColumns && !ws.level_sweeps;
+    const bool narrow = kk <= kFlowColumns && !ws.level_sweeps &&
+                        (!use_fp32 || plan.w_size <= kFlowFp32Entries);
     const WaitClaim claim(narrow && !speculate, false);
     const bool claimed = narrow && (speculate ? ws.flows : claim.held());
     while (rounds < max_rounds) {

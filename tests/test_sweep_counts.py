@@ -101,3 +101,22 @@ def test_rounds_that_wait_for_their_verdicts(cuda, patience):
     solver.diffuse(rhs, cuda.empty_like(rhs))
     flows, levels, given_up = (a - b for a, b in zip(_counts(solver), before))
     assert given_up == 0 and (flows > 0) == (patience is None) and (levels > 0) == (patience == 0)
+
+
+@pytest.mark.parametrize("columns", [1, 4])
+def test_many_fp32_entries_sweep_level_by_level(cuda, columns):
+    """A torus of 160,000 rows stores 38.3 million entries, past the 2^25 of FP32 blocks that sweep in
+    one launch."""
+    from ordito_amd import creation
+
+    mesh = creation.torus(400, 400, 1.0, 0.3, 0.1, 4)
+    fields = {}
+    for precision in ("mixed", "fp64"):
+        trimesh, solver = _solver(cuda, mesh, "meshlab", precision, None)
+        assert solver.plan_stats()["solve_block_entries"] > 1 << 25
+        fields[precision] = solver.geodesic(_sets(cuda, trimesh.n_vertices, columns)).cpu().numpy()
+        flows, levels, given_up = _counts(solver)
+        assert given_up == 0
+        assert (flows == 0 and levels > 0) if precision == "mixed" else (flows == 2 and levels == 0)
+    for got, want in zip(fields["mixed"], fields["fp64"]):
+        assert np.max(np.abs(got - want)) <= 1e-6 * np.ptp(want)
