@@ -493,9 +493,9 @@ HostGather gather_lists(const Plan& plan) {
 void validate_sweeps(const Plan& plan, int32_t target_tasks) {
   auto fail = [](const std::string& what) { throw Error{HG_ERR_RUNTIME, "plan check: " + what}; };
   const int64_t S = plan.n_super;
-  for (int dir = 0; dir < 2; ++dir) {
-    const bool forward = dir == 0;
-    const HostSweep h = sweep_tasks(plan, forward, target_tasks);
+  for (int list = 0; list < 4; ++list) {
+    const bool forward = list % 2 == 0;
+    const HostSweep h = sweep_tasks(plan, forward, sweep_targets(target_tasks)[list / 2]);
     std::vector<int64_t> covered(S, 0);
     for (size_t t = 0; t < h.s.size(); ++t) {
       const int32_t s = h.s[t];
@@ -758,7 +758,7 @@ void upload_sweep(const Plan& plan, bool forward, const HostSweep& h,
 
 void DevicePlan::upload_sweeps(const Plan& plan, int32_t target_tasks, hipStream_t stream) {
   for (int list = 0; list < 2; ++list) {
-    const int32_t target = list == 0 ? target_tasks : std::max(1, target_tasks / 4);
+    const int32_t target = sweep_targets(target_tasks)[list];
     const HostSweep hf = sweep_tasks(plan, true, target);
     const HostSweep hb = sweep_tasks(plan, false, target);
     max_slots[list] = std::max(hf.max_slots, hb.max_slots);

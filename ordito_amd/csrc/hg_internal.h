@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cstdint>
 #include <future>
 #include <memory>
@@ -203,6 +204,10 @@ struct HostSweep {
 // dimension until it has about that many tasks (a few per compute unit by default).
 constexpr int32_t kDefaultSplitTarget = 1024;
 HostSweep sweep_tasks(const Plan& plan, bool forward, int32_t target_tasks = kDefaultSplitTarget);
+// The targets of a plan's two task lists (DevicePlan): for up to 16 columns, and for more.
+inline std::array<int32_t, 2> sweep_targets(int32_t target_tasks) {
+  return {target_tasks, std::max(1, target_tasks / 4)};
+}
 
 // The forward sweep's gather lists: for each front-vector row (vec_off[s] + position) the rows of
 // the children's update vectors that add into it, and the first two of them inline per position
