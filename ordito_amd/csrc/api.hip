@@ -120,11 +120,9 @@ struct hg_mesh {
   int32_t check_rounds = kHeatCheckRounds;
   double change_tolerance = kHeatChangeTolerance;
   int32_t settle_window = 0;
-  // Speculative refinement (FP64 factors): the verdicts of the first rounds of the heat, pinned and
-  // Poisson solves of a call, [system][chunk], read at the call's last synchronization.
   // A call's flags, on the device and read back by its last copy: [0] a source out of range, then the
-  // speculated verdicts of the heat, rim-pinned and Poisson solves, spec_chunks each. Behind them the
-  // bitmap of the rows with a source (launch_seed).
+  // speculated verdicts (arm_speculation) of the heat, rim-pinned and Poisson solves, spec_chunks each.
+  // Behind them the bitmap of the rows with a source (launch_seed).
   DeviceArray<int32_t> d_flags;
   PinnedArray<int32_t> h_flags;
   bool speculating = false;
@@ -148,8 +146,8 @@ struct hg_mesh {
   NullSpace null_space;
   DeviceArray<int32_t> d_sources, invalid;
   DeviceArray<int64_t> d_owner, d_offsets;
-  // A call's offsets, output slots (a pointer a 64-column chunk) and source owners, staged for one
-  // asynchronous upload.
+  // A call's offsets, output slots (a pointer a 64-column chunk, read by the finishing kernel, so that a
+  // replayed graph writes to each call's buffer) and source owners, staged for one asynchronous upload.
   PinnedArray<int64_t> h_stage;
   DeviceArray<int64_t> d_stage;
   const int64_t* query_offsets = nullptr;  // into d_stage, or d_offsets of packed meshes
@@ -158,8 +156,6 @@ struct hg_mesh {
   int64_t owner_capacity = 0;
   bool sources_on_device = false;  // query_offsets[k] holds this call's source count
   int64_t host_sources = 0;        // the source count where it does not
-  // The distance's destination per 64-column chunk, read by the finishing kernel (so a replayed
-  // graph writes to each call's buffer), staged in pinned memory.
   // Replay of the factored FP64 path: one instantiated graph per column count, and a second for the
   // narrow calls that find the device claimed (FlowScope) and sweep level by level; valid while every
   // buffer it names is the one it was captured with (signature) and no state change intervened.

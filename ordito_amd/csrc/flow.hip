@@ -14,9 +14,10 @@
 // all the same, and a launch that gave up reports it (kFlowAborted in the pending word), upon
 // which the solve starts over level by level.
 //
-// Both sweeps of a query, level by level and now: icosphere(4) 4 x 45 -> 4 x 19 us (its 12 levels
-// are 24 hand-overs of 1.5 us), icosphere(7) 730 -> 320 us, the 524,288-row torus 1.77 ms -> 830 us
-// (its inverse factors, 1.23 GB read of 1.54 stored, at 1.5 TB/s level by level, 3 now).
+// Both sweeps of a one-source query, level by level before this and now: icosphere(4) 180 -> 39 us (its
+// three levels are six hand-overs of about 2.5 us a sweep), icosphere(7) 730 -> 248 us (the heat step's,
+// over the fronts its source reaches, 105), the 524,288-row torus 1.77 ms -> 632 us (216 and 416: the
+// second reads 1.49 GB, at 3.6 TB/s where 1.5).
 //
 // A forward task is 256 / LN rows of a front, LN threads a row splitting the inner range; a
 // backward task is 16 * PASS columns, sixteen lanes a column along its rows. Every output is one

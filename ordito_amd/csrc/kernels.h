@@ -189,8 +189,7 @@ inline int64_t seed_words(int64_t n) { return (n + 31) / 32; }
 void launch_seed(const int32_t* sources, const int64_t* owner, int64_t n_entries,
                  const int64_t* count_at, int64_t n, int64_t k, const int32_t* row_of, double* u0,
                  int32_t* flags, int64_t n_flags, hipStream_t stream);
-// Zeroes `bytes` (whole 32-bit words) with a kernel (graph-capturable, unlike a memset node).
-// Zeroes p's bytes, and q's (multiples of 4).
+// Zeroes p's bytes, and q's (whole 32-bit words), with a kernel (graph-capturable, unlike a memset node).
 void launch_zero(void* p, int64_t bytes, hipStream_t stream, void* q = nullptr, int64_t q_bytes = 0);
 // Per face, kFaceGeom doubles: two of the gradient basis vectors a_k = N x e_k (the third is minus
 // their sum) and the three corners' integration vectors.
