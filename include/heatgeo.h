@@ -168,9 +168,8 @@ int hg_factored(hg_mesh* mesh, int32_t* out_systems);
 /*
  * Graph replay of hg_geodesic (no counterpart in the reference, whose kernels are launched one by
  * one): with every system factored in FP64 and timing off, the whole path (seeds, refined sweeps,
- * divergence, Poisson, finish) is captured once per column count (a second time where other calls keep
- * a narrow one from its one-launch sweeps) as a HIP graph on a stream of the library's own and
- * replayed, the call's sources, offsets and output reaching it through staged
+ * divergence, Poisson, finish) is captured once per column count as a HIP graph on a stream of the
+ * library's own and replayed, the call's sources, offsets and output reaching it through staged
  * buffers. On by default; enable = 0 solves eagerly. A capture that fails leaves the mesh eager.
  * hg_graph_state reports the graphs held and whether a capture failed.
  */

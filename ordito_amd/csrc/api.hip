@@ -7,7 +7,6 @@
 #include <limits>
 #include <map>
 #include <mutex>
-#include <utility>
 
 #include "cholesky.h"
 #include "multigrid.h"
@@ -156,8 +155,7 @@ struct hg_mesh {
   int64_t owner_capacity = 0;
   bool sources_on_device = false;  // query_offsets[k] holds this call's source count
   int64_t host_sources = 0;        // the source count where it does not
-  // Replay of the factored FP64 path: one instantiated graph per column count, and a second for the
-  // narrow calls that find the device claimed (FlowScope) and sweep level by level; valid while every
+  // Replay of the factored FP64 path: one instantiated graph per column count, valid while every
   // buffer it names is the one it was captured with (signature) and no state change intervened.
   struct Graph {
     hipGraphExec_t exec = nullptr;
@@ -170,7 +168,7 @@ struct hg_mesh {
       if (exec) (void)hipGraphExecDestroy(exec);
     }
   };
-  std::map<std::pair<int64_t, bool>, std::unique_ptr<Graph>> graphs;  // by columns and claim
+  std::map<int64_t, std::unique_ptr<Graph>> graphs;
   bool use_graphs = true;
   bool graphs_broken = false;  // a capture failed: this mesh runs eagerly from then on
   int64_t field_capacity = 0;
@@ -1146,15 +1144,18 @@ thread_local SideStream t_side_stream;
 // device for themselves (refined_solve).
 struct FlowScope {
   hg_mesh& m;
+  const bool wanted;
   WaitClaim claim;
   FlowScope(hg_mesh& mesh, bool speculates, int64_t k)
       : m(mesh),
-        claim(speculates && k > 0 && (k + kFieldChunk - 1) % kFieldChunk < kFlowColumns &&
-                  !mesh.solve.level_sweeps,
-              false) {
+        wanted(speculates && k > 0 && (k + kFieldChunk - 1) % kFieldChunk < kFlowColumns &&
+               !mesh.solve.level_sweeps),
+        claim(wanted, false) {
     m.solve.flows = claim.held();
   }
   ~FlowScope() { m.solve.flows = false; }
+  // A captured call sweeps as the claim allows.
+  bool as_captured() const { return !wanted || claim.held(); }
 };
 
 bool run_graph(hg_mesh& m, const int64_t* offsets, int64_t k, double* d_out, int32_t precision) {
@@ -1166,7 +1167,7 @@ bool run_graph(hg_mesh& m, const int64_t* offsets, int64_t k, double* d_out, int
   // The uploads on the caller's stream come first.
   HG_HIP(hipEventRecord(gs.ready, m.stream));
   HG_HIP(hipStreamWaitEvent(gs.stream, gs.ready, 0));
-  std::unique_ptr<hg_mesh::Graph>& g = m.graphs[{k, m.solve.flows}];
+  std::unique_ptr<hg_mesh::Graph>& g = m.graphs[k];
   if (!g || g->signature != graph_signature(m, k)) {
     g.reset();
     auto graph = std::make_unique<hg_mesh::Graph>();
@@ -1923,7 +1924,7 @@ int hg_geodesic(hg_mesh* mesh, const int32_t* d_sources, const int64_t* source_o
     const bool factored = ready_factors(m, mode, precision);
     FlowScope flow(m, factored && precision == HG_PRECISION_FP64, k);
     bool done = false;
-    if (replays) done = run_graph(m, source_offsets, k, d_out, precision);
+    if (replays && flow.as_captured()) done = run_graph(m, source_offsets, k, d_out, precision);
     if (!done) {
       for (bool speculate : {precision == HG_PRECISION_FP64, false}) {
         m.stats = hg_solve_stats{};

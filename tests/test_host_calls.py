@@ -183,33 +183,6 @@ def preparation_leaves_the_device_unclaimed(lib: Library) -> None:
     assert swept() == 1
 
 
-def a_narrow_query_replays_whoever_holds_the_device(lib: Library) -> None:
-    """A narrow query replays a graph with the device claimed by another call as without: one captured
-    with its sweeps level by level, kept beside the one with them in one launch each."""
-    small, large = lib.mesh(300), lib.mesh(2000)
-    kernels = ("flow_kernel", "fwd_tile_kernel", "graph")
-
-    def query():
-        before = [lib.fake.fake_thread_launches(k.encode()) for k in kernels]
-        lib.geodesic(small, 300, 1)
-        return [lib.fake.fake_thread_launches(k.encode()) - b for k, b in zip(kernels, before)]
-
-    for _ in range(2):
-        query()
-    assert query() == [0, 0, 1]
-    for first in (True, False):
-        with _held(lib, "cg_resident_kernel", lambda: lib.solve_poisson(large, 2000, 1)):
-            if first:
-                flows, tiles, graphs = _beside(query)["value"]
-                assert flows == 0 and tiles > 0 and graphs == 1
-            for _ in range(2):
-                assert _beside(query)["value"] == [0, 0, 1]
-        assert query() == [0, 0, 1]
-    held = ctypes.c_int64()
-    lib.call("hg_graph_state", small, ctypes.byref(held), None)
-    assert held.value == 2
-
-
 def workspaces_after_a_failed_allocation(lib: Library) -> None:
     """A call that could not allocate says so, holds no more than the mesh counts, and leaves
     workspaces that a narrower call can trust: none of theirs is missing."""
@@ -328,10 +301,6 @@ def test_iterations_of_one_block_run_beside_others(tmp_path):
 
 def test_preparation_leaves_the_device_unclaimed(tmp_path):
     _alone("preparation_leaves_the_device_unclaimed", tmp_path)
-
-
-def test_a_narrow_query_replays_whoever_holds_the_device(tmp_path):
-    _alone("a_narrow_query_replays_whoever_holds_the_device", tmp_path)
 
 
 if __name__ == "__main__":
