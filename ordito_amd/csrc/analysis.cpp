@@ -179,7 +179,12 @@ struct Dissector {
 // cost more. One query's call, unmerged and so: icosphere(4) 172 and 142 us, icosphere(7) 434 and 403, a
 // torus of 524,288 860 and 842, icosphere(8) (655,362 rows) 980 and 962. 64 columns there: 300 and 241,
 // 1,217 and 1,167, 2,880 and 2,802, 3,364 and 3,285. 16 columns on icosphere(9) would take 5,306 us
-// merged to 128 columns and 5,488 to 256, against 5,147.
+// merged to 128 columns and 5,488 to 256, against 5,147. Where the ranges meet, 128 and 256 columns: the
+// torus of 524,288 rows at one, 16 and 64 columns 837 and 835, 1,440 and 1,373, 2,797 and 2,720;
+// icosphere(8) 863 and 927, 1,598 and 1,569, 3,233 and 3,182.
+// A merged front eliminates its children's columns one after the other: factor() takes 3.1 ms unmerged and
+// 3.5 so at 12,000 rows, 3.6 and 4.0 at 27,600, 16.8 and 17.3 at 524,288. (128 columns there would cost it
+// nothing, and a query of 16 columns on icosphere(5) 318 us instead of 265.)
 int32_t default_merge_rows(int64_t n) {
   return n <= (int64_t{1} << 19) ? 256 : n <= (int64_t{1} << 20) ? 128 : 0;
 }
